@@ -80,19 +80,17 @@ struct Lay {
 
 // LDS layout kinds: how many tiles / broadcast vectors a worker of each
 // kernel needs and whether the block stages the model constants F, LQ, N1z.
-// The *T kinds are the throughput forms of the three scan combines: the same
-// LDS needs, but one lane per matrix row and the narrowest worker that holds
-// the 2D rows (several combines per wavefront), for scan levels wide enough
-// to fill the chip, where the per-pivot work that every lane of a worker
-// repeats, not the latency of one combine, sets the time.
-enum LdsKind : int { kLdsFull = 0, kLdsState, kLdsSmooth, kLdsLeaf, kLdsPost, kLdsSeq, kLdsLeaf1, kLdsFullT,
-                     kLdsStateT, kLdsSmoothT };
+// kLdsFull and kLdsState are the filter combines of D > 16 (pof_row16.hpp has
+// those of D <= 16).  kLdsSmoothT is the throughput form of the smoother
+// combine: the same LDS needs, but one lane per matrix row and the narrowest
+// worker that holds the 2D rows (several combines per wavefront), for scan
+// levels wide enough to fill the chip, where the per-pivot work that every
+// lane of a worker repeats, not the latency of one combine, sets the time.
+enum LdsKind : int { kLdsFull = 0, kLdsState, kLdsSmooth, kLdsLeaf, kLdsPost, kLdsSeq, kLdsLeaf1, kLdsSmoothT };
 
 // the latency-oriented kind of a throughput kind (same LDS needs)
-constexpr int base_kind(int K) {
-  return (K == kLdsFullT) ? kLdsFull : (K == kLdsStateT) ? kLdsState : (K == kLdsSmoothT) ? kLdsSmooth : K;
-}
-constexpr bool is_throughput_kind(int K) { return K == kLdsFullT || K == kLdsStateT || K == kLdsSmoothT; }
+constexpr int base_kind(int K) { return (K == kLdsSmoothT) ? kLdsSmooth : K; }
+constexpr bool is_throughput_kind(int K) { return K == kLdsSmoothT; }
 
 // Widest observation dimension of the per-worker engines.
 constexpr int kMaxObs = 4;
@@ -132,13 +130,11 @@ constexpr int kind_width() {
   return is_throughput_kind(K) ? pow2_at_least(2 * D, 8) : 0;
 }
 
-// State dimensions whose scan combines form their D x D tile products on the FP64 matrix cores
+// State dimensions whose smoother combines form their D x D tile products on the FP64 matrix cores
 // (v_mfma_f64_16x16x4f64, one 16 x 16 tile): whole-wavefront workers (rows over two lanes,
 // D > 8) that stage operands in one more LDS tile.  D = 9 .. 11 keep their throughput forms,
 // which the autotuner picks on wide levels and whose results must stay bitwise equal to the
-// latency form's (the matrix core sums in an order of its own).  At D = 15 the extra tile costs
-// one of twelve resident up-sweep workers per CU (LDS), and the products save 14% of the
-// up-sweep's instructions: the batch's D = 15 group gained (6.26 -> 6.16 s for the batch).
+// latency form's (the matrix core sums in an order of its own).
 template <int D>
 constexpr bool mfma_products() {
   return D == 12 || D == 15 || D == 16;
@@ -156,10 +152,7 @@ struct Geo : Lay<D_, kind_split<D_, K>(), kind_width<D_, K>()> {
   static constexpr int TILE = D_ * L::LD;
   // tiles per worker; the combines with matrix-core products stage operands and results in one more
   static constexpr int NT =
-      LdsNeeds<K>::NT + ((mfma_products<D_>() && (base_kind(K) == kLdsFull || base_kind(K) == kLdsState ||
-                                                   base_kind(K) == kLdsSmooth))
-                             ? 1
-                             : 0);
+      LdsNeeds<K>::NT + ((mfma_products<D_>() && base_kind(K) == kLdsSmooth) ? 1 : 0);
   static constexpr int NV = LdsNeeds<K>::NV;        // broadcast vectors per worker (2D entries each)
   // pivot-row broadcast of two matrices of 2 DP columns; the throughput kinds broadcast rows in the
   // padded layout of the latency kinds' split (whose reduction order they reproduce)
@@ -1357,7 +1350,7 @@ __device__ void filter_element(const Ctx<D, SS>& cx, const ModelArgs& a, int k,
 }
 
 // ---------------------------------------------------------- filter operators
-// Full combine (pof/parallel_filtsmooth/filter.py:117-142): e = e1 o e2, e1
+// Full combine (pof/parallel_filtsmooth/filter.py:117-142) for D > 16: e = e1 o e2, e1
 // earlier.  Reads e1 at index i1 of `x1`, e2 at index i2 of `x2`, writes index
 // o of `y`.  If `state_only`, e1 is a prefix state (b1, U1) read from
 // (s1.m, s1.L) and only (b, U) of the result are produced, into (so.m, so.L).
@@ -1434,20 +1427,10 @@ __device__ void filter_combine(const Ctx<D, SS>& cx, const FiltArrays& x1, const
     }
   }
   // Xi_ = [[U1^T Z2, I], [Z2, 0]]: rows 0..2D-1, column blocks (D, D)
-  // the combines of mfma_products<D>() (latency form) form their tile products on the matrix
-  // cores, staging row operands and results in one more LDS tile
-  constexpr bool MP = mfma_products<D>() && S == split_of<D>();
-  double* TS = MP ? cx.tile(state_only ? 4 : 5) : nullptr;
   double xr[2 * NL];
   {
     double t1[NL];
-    if constexpr (MP) {
-      tile_mfma<D, LD, true, false>(TU1, TZ2, TX11);  // U1^T Z2 (TX11 is free until Xi11 is stored)
-      wsync();
-      load_dist<S, D>(t1, TX11 + rr * LD, s);
-    } else {
-      tile_t_times_tile<S, D, D, LD>(rr, TU1, TZ2, s, t1);
-    }
+    tile_t_times_tile<S, D, D, LD>(rr, TU1, TZ2, s, t1);
     double zr[NL];
     const int r2 = (r >= D && r < 2 * D) ? r - D : 0;
     load_dist<S, D>(zr, TZ2 + r2 * LD, s);
@@ -1492,32 +1475,13 @@ __device__ void filter_combine(const Ctx<D, SS>& cx, const FiltArrays& x1, const
 
   // MT = A2 U1 Xi11^-T ; W = A2 - MT Xi21^T
   double mt[NL], wr[NL];
-  if constexpr (MP) {
-    stage_row<S, D, LD>(TS, r, s, a2);
-    wsync();
-    tile_mfma<D, LD, false, false>(TS, TU1, TS);  // A2 U1
-    wsync();
-    load_dist<S, D>(mt, TS + rr * LD, s);
-  } else {
+  {
     double a2f[D];
     gather<S, D>(a2, a2f);
     row_times_tile<S, D, D, LD>(a2f, TU1, s, mt);
   }
   rsolve_lowerT_s<S, D, LD>(mt, TX11, s);
-  if constexpr (MP) {
-    wsync();  // every row has read A2 U1
-    stage_row<S, D, LD>(TS, r, s, mt);
-    wsync();
-    tile_mfma<D, LD, false, true>(TS, TX21, TS);  // MT Xi21^T
-    wsync();
-    double p[NL];
-    load_dist<S, D>(p, TS + rr * LD, s);
-#pragma unroll
-    for (int t = 0; t < NL; ++t) {
-      wr[t] = (t * S + s < D) ? a2[t] - p[t] : 0.0;
-      pin1(wr[t]);
-    }
-  } else {
+  {
     double mtf[D];
     gather<S, D>(mt, mtf);
 #pragma unroll
@@ -1566,13 +1530,7 @@ __device__ void filter_combine(const Ctx<D, SS>& cx, const FiltArrays& x1, const
     wsync();
     eo = eta1r + lds_dot<S, D, LD, VS>(TA1 + rr, Vs3, s);
     pin1(eo);
-    if constexpr (MP) {
-      wsync();  // every row has read MT Xi21^T
-      stage_row<S, D, LD>(TS, r, s, wr);
-      wsync();
-      tile_mfma<D, LD, false, false>(TS, TA1, TU1);  // A = W A1 into U1's tile: U1's last reads were above
-      wsync();
-    } else {
+    {
       double wf[D];
       gather<S, D>(wr, wf);
       double ar[NL];
@@ -1589,11 +1547,7 @@ __device__ void filter_combine(const Ctx<D, SS>& cx, const FiltArrays& x1, const
   double jr[2 * NL];
   {
     double tz[NL];
-    if constexpr (!state_only && MP) {
-      tile_mfma<D, LD, true, false>(TA1, TX22, TS);  // A1^T Xi22
-      wsync();
-      load_dist<S, D>(tz, TS + rz * LD, s);
-    } else if constexpr (!state_only) {
+    if constexpr (!state_only) {
       tile_t_times_tile<S, D, D, LD>(rz, TA1, TX22, s, tz);
     } else {
       zero(tz);

@@ -21,6 +21,7 @@
 #include "pof_core.hpp"
 #include "pof_engine.hpp"
 #include "pof_linearization.hpp"
+#include "pof_row16.hpp"
 
 namespace pof {
 
@@ -138,34 +139,11 @@ k_filter_leaf(GroupArgs g, LaunchMap lm) {
   }
 }
 
-// Waves per SIMD the up- and down-sweep combines are compiled for: 5 at D = 10,
-// the natural allocation elsewhere.  A 4-wave budget (128 VGPRs) for the D = 12
-// up-sweep or the D = 15 down-sweep spills (24 and 44 bytes per lane) and is no
-// faster than their natural 3 waves.
+// Up-sweep: out[i] = in[2i] o in[2i+1], D > 16
 template <int D>
-constexpr int up_min_waves() {
-  return (D == 10) ? 5 : 1;
-}
-template <int D>
-constexpr int down_min_waves() {
-  return (D == 10) ? 5 : 1;
-}
-
-// Waves per SIMD of a scan kernel of kind K: the tuned bound of the
-// latency-oriented kinds; at least 2 for the throughput kinds, whose natural
-// allocation can exceed half the register file (D = 15: 256 VGPRs + 4 AGPRs,
-// one wave per SIMD).
-template <int D, int K>
-constexpr int scan_min_waves() {
-  return (K == kLdsFull) ? up_min_waves<D>() : (K == kLdsState) ? down_min_waves<D>() : is_throughput_kind(K) ? 2 : 1;
-}
-
-// Up-sweep: out[i] = in[2i] o in[2i+1]  (K: kLdsFull, or kLdsFullT on wide levels)
-template <int D, int K>
-__global__ __launch_bounds__((Geo<D, K>::BLOCK), (scan_min_waves<D, K>())) void k_filter_up(GroupArgs g, LaunchMap lm,
-                                                                                            int l) {
+__global__ __launch_bounds__((Geo<D, kLdsFull>::BLOCK)) void k_filter_up(GroupArgs g, LaunchMap lm, int l) {
   extern __shared__ double smem[];
-  auto cx = make_ctx<D, K>(g.F, g.LQ, g.N1z, smem);
+  auto cx = make_ctx<D, kLdsFull>(g.F, g.LQ, g.N1z, smem);
   int j, i;
   if (!locate(lm, cx.wid, j, i)) return;
   const long long N = g.Ns[j], base = g.base[j];
@@ -178,11 +156,10 @@ __global__ __launch_bounds__((Geo<D, K>::BLOCK), (scan_min_waves<D, K>())) void 
 // Down-sweep of level l: positions 2i and 2i+1 of the level-l prefix states.
 //   p[0] = state(e[0]); p[2i+1] = up[i]; p[2i] = up[i-1] o e[2i]  (i >= 1)
 // With top != 0 (a level of one element) only p[0] = state(e[0]) is written.
-template <int D, int K>
-__global__ __launch_bounds__((Geo<D, K>::BLOCK), (scan_min_waves<D, K>())) void k_filter_down(GroupArgs g,
-                                                                                            LaunchMap lm, int l) {
+template <int D>
+__global__ __launch_bounds__((Geo<D, kLdsState>::BLOCK)) void k_filter_down(GroupArgs g, LaunchMap lm, int l) {
   extern __shared__ double smem[];
-  auto cx = make_ctx<D, K>(g.F, g.LQ, g.N1z, smem);
+  auto cx = make_ctx<D, kLdsState>(g.F, g.LQ, g.N1z, smem);
   int j, i;
   if (!locate(lm, cx.wid, j, i)) return;
   const long long N = g.Ns[j], base = g.base[j];
@@ -210,6 +187,50 @@ __global__ __launch_bounds__((Geo<D, K>::BLOCK), (scan_min_waves<D, K>())) void 
     load_dist<S, D>(u, up.L + ((size_t)i * D + r) * D, sb);
     store_dist<S, D>(p.L + ((size_t)j1 * D + r) * D, u, sb);
     if (sb == 0) p.m[(size_t)j1 * D + r] = up.m[(size_t)i * D + r];
+  }
+}
+
+// The same two sweeps with one row per lane (pof_row16.hpp), D <= 16.  DZ: nonzero columns of the
+// level's elements' Z (d at level 0, D above).
+template <int D, int DZ>
+__global__ __launch_bounds__(r16::kBlock, 2) void k_filter_up16(GroupArgs g, LaunchMap lm, int l) {
+  int j, i;
+  if (!locate(lm, blockIdx.x * r16::kPerBlock + threadIdx.x / r16::kRow, j, i)) return;
+  const long long N = g.Ns[j], base = g.base[j];
+  const FiltArrays in = at(g.fel, base + lev_off(N, l), D);
+  const FiltArrays out = at(g.fel, base + lev_off(N, l + 1), D);
+  StateArrays none{};
+  r16::filter_combine<D, DZ, false>(threadIdx.x % r16::kRow, in, none, 2 * (size_t)i, in, 2 * (size_t)i + 1, out, none,
+                                    (size_t)i);
+}
+
+template <int D, int DZ>
+__global__ __launch_bounds__(r16::kBlock, 2) void k_filter_down16(GroupArgs g, LaunchMap lm, int l) {
+  int j, i;
+  if (!locate(lm, blockIdx.x * r16::kPerBlock + threadIdx.x / r16::kRow, j, i)) return;
+  const long long N = g.Ns[j], base = g.base[j];
+  const int n = (int)(N >> l);
+  const FiltArrays el = at(g.fel, base + lev_off(N, l), D);
+  const StateArrays p = at(g.fpre, base + lev_off(N, l), D);
+  const StateArrays up = (l + 1 < n_levels(N)) ? at(g.fpre, base + lev_off(N, l + 1), D) : StateArrays{};
+  const int r = threadIdx.x % r16::kRow;
+  const int j0 = 2 * i, j1 = j0 + 1;
+  if (j1 < n && r < D) {
+    double u[D];
+    r16::load_row16<D>(u, up.L + ((size_t)i * D + r) * D);
+    r16::store_row16<D>(p.L + ((size_t)j1 * D + r) * D, u);
+    p.m[(size_t)j1 * D + r] = up.m[(size_t)i * D + r];
+  }
+  if (j0 == 0) {
+    if (r < D) {
+      double u[D];
+      r16::load_row16<D>(u, el.U + r * D);
+      r16::store_row16<D>(p.L + r * D, u);
+      p.m[r] = el.b[r];
+    }
+  } else {
+    FiltArrays none{};
+    r16::filter_combine<D, DZ, true>(r, none, up, (size_t)i - 1, el, (size_t)j0, none, p, (size_t)j0);
   }
 }
 
@@ -912,6 +933,9 @@ inline unsigned grid_workers(size_t nworkers) {
   hipLaunchKernelGGL(kernel, dim3((grid_workers<D, K>(nworkers))), dim3((Geo<D, K>::BLOCK)),        \
                      (Geo<D, K>::lds_bytes()), __VA_ARGS__)
 
+#define POF_LAUNCH16(kernel, nworkers, ...)                                                              \
+  hipLaunchKernelGGL(kernel, dim3(((nworkers) + r16::kPerBlock - 1) / r16::kPerBlock), dim3(r16::kBlock), 0, __VA_ARGS__)
+
 namespace {
 // With a timer, event i+1 is recorded after launch i (event 0 before the first).
 struct Rec {
@@ -996,14 +1020,27 @@ hipError_t run_iteration(const GroupArgs& g, const LaunchPlan& p, double* scal, 
   for (int l = 0; l + 1 < p.fl; ++l) {
     const int nw = p.fup_total[l];
     if (nw == 0) continue;
-    POF_LAUNCH_LEVEL(k_filter_up, kLdsFull, kLdsFullT, p.tune.filter_up, nw, st, g, p.map(p.fup_off[l], nw), l);
+    if constexpr (D <= r16::kRow) {
+      if (l == 0)
+        POF_LAUNCH16((k_filter_up16<D, d>), nw, st, g, p.map(p.fup_off[l], nw), l);
+      else
+        POF_LAUNCH16((k_filter_up16<D, D>), nw, st, g, p.map(p.fup_off[l], nw), l);
+    } else {
+      POF_LAUNCH((k_filter_up<D>), kLdsFull, nw, st, g, p.map(p.fup_off[l], nw), l);
+    }
     rec(kKFilterUp, nw);
   }
   for (int l = p.fl - 1; l >= 0; --l) {
     const int nw = p.fdn_total[l];
     if (nw == 0) continue;
-    POF_LAUNCH_LEVEL(k_filter_down, kLdsState, kLdsStateT, p.tune.filter_down, nw, st, g, p.map(p.fdn_off[l], nw),
-                     l);
+    if constexpr (D <= r16::kRow) {
+      if (l == 0)
+        POF_LAUNCH16((k_filter_down16<D, d>), nw, st, g, p.map(p.fdn_off[l], nw), l);
+      else
+        POF_LAUNCH16((k_filter_down16<D, D>), nw, st, g, p.map(p.fdn_off[l], nw), l);
+    } else {
+      POF_LAUNCH((k_filter_down<D>), kLdsState, nw, st, g, p.map(p.fdn_off[l], nw), l);
+    }
     rec(kKFilterDown, nw - p.fdn_ivps[l]);
   }
   // ---- smoother elements + observation statistics

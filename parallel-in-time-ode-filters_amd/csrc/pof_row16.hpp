@@ -1,0 +1,491 @@
+// Scan combines with one matrix row per lane and sixteen lanes per worker (CDNA3/4, D <= 16).
+//
+// A worker is one DPP row: the 16 lanes l & ~15 .. l | 15 of a wavefront, four workers to a
+// wavefront.  Lane r < D holds row r of every matrix of the element in registers.  What one lane
+// needs of another's row arrives as the broadcast operand of the multiply-add that uses it
+// (v_fmac_f64_dpp with row_newbcast: the one DPP control that 64-bit operations take, at the
+// rate of a plain v_fma_f64: 3.97 and 4.18 ns per operation of one wave, 2.3 ns and 2.3 ns at four
+// waves per SIMD), so nothing passes through LDS and no worker waits for another.  The scalar part
+// of a Householder pivot (square root, reciprocal, selects) is issued once for the wavefront's four
+// combines.
+//
+// Against rows split over two lanes of a whole-wavefront worker, with each pivot row passed through
+// LDS and every lane repeating the pivot's scalar part: about 5,300 instructions per combine became
+// about 5,600 per four, and at D = 12 a level of 32,768 combines went from 364 to 107 us (up) and
+// from 205 to 70 us (down), the latency of one combine from 19 to 14 us and from 13 to 9.7 us.  What
+// bounds it is FP64 issue: two waves per SIMD (248 registers), 2.5 ns per instruction.
+//
+// Lanes r >= D of a row repeat row 0; only lanes r < D are ever the source of a broadcast or store.
+// A whole row is active or not (a worker past the end returns as a whole), so a broadcast never
+// reads an inactive lane.
+#pragma once
+
+#include <hip/hip_runtime.h>
+
+#include <type_traits>
+
+#include "pof_core.hpp"
+
+#pragma clang fp contract(off)
+
+namespace pof {
+namespace r16 {
+
+constexpr int kRow = 16;            // lanes per worker
+constexpr int kBlock = 64;          // threads per block: one wavefront
+constexpr int kPerBlock = kBlock / kRow;
+
+// ------------------------------------------------------------- broadcasts
+__device__ double update_dpp_f64(double, double, int, int, int, bool) __asm("llvm.amdgcn.update.dpp.f64");
+
+// Lane L's value in every lane of its row.
+template <int L>
+__device__ __forceinline__ double bcast(double v) {
+  return update_dpp_f64(v, v, 0x150 + L, 0xf, 0xf, true);
+}
+
+// y += (lane l's p) * x.  A DPP operand must not have been written by the two instructions before
+// (the hardware does not wait for it and the compiler does not look into an asm statement), hence
+// the s_nop at the head of each group; within a group no source is a result.
+#define POF_FMAC(y, p, x, l) \
+  "v_fmac_f64_dpp %[" #y "], %[" #p "], %[" #x "] row_newbcast:%[" #l "] row_mask:0xf bank_mask:0xf\n"
+
+// y[c] += bcast_L(p[c]) x, c < N
+template <int L, int N>
+__device__ __forceinline__ void fma_rows(double* y, const double* p, double x) {
+  if constexpr (N >= 8) {
+    asm("s_nop 1\n" POF_FMAC(y0, p0, x, l) POF_FMAC(y1, p1, x, l) POF_FMAC(y2, p2, x, l) POF_FMAC(y3, p3, x, l)
+            POF_FMAC(y4, p4, x, l) POF_FMAC(y5, p5, x, l) POF_FMAC(y6, p6, x, l) POF_FMAC(y7, p7, x, l)
+        : [y0] "+v"(y[0]), [y1] "+v"(y[1]), [y2] "+v"(y[2]), [y3] "+v"(y[3]), [y4] "+v"(y[4]), [y5] "+v"(y[5]),
+          [y6] "+v"(y[6]), [y7] "+v"(y[7])
+        : [p0] "v"(p[0]), [p1] "v"(p[1]), [p2] "v"(p[2]), [p3] "v"(p[3]), [p4] "v"(p[4]), [p5] "v"(p[5]),
+          [p6] "v"(p[6]), [p7] "v"(p[7]), [x] "v"(x), [l] "n"(L));
+    if constexpr (N > 8) fma_rows<L, N - 8>(y + 8, p + 8, x);
+  } else if constexpr (N >= 4) {
+    asm("s_nop 1\n" POF_FMAC(y0, p0, x, l) POF_FMAC(y1, p1, x, l) POF_FMAC(y2, p2, x, l) POF_FMAC(y3, p3, x, l)
+        : [y0] "+v"(y[0]), [y1] "+v"(y[1]), [y2] "+v"(y[2]), [y3] "+v"(y[3])
+        : [p0] "v"(p[0]), [p1] "v"(p[1]), [p2] "v"(p[2]), [p3] "v"(p[3]), [x] "v"(x), [l] "n"(L));
+    if constexpr (N > 4) fma_rows<L, N - 4>(y + 4, p + 4, x);
+  } else if constexpr (N >= 2) {
+    asm("s_nop 1\n" POF_FMAC(y0, p0, x, l) POF_FMAC(y1, p1, x, l)
+        : [y0] "+v"(y[0]), [y1] "+v"(y[1])
+        : [p0] "v"(p[0]), [p1] "v"(p[1]), [x] "v"(x), [l] "n"(L));
+    if constexpr (N > 2) fma_rows<L, N - 2>(y + 2, p + 2, x);
+  } else if constexpr (N == 1) {
+    asm("s_nop 1\n" POF_FMAC(y0, p0, x, l) : [y0] "+v"(y[0]) : [p0] "v"(p[0]), [x] "v"(x), [l] "n"(L));
+  }
+}
+
+// y[c] += bcast_L(y[c]) x, c < N (lane L's own values feed the products before they change)
+template <int L, int N>
+__device__ __forceinline__ void fma_self(double* y, double x) {
+  if constexpr (N >= 8) {
+    asm("s_nop 1\n" POF_FMAC(y0, y0, x, l) POF_FMAC(y1, y1, x, l) POF_FMAC(y2, y2, x, l) POF_FMAC(y3, y3, x, l)
+            POF_FMAC(y4, y4, x, l) POF_FMAC(y5, y5, x, l) POF_FMAC(y6, y6, x, l) POF_FMAC(y7, y7, x, l)
+        : [y0] "+v"(y[0]), [y1] "+v"(y[1]), [y2] "+v"(y[2]), [y3] "+v"(y[3]), [y4] "+v"(y[4]), [y5] "+v"(y[5]),
+          [y6] "+v"(y[6]), [y7] "+v"(y[7])
+        : [x] "v"(x), [l] "n"(L));
+    if constexpr (N > 8) fma_self<L, N - 8>(y + 8, x);
+  } else if constexpr (N >= 4) {
+    asm("s_nop 1\n" POF_FMAC(y0, y0, x, l) POF_FMAC(y1, y1, x, l) POF_FMAC(y2, y2, x, l) POF_FMAC(y3, y3, x, l)
+        : [y0] "+v"(y[0]), [y1] "+v"(y[1]), [y2] "+v"(y[2]), [y3] "+v"(y[3])
+        : [x] "v"(x), [l] "n"(L));
+    if constexpr (N > 4) fma_self<L, N - 4>(y + 4, x);
+  } else if constexpr (N >= 2) {
+    asm("s_nop 1\n" POF_FMAC(y0, y0, x, l) POF_FMAC(y1, y1, x, l)
+        : [y0] "+v"(y[0]), [y1] "+v"(y[1])
+        : [x] "v"(x), [l] "n"(L));
+    if constexpr (N > 2) fma_self<L, N - 2>(y + 2, x);
+  } else if constexpr (N == 1) {
+    asm("s_nop 1\n" POF_FMAC(y0, y0, x, l) : [y0] "+v"(y[0]) : [x] "v"(x), [l] "n"(L));
+  }
+}
+
+// y[c] += bcast_{L + c}(p) x, c < N
+template <int L, int N>
+__device__ __forceinline__ void fma_lanes(double* y, double p, double x) {
+  if constexpr (N >= 4) {
+    asm("s_nop 1\n" POF_FMAC(y0, p, x, l0) POF_FMAC(y1, p, x, l1) POF_FMAC(y2, p, x, l2) POF_FMAC(y3, p, x, l3)
+        : [y0] "+v"(y[0]), [y1] "+v"(y[1]), [y2] "+v"(y[2]), [y3] "+v"(y[3])
+        : [p] "v"(p), [x] "v"(x), [l0] "n"(L), [l1] "n"(L + 1), [l2] "n"(L + 2), [l3] "n"(L + 3));
+    if constexpr (N > 4) fma_lanes<L + 4, N - 4>(y + 4, p, x);
+  } else if constexpr (N >= 2) {
+    asm("s_nop 1\n" POF_FMAC(y0, p, x, l0) POF_FMAC(y1, p, x, l1)
+        : [y0] "+v"(y[0]), [y1] "+v"(y[1])
+        : [p] "v"(p), [x] "v"(x), [l0] "n"(L), [l1] "n"(L + 1));
+    if constexpr (N > 2) fma_lanes<L + 2, N - 2>(y + 2, p, x);
+  } else if constexpr (N == 1) {
+    asm("s_nop 1\n" POF_FMAC(y0, p, x, l0) : [y0] "+v"(y[0]) : [p] "v"(p), [x] "v"(x), [l0] "n"(L));
+  }
+}
+
+// s[c & 1] += bcast_L(p[c]) q[c], c = C .. C + N - 1: even and odd columns in a sum each
+template <int L, int N, int C = 0>
+__device__ __forceinline__ void dot_rows(double (&s)[2], const double* p, const double* q) {
+  double& e = s[C & 1];
+  double& o = s[(C + 1) & 1];
+  if constexpr (N >= 4) {
+    asm("s_nop 1\n" POF_FMAC(e, p0, q0, l) POF_FMAC(o, p1, q1, l) POF_FMAC(e, p2, q2, l) POF_FMAC(o, p3, q3, l)
+        : [e] "+v"(e), [o] "+v"(o)
+        : [p0] "v"(p[C]), [p1] "v"(p[C + 1]), [p2] "v"(p[C + 2]), [p3] "v"(p[C + 3]), [q0] "v"(q[C]),
+          [q1] "v"(q[C + 1]), [q2] "v"(q[C + 2]), [q3] "v"(q[C + 3]), [l] "n"(L));
+    if constexpr (N > 4) dot_rows<L, N - 4, C + 4>(s, p, q);
+  } else if constexpr (N >= 2) {
+    asm("s_nop 1\n" POF_FMAC(e, p0, q0, l) POF_FMAC(o, p1, q1, l)
+        : [e] "+v"(e), [o] "+v"(o)
+        : [p0] "v"(p[C]), [p1] "v"(p[C + 1]), [q0] "v"(q[C]), [q1] "v"(q[C + 1]), [l] "n"(L));
+    if constexpr (N > 2) dot_rows<L, N - 2, C + 2>(s, p, q);
+  } else if constexpr (N == 1) {
+    asm("s_nop 1\n" POF_FMAC(e, p0, q0, l) : [e] "+v"(e) : [p0] "v"(p[C]), [q0] "v"(q[C]), [l] "n"(L));
+  }
+}
+
+// sum_{k < N} bcast_k(v) x[k]: a row (or, of a transposed matrix, a column) times a vector whose
+// entry k sits in lane k; even and odd k in a sum each
+template <int N, int K = 0>
+__device__ __forceinline__ void dot_lanes_(double (&s)[2], const double* x, double v) {
+  if constexpr (N >= 4) {
+    asm("s_nop 1\n" POF_FMAC(e, v, x0, l0) POF_FMAC(o, v, x1, l1) POF_FMAC(e, v, x2, l2) POF_FMAC(o, v, x3, l3)
+        : [e] "+v"(s[0]), [o] "+v"(s[1])
+        : [v] "v"(v), [x0] "v"(x[K]), [x1] "v"(x[K + 1]), [x2] "v"(x[K + 2]), [x3] "v"(x[K + 3]), [l0] "n"(K),
+          [l1] "n"(K + 1), [l2] "n"(K + 2), [l3] "n"(K + 3));
+    dot_lanes_<N - 4, K + 4>(s, x, v);
+  } else if constexpr (N >= 2) {
+    asm("s_nop 1\n" POF_FMAC(e, v, x0, l0) POF_FMAC(o, v, x1, l1)
+        : [e] "+v"(s[0]), [o] "+v"(s[1])
+        : [v] "v"(v), [x0] "v"(x[K]), [x1] "v"(x[K + 1]), [l0] "n"(K), [l1] "n"(K + 1));
+    dot_lanes_<N - 2, K + 2>(s, x, v);
+  } else if constexpr (N == 1) {
+    asm("s_nop 1\n" POF_FMAC(e, v, x0, l0) : [e] "+v"(s[0]) : [v] "v"(v), [x0] "v"(x[K]), [l0] "n"(K));
+  }
+}
+template <int N>
+__device__ __forceinline__ double dot_lanes(const double* x, double v, double init = 0.0) {
+  double s[2] = {init, 0.0};
+  dot_lanes_<N>(s, x, v);
+  return s[0] + s[1];
+}
+
+// ------------------------------------------------------------- compile-time loops
+template <int I, int N, class F>
+__device__ __forceinline__ void unroll(F&& f) {
+  if constexpr (I < N) {
+    f(std::integral_constant<int, I>{});
+    unroll<I + 1, N>(f);
+  }
+}
+template <int I, int N, class F>  // I, I - 1, ..., N
+__device__ __forceinline__ void unroll_down(F&& f) {
+  if constexpr (I >= N) {
+    f(std::integral_constant<int, I>{});
+    unroll_down<I - 1, N>(f);
+  }
+}
+
+// ------------------------------------------------------------- products
+// y[c] += sum_k x[k] (row k of B)[c] over the columns c < min(N, k + LOW) of row k (LOW = 1: B lower
+// triangular; LOW >= N: full)
+template <int K, int N, int LOW>
+__device__ __forceinline__ void mul_rows(double (&y)[N], const double* x, const double* B) {
+  unroll<0, K>([&](auto k) {
+    constexpr int kk = decltype(k)::value;
+    fma_rows<kk, (kk + LOW < N) ? kk + LOW : N>(y, B, x[kk]);
+  });
+}
+
+// ------------------------------------------------------------- Householder pivot
+// The scalar part of a pivot with entry alpha and squared tail sig, as LAPACK dlarfg:
+// beta = -sign(alpha) sqrt(alpha^2 + sig), v = [1, tail / (alpha - beta)], tau = (beta - alpha) / beta.
+// Applied to another row with entry a at the pivot and product `dot` with the tail:
+//   w = a + dot / (alpha - beta),  entry -= tau w,  tail -= tau w / (alpha - beta) tail,
+// and tau / (alpha - beta) = -1 / beta, so one reciprocal serves.
+// rb = -1 / beta = sign(alpha) / norm, den = alpha - beta, sc = 1 / den.
+struct Pivot {
+  double beta, rb, den, sc;
+};
+
+// norm and 1 / norm of x > 0: the hardware's estimate y (about 2^-24) and one third-order step,
+// e = 1 - x y^2, (1 - e)^(-1/2) = 1 + e / 2 + 3 e^2 / 8 + O(e^3): 2^-72 before rounding.
+__device__ __forceinline__ void norm_rnorm(double x, double& n, double& rn) {
+  const double y = __builtin_amdgcn_rsq(x);
+  const double g = x * y;
+  const double e = fma(-g, y, 1.0);
+  const double q = e * fma(e, 0.375, 0.5);
+  n = fma(g, q, g);
+  rn = fma(y, q, y);
+}
+
+// 1 / x for normal x: the estimate and one third-order step (1 + e + e^2)
+__device__ __forceinline__ double rcp3(double x) {
+  const double r = __builtin_amdgcn_rcp(x);
+  const double e = fma(-x, r, 1.0);
+  return fma(r, fma(e, e, e), r);
+}
+
+// A pivot whose tail cannot vanish.
+__device__ __forceinline__ Pivot pivot_nz(double alpha, double sig) {
+  Pivot p;
+  double n, rn;
+  norm_rnorm(fma(alpha, alpha, sig), n, rn);
+  p.beta = -copysign(n, alpha);  // Fortran SIGN: honours the sign of -0.0
+  p.den = alpha - p.beta;
+  p.sc = rcp3(p.den);
+  p.rb = copysign(rn, alpha);
+  return p;
+}
+
+// Any pivot: a zero tail leaves the row (tau = 0, beta = alpha).
+__device__ __forceinline__ Pivot pivot(double alpha, double sig) {
+  const bool nz = sig != 0.0;
+  Pivot p = pivot_nz(nz ? alpha : 1.0, nz ? sig : 1.0);
+  p.beta = nz ? p.beta : alpha;
+  p.rb = nz ? p.rb : 0.0;
+  return p;
+}
+
+// ------------------------------------------------------------- LQ, one row set
+// LQ of a D-row matrix [B1 | B2] (B1 first-block columns a, B2 second-block columns b, rows in lanes
+// 0 .. D - 1): on return a holds the lower triangle of the factor in its columns <= row (entries
+// above are left over and not cleared).  Row r of the second block is zero beyond column
+// max(r, W2).  B1 >= D.
+template <int D, int B1, int B2, int W2>
+__device__ __forceinline__ void lq1(double (&a)[B1], double* b, int r) {
+  unroll<0, D>([&](auto ic) {
+    constexpr int i = decltype(ic)::value;
+    constexpr int n1 = B1 - 1 - i;
+    constexpr int band = (i > W2 ? i : W2) + 1;
+    constexpr int n2 = (band < B2) ? band : B2;
+    if constexpr (n1 + n2 > 0) {
+      double s[2] = {0.0, 0.0};
+      dot_rows<i, n1, i + 1>(s, a, a);
+      dot_rows<i, n2, 0>(s, b, b);
+      const double dot = s[0] + s[1];
+      const Pivot p = pivot(bcast<i>(a[i]), bcast<i>(dot));
+      const double tws = p.rb * fma(p.sc, dot, a[i]);
+      a[i] = (r == i) ? p.beta : fma(-p.den, tws, a[i]);
+      fma_self<i, n1>(a + i + 1, -tws);
+      fma_self<i, n2>(b, -tws);
+    }
+  });
+}
+
+// ------------------------------------------------------------- memory
+// Row of N contiguous doubles (16-byte accesses where every row of an N-column matrix is aligned)
+template <int N>
+__device__ __forceinline__ void load_row16(double (&x)[N], const double* p) {
+  if constexpr (N % 2 == 0) {
+#pragma unroll
+    for (int i = 0; i < N; i += 2) {
+      const double2 v = *reinterpret_cast<const double2*>(p + i);
+      x[i] = v.x;
+      x[i + 1] = v.y;
+    }
+  } else {
+#pragma unroll
+    for (int i = 0; i < N; ++i) x[i] = p[i];
+  }
+}
+template <int N>
+__device__ __forceinline__ void store_row16(double* p, const double (&x)[N]) {
+  if constexpr (N % 2 == 0) {
+#pragma unroll
+    for (int i = 0; i < N; i += 2) *reinterpret_cast<double2*>(p + i) = make_double2(x[i], x[i + 1]);
+  } else {
+#pragma unroll
+    for (int i = 0; i < N; ++i) p[i] = x[i];
+  }
+}
+// column r of an N x N matrix: the lanes of a row read one matrix row together
+template <int N>
+__device__ __forceinline__ void load_col16(double (&x)[N], const double* M, int r) {
+#pragma unroll
+  for (int k = 0; k < N; ++k) x[k] = M[k * N + r];
+}
+// the lower triangle of a factor, its strict upper part cleared
+template <int N>
+__device__ __forceinline__ void store_lower16(double* p, double (&x)[N], int r) {
+#pragma unroll
+  for (int c = 1; c < N; ++c) x[c] = (c > r) ? 0.0 : x[c];
+  store_row16(p, x);
+}
+
+// ------------------------------------------------------------- filter combine
+// pof/parallel_filtsmooth/filter.py:117-142, as filter_combine() of pof_core.hpp: e = e1 o e2, e1
+// earlier.  SO (state only): e1 is a prefix state (s1.m, s1.L) and (so.m, so.L) receives the result.
+//
+// DZ: nonzero columns of the elements' Z: d at a leaf level ([Zr | 0]), D above it (lower
+// triangular).  Columns of zeros are left out of every sum and update (they add exact zeros); at a
+// leaf level this leaves pivot i of the Xi factorisation max(d - 1 - i, 0) + i tail columns instead
+// of D - 1 in each of its four passes.
+//
+// Xi = [[U1^T Z2, I], [Z2, 0]], rows 0 .. D - 1 (a) and D .. 2D - 1 (b) of a lane's two row sets.
+// Column i of the second block is still the identity's when pivot i comes: it adds 1 to the pivot
+// row's squared tail (so no tail vanishes) and its update is -tau w v_i without a product.
+template <int D, int DZ, bool SO>
+__device__ __forceinline__ void filter_combine(int r, const FiltArrays& x1, const StateArrays& s1, size_t i1,
+                                               const FiltArrays& x2, size_t i2, const FiltArrays& y,
+                                               const StateArrays& so, size_t o) {
+  constexpr size_t DD = (size_t)D * D;
+  constexpr bool kLeaf = DZ < D;
+  constexpr int kLow = kLeaf ? D : 1;  // Z2's row k holds columns < min(DZ, k + kLow)
+  const bool act = r < D;
+  const int rr = act ? r : 0;
+  const double* U1 = (SO ? s1.L : x1.U) + i1 * DD;
+  const double* A2 = x2.A + i2 * DD;
+  const double* Z2 = x2.Z + i2 * DD;
+  const double b1r = (SO ? s1.m : x1.b)[i1 * D + rr];
+  const double eta2r = x2.eta[i2 * D + rr];
+
+  double u, s2 = 0.0, uu = 0.0;
+  double a1[D], b1[D], b2[D], rd = 0.0;  // Xi11, Xi21, Xi22; rd: 1 / Xi11[r][r] in lane r
+  {
+    double a2[D];
+    {
+      double u1t[D], z2[D];
+      load_col16<D>(u1t, U1, rr);
+      if constexpr (kLeaf) {
+#pragma unroll
+        for (int c = 0; c < DZ; ++c) z2[c] = Z2[rr * D + c];
+      } else {
+        load_row16<D>(z2, Z2 + rr * D);
+      }
+      if constexpr (!SO) {
+        // s2 = eta2 - Z2 (Z2^T b1), uu = U1^T s2
+        double z2t[D];
+        load_col16<D>(z2t, Z2, rr);
+        const double t = dot_lanes<D>(z2t, b1r);
+        s2 = eta2r - dot_lanes<DZ>(z2, t);
+        uu = dot_lanes<D>(u1t, s2);
+      }
+      u = dot_lanes<D>(u1t, eta2r);
+      double x[DZ];
+      zero(x);
+      mul_rows<D, DZ, kLow>(x, u1t, z2);
+#pragma unroll
+      for (int c = 0; c < DZ; ++c) {
+        a1[c] = x[c];
+        b1[c] = z2[c];
+      }
+    }
+    unroll<0, D>([&](auto ic) {
+      constexpr int i = decltype(ic)::value;
+      constexpr int n1 = (i < DZ) ? DZ - 1 - i : 0;
+      double sa[2] = {0.0, 0.0}, sb[2] = {0.0, 0.0};
+      dot_rows<i, n1, i + 1>(sa, a1, a1);
+      dot_rows<i, n1, i + 1>(sb, a1, b1);
+      dot_rows<i, i, 0>(sa, a2, a2);
+      dot_rows<i, i, 0>(sb, a2, b2);
+      const double da = sa[0] + sa[1], db = sb[0] + sb[1];
+      const double sig = bcast<i>(da) + 1.0;
+      double ta, tb;
+      if constexpr (i < DZ) {
+        const Pivot p = pivot_nz(bcast<i>(a1[i]), sig);
+        ta = p.rb * fma(p.sc, da, a1[i]);
+        tb = p.rb * fma(p.sc, db, b1[i]);
+        a1[i] = fma(-p.den, ta, a1[i]);
+        b1[i] = fma(-p.den, tb, b1[i]);
+        rd = (r == i) ? -p.rb : rd;
+      } else {
+        // column i of the first block is zero: alpha = 0, den = norm, beta = -norm
+        double n, rn;
+        norm_rnorm(sig, n, rn);
+        const double wa = rn * da, wb = rn * db;
+        ta = rn * wa;
+        tb = rn * wb;
+        a1[i] = -wa;
+        b1[i] = -wb;
+        rd = (r == i) ? -rn : rd;
+      }
+      fma_rows<i, n1>(b1 + i + 1, a1 + i + 1, -tb);
+      fma_rows<i, i>(b2, a2, -tb);
+      fma_self<i, n1>(a1 + i + 1, -ta);
+      fma_self<i, i>(a2, -ta);
+      a2[i] = -ta;
+      b2[i] = -tb;
+    });
+  }
+
+  // MT = A2 U1 Xi11^-T, W = A2 - MT Xi21^T, b = W (b1 + U1 u) + b2
+  double mt[D], w[D];
+  zero(mt);
+  double sv;
+  {
+    double u1[D];
+    load_row16<D>(w, A2 + rr * D);
+    load_row16<D>(u1, U1 + rr * D);
+    mul_rows<D, D, 1>(mt, w, u1);
+    sv = dot_lanes<D>(u1, u, b1r);
+  }
+  unroll<0, D>([&](auto jc) {
+    constexpr int j = decltype(jc)::value;
+    mt[j] = mt[j] * bcast<j>(rd);
+    fma_lanes<j + 1, D - 1 - j>(mt + j + 1, a1[j], -mt[j]);
+  });
+  unroll<0, D>([&](auto jc) {
+    constexpr int j = decltype(jc)::value;
+    fma_lanes<0, D>(w, b1[j], -mt[j]);
+  });
+  const double bo = dot_lanes<D>(w, sv, x2.b[i2 * D + rr]);
+
+  if constexpr (!SO) {
+    // A = W A1
+    const double* A1 = x1.A + i1 * DD;
+    {
+      double ar[D], a[D];
+      load_row16<D>(ar, A1 + rr * D);
+      zero(a);
+      mul_rows<D, D, D>(a, w, ar);
+      if (act) store_row16<D>(y.A + (o * D + r) * D, a);
+    }
+    // eta = A1^T (s2 - Xi21 Xi11^-1 U1^T s2) + eta1
+    double w2 = 0.0;
+    {
+      double x = uu;
+      unroll<0, D>([&](auto jc) {
+        constexpr int j = decltype(jc)::value;
+        const double wj = bcast<j>(x * rd);
+        w2 = (r == j) ? wj : w2;
+        x = fma(-a1[j], wj, x);
+      });
+    }
+    const double s3 = s2 - dot_lanes<D>(b1, w2);
+    // Xi22 triangular, then Z = tria([A1^T Xi22 | Z1])
+    lq1<D, D, 0, 0>(b2, nullptr, r);
+    double z[D];
+    {
+      double a1t[D];
+      load_col16<D>(a1t, A1, rr);
+      const double eo = dot_lanes<D>(a1t, s3, x1.eta[i1 * D + rr]);
+      if (act) y.eta[o * D + r] = eo;
+      zero(z);
+      mul_rows<D, D, 1>(z, a1t, b2);
+    }
+    {
+      double z1[DZ];
+      const double* Z1 = x1.Z + i1 * DD;
+      if constexpr (kLeaf) {
+#pragma unroll
+        for (int c = 0; c < DZ; ++c) z1[c] = Z1[rr * D + c];
+      } else {
+        load_row16<DZ>(z1, Z1 + rr * D);
+      }
+      lq1<D, D, DZ, kLeaf ? DZ - 1 : 0>(z, z1, r);
+    }
+    if (act) store_lower16<D>(y.Z + (o * D + r) * D, z, r);
+  }
+  // U = tria([MT | U2])
+  {
+    double u2[D];
+    load_row16<D>(u2, x2.U + (i2 * D + rr) * D);
+    lq1<D, D, D, 0>(mt, u2, r);
+  }
+  if (act) {
+    (SO ? so.m : y.b)[o * D + r] = bo;
+    store_lower16<D>((SO ? so.L : y.U) + (o * D + r) * D, mt, r);
+  }
+}
+
+}  // namespace r16
+}  // namespace pof
+
+#pragma clang fp contract(fast)
