@@ -1007,22 +1007,23 @@ struct Obs<D, d, true> {
 
   __device__ __forceinline__ void load(const ModelArgs& a, int k) { load_at(a, a.lin + (size_t)(k + 1) * D); }
   // linearise at the (preconditioned) state mean m
-  __device__ __forceinline__ void load_at(const ModelArgs& a, const double* m) {
+  __device__ __forceinline__ void load_at(const ModelArgs& a, const double* m) { load_at(a.kind, a.params, a.Pd, m); }
+  __device__ __forceinline__ void load_at(int kind, const double* params, const double* Pd, const double* m) {
     double y[d];
 #pragma unroll
-    for (int i = 0; i < d; ++i) y[i] = a.Pd[i * q1] * m[i * q1];
+    for (int i = 0; i < d; ++i) y[i] = Pd[i * q1] * m[i * q1];
     double f[d];
     double J[d][d];
-    field_and_jacobian<d>(a.kind, a.params, y, f, J);
+    field_and_jacobian<d>(kind, params, y, f, J);
 #pragma unroll
     for (int i = 0; i < d; ++i) {
       double acc = 0.0;
 #pragma unroll
       for (int l = 0; l < d; ++l) {
-        hc[i][l] = -J[i][l] * a.Pd[l * q1];
+        hc[i][l] = -J[i][l] * Pd[l * q1];
         acc = fma(J[i][l], y[l], acc);
       }
-      hd[i] = a.Pd[i * q1 + 1];
+      hd[i] = Pd[i * q1 + 1];
       c[i] = acc - f[i];
     }
   }

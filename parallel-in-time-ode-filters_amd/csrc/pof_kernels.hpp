@@ -96,25 +96,11 @@ __device__ __forceinline__ ModelArgs view(const GroupArgs& g, int j) {
 }
 
 // ------------------------------------------------------------------ kernels
-// Launch bounds of the element kernels on the IEKS path (EK1), where LDS
-// allows more waves per SIMD than their natural register allocation: the
-// bound trades a small spill for occupancy.  Measured to pay at D = 12 only
-// (leaf 3 -> 4, post 2 -> 3 waves, +0.9% on Lorenz-63 Ns = 65536); the same
-// bounds on leaf<15>, post<10> and post<15> ran slower.
-template <int D, bool EK1>
-constexpr int leaf_min_waves(bool first) {
-  return (first || !EK1) ? 1 : (D == 12) ? 4 : 1;
-}
-template <int D, bool EK1>
-constexpr int post_min_waves() {
-  return !EK1 ? 1 : (D == 12) ? 3 : 1;
-}
-
-// Leaf elements.  FIRST: element 0 of each IVP (it carries the prior x0;
+// Leaf elements, D > 16.  FIRST: element 0 of each IVP (it carries the prior x0;
 // one work item per IVP); otherwise work item i builds element i + 1.
 template <int D, int d, bool EK1, bool FIRST>
-__global__ __launch_bounds__((Geo<D, FIRST ? kLdsLeaf1 : kLdsLeaf>::BLOCK), (leaf_min_waves<D, EK1>(FIRST))) void
-k_filter_leaf(GroupArgs g, LaunchMap lm) {
+__global__ __launch_bounds__((Geo<D, FIRST ? kLdsLeaf1 : kLdsLeaf>::BLOCK)) void k_filter_leaf(GroupArgs g,
+                                                                                              LaunchMap lm) {
   extern __shared__ double smem[];
   auto cx = make_ctx<D, FIRST ? kLdsLeaf1 : kLdsLeaf>(g.F, g.LQ, g.N1z, smem);
   int j, k;
@@ -234,6 +220,14 @@ __global__ __launch_bounds__(r16::kBlock, 2) void k_filter_down16(GroupArgs g, L
   }
 }
 
+// Elements 0 .. Ns - 1, one row per lane, D <= 16.
+template <int D, int d, bool EK1>
+__global__ __launch_bounds__(r16::kBlock, 2) void k_filter_leaf16(GroupArgs g, LaunchMap lm) {
+  int j, k;
+  if (!locate(lm, blockIdx.x * r16::kPerBlock + threadIdx.x / r16::kRow, j, k)) return;
+  r16::filter_element<D, d, EK1>(threadIdx.x % r16::kRow, g, j, k, at(g.fel, g.base[j], D));
+}
+
 // Per filtered state s = 0..Ns: smoother element (smoother.py:37-50) stored at
 // reversed index Ns - s (terminal element (m, 0, L) for s = Ns), and for
 // s < Ns the predicted observation statistics of filter.py:84-114:
@@ -246,9 +240,7 @@ __global__ __launch_bounds__(r16::kBlock, 2) void k_filter_down16(GroupArgs g, L
 // smoother elements without observation statistics (smoother on its own).
 enum PostMode : int { kPostFull = 0, kPostDm = 1, kPostNoObs = 2 };
 template <int D, int d, bool EK1>
-__global__ __launch_bounds__((Geo<D, kLdsPost>::BLOCK), (post_min_waves<D, EK1>())) void k_filter_post(GroupArgs g,
-                                                                                                      LaunchMap lm,
-                                                                                                      int mode) {
+__global__ __launch_bounds__((Geo<D, kLdsPost>::BLOCK)) void k_filter_post(GroupArgs g, LaunchMap lm, int mode) {
   extern __shared__ double smem[];
   auto cx = make_ctx<D, kLdsPost>(g.F, g.LQ, g.N1z, smem);
   using L = Lay<D, decltype(cx)::S>;
@@ -424,6 +416,35 @@ __global__ __launch_bounds__((Geo<D, kLdsPost>::BLOCK), (post_min_waves<D, EK1>(
     store_dist<S, D>(sel.E + (ro * D + r) * D, e, sb);
   }
   wsync();
+}
+
+// The same with one row per lane, D <= 16.
+template <int D, int d, bool EK1>
+__global__ __launch_bounds__(r16::kBlock, 2) void k_filter_post16(GroupArgs g, LaunchMap lm, int mode) {
+  int j, s;
+  if (!locate(lm, blockIdx.x * r16::kPerBlock + threadIdx.x / r16::kRow, j, s)) return;
+  const long long base = g.base[j];
+  const int Ns = g.Ns[j];
+  const StateArrays pre0 = at(g.fpre, base, D);
+  const SmoArrays sel = at(g.sel, base, D);
+  const int r = threadIdx.x % r16::kRow;
+  const double* mp = (s == 0) ? g.x0m + (size_t)j * D : pre0.m + (size_t)(s - 1) * D;
+  const double* Lp = (s == 0) ? g.x0L + (size_t)j * D * D : pre0.L + (size_t)(s - 1) * D * D;
+  const size_t ro = (size_t)(Ns - s);
+  if (s == Ns) {
+    if (r < D) {
+      double x[D];
+      r16::load_row16<D>(x, Lp + r * D);
+      r16::store_row16<D>(sel.Dm + (ro * D + r) * D, x);
+      zero(x);
+      r16::store_row16<D>(sel.E + (ro * D + r) * D, x);
+      sel.g[ro * D + r] = mp[r];
+    }
+    return;
+  }
+  const bool dm = mode == kPostDm;
+  r16::filter_post<D, d, EK1>(r, g, j, s, mp, Lp, mode == kPostFull, dm, dm || g.wchol[j] != 0, sel, ro, g.t_ssq + base,
+                              g.t_nll + base);
 }
 
 // Smoother up-sweep
@@ -987,15 +1008,24 @@ void smooth_scan(const GroupArgs& g, const LaunchPlan& p, hipStream_t st, Rec& r
   }
 }
 
+// k_filter_post of every filtered state
+template <int D, int d, bool EK1>
+void launch_post(const GroupArgs& g, const LaunchPlan& p, int mode, hipStream_t st) {
+  const LaunchMap lm = p.map(p.pts_off, p.pts_total);
+  if constexpr (D <= r16::kRow)
+    POF_LAUNCH16((k_filter_post16<D, d, EK1>), p.pts_total, st, g, lm, mode);
+  else
+    POF_LAUNCH((k_filter_post<D, d, EK1>), kLdsPost, p.pts_total, st, g, lm, mode);
+}
+
 template <int D, int d>
 hipError_t run_smooth_chol(const GroupArgs& g, const LaunchPlan& p, hipStream_t st, KernelTimer* t) {
   Rec rec(t, st);
   // the smoother elements' D of the last (means-only) iteration, then the factor scan
-  if (g.affine) {
-    POF_LAUNCH((k_filter_post<D, d, false>), kLdsPost, p.pts_total, st, g, p.map(p.pts_off, p.pts_total), kPostDm);
-  } else {
-    POF_LAUNCH((k_filter_post<D, d, true>), kLdsPost, p.pts_total, st, g, p.map(p.pts_off, p.pts_total), kPostDm);
-  }
+  if (g.affine)
+    launch_post<D, d, false>(g, p, kPostDm, st);
+  else
+    launch_post<D, d, true>(g, p, kPostDm, st);
   rec(kKFilterPost, p.leaf_total);
   smooth_scan<D>(g, p, st, rec);
   return hipGetLastError();
@@ -1005,7 +1035,12 @@ template <int D, int d>
 hipError_t run_iteration(const GroupArgs& g, const LaunchPlan& p, double* scal, hipStream_t st, KernelTimer* t) {
   Rec rec(t, st);
   // ---- filter: leaf elements, up-sweep, down-sweep
-  if (g.affine) {
+  if constexpr (D <= r16::kRow) {
+    if (g.affine)
+      POF_LAUNCH16((k_filter_leaf16<D, d, false>), p.leaf_total, st, g, p.map(p.leaf_off, p.leaf_total));
+    else
+      POF_LAUNCH16((k_filter_leaf16<D, d, true>), p.leaf_total, st, g, p.map(p.leaf_off, p.leaf_total));
+  } else if (g.affine) {
     POF_LAUNCH((k_filter_leaf<D, d, false, true>), kLdsLeaf1, p.one_total, st, g, p.map(p.one_off, p.one_total));
     if (p.leaf1_total > 0)
       POF_LAUNCH((k_filter_leaf<D, d, false, false>), kLdsLeaf, p.leaf1_total, st, g,
@@ -1044,11 +1079,10 @@ hipError_t run_iteration(const GroupArgs& g, const LaunchPlan& p, double* scal, 
     rec(kKFilterDown, nw - p.fdn_ivps[l]);
   }
   // ---- smoother elements + observation statistics
-  if (g.affine) {
-    POF_LAUNCH((k_filter_post<D, d, false>), kLdsPost, p.pts_total, st, g, p.map(p.pts_off, p.pts_total), kPostFull);
-  } else {
-    POF_LAUNCH((k_filter_post<D, d, true>), kLdsPost, p.pts_total, st, g, p.map(p.pts_off, p.pts_total), kPostFull);
-  }
+  if (g.affine)
+    launch_post<D, d, false>(g, p, kPostFull, st);
+  else
+    launch_post<D, d, true>(g, p, kPostFull, st);
   rec(kKFilterPost, p.leaf_total);
   // ---- smoother scan (reversed order)
   smooth_scan<D>(g, p, st, rec);
@@ -1101,8 +1135,7 @@ hipError_t run_smooth_only(const GroupArgs& g, const LaunchPlan& p, double* scal
     POF_LAUNCH((k_seq_smooth<D>), kLdsSeq, p.one_total, st, g, p.map(p.one_off, p.one_total));
     rec(kKSmoothUp, p.leaf_total);
   } else {
-    POF_LAUNCH((k_filter_post<D, d, false>), kLdsPost, p.pts_total, st, g, p.map(p.pts_off, p.pts_total),
-               kPostNoObs);
+    launch_post<D, d, false>(g, p, kPostNoObs, st);
     rec(kKFilterPost, p.leaf_total);
     smooth_scan<D>(g, p, st, rec);
   }

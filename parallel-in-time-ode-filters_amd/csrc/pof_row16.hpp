@@ -46,7 +46,9 @@ __device__ __forceinline__ double bcast(double v) {
 
 // y += (lane l's p) * x.  A DPP operand must not have been written by the two instructions before
 // (the hardware does not wait for it and the compiler does not look into an asm statement), hence
-// the s_nop at the head of each group; within a group no source is a result.
+// the s_nop at the head of each group; within a group no source is a result.  Results are early
+// clobbers: an input that holds the same value as a result's initial one (two zeros) must not share
+// its register.
 #define POF_FMAC(y, p, x, l) \
   "v_fmac_f64_dpp %[" #y "], %[" #p "], %[" #x "] row_newbcast:%[" #l "] row_mask:0xf bank_mask:0xf\n"
 
@@ -54,25 +56,25 @@ __device__ __forceinline__ double bcast(double v) {
 template <int L, int N>
 __device__ __forceinline__ void fma_rows(double* y, const double* p, double x) {
   if constexpr (N >= 8) {
-    asm("s_nop 1\n" POF_FMAC(y0, p0, x, l) POF_FMAC(y1, p1, x, l) POF_FMAC(y2, p2, x, l) POF_FMAC(y3, p3, x, l)
+    asm volatile("s_nop 1\n" POF_FMAC(y0, p0, x, l) POF_FMAC(y1, p1, x, l) POF_FMAC(y2, p2, x, l) POF_FMAC(y3, p3, x, l)
             POF_FMAC(y4, p4, x, l) POF_FMAC(y5, p5, x, l) POF_FMAC(y6, p6, x, l) POF_FMAC(y7, p7, x, l)
-        : [y0] "+v"(y[0]), [y1] "+v"(y[1]), [y2] "+v"(y[2]), [y3] "+v"(y[3]), [y4] "+v"(y[4]), [y5] "+v"(y[5]),
-          [y6] "+v"(y[6]), [y7] "+v"(y[7])
+        : [y0] "+&v"(y[0]), [y1] "+&v"(y[1]), [y2] "+&v"(y[2]), [y3] "+&v"(y[3]), [y4] "+&v"(y[4]), [y5] "+&v"(y[5]),
+          [y6] "+&v"(y[6]), [y7] "+&v"(y[7])
         : [p0] "v"(p[0]), [p1] "v"(p[1]), [p2] "v"(p[2]), [p3] "v"(p[3]), [p4] "v"(p[4]), [p5] "v"(p[5]),
           [p6] "v"(p[6]), [p7] "v"(p[7]), [x] "v"(x), [l] "n"(L));
     if constexpr (N > 8) fma_rows<L, N - 8>(y + 8, p + 8, x);
   } else if constexpr (N >= 4) {
-    asm("s_nop 1\n" POF_FMAC(y0, p0, x, l) POF_FMAC(y1, p1, x, l) POF_FMAC(y2, p2, x, l) POF_FMAC(y3, p3, x, l)
-        : [y0] "+v"(y[0]), [y1] "+v"(y[1]), [y2] "+v"(y[2]), [y3] "+v"(y[3])
+    asm volatile("s_nop 1\n" POF_FMAC(y0, p0, x, l) POF_FMAC(y1, p1, x, l) POF_FMAC(y2, p2, x, l) POF_FMAC(y3, p3, x, l)
+        : [y0] "+&v"(y[0]), [y1] "+&v"(y[1]), [y2] "+&v"(y[2]), [y3] "+&v"(y[3])
         : [p0] "v"(p[0]), [p1] "v"(p[1]), [p2] "v"(p[2]), [p3] "v"(p[3]), [x] "v"(x), [l] "n"(L));
     if constexpr (N > 4) fma_rows<L, N - 4>(y + 4, p + 4, x);
   } else if constexpr (N >= 2) {
-    asm("s_nop 1\n" POF_FMAC(y0, p0, x, l) POF_FMAC(y1, p1, x, l)
-        : [y0] "+v"(y[0]), [y1] "+v"(y[1])
+    asm volatile("s_nop 1\n" POF_FMAC(y0, p0, x, l) POF_FMAC(y1, p1, x, l)
+        : [y0] "+&v"(y[0]), [y1] "+&v"(y[1])
         : [p0] "v"(p[0]), [p1] "v"(p[1]), [x] "v"(x), [l] "n"(L));
     if constexpr (N > 2) fma_rows<L, N - 2>(y + 2, p + 2, x);
   } else if constexpr (N == 1) {
-    asm("s_nop 1\n" POF_FMAC(y0, p0, x, l) : [y0] "+v"(y[0]) : [p0] "v"(p[0]), [x] "v"(x), [l] "n"(L));
+    asm volatile("s_nop 1\n" POF_FMAC(y0, p0, x, l) : [y0] "+&v"(y[0]) : [p0] "v"(p[0]), [x] "v"(x), [l] "n"(L));
   }
 }
 
@@ -80,24 +82,24 @@ __device__ __forceinline__ void fma_rows(double* y, const double* p, double x) {
 template <int L, int N>
 __device__ __forceinline__ void fma_self(double* y, double x) {
   if constexpr (N >= 8) {
-    asm("s_nop 1\n" POF_FMAC(y0, y0, x, l) POF_FMAC(y1, y1, x, l) POF_FMAC(y2, y2, x, l) POF_FMAC(y3, y3, x, l)
+    asm volatile("s_nop 1\n" POF_FMAC(y0, y0, x, l) POF_FMAC(y1, y1, x, l) POF_FMAC(y2, y2, x, l) POF_FMAC(y3, y3, x, l)
             POF_FMAC(y4, y4, x, l) POF_FMAC(y5, y5, x, l) POF_FMAC(y6, y6, x, l) POF_FMAC(y7, y7, x, l)
-        : [y0] "+v"(y[0]), [y1] "+v"(y[1]), [y2] "+v"(y[2]), [y3] "+v"(y[3]), [y4] "+v"(y[4]), [y5] "+v"(y[5]),
-          [y6] "+v"(y[6]), [y7] "+v"(y[7])
+        : [y0] "+&v"(y[0]), [y1] "+&v"(y[1]), [y2] "+&v"(y[2]), [y3] "+&v"(y[3]), [y4] "+&v"(y[4]), [y5] "+&v"(y[5]),
+          [y6] "+&v"(y[6]), [y7] "+&v"(y[7])
         : [x] "v"(x), [l] "n"(L));
     if constexpr (N > 8) fma_self<L, N - 8>(y + 8, x);
   } else if constexpr (N >= 4) {
-    asm("s_nop 1\n" POF_FMAC(y0, y0, x, l) POF_FMAC(y1, y1, x, l) POF_FMAC(y2, y2, x, l) POF_FMAC(y3, y3, x, l)
-        : [y0] "+v"(y[0]), [y1] "+v"(y[1]), [y2] "+v"(y[2]), [y3] "+v"(y[3])
+    asm volatile("s_nop 1\n" POF_FMAC(y0, y0, x, l) POF_FMAC(y1, y1, x, l) POF_FMAC(y2, y2, x, l) POF_FMAC(y3, y3, x, l)
+        : [y0] "+&v"(y[0]), [y1] "+&v"(y[1]), [y2] "+&v"(y[2]), [y3] "+&v"(y[3])
         : [x] "v"(x), [l] "n"(L));
     if constexpr (N > 4) fma_self<L, N - 4>(y + 4, x);
   } else if constexpr (N >= 2) {
-    asm("s_nop 1\n" POF_FMAC(y0, y0, x, l) POF_FMAC(y1, y1, x, l)
-        : [y0] "+v"(y[0]), [y1] "+v"(y[1])
+    asm volatile("s_nop 1\n" POF_FMAC(y0, y0, x, l) POF_FMAC(y1, y1, x, l)
+        : [y0] "+&v"(y[0]), [y1] "+&v"(y[1])
         : [x] "v"(x), [l] "n"(L));
     if constexpr (N > 2) fma_self<L, N - 2>(y + 2, x);
   } else if constexpr (N == 1) {
-    asm("s_nop 1\n" POF_FMAC(y0, y0, x, l) : [y0] "+v"(y[0]) : [x] "v"(x), [l] "n"(L));
+    asm volatile("s_nop 1\n" POF_FMAC(y0, y0, x, l) : [y0] "+&v"(y[0]) : [x] "v"(x), [l] "n"(L));
   }
 }
 
@@ -105,17 +107,17 @@ __device__ __forceinline__ void fma_self(double* y, double x) {
 template <int L, int N>
 __device__ __forceinline__ void fma_lanes(double* y, double p, double x) {
   if constexpr (N >= 4) {
-    asm("s_nop 1\n" POF_FMAC(y0, p, x, l0) POF_FMAC(y1, p, x, l1) POF_FMAC(y2, p, x, l2) POF_FMAC(y3, p, x, l3)
-        : [y0] "+v"(y[0]), [y1] "+v"(y[1]), [y2] "+v"(y[2]), [y3] "+v"(y[3])
+    asm volatile("s_nop 1\n" POF_FMAC(y0, p, x, l0) POF_FMAC(y1, p, x, l1) POF_FMAC(y2, p, x, l2) POF_FMAC(y3, p, x, l3)
+        : [y0] "+&v"(y[0]), [y1] "+&v"(y[1]), [y2] "+&v"(y[2]), [y3] "+&v"(y[3])
         : [p] "v"(p), [x] "v"(x), [l0] "n"(L), [l1] "n"(L + 1), [l2] "n"(L + 2), [l3] "n"(L + 3));
     if constexpr (N > 4) fma_lanes<L + 4, N - 4>(y + 4, p, x);
   } else if constexpr (N >= 2) {
-    asm("s_nop 1\n" POF_FMAC(y0, p, x, l0) POF_FMAC(y1, p, x, l1)
-        : [y0] "+v"(y[0]), [y1] "+v"(y[1])
+    asm volatile("s_nop 1\n" POF_FMAC(y0, p, x, l0) POF_FMAC(y1, p, x, l1)
+        : [y0] "+&v"(y[0]), [y1] "+&v"(y[1])
         : [p] "v"(p), [x] "v"(x), [l0] "n"(L), [l1] "n"(L + 1));
     if constexpr (N > 2) fma_lanes<L + 2, N - 2>(y + 2, p, x);
   } else if constexpr (N == 1) {
-    asm("s_nop 1\n" POF_FMAC(y0, p, x, l0) : [y0] "+v"(y[0]) : [p] "v"(p), [x] "v"(x), [l0] "n"(L));
+    asm volatile("s_nop 1\n" POF_FMAC(y0, p, x, l0) : [y0] "+&v"(y[0]) : [p] "v"(p), [x] "v"(x), [l0] "n"(L));
   }
 }
 
@@ -125,18 +127,18 @@ __device__ __forceinline__ void dot_rows(double (&s)[2], const double* p, const 
   double& e = s[C & 1];
   double& o = s[(C + 1) & 1];
   if constexpr (N >= 4) {
-    asm("s_nop 1\n" POF_FMAC(e, p0, q0, l) POF_FMAC(o, p1, q1, l) POF_FMAC(e, p2, q2, l) POF_FMAC(o, p3, q3, l)
-        : [e] "+v"(e), [o] "+v"(o)
+    asm volatile("s_nop 1\n" POF_FMAC(e, p0, q0, l) POF_FMAC(o, p1, q1, l) POF_FMAC(e, p2, q2, l) POF_FMAC(o, p3, q3, l)
+        : [e] "+&v"(e), [o] "+&v"(o)
         : [p0] "v"(p[C]), [p1] "v"(p[C + 1]), [p2] "v"(p[C + 2]), [p3] "v"(p[C + 3]), [q0] "v"(q[C]),
           [q1] "v"(q[C + 1]), [q2] "v"(q[C + 2]), [q3] "v"(q[C + 3]), [l] "n"(L));
     if constexpr (N > 4) dot_rows<L, N - 4, C + 4>(s, p, q);
   } else if constexpr (N >= 2) {
-    asm("s_nop 1\n" POF_FMAC(e, p0, q0, l) POF_FMAC(o, p1, q1, l)
-        : [e] "+v"(e), [o] "+v"(o)
+    asm volatile("s_nop 1\n" POF_FMAC(e, p0, q0, l) POF_FMAC(o, p1, q1, l)
+        : [e] "+&v"(e), [o] "+&v"(o)
         : [p0] "v"(p[C]), [p1] "v"(p[C + 1]), [q0] "v"(q[C]), [q1] "v"(q[C + 1]), [l] "n"(L));
     if constexpr (N > 2) dot_rows<L, N - 2, C + 2>(s, p, q);
   } else if constexpr (N == 1) {
-    asm("s_nop 1\n" POF_FMAC(e, p0, q0, l) : [e] "+v"(e) : [p0] "v"(p[C]), [q0] "v"(q[C]), [l] "n"(L));
+    asm volatile("s_nop 1\n" POF_FMAC(e, p0, q0, l) : [e] "+&v"(e) : [p0] "v"(p[C]), [q0] "v"(q[C]), [l] "n"(L));
   }
 }
 
@@ -145,18 +147,18 @@ __device__ __forceinline__ void dot_rows(double (&s)[2], const double* p, const 
 template <int N, int K = 0>
 __device__ __forceinline__ void dot_lanes_(double (&s)[2], const double* x, double v) {
   if constexpr (N >= 4) {
-    asm("s_nop 1\n" POF_FMAC(e, v, x0, l0) POF_FMAC(o, v, x1, l1) POF_FMAC(e, v, x2, l2) POF_FMAC(o, v, x3, l3)
-        : [e] "+v"(s[0]), [o] "+v"(s[1])
+    asm volatile("s_nop 1\n" POF_FMAC(e, v, x0, l0) POF_FMAC(o, v, x1, l1) POF_FMAC(e, v, x2, l2) POF_FMAC(o, v, x3, l3)
+        : [e] "+&v"(s[0]), [o] "+&v"(s[1])
         : [v] "v"(v), [x0] "v"(x[K]), [x1] "v"(x[K + 1]), [x2] "v"(x[K + 2]), [x3] "v"(x[K + 3]), [l0] "n"(K),
           [l1] "n"(K + 1), [l2] "n"(K + 2), [l3] "n"(K + 3));
     dot_lanes_<N - 4, K + 4>(s, x, v);
   } else if constexpr (N >= 2) {
-    asm("s_nop 1\n" POF_FMAC(e, v, x0, l0) POF_FMAC(o, v, x1, l1)
-        : [e] "+v"(s[0]), [o] "+v"(s[1])
+    asm volatile("s_nop 1\n" POF_FMAC(e, v, x0, l0) POF_FMAC(o, v, x1, l1)
+        : [e] "+&v"(s[0]), [o] "+&v"(s[1])
         : [v] "v"(v), [x0] "v"(x[K]), [x1] "v"(x[K + 1]), [l0] "n"(K), [l1] "n"(K + 1));
     dot_lanes_<N - 2, K + 2>(s, x, v);
   } else if constexpr (N == 1) {
-    asm("s_nop 1\n" POF_FMAC(e, v, x0, l0) : [e] "+v"(s[0]) : [v] "v"(v), [x0] "v"(x[K]), [l0] "n"(K));
+    asm volatile("s_nop 1\n" POF_FMAC(e, v, x0, l0) : [e] "+&v"(s[0]) : [v] "v"(v), [x0] "v"(x[K]), [l0] "n"(K));
   }
 }
 template <int N>
@@ -181,6 +183,12 @@ __device__ __forceinline__ void unroll_down(F&& f) {
     unroll_down<I - 1, N>(f);
   }
 }
+
+// x is formed here (not recomputed from its operands where it is used, which would hold all of them)
+__device__ __forceinline__ void keep(double& x) { asm volatile("" : "+v"(x)); }
+
+// End of a phase: later loads are not moved above it (they would hold registers through the phase).
+__device__ __forceinline__ void phase() { asm volatile("" ::: "memory"); }
 
 // ------------------------------------------------------------- products
 // y[c] += sum_k x[k] (row k of B)[c] over the columns c < min(N, k + LOW) of row k (LOW = 1: B lower
@@ -269,6 +277,38 @@ __device__ __forceinline__ void lq1(double (&a)[B1], double* b, int r) {
   });
 }
 
+// The remaining pivots of a square factor whose rows r < D have N <= D columns that may be nonzero
+// (the rest zero): a zero column after a zero tail is left as it is.
+template <int D, int N>
+__device__ __forceinline__ void lq_rows(double (&a)[D], int r) {
+  unroll<0, N - 1>([&](auto ic) {
+    constexpr int i = decltype(ic)::value;
+    constexpr int n = N - 1 - i;
+    double s[2] = {0.0, 0.0};
+    dot_rows<i, n, i + 1>(s, a, a);
+    const double dot = s[0] + s[1];
+    const Pivot p = pivot(bcast<i>(a[i]), bcast<i>(dot));
+    const double tws = p.rb * fma(p.sc, dot, a[i]);
+    a[i] = (r == i) ? p.beta : fma(-p.den, tws, a[i]);
+    fma_self<i, n>(a + i + 1, -tws);
+  });
+}
+// LQ of a matrix of NR rows (lanes 0 .. NR - 1) and N > NR columns
+template <int NR, int N>
+__device__ __forceinline__ void lq_top(double (&a)[N], int r) {
+  unroll<0, NR>([&](auto ic) {
+    constexpr int i = decltype(ic)::value;
+    constexpr int n = N - 1 - i;
+    double s[2] = {0.0, 0.0};
+    dot_rows<i, n, i + 1>(s, a, a);
+    const double dot = s[0] + s[1];
+    const Pivot p = pivot(bcast<i>(a[i]), bcast<i>(dot));
+    const double tws = p.rb * fma(p.sc, dot, a[i]);
+    a[i] = (r == i) ? p.beta : fma(-p.den, tws, a[i]);
+    fma_self<i, n>(a + i + 1, -tws);
+  });
+}
+
 // ------------------------------------------------------------- memory
 // Row of N contiguous doubles (16-byte accesses where every row of an N-column matrix is aligned)
 template <int N>
@@ -313,7 +353,7 @@ __device__ __forceinline__ void store_lower16(double* p, double (&x)[N], int r) 
 // pof/parallel_filtsmooth/filter.py:117-142, as filter_combine() of pof_core.hpp: e = e1 o e2, e1
 // earlier.  SO (state only): e1 is a prefix state (s1.m, s1.L) and (so.m, so.L) receives the result.
 //
-// DZ: nonzero columns of the elements' Z: d at a leaf level ([Zr | 0]), D above it (lower
+// DZ: columns of the elements' Z: d at a leaf level ([Zr | 0] stored as Zr), D above it (lower
 // triangular).  Columns of zeros are left out of every sum and update (they add exact zeros); at a
 // leaf level this leaves pivot i of the Xi factorisation max(d - 1 - i, 0) + i tail columns instead
 // of D - 1 in each of its four passes.
@@ -345,14 +385,20 @@ __device__ __forceinline__ void filter_combine(int r, const FiltArrays& x1, cons
       load_col16<D>(u1t, U1, rr);
       if constexpr (kLeaf) {
 #pragma unroll
-        for (int c = 0; c < DZ; ++c) z2[c] = Z2[rr * D + c];
+        for (int c = 0; c < DZ; ++c) z2[c] = Z2[rr * DZ + c];
       } else {
         load_row16<D>(z2, Z2 + rr * D);
       }
       if constexpr (!SO) {
         // s2 = eta2 - Z2 (Z2^T b1), uu = U1^T s2
         double z2t[D];
-        load_col16<D>(z2t, Z2, rr);
+        if constexpr (kLeaf) {
+          const int rz = (r < DZ) ? r : 0;  // lanes past the last column hold no entry of Z2^T b1
+#pragma unroll
+          for (int k = 0; k < D; ++k) z2t[k] = Z2[k * DZ + rz];
+        } else {
+          load_col16<D>(z2t, Z2, rr);
+        }
         const double t = dot_lanes<D>(z2t, b1r);
         s2 = eta2r - dot_lanes<DZ>(z2, t);
         uu = dot_lanes<D>(u1t, s2);
@@ -385,6 +431,7 @@ __device__ __forceinline__ void filter_combine(int r, const FiltArrays& x1, cons
         a1[i] = fma(-p.den, ta, a1[i]);
         b1[i] = fma(-p.den, tb, b1[i]);
         rd = (r == i) ? -p.rb : rd;
+        keep(rd);
       } else {
         // column i of the first block is zero: alpha = 0, den = norm, beta = -norm
         double n, rn;
@@ -395,6 +442,7 @@ __device__ __forceinline__ void filter_combine(int r, const FiltArrays& x1, cons
         a1[i] = -wa;
         b1[i] = -wb;
         rd = (r == i) ? -rn : rd;
+        keep(rd);
       }
       fma_rows<i, n1>(b1 + i + 1, a1 + i + 1, -tb);
       fma_rows<i, i>(b2, a2, -tb);
@@ -465,7 +513,7 @@ __device__ __forceinline__ void filter_combine(int r, const FiltArrays& x1, cons
       const double* Z1 = x1.Z + i1 * DD;
       if constexpr (kLeaf) {
 #pragma unroll
-        for (int c = 0; c < DZ; ++c) z1[c] = Z1[rr * D + c];
+        for (int c = 0; c < DZ; ++c) z1[c] = Z1[rr * DZ + c];
       } else {
         load_row16<DZ>(z1, Z1 + rr * D);
       }
@@ -482,6 +530,401 @@ __device__ __forceinline__ void filter_combine(int r, const FiltArrays& x1, cons
   if (act) {
     (SO ? so.m : y.b)[o * D + r] = bo;
     store_lower16<D>((SO ? so.L : y.U) + (o * D + r) * D, mt, r);
+  }
+}
+
+// ------------------------------------------------------------- observation model
+// Affine observation y = H x + c of one element, noise factor R (zero for EK1).  EK1 (Obs of
+// pof_core.hpp): row i of H is hc[i][l] at the columns l q1 and hd[i] at column i q1 + 1, the same
+// in every lane.  Otherwise lane i < d holds row i of the caller's H and R.
+template <int D, int d, bool EK1>
+struct ObsRow;
+
+template <int D, int d>
+struct ObsRow<D, d, true> {
+  static constexpr int q1 = D / d;
+  static constexpr int NR = 0;  // noise columns
+  Obs<D, d, true> o;
+  double c[d];
+  // (the parameters are read where they are: a local copy indexed by the field's cases would go through scratch)
+  __device__ __forceinline__ void load(const GroupArgs& g, int j, int k, int) {
+    const double* lin = (g.cur[j] ? g.means1 : g.means0) + (size_t)g.base[j] * D;
+    o.load_at(g.kind[j], g.params + (size_t)j * kMaxParams, g.Pd + (size_t)j * D, lin + (size_t)(k + 1) * D);
+#pragma unroll
+    for (int i = 0; i < d; ++i) c[i] = o.c[i];
+  }
+  __device__ __forceinline__ double r_at(int) const { return 0.0; }
+  // out[c] += (H M)[r][c] for r < d, M's row j (columns < j + LOW) in lane j
+  template <int LOW>
+  __device__ __forceinline__ void times_rows(int r, const double (&M)[D], double (&out)[D]) const {
+    unroll<0, d>([&](auto lc) {
+      constexpr int l = decltype(lc)::value;
+      double h = o.hc[0][l];
+#pragma unroll
+      for (int i = 1; i < d; ++i) h = (r == i) ? o.hc[i][l] : h;
+      constexpr int n = (l * q1 + LOW < D) ? l * q1 + LOW : D;
+      fma_rows<l * q1, n>(out, M, h);
+    });
+    unroll<0, d>([&](auto ic) {
+      constexpr int i = decltype(ic)::value;
+      constexpr int n = (i * q1 + 1 + LOW < D) ? i * q1 + 1 + LOW : D;
+      fma_rows<i * q1 + 1, n>(out, M, (r == i) ? o.hd[i] : 0.0);
+    });
+  }
+  // y[i] = c_i + (H v)_i, v's entry j in lane j
+  __device__ __forceinline__ void predict(double v, double (&y)[d]) const {
+    double p[d], n[d];
+    unroll<0, d>([&](auto lc) {
+      constexpr int l = decltype(lc)::value;
+      p[l] = bcast<l * q1>(v);
+      n[l] = bcast<l * q1 + 1>(v);
+    });
+#pragma unroll
+    for (int i = 0; i < d; ++i) {
+      double h = o.hc[i][0] * p[0];
+#pragma unroll
+      for (int l = 1; l < d; ++l) h = fma(o.hc[i][l], p[l], h);
+      y[i] = c[i] + fma(o.hd[i], n[i], h);
+    }
+  }
+  // y[i] = (H F)[i][r]
+  __device__ __forceinline__ void times_col(const double* F, int r, double (&y)[d]) const {
+    double p[d];
+#pragma unroll
+    for (int l = 0; l < d; ++l) p[l] = F[(l * q1) * D + r];
+#pragma unroll
+    for (int i = 0; i < d; ++i) {
+      double h = o.hc[i][0] * p[0];
+#pragma unroll
+      for (int l = 1; l < d; ++l) h = fma(o.hc[i][l], p[l], h);
+      y[i] = fma(o.hd[i], F[(i * q1 + 1) * D + r], h);
+    }
+  }
+  // x[c] -= (K H M)[c] for the lane's row K of a gain
+  __device__ __forceinline__ void sub_gain(const double (&K)[d], const double (&M)[D], double (&x)[D]) const {
+    unroll<0, d>([&](auto lc) {
+      constexpr int l = decltype(lc)::value;
+      double h = 0.0;
+#pragma unroll
+      for (int i = 0; i < d; ++i) h = fma(K[i], o.hc[i][l], h);
+      fma_rows<l * q1, D>(x, M, -h);
+    });
+    unroll<0, d>([&](auto ic) {
+      constexpr int i = decltype(ic)::value;
+      fma_rows<i * q1 + 1, D>(x, M, -(K[i] * o.hd[i]));
+    });
+  }
+};
+
+template <int D, int d>
+struct ObsRow<D, d, false> {
+  static constexpr int NR = d;
+  double h[D], R[d], c[d];
+  __device__ __forceinline__ void load(const GroupArgs& g, int, int k, int r) {
+    const int i = (r < d) ? r : 0;
+    const double* H = g.Hx + ((size_t)k * d + i) * D;
+#pragma unroll
+    for (int j = 0; j < D; ++j) h[j] = (r < d) ? H[j] : 0.0;
+#pragma unroll
+    for (int j = 0; j < d; ++j) R[j] = (g.Rx && r < d) ? g.Rx[((size_t)k * d + i) * d + j] : 0.0;
+#pragma unroll
+    for (int j = 0; j < d; ++j) c[j] = g.cx[(size_t)k * d + j];
+  }
+  __device__ __forceinline__ double r_at(int j) const { return R[j]; }
+  template <int LOW>
+  __device__ __forceinline__ void times_rows(int, const double (&M)[D], double (&out)[D]) const {
+    mul_rows<D, D, LOW>(out, h, M);
+  }
+  __device__ __forceinline__ void predict(double v, double (&y)[d]) const {
+    const double s = dot_lanes<D>(h, v);
+    unroll<0, d>([&](auto ic) { y[decltype(ic)::value] = c[decltype(ic)::value] + bcast<decltype(ic)::value>(s); });
+  }
+  __device__ __forceinline__ void times_col(const double* F, int r, double (&y)[d]) const {
+    double f[D];
+    load_col16<D>(f, F, r);
+    unroll<0, d>([&](auto ic) {
+      double s[2] = {0.0, 0.0};
+      dot_rows<decltype(ic)::value, D>(s, h, f);
+      y[decltype(ic)::value] = s[0] + s[1];
+    });
+  }
+  __device__ __forceinline__ void sub_gain(const double (&K)[d], const double (&M)[D], double (&x)[D]) const {
+    double kh[D];
+    zero(kh);
+    unroll<0, d>([&](auto ic) { fma_rows<decltype(ic)::value, D>(kh, h, -K[decltype(ic)::value]); });
+    mul_rows<D, D, D>(x, kh, M);
+  }
+};
+
+// A d x d lower triangular factor held by lanes 0 .. d - 1 (row i in lane i), the same in every lane
+// of the row: entries and reciprocal diagonal.
+template <int d>
+struct Small {
+  double l[d][d], rd[d];
+  template <int N>
+  __device__ __forceinline__ void load(const double (&rows)[N]) {
+    unroll<0, d>([&](auto ic) {
+      constexpr int i = decltype(ic)::value;
+      unroll<0, i + 1>([&](auto jc) { l[i][decltype(jc)::value] = bcast<i>(rows[decltype(jc)::value]); });
+      rd[i] = 1.0 / l[i][i];
+    });
+  }
+  // x = L^-1 x
+  __device__ __forceinline__ void solve(double (&x)[d]) const {
+#pragma unroll
+    for (int j = 0; j < d; ++j) {
+#pragma unroll
+      for (int i = 0; i < j; ++i) x[j] = fma(-x[i], l[j][i], x[j]);
+      x[j] *= rd[j];
+    }
+  }
+  // x = L^-T x (the row vector x L^-1)
+  __device__ __forceinline__ void solve_t(double (&x)[d]) const {
+#pragma unroll
+    for (int j = d - 1; j >= 0; --j) {
+#pragma unroll
+      for (int i = j + 1; i < d; ++i) x[j] = fma(-x[i], l[i][j], x[j]);
+      x[j] *= rd[j];
+    }
+  }
+};
+
+// ------------------------------------------------------------- filter element
+// _get_element (pof/parallel_filtsmooth/filter.py:50-81) for element k, as filter_element() of
+// pof_core.hpp; element 0 carries the prior (x0m, x0L), the others a zero one.  The element's
+// Z = [Zr | 0] is stored as its d columns alone, rows packed ([D, d] at the element's place).
+//
+// Psi = tria([[H N1, R], [N1, 0]]): the d rows of the first block row in t, the D rows of the second
+// in n.  The first d pivots leave Psi11 (t) and Psi21 (n's first d columns), the rest U = Psi22.
+// Without noise the last d columns are zero throughout and are left out.
+template <int D, int d, bool EK1>
+__device__ __forceinline__ void filter_element(int r, const GroupArgs& g, int j, int k, const FiltArrays& out) {
+  using O = ObsRow<D, d, EK1>;
+  constexpr int NR = O::NR, NC = D + NR;
+  constexpr size_t DD = (size_t)D * D;
+  const bool act = r < D;
+  const int rr = act ? r : 0;
+  O ob;
+  ob.load(g, j, k, r);
+  double f[D];
+  load_row16<D>(f, g.F + rr * D);
+  double n[NC];
+  double m1 = 0.0;
+  {
+    double n1[D];
+    load_row16<D>(n1, g.N1z + rr * D);
+    if (k == 0) {
+      m1 = dot_lanes<D>(f, g.x0m[(size_t)j * D + rr]);
+      double l0[D];
+      load_row16<D>(l0, g.x0L + (size_t)j * DD + rr * D);
+      bool nz = false;
+#pragma unroll
+      for (int c = 0; c < D; ++c) nz = nz || l0[c] != 0.0;
+      // N1 = tria([F L0 | LQ]); of a zero L0 it is N1z
+      if ((__ballot(nz) >> ((threadIdx.x & 63) & ~(kRow - 1))) & 0xffffull) {
+        double lq[D];
+        load_row16<D>(lq, g.LQ + rr * D);
+        zero(n1);
+        mul_rows<D, D, D>(n1, f, l0);
+        lq1<D, D, D, D>(n1, lq, r);
+#pragma unroll
+        for (int c = 1; c < D; ++c) n1[c] = (c > r) ? 0.0 : n1[c];
+      }
+    }
+#pragma unroll
+    for (int c = 0; c < D; ++c) n[c] = n1[c];
+  }
+#pragma unroll
+  for (int c = D; c < NC; ++c) n[c] = 0.0;
+  double t[NC];
+  {
+    double hn[D];
+    zero(hn);
+    double n1[D];
+#pragma unroll
+    for (int c = 0; c < D; ++c) n1[c] = n[c];
+    ob.template times_rows<1>(r, n1, hn);
+#pragma unroll
+    for (int c = 0; c < D; ++c) t[c] = hn[c];
+  }
+#pragma unroll
+  for (int c = D; c < NC; ++c) t[c] = ob.r_at(c - D);
+  unroll<0, d>([&](auto ic) {
+    constexpr int i = decltype(ic)::value;
+    constexpr int nt = NC - 1 - i;
+    double st[2] = {0.0, 0.0}, sn[2] = {0.0, 0.0};
+    dot_rows<i, nt, i + 1>(st, t, t);
+    dot_rows<i, nt, i + 1>(sn, t, n);
+    const double dt = st[0] + st[1], dn = sn[0] + sn[1];
+    const Pivot p = pivot(bcast<i>(t[i]), bcast<i>(dt));
+    const double tt = p.rb * fma(p.sc, dt, t[i]), tn = p.rb * fma(p.sc, dn, n[i]);
+    t[i] = (r == i) ? p.beta : fma(-p.den, tt, t[i]);
+    n[i] = fma(-p.den, tn, n[i]);
+    fma_rows<i, nt>(n + i + 1, t + i + 1, -tn);
+    fma_self<i, nt>(t + i + 1, -tt);
+  });
+  Small<d> p11;
+  p11.load(t);
+  // gain K = Psi21 Psi11^-1; A = F - K H F, b = m1 - K (H m1 + c)
+  double K[d];
+#pragma unroll
+  for (int i = 0; i < d; ++i) K[i] = n[i];
+  p11.solve_t(K);
+  const size_t o = (size_t)k * D + rr;
+  {
+    double A[D];
+#pragma unroll
+    for (int c = 0; c < D; ++c) A[c] = f[c];
+    ob.sub_gain(K, f, A);
+    if (act) store_row16<D>(out.A + o * D, A);
+  }
+  {
+    double y[d];
+    ob.predict(m1, y);  // m1 = 0 without a prior
+    double b = m1;
+#pragma unroll
+    for (int i = 0; i < d; ++i) b = fma(-K[i], y[i], b);
+    // Z row = (Psi11^-1 (H F)[:, r])^T, eta = -Z Psi11^-1 c
+    double z[d], w[d];
+    ob.times_col(g.F, rr, z);
+    p11.solve(z);
+#pragma unroll
+    for (int i = 0; i < d; ++i) w[i] = ob.c[i];
+    p11.solve(w);
+    double e = 0.0;
+#pragma unroll
+    for (int i = 0; i < d; ++i) e = fma(-z[i], w[i], e);
+    if (act) {
+      out.b[o] = b;
+      out.eta[o] = e;
+#pragma unroll
+      for (int i = 0; i < d; ++i) out.Z[(size_t)k * DD + r * d + i] = z[i];
+    }
+  }
+  // U = Psi22: the remaining pivots, rows of n in the columns from d on (NR < d: the last columns zero)
+  {
+    double u[D];
+#pragma unroll
+    for (int c = 0; c < D; ++c) u[c] = (d + c < NC) ? n[(d + c < NC) ? d + c : 0] : 0.0;
+    lq_rows<D, NC - d>(u, r);
+    if (act) store_lower16<D>(out.U + o * D, u, r);
+  }
+}
+
+// ------------------------------------------------------------- smoother element, statistics
+// Smoother element of filtered state (m, L) (pof/parallel_filtsmooth/smoother.py:37-50) and, with
+// OBS, the predicted observation's statistics (filter.py:84-114): see k_filter_post.
+//   Phi = tria([[F L, LQ], [L, 0]]), E = Phi21 Phi11^-1, g = m - E F m, D = Phi22,
+//   S = tria([H Phi11 | R]), yhat = H F m + c.
+// LOWL: L and LQ are lower triangular with LQ's diagonal nonzero (the solver's own model).
+// The observation model is read once the smoother element is stored, so that its values are not held
+// in registers through the factorisation.
+template <int D, int d, bool EK1>
+__device__ __forceinline__ void filter_post(int r, const GroupArgs& g, int j, int s, const double* mp, const double* Lp,
+                                            bool obs, bool dm_only, bool wc, const SmoArrays& sel, size_t ro,
+                                            double* t_ssq, double* t_nll) {
+  using O = ObsRow<D, d, EK1>;
+  constexpr int NR = O::NR;
+  const bool act = r < D;
+  const int rr = act ? r : 0;
+  double a1[D], b1[D], b2[D], fm, mr, rd = 0.0;
+  {
+    double a2[D], f[D];
+    mr = mp[rr];
+    load_row16<D>(b1, Lp + rr * D);
+    load_row16<D>(f, g.F + rr * D);
+    load_row16<D>(a2, g.LQ + rr * D);
+    fm = dot_lanes<D>(f, mr);
+    zero(a1);
+    mul_rows<D, D, EK1 ? 1 : D>(a1, f, b1);
+    zero(b2);
+    unroll<0, D>([&](auto ic) {
+      constexpr int i = decltype(ic)::value;
+      constexpr int n1 = D - 1 - i, n2 = EK1 ? i + 1 : D;
+      double sa[2] = {0.0, 0.0}, sb[2] = {0.0, 0.0};
+      dot_rows<i, n1, i + 1>(sa, a1, a1);
+      dot_rows<i, n1, i + 1>(sb, a1, b1);
+      dot_rows<i, n2, 0>(sa, a2, a2);
+      dot_rows<i, (EK1 ? i : D), 0>(sb, a2, b2);
+      const double da = sa[0] + sa[1], db = sb[0] + sb[1];
+      const double alpha = bcast<i>(a1[i]), sig = bcast<i>(da);
+      const Pivot p = EK1 ? pivot_nz(alpha, sig) : pivot(alpha, sig);
+      const double ta = p.rb * fma(p.sc, da, a1[i]), tb = p.rb * fma(p.sc, db, b1[i]);
+      a1[i] = (r == i) ? p.beta : fma(-p.den, ta, a1[i]);
+      b1[i] = fma(-p.den, tb, b1[i]);
+      const double rp = EK1 ? -p.rb : 1.0 / p.beta;
+      rd = (r == i) ? rp : rd;
+      keep(rd);
+      keep(a1[i]);
+      keep(b1[i]);
+      fma_rows<i, n1>(b1 + i + 1, a1 + i + 1, -tb);
+      fma_rows<i, n2>(b2, a2, -tb);
+      fma_self<i, n1>(a1 + i + 1, -ta);
+      fma_self<i, n2>(a2, -ta);
+    });
+  }
+  phase();
+  if (wc) {
+    lq1<D, D, 0, 0>(b2, nullptr, r);
+    if (act) store_lower16<D>(sel.Dm + (ro * D + r) * D, b2, r);
+  }
+  if (dm_only) return;
+  // E = Phi21 Phi11^-1
+  unroll_down<D - 1, 0>([&](auto jc) {
+    constexpr int j = decltype(jc)::value;
+    b1[j] = b1[j] * bcast<j>(rd);
+    fma_rows<j, j>(b1, a1, -b1[j]);
+  });
+  const double gr = mr - dot_lanes<D>(b1, fm);
+  if (act) {
+    store_row16<D>(sel.E + (ro * D + r) * D, b1);
+    sel.g[ro * D + r] = gr;
+  }
+  if (!obs) {
+    if (r == 0) {
+      t_ssq[s] = 0.0;
+      t_nll[s] = 0.0;
+    }
+    return;
+  }
+  phase();
+  O ob;
+  ob.load(g, j, s, r);
+  double sr[D + NR];
+  {
+    double h[D];
+    zero(h);
+    ob.template times_rows<1>(r, a1, h);
+#pragma unroll
+    for (int c = 0; c < D; ++c) sr[c] = h[c];
+#pragma unroll
+    for (int c = D; c < D + NR; ++c) sr[c] = ob.r_at(c - D);
+  }
+  lq_top<d, D + NR>(sr, r);
+  Small<d> S;
+  S.load(sr);
+  double yh[d], w[d];
+  ob.predict(fm, yh);
+#pragma unroll
+  for (int i = 0; i < d; ++i) w[i] = yh[i];
+  S.solve_t(w);   // S^T w = yhat
+  S.solve(yh);    // S y = yhat
+  // lane i < d takes the logarithm of its own diagonal entry
+  double di = S.l[0][0];
+#pragma unroll
+  for (int i = 1; i < d; ++i) di = (r == i) ? S.l[i][i] : di;
+  const double lg = log(fabs(di));
+  double ss = 0.0, nn = 0.0, ld = 0.0;
+  unroll<0, d>([&](auto ic) {
+    constexpr int i = decltype(ic)::value;
+    ss = fma(w[i], w[i], ss);
+    nn = fma(yh[i], yh[i], nn);
+    ld += bcast<i>(lg);
+  });
+  if (r == 0) {
+    t_ssq[s] = ss;
+    // -loglik = 0.5 |S^-1 y|^2 + sum log|S_ii| + d log(2 pi) / 2
+    t_nll[s] = 0.5 * nn + (ld + d * log(2.0 * M_PI) / 2.0);
   }
 }
 
