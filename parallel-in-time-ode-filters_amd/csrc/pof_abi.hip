@@ -755,6 +755,8 @@ void range_free(pof_batch* b, long long start, long long len) {
 // Append the launch tables of IVP slots `ids` to h; offsets in p are relative
 // to `at` (the tables' position in the device buffer is set after upload).
 int plan_tables(pof_batch* b, const std::vector<int>& ids, std::vector<int>& h, LaunchPlan& p) {
+  const auto tu = b->ctx->tuning.find(b->D);
+  const Tuning tune = (tu != b->ctx->tuning.end()) ? tu->second : Tuning{};
   const int at = (int)h.size();
   const int m = (int)ids.size();
   h.insert(h.end(), ids.begin(), ids.end());
@@ -786,14 +788,49 @@ int plan_tables(pof_batch* b, const std::vector<int>& ids, std::vector<int>& h, 
   table([](long long N) { return N - 1; }, p.leaf1_off, p.leaf1_total, nullptr);
   table([](long long N) { return N + 1; }, p.pts_off, p.pts_total, nullptr);
   table([](long long N) { return (N + 1 + kChunk - 1) / kChunk; }, p.chunk_off, p.chunk_total, nullptr);
-  for (int l = 0; l + 1 < p.fl; ++l)
-    table([l](long long N) { return N >> (l + 1); }, p.fup_off[l], p.fup_total[l], nullptr);
-  for (int l = 0; l < p.fl; ++l)
-    table([l](long long N) { return ((N >> l) + 1) / 2; }, p.fdn_off[l], p.fdn_total[l], &p.fdn_ivps[l]);
-  for (int l = 0; l + 1 < p.sl; ++l)
-    table([l](long long N) { return (N + 1) >> (l + 1); }, p.sup_off[l], p.sup_total[l], nullptr);
-  for (int l = 0; l < p.sl; ++l)
-    table([l](long long N) { return (((N + 1) >> l) + 1) / 2; }, p.sdn_off[l], p.sdn_total[l], &p.sdn_ivps[l]);
+  // combines of a level: n0 >> (l + 1) on the way up, ((n0 >> l) + 1) / 2 pairs on the way down (the pairs
+  // with 2 i = 0 combine nothing), n0 = Ns for the filter and Ns + 1 for the smoother
+  auto up_count = [](long long n0, int l) { return n0 >> (l + 1); };
+  auto down_count = [](long long n0, int l) { return ((n0 >> l) + 1) / 2; };
+  if (b->D <= 16) {
+    // stages: a level as wide as the sweep's width alone, and the filter's level 0 (whose elements' Z has
+    // fewer columns); narrower ones together
+    auto stages = [&](auto count, int n1, int levels, int width, bool down, Stage* st, int& ns) {
+      ns = 0;
+      for (int l = 0; l < levels;) {
+        Stage& g = st[ns++];
+        auto total = [&](int lv) {
+          long long c = 0;
+          for (int id : ids) c += count((long long)b->hNs[id] + n1, lv);
+          return c;
+        };
+        g.l0 = l;
+        g.nlev = (total(l) >= width || (n1 == 0 && l == 0)) ? 1 : std::min(kStageLevels, levels - l);
+        table([&](long long N) { return (count(N + n1, l) + kStageWorkers - 1) / kStageWorkers; }, g.off, g.blocks,
+              nullptr);
+        g.work = 0;
+        for (int t = 0; t < g.nlev; ++t) g.work += total(l + t);
+        if (down)
+          for (int t = 0; t < g.nlev; ++t)
+            for (int id : ids) g.work -= (((long long)b->hNs[id] + n1) >> (l + t)) > 0 ? 1 : 0;
+        l += g.nlev;
+      }
+      if (down) std::reverse(st, st + ns);
+    };
+    stages(up_count, 0, p.fl - 1, tune.filter_up, false, p.fup, p.n_fup);
+    stages(down_count, 0, p.fl, tune.filter_down, true, p.fdn, p.n_fdn);
+    stages(up_count, 1, p.sl - 1, tune.smooth_up, false, p.sup, p.n_sup);
+    stages(down_count, 1, p.sl, tune.smooth_down, true, p.sdn, p.n_sdn);
+  } else {
+    for (int l = 0; l + 1 < p.fl; ++l)
+      table([&](long long N) { return up_count(N, l); }, p.fup_off[l], p.fup_total[l], nullptr);
+    for (int l = 0; l < p.fl; ++l)
+      table([&](long long N) { return down_count(N, l); }, p.fdn_off[l], p.fdn_total[l], &p.fdn_ivps[l]);
+    for (int l = 0; l + 1 < p.sl; ++l)
+      table([&](long long N) { return up_count(N + 1, l); }, p.sup_off[l], p.sup_total[l], nullptr);
+    for (int l = 0; l < p.sl; ++l)
+      table([&](long long N) { return down_count(N + 1, l); }, p.sdn_off[l], p.sdn_total[l], &p.sdn_ivps[l]);
+  }
   return overflow ? POF_E_ARG : POF_OK;
 }
 
@@ -941,8 +978,6 @@ int batch_launch(pof_batch* b) {
     b->hmaps.clear();
     int rc = plan_tables(b, b->active, b->hmaps, b->plan);
     if (rc != POF_OK) return set_err(ctx, rc, "launch tables overflow");
-    const auto tu = ctx->tuning.find(b->D);
-    if (tu != ctx->tuning.end()) b->plan.tune = tu->second;
     b->tune_version = ctx->tune_version;
     if (b->hmaps.size() > b->maps_cap) {
       HIP_TRY(hipStreamSynchronize(b->st));

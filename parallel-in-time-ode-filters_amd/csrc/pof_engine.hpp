@@ -35,21 +35,32 @@ struct KernelTimer {
   bool ready = false;
 };
 
-// Scan-level widths (work items per launch) from which each scan kernel runs
-// in its throughput form (one lane per matrix row, several combines per
-// wavefront) instead of its latency form (rows split over several lanes).
-// Only state dimensions whose latency form splits rows (D <= 16) have both.
+// Scan-level widths (combines per level, summed over the batch's IVPs) from which a scan level of a
+// state dimension D <= 16 is a launch of its own; narrower levels, bound by the latency of one
+// combine, share launches of up to kStageLevels levels.  The default is one wavefront of four
+// combines on each of the chip's 1,024 SIMDs.
 struct Tuning {
-  int filter_up = 1 << 30;
-  int filter_down = 1 << 30;
-  int smooth_up = 1 << 30;
-  int smooth_down = 1 << 30;
+  int filter_up = 4096;
+  int filter_down = 4096;
+  int smooth_up = 4096;
+  int smooth_down = 4096;
+};
+
+// A launch of a scan with one row per lane (D <= 16): nlev consecutive levels from l0 (the one with
+// the most entries), in blocks of kStageWorkers workers.  Block b of an IVP owns the combines
+// [b c, (b + 1) c) of each level, c = kStageWorkers >> (level - l0): in the up-sweep their inputs, in the
+// down-sweep their prefixes, are the block's own (but for one prefix, that of everything before the block).
+constexpr int kStageWorkers = 16;
+constexpr int kStageLevels = 5;  // kStageWorkers >> (kStageLevels - 1) = 1
+struct Stage {
+  int l0 = 0, nlev = 0;
+  int off = 0, blocks = 0;  // table of blocks per IVP
+  long long work = 0;       // combines
 };
 
 // Launch maps of one active set of a group (host view of a device int buffer):
 // the active IVP ids, then one prefix table per launch kind and level.
 struct LaunchPlan {
-  Tuning tune;
   const int* dev = nullptr;  // device buffer
   int m = 0;                 // active IVPs
   int fl = 0, sl = 0;        // filter / smoother levels (maximum over the active IVPs)
@@ -58,6 +69,10 @@ struct LaunchPlan {
   int leaf1_off = 0, leaf1_total = 0;  // Ns - 1 (the other elements)
   int pts_off = 0, pts_total = 0;      // Ns + 1
   int chunk_off = 0, chunk_total = 0;  // ceil((Ns + 1) / kChunk)
+  // D <= 16: the stages of the four sweeps, in launch order
+  int n_fup = 0, n_fdn = 0, n_sup = 0, n_sdn = 0;
+  Stage fup[kMaxLevels], fdn[kMaxLevels], sup[kMaxLevels], sdn[kMaxLevels];
+  // D > 16: a table per level
   int fup_off[kMaxLevels] = {}, fup_total[kMaxLevels] = {};  // Ns >> (l + 1)
   int fdn_off[kMaxLevels] = {}, fdn_total[kMaxLevels] = {};  // ((Ns >> l) + 1) / 2
   int sup_off[kMaxLevels] = {}, sup_total[kMaxLevels] = {};  // (Ns + 1) >> (l + 1)

@@ -176,47 +176,75 @@ __global__ __launch_bounds__((Geo<D, kLdsState>::BLOCK)) void k_filter_down(Grou
   }
 }
 
-// The same two sweeps with one row per lane (pof_row16.hpp), D <= 16.  DZ: nonzero columns of the
-// level's elements' Z (d at level 0, D above).
-template <int D, int DZ>
-__global__ __launch_bounds__(r16::kBlock, 2) void k_filter_up16(GroupArgs g, LaunchMap lm, int l) {
-  int j, i;
-  if (!locate(lm, blockIdx.x * r16::kPerBlock + threadIdx.x / r16::kRow, j, i)) return;
-  const long long N = g.Ns[j], base = g.base[j];
-  const FiltArrays in = at(g.fel, base + lev_off(N, l), D);
-  const FiltArrays out = at(g.fel, base + lev_off(N, l + 1), D);
-  StateArrays none{};
-  r16::filter_combine<D, DZ, false>(threadIdx.x % r16::kRow, in, none, 2 * (size_t)i, in, 2 * (size_t)i + 1, out, none,
-                                    (size_t)i);
-}
+// The same two sweeps with one row per lane (pof_row16.hpp), D <= 16, a stage of levels per launch:
+// block b of an IVP takes the combines [b c, (b + 1) c) of level l0 + t, c = 16 >> t, whose inputs it
+// formed itself one level before.  Worker w of a block is DPP row w / 4 of wavefront w % 4, so that
+// up to four combines of a level run on a SIMD each.  A launch costs 1.6 us replayed from a graph
+// and its first wavefronts start cold; at D = 3 a level's combine takes about as long.
+// DZ: columns of the elements' Z: d at level 0, which is a stage of its own (with a second combine for the
+// levels above, the kernel's registers would spill at D = 15 and 16), D above.
+__device__ __forceinline__ int stage_worker() { return ((threadIdx.x & 63) >> 4) * 4 + (threadIdx.x >> 6); }
 
 template <int D, int DZ>
-__global__ __launch_bounds__(r16::kBlock, 2) void k_filter_down16(GroupArgs g, LaunchMap lm, int l) {
-  int j, i;
-  if (!locate(lm, blockIdx.x * r16::kPerBlock + threadIdx.x / r16::kRow, j, i)) return;
-  const long long N = g.Ns[j], base = g.base[j];
-  const int n = (int)(N >> l);
-  const FiltArrays el = at(g.fel, base + lev_off(N, l), D);
-  const StateArrays p = at(g.fpre, base + lev_off(N, l), D);
-  const StateArrays up = (l + 1 < n_levels(N)) ? at(g.fpre, base + lev_off(N, l + 1), D) : StateArrays{};
-  const int r = threadIdx.x % r16::kRow;
-  const int j0 = 2 * i, j1 = j0 + 1;
-  if (j1 < n && r < D) {
-    double u[D];
-    r16::load_row16<D>(u, up.L + ((size_t)i * D + r) * D);
-    r16::store_row16<D>(p.L + ((size_t)j1 * D + r) * D, u);
-    p.m[(size_t)j1 * D + r] = up.m[(size_t)i * D + r];
-  }
-  if (j0 == 0) {
-    if (r < D) {
-      double u[D];
-      r16::load_row16<D>(u, el.U + r * D);
-      r16::store_row16<D>(p.L + r * D, u);
-      p.m[r] = el.b[r];
+__global__ __launch_bounds__(r16::kStageBlock, 2) void k_filter_up16(GroupArgs g, LaunchMap lm, int l0, int nlev) {
+  if constexpr (DZ != D) l0 = 0, nlev = 1;
+  int j, b;
+  if (!locate(lm, blockIdx.x, j, b)) return;
+  const long long N = g.Ns[j];
+  const int r = threadIdx.x % r16::kRow, w = stage_worker();
+  long long off = g.base[j] + lev_off(N, l0);
+  StateArrays none{};
+  for (int t = 0; t < nlev; ++t) {
+    const int c = kStageWorkers >> t;
+    const long long i = (long long)b * c + w, next = off + (N >> (l0 + t));
+    if (w < c && i < N >> (l0 + t + 1)) {
+      const FiltArrays in = at(g.fel, off, D), out = at(g.fel, next, D);
+      r16::filter_combine<D, DZ, false>(r, in, none, 2 * (size_t)i, in, 2 * (size_t)i + 1, out, none, (size_t)i);
     }
-  } else {
-    FiltArrays none{};
-    r16::filter_combine<D, DZ, true>(r, none, up, (size_t)i - 1, el, (size_t)j0, none, p, (size_t)j0);
+    off = next;
+    if (t + 1 < nlev) __syncthreads();
+  }
+}
+
+// Pair i of level l: p[2i + 1] = up[i], p[2i] = up[i - 1] o e[2i] (p[0] = e[0]'s state).  up[i - 1] of a
+// block's first pair belongs to the block before, which copies it down from the stage's top level:
+// it is read there.
+template <int D, int DZ>
+__global__ __launch_bounds__(r16::kStageBlock, 2) void k_filter_down16(GroupArgs g, LaunchMap lm, int l0, int nlev) {
+  if constexpr (DZ != D) l0 = 0, nlev = 1;
+  int j, b;
+  if (!locate(lm, blockIdx.x, j, b)) return;
+  const long long N = g.Ns[j], base = g.base[j];
+  const int r = threadIdx.x % r16::kRow, w = stage_worker();
+  for (int t = nlev - 1; t >= 0; --t) {
+    const int l = l0 + t, c = kStageWorkers >> t;
+    const long long i = (long long)b * c + w, n = N >> l;
+    if (w < c && i < (n + 1) / 2) {
+      const long long o = base + lev_off(N, l);
+      const StateArrays p = at(g.fpre, o, D), up = at(g.fpre, o + n, D);
+      if (2 * i + 1 < n && r < D) {
+        double u[D];
+        r16::load_row16<D>(u, up.L + (i * D + r) * D);
+        r16::store_row16<D>(p.L + ((2 * i + 1) * D + r) * D, u);
+        p.m[(2 * i + 1) * D + r] = up.m[i * D + r];
+      }
+      const FiltArrays el = at(g.fel, o, D);
+      if (i == 0) {
+        if (r < D) {
+          double u[D];
+          r16::load_row16<D>(u, el.U + r * D);
+          r16::store_row16<D>(p.L + r * D, u);
+          p.m[r] = el.b[r];
+        }
+      } else {
+        const bool first = w == 0 && t + 1 < nlev;
+        const StateArrays s = first ? at(g.fpre, base + lev_off(N, l0 + nlev), D) : up;
+        const size_t is = (size_t)(first ? (long long)b * (kStageWorkers >> (nlev - 1)) - 1 : i - 1);
+        FiltArrays none{};
+        r16::filter_combine<D, DZ, true>(r, none, s, is, el, 2 * (size_t)i, none, p, 2 * (size_t)i);
+      }
+    }
+    if (t > 0) __syncthreads();
   }
 }
 
@@ -447,11 +475,11 @@ __global__ __launch_bounds__(r16::kBlock, 2) void k_filter_post16(GroupArgs g, L
                               g.t_nll + base);
 }
 
-// Smoother up-sweep
-template <int D, int K>
-__global__ __launch_bounds__((Geo<D, K>::BLOCK)) void k_smooth_up(GroupArgs g, LaunchMap lm, int l) {
+// Smoother up-sweep, D > 16
+template <int D>
+__global__ __launch_bounds__((Geo<D, kLdsSmooth>::BLOCK)) void k_smooth_up(GroupArgs g, LaunchMap lm, int l) {
   extern __shared__ double smem[];
-  auto cx = make_ctx<D, K>(g.F, g.LQ, g.N1z, smem);
+  auto cx = make_ctx<D, kLdsSmooth>(g.F, g.LQ, g.N1z, smem);
   int j, i;
   if (!locate(lm, cx.wid, j, i)) return;
   const long long n0 = (long long)g.Ns[j] + 1, base = g.base[j];
@@ -463,10 +491,10 @@ __global__ __launch_bounds__((Geo<D, K>::BLOCK)) void k_smooth_up(GroupArgs g, L
                              with_chol != 0);
 }
 
-template <int D, int K>
-__global__ __launch_bounds__((Geo<D, K>::BLOCK)) void k_smooth_down(GroupArgs g, LaunchMap lm, int l) {
+template <int D>
+__global__ __launch_bounds__((Geo<D, kLdsSmooth>::BLOCK)) void k_smooth_down(GroupArgs g, LaunchMap lm, int l) {
   extern __shared__ double smem[];
-  auto cx = make_ctx<D, K>(g.F, g.LQ, g.N1z, smem);
+  auto cx = make_ctx<D, kLdsSmooth>(g.F, g.LQ, g.N1z, smem);
   int j, i;
   if (!locate(lm, cx.wid, j, i)) return;
   const long long n0 = (long long)g.Ns[j] + 1, base = g.base[j];
@@ -499,6 +527,72 @@ __global__ __launch_bounds__((Geo<D, K>::BLOCK)) void k_smooth_down(GroupArgs g,
       load_dist<S, D>(u, up.L + ((size_t)i * D + r) * D, sb);
       store_dist<S, D>(p.L + ((size_t)j1 * D + r) * D, u, sb);
     }
+  }
+}
+
+// The smoother's sweeps with one row per lane, D <= 16: stages as k_filter_up16 and k_filter_down16.
+template <int D>
+__global__ __launch_bounds__(r16::kStageBlock) void k_smooth_up16(GroupArgs g, LaunchMap lm, int l0, int nlev) {
+  int j, b;
+  if (!locate(lm, blockIdx.x, j, b)) return;
+  const long long n0 = (long long)g.Ns[j] + 1;
+  const int r = threadIdx.x % r16::kRow, w = stage_worker();
+  const bool wc = g.wchol[j] != 0;
+  long long off = g.base[j] + lev_off(n0, l0);
+  StateArrays none{};
+  for (int t = 0; t < nlev; ++t) {
+    const int c = kStageWorkers >> t;
+    const long long i = (long long)b * c + w, next = off + (n0 >> (l0 + t));
+    if (w < c && i < n0 >> (l0 + t + 1)) {
+      const SmoArrays in = at(g.sel, off, D);
+      r16::smoother_combine<D, false>(r, in, none, 2 * (size_t)i, in, 2 * (size_t)i + 1, at(g.sel, next, D), none,
+                                      (size_t)i, wc);
+    }
+    off = next;
+    if (t + 1 < nlev) __syncthreads();
+  }
+}
+
+template <int D>
+__global__ __launch_bounds__(r16::kStageBlock) void k_smooth_down16(GroupArgs g, LaunchMap lm, int l0, int nlev) {
+  int j, b;
+  if (!locate(lm, blockIdx.x, j, b)) return;
+  const long long n0 = (long long)g.Ns[j] + 1, base = g.base[j];
+  const int r = threadIdx.x % r16::kRow, w = stage_worker();
+  const bool wc = g.wchol[j] != 0;
+  for (int t = nlev - 1; t >= 0; --t) {
+    const int l = l0 + t, c = kStageWorkers >> t;
+    const long long i = (long long)b * c + w, n = n0 >> l;
+    if (w < c && i < (n + 1) / 2) {
+      const long long o = base + lev_off(n0, l);
+      const StateArrays p = at(g.spre, o, D), up = at(g.spre, o + n, D);
+      if (2 * i + 1 < n && r < D) {
+        p.m[(2 * i + 1) * D + r] = up.m[i * D + r];
+        if (wc) {
+          double u[D];
+          r16::load_row16<D>(u, up.L + (i * D + r) * D);
+          r16::store_row16<D>(p.L + ((2 * i + 1) * D + r) * D, u);
+        }
+      }
+      const SmoArrays el = at(g.sel, o, D);
+      if (i == 0) {
+        if (r < D) {
+          p.m[r] = el.g[r];
+          if (wc) {
+            double u[D];
+            r16::load_row16<D>(u, el.Dm + r * D);
+            r16::store_row16<D>(p.L + r * D, u);
+          }
+        }
+      } else {
+        const bool first = w == 0 && t + 1 < nlev;
+        const StateArrays s = first ? at(g.spre, base + lev_off(n0, l0 + nlev), D) : up;
+        const size_t is = (size_t)(first ? (long long)b * (kStageWorkers >> (nlev - 1)) - 1 : i - 1);
+        SmoArrays none{};
+        r16::smoother_combine<D, true>(r, none, s, is, el, 2 * (size_t)i, none, p, 2 * (size_t)i, wc);
+      }
+    }
+    if (t > 0) __syncthreads();
   }
 }
 
@@ -978,33 +1072,71 @@ struct Rec {
 };
 }  // namespace
 
-// Launch one scan level: the throughput kind KT when the level has at least
-// `thr` work items (and the kinds differ at this D), else the latency kind KL.
-#define POF_LAUNCH_LEVEL(kernel, KL, KT, thr, nw, ...)                                        \
-  do {                                                                                          \
-    if constexpr (has_throughput_kinds<D>()) {                                                  \
-      if ((nw) >= (thr)) {                                                                      \
-        POF_LAUNCH((kernel<D, KT>), KT, nw, __VA_ARGS__);                                       \
-        break;                                                                                  \
-      }                                                                                         \
-    }                                                                                           \
-    POF_LAUNCH((kernel<D, KL>), KL, nw, __VA_ARGS__);                                           \
-  } while (0)
+// One launch per stage of a sweep
+#define POF_LAUNCH_STAGE(kernel, sg, ...) \
+  hipLaunchKernelGGL(kernel, dim3((sg).blocks), dim3(r16::kStageBlock), 0, __VA_ARGS__, (sg).l0, (sg).nlev)
 
 template <int D>
 void smooth_scan(const GroupArgs& g, const LaunchPlan& p, hipStream_t st, Rec& rec) {
-  for (int l = 0; l + 1 < p.sl; ++l) {
-    const int nw = p.sup_total[l];
-    if (nw == 0) continue;
-    POF_LAUNCH_LEVEL(k_smooth_up, kLdsSmooth, kLdsSmoothT, p.tune.smooth_up, nw, st, g, p.map(p.sup_off[l], nw), l);
-    rec(kKSmoothUp, nw);
+  if constexpr (D <= r16::kRow) {
+    for (int k = 0; k < p.n_sup; ++k) {
+      const Stage& s = p.sup[k];
+      POF_LAUNCH_STAGE(k_smooth_up16<D>, s, st, g, p.map(s.off, s.blocks));
+      rec(kKSmoothUp, s.work);
+    }
+    for (int k = 0; k < p.n_sdn; ++k) {
+      const Stage& s = p.sdn[k];
+      POF_LAUNCH_STAGE(k_smooth_down16<D>, s, st, g, p.map(s.off, s.blocks));
+      rec(kKSmoothDown, s.work);
+    }
+  } else {
+    for (int l = 0; l + 1 < p.sl; ++l) {
+      const int nw = p.sup_total[l];
+      if (nw == 0) continue;
+      POF_LAUNCH((k_smooth_up<D>), kLdsSmooth, nw, st, g, p.map(p.sup_off[l], nw), l);
+      rec(kKSmoothUp, nw);
+    }
+    for (int l = p.sl - 1; l >= 0; --l) {
+      const int nw = p.sdn_total[l];
+      if (nw == 0) continue;
+      POF_LAUNCH((k_smooth_down<D>), kLdsSmooth, nw, st, g, p.map(p.sdn_off[l], nw), l);
+      rec(kKSmoothDown, nw - p.sdn_ivps[l]);
+    }
   }
-  for (int l = p.sl - 1; l >= 0; --l) {
-    const int nw = p.sdn_total[l];
-    if (nw == 0) continue;
-    POF_LAUNCH_LEVEL(k_smooth_down, kLdsSmooth, kLdsSmoothT, p.tune.smooth_down, nw, st, g, p.map(p.sdn_off[l], nw),
-                     l);
-    rec(kKSmoothDown, nw - p.sdn_ivps[l]);
+}
+
+template <int D, int d>
+void filter_scan(const GroupArgs& g, const LaunchPlan& p, hipStream_t st, Rec& rec) {
+  if constexpr (D <= r16::kRow) {
+    for (int k = 0; k < p.n_fup; ++k) {
+      const Stage& s = p.fup[k];
+      if (s.l0 == 0)
+        POF_LAUNCH_STAGE((k_filter_up16<D, d>), s, st, g, p.map(s.off, s.blocks));
+      else
+        POF_LAUNCH_STAGE((k_filter_up16<D, D>), s, st, g, p.map(s.off, s.blocks));
+      rec(kKFilterUp, s.work);
+    }
+    for (int k = 0; k < p.n_fdn; ++k) {
+      const Stage& s = p.fdn[k];
+      if (s.l0 == 0)
+        POF_LAUNCH_STAGE((k_filter_down16<D, d>), s, st, g, p.map(s.off, s.blocks));
+      else
+        POF_LAUNCH_STAGE((k_filter_down16<D, D>), s, st, g, p.map(s.off, s.blocks));
+      rec(kKFilterDown, s.work);
+    }
+  } else {
+    for (int l = 0; l + 1 < p.fl; ++l) {
+      const int nw = p.fup_total[l];
+      if (nw == 0) continue;
+      POF_LAUNCH((k_filter_up<D>), kLdsFull, nw, st, g, p.map(p.fup_off[l], nw), l);
+      rec(kKFilterUp, nw);
+    }
+    for (int l = p.fl - 1; l >= 0; --l) {
+      const int nw = p.fdn_total[l];
+      if (nw == 0) continue;
+      POF_LAUNCH((k_filter_down<D>), kLdsState, nw, st, g, p.map(p.fdn_off[l], nw), l);
+      rec(kKFilterDown, nw - p.fdn_ivps[l]);
+    }
   }
 }
 
@@ -1052,32 +1184,7 @@ hipError_t run_iteration(const GroupArgs& g, const LaunchPlan& p, double* scal, 
                  p.map(p.leaf1_off, p.leaf1_total));
   }
   rec(kKFilterLeaf, p.leaf_total);
-  for (int l = 0; l + 1 < p.fl; ++l) {
-    const int nw = p.fup_total[l];
-    if (nw == 0) continue;
-    if constexpr (D <= r16::kRow) {
-      if (l == 0)
-        POF_LAUNCH16((k_filter_up16<D, d>), nw, st, g, p.map(p.fup_off[l], nw), l);
-      else
-        POF_LAUNCH16((k_filter_up16<D, D>), nw, st, g, p.map(p.fup_off[l], nw), l);
-    } else {
-      POF_LAUNCH((k_filter_up<D>), kLdsFull, nw, st, g, p.map(p.fup_off[l], nw), l);
-    }
-    rec(kKFilterUp, nw);
-  }
-  for (int l = p.fl - 1; l >= 0; --l) {
-    const int nw = p.fdn_total[l];
-    if (nw == 0) continue;
-    if constexpr (D <= r16::kRow) {
-      if (l == 0)
-        POF_LAUNCH16((k_filter_down16<D, d>), nw, st, g, p.map(p.fdn_off[l], nw), l);
-      else
-        POF_LAUNCH16((k_filter_down16<D, D>), nw, st, g, p.map(p.fdn_off[l], nw), l);
-    } else {
-      POF_LAUNCH((k_filter_down<D>), kLdsState, nw, st, g, p.map(p.fdn_off[l], nw), l);
-    }
-    rec(kKFilterDown, nw - p.fdn_ivps[l]);
-  }
+  filter_scan<D, d>(g, p, st, rec);
   // ---- smoother elements + observation statistics
   if (g.affine)
     launch_post<D, d, false>(g, p, kPostFull, st);

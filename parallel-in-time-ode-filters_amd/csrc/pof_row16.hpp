@@ -25,6 +25,7 @@
 #include <type_traits>
 
 #include "pof_core.hpp"
+#include "pof_engine.hpp"
 
 #pragma clang fp contract(off)
 
@@ -32,8 +33,9 @@ namespace pof {
 namespace r16 {
 
 constexpr int kRow = 16;            // lanes per worker
-constexpr int kBlock = 64;          // threads per block: one wavefront
+constexpr int kBlock = 64;          // threads per block of the element kernels: one wavefront
 constexpr int kPerBlock = kBlock / kRow;
+constexpr int kStageBlock = kStageWorkers * kRow;  // threads per block of the scan stages: four wavefronts
 
 // ------------------------------------------------------------- broadcasts
 __device__ double update_dpp_f64(double, double, int, int, int, bool) __asm("llvm.amdgcn.update.dpp.f64");
@@ -530,6 +532,40 @@ __device__ __forceinline__ void filter_combine(int r, const FiltArrays& x1, cons
   if (act) {
     (SO ? so.m : y.b)[o * D + r] = bo;
     store_lower16<D>((SO ? so.L : y.U) + (o * D + r) * D, mt, r);
+  }
+}
+
+// ------------------------------------------------------------- smoother combine
+// pof/parallel_filtsmooth/smoother.py:53-63 under reverse=True, as smoother_combine() of pof_core.hpp:
+// e1 is the aggregate later in time, (g, E, D) = (E2 g1 + g2, E2 E1, tria([E2 D1 | D2])); SO: (m, L) =
+// (E2 m1 + g2, tria([E2 L1 | D2])).  wc = false: no factors (means-only iterations).
+template <int D, bool SO>
+__device__ __forceinline__ void smoother_combine(int r, const SmoArrays& x1, const StateArrays& s1, size_t i1,
+                                                 const SmoArrays& x2, size_t i2, const SmoArrays& y,
+                                                 const StateArrays& so, size_t o, bool wc) {
+  constexpr size_t DD = (size_t)D * D;
+  const bool act = r < D;
+  const int rr = act ? r : 0;
+  double e2[D];
+  load_row16<D>(e2, x2.E + i2 * DD + rr * D);
+  const double g1 = (SO ? s1.m : x1.g)[i1 * D + rr];
+  const double g = x2.g[i2 * D + rr] + dot_lanes<D>(e2, g1);
+  if (act) (SO ? so.m : y.g)[o * D + r] = g;
+  if constexpr (!SO) {
+    double e1[D], e[D];
+    load_row16<D>(e1, x1.E + i1 * DD + rr * D);
+    zero(e);
+    mul_rows<D, D, D>(e, e2, e1);
+    if (act) store_row16<D>(y.E + o * DD + r * D, e);
+  }
+  if (wc) {
+    double d1[D], d2[D], t[D];
+    load_row16<D>(d1, (SO ? s1.L : x1.Dm) + i1 * DD + rr * D);
+    load_row16<D>(d2, x2.Dm + i2 * DD + rr * D);
+    zero(t);
+    mul_rows<D, D, D>(t, e2, d1);  // the first aggregate's D may be a caller's factor, not triangular
+    lq1<D, D, D, 0>(t, d2, r);
+    if (act) store_lower16<D>((SO ? so.L : y.Dm) + o * DD + r * D, t, r);
   }
 }
 

@@ -1,13 +1,14 @@
-"""Autotuner of the scan kernels' forms (no counterpart in the reference).
+"""Autotuner of the scan levels' launches (no counterpart in the reference).
 
-Every scan kernel of state dimension D <= 16 (filter up-sweep and down-sweep,
-smoother up-sweep and down-sweep) exists in two forms with bitwise equal
-results: a latency form, a matrix row split over 2 or 4 lanes and one combine
-per wavefront, fastest when a scan level holds too few combines to fill the
-chip; and a throughput form, one lane per row and several combines per
-wavefront, fewer instructions per combine when a level is wide.  The library
-picks the throughput form for a level with at least ``widths[k]`` work items
-(summed over a batch's IVPs); ``pof_tuning_set`` sets the four widths per D.
+A level of a scan sweep (filter up-sweep and down-sweep, smoother up-sweep and
+down-sweep; state dimension D <= 16) either has a launch of its own, in which
+the chip is full of its combines (the throughput form), or shares a launch with
+the levels above it, each block of 16 workers carrying its combines through up
+to five levels (the latency form: fewer launches, but half the workers drop out
+at every level).  A combine is the same code either way, so results are bitwise
+equal.  The library takes the throughput form for a level with at least
+``widths[k]`` work items (summed over a batch's IVPs); ``pof_tuning_set`` sets
+the four widths per D.
 
 :func:`tune` measures, per (D, d) kernel instantiation, the per-class kernel
 time (HIP events around every launch, ``pof_profile_*``) of two synthetic
@@ -27,15 +28,14 @@ from . import _lib
 
 CACHE = Path(__file__).resolve().with_name("tuning_gfx950.json")
 NEVER = 1 << 30
-CANDIDATES = (NEVER, 65536, 16384, 4096, 1024)
+CANDIDATES = (NEVER, 32768, 16384, 8192, 4096, 2048, 1024)
 CLASSES = ("filter_up", "filter_down", "smooth_up", "smooth_down")
-# (D, d) pairs whose latency form splits rows (D <= 16), with the order q = D / d - 1 <= 4 that a
-# device problem of dimension d takes
+# a device problem of each dimension d, taken with the orders q = D / d - 1 <= 4 that keep D <= 16
 _FIELDS = {1: "logistic", 2: "fhn_classic", 3: "lorenz63", 4: "lorenz96"}
 
 
 def set_widths(D, widths, ctx=None):
-    """Level widths from which the four scan kernels of dimension D run in their throughput form."""
+    """Level widths from which the four scan sweeps of dimension D give a level a launch of its own."""
     ctx = ctx if ctx is not None else _lib.context()
     arr = (ctypes.c_int32 * 4)(*[int(w) for w in widths])
     _lib.check(_lib.load().pof_tuning_set(ctx, int(D), arr), ctx, "pof_tuning_set")
@@ -139,7 +139,7 @@ def tune(pairs=None, candidates=CANDIDATES, iters=2, write=True, path=CACHE, log
         widths[D] = [min(per[k], key=lambda w: per[k][w]) for k in CLASSES]
         set_widths(D, widths[D], ctx)
     cache = {
-        "what": "scan-level widths from which each scan kernel runs in its throughput form, per state dimension "
+        "what": "scan-level widths from which a level of each sweep has a launch of its own, per state dimension "
                 "D: [filter_up, filter_down, smooth_up, smooth_down]; 1073741824 = never",
         "device": torch.cuda.get_device_name(0),
         "workloads": "per (D, d): one IVP of Ns = 2^15 and a batch of 96 IVPs of Ns = 2^12, "

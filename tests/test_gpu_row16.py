@@ -2,7 +2,8 @@
 
 A random linear-Gaussian model with observation noise, so that every factor is well defined, for each state
 dimension the kernels exist for, on grids around the places where the work can go wrong: a single element,
-levels of odd length, fewer combines than a wavefront's four workers, one more and one less than a full block.
+levels of odd length, fewer combines than a wavefront's four workers, one more and one less than a full block, stages of
+several levels over one block and over many (a block's first prefix comes from the block before), several stages.
 Both sides run the same scan in float64.  How far rounding may take two such runs apart is the model's conditioning,
 which ranges over six orders of magnitude here (order 5: 3e-10 between the oracle's own parallel and sequential
 filters): the tolerance of each result is 20 times the oracle's own change when its inputs move by 1e-15 relative, and
@@ -15,7 +16,7 @@ pytestmark = pytest.mark.gpu
 
 PAIRS = [(1, 1), (1, 2), (1, 3), (1, 4), (1, 5), (2, 1), (2, 2), (2, 3), (2, 4), (2, 5), (3, 1), (3, 2), (3, 3), (3, 4),
          (4, 1), (4, 2), (4, 3)]
-STEPS = [1, 2, 3, 4, 5, 7, 8, 9, 31, 33, 130]
+STEPS = [1, 2, 3, 4, 5, 7, 8, 9, 31, 33, 130, 515, 1100]
 
 
 def gram(c):
