@@ -446,7 +446,8 @@ struct pof_batch {
   // writable device tables (g holds the same pointers)
   double *F = nullptr, *LQ = nullptr, *N1z = nullptr, *Pd = nullptr, *x0m = nullptr, *x0L = nullptr;
   double* cvec = nullptr;  // [slots, D] the state of a constant initial trajectory
-  double *params = nullptr, *scale = nullptr, *scal_dev = nullptr, *scal_host = nullptr;
+  double *params = nullptr, *scale = nullptr, *scal_host = nullptr;  // pinned, written by the last kernel
+  double* scal_dev = nullptr;   // its device address
   int *kind = nullptr, *Ns = nullptr, *cur = nullptr, *wchol = nullptr, *pfull = nullptr;
   long long* base = nullptr;
   double** outp = nullptr;  // [4, slots]: means, chols, full means, full chols
@@ -536,12 +537,6 @@ __global__ void k_fill_rows(double* m, const double* v, long long n, int D) {
   if (e < n * D) m[e] = v[e % D];
 }
 
-// After an iteration: every active IVP's result buffer becomes its next linearisation point.
-__global__ void k_flip_cur(int* cur, const int* ivp, int m) {
-  const int a = blockIdx.x * blockDim.x + threadIdx.x;
-  if (a < m) cur[ivp[a]] ^= 1;
-}
-
 // after an instrumented run: accumulate event intervals per kernel class
 hipError_t collect_timing(pof_ctx* ctx, hipStream_t st) {
   if (!ctx->profiling) return hipSuccess;
@@ -600,8 +595,8 @@ hipError_t dalloc(pof_batch* b, size_t n, T** out) {
 // Device bytes of a batch of `entries` entries and `slots` IVPs with state dimension D.
 size_t batch_bytes(int D, long long entries, int slots) {
   const size_t DD = (size_t)D * D;
-  const size_t per_entry = 8 * (7 * DD + 7 * (size_t)D + 4);
-  const size_t per_slot = 8 * (2 * D + DD + kMaxParams + 1 + 8 + 4) + 4 * 4 + 8;
+  const size_t per_entry = 8 * (7 * DD + 7 * (size_t)D + 2);
+  const size_t per_slot = 8 * (2 * D + DD + kMaxParams + 1 + 4) + 4 * 4 + 8;
   return per_entry * (size_t)entries + per_slot * (size_t)slots + 8 * 4 * ((size_t)entries / kChunk + slots + 1);
 }
 
@@ -630,18 +625,21 @@ int batch_new(pof_ctx* ctx, int D, int d, long long entries, int slots, bool aff
   hipError_t he = hipSuccess;
 #define POF_A(ptr, count)                       \
   if (he == hipSuccess) he = dalloc(b, (count), &(ptr));
-  double *fA, *fb, *fU, *feta, *fZ, *pm, *pL, *sg, *sE, *sD, *qm, *qL, *m0, *m1, *ts, *tn, *to, *tv, *part;
+  double *fA, *fb, *fU, *feta, *fZ, *pm, *pL, *sg, *sE, *sD, *qm, *qL, *m0, *m1, *ts, *tn, *part;
   POF_A(fA, n * DD) POF_A(fb, n * D) POF_A(fU, n * DD) POF_A(feta, n * D) POF_A(fZ, n * DD)
   POF_A(pm, n * D) POF_A(pL, n * DD)
   POF_A(sg, n * D) POF_A(sE, n * DD) POF_A(sD, n * DD) POF_A(qm, n * D) POF_A(qL, n * DD)
-  POF_A(m0, n * D) POF_A(m1, n * D) POF_A(ts, n) POF_A(tn, n) POF_A(to, n) POF_A(tv, n)
+  POF_A(m0, n * D) POF_A(m1, n * D) POF_A(ts, n) POF_A(tn, n)
   POF_A(part, 4 * (n / kChunk + S + 1))
   POF_A(b->F, DD) POF_A(b->LQ, DD) POF_A(b->N1z, DD) POF_A(b->Pd, S * D) POF_A(b->x0m, S * D)
-  POF_A(b->x0L, S * DD) POF_A(b->params, S * kMaxParams) POF_A(b->scale, S) POF_A(b->scal_dev, S * 8)
+  POF_A(b->x0L, S * DD) POF_A(b->params, S * kMaxParams) POF_A(b->scale, S)
   POF_A(b->kind, S) POF_A(b->Ns, S) POF_A(b->cur, S) POF_A(b->wchol, S) POF_A(b->base, S) POF_A(b->outp, 4 * S)
   POF_A(b->pfull, S) POF_A(b->cvec, S * D)
 #undef POF_A
-  if (he == hipSuccess) he = hipHostMalloc((void**)&b->scal_host, S * 8 * sizeof(double));
+  // the iteration's scalars go straight to host memory: no copy behind the last kernel
+  if (he == hipSuccess)
+    he = hipHostMalloc((void**)&b->scal_host, S * 8 * sizeof(double), hipHostMallocMapped | hipHostMallocCoherent);
+  if (he == hipSuccess) he = hipHostGetDevicePointer((void**)&b->scal_dev, b->scal_host, 0);
   if (he == hipSuccess) he = hipStreamCreateWithFlags(&b->own_st, hipStreamNonBlocking);
   if (he == hipSuccess) he = hipEventCreateWithFlags(&b->ev, hipEventDisableTiming);
   if (he == hipSuccess) he = hipEventCreateWithFlags(&b->join_ev, hipEventDisableTiming);
@@ -670,8 +668,6 @@ int batch_new(pof_ctx* ctx, int D, int d, long long entries, int slots, bool aff
   g.spre = StateArrays{qm, qL};
   g.t_ssq = ts;
   g.t_nll = tn;
-  g.t_obj = to;
-  g.t_viol = tv;
   g.part = part;
   g.out_means = b->outp;
   g.out_chols = b->outp + S;
@@ -757,13 +753,21 @@ void range_free(pof_batch* b, long long start, long long len) {
 int plan_tables(pof_batch* b, const std::vector<int>& ids, std::vector<int>& h, LaunchPlan& p) {
   const auto tu = b->ctx->tuning.find(b->D);
   const Tuning tune = (tu != b->ctx->tuning.end()) ? tu->second : Tuning{};
+  static_assert(sizeof(IvpRec) == 4 * sizeof(int), "records are laid out in the table of ints");
+  h.resize((h.size() + 3) / 4 * 4);  // records are aligned to 16 bytes
   const int at = (int)h.size();
   const int m = (int)ids.size();
-  h.insert(h.end(), ids.begin(), ids.end());
+  for (int id : ids) {
+    const IvpRec rec{id, b->hNs[id], b->hbase[id]};
+    int v[4];
+    std::memcpy(v, &rec, sizeof v);
+    h.insert(h.end(), v, v + 4);
+  }
   long long maxNs = 1;
   for (int id : ids) maxNs = std::max<long long>(maxNs, b->hNs[id]);
   p = LaunchPlan{};
   p.m = m;
+  if (m > 0) std::memcpy(&p.first, &h[at], sizeof p.first);
   p.fl = n_levels_host(maxNs);
   p.sl = n_levels_host(maxNs + 1);
   if (p.sl > kMaxLevels) return POF_E_ARG;
@@ -920,9 +924,7 @@ hipError_t launch_iteration(pof_batch* b, KernelTimer* tm) {
     e = b->e->seq_iteration(b->g, b->plan, b->scal_dev, b->mode == 2 ? 1 : 0, b->st, tm);
   else
     e = b->e->iteration(b->g, b->plan, b->scal_dev, b->st, tm);
-  if (e != hipSuccess) return e;
-  hipLaunchKernelGGL(k_flip_cur, dim3((b->plan.m + 255) / 256), dim3(256), 0, b->st, b->cur, b->plan.dev, b->plan.m);
-  return hipGetLastError();
+  return e;
 }
 
 // The caller has drained b->st (settle): no replay of the graph is in flight.
@@ -1091,8 +1093,6 @@ int batch_launch(pof_batch* b) {
   for (int j : b->active) b->hcur[j] ^= 1;  // host mirror of the flip
   HIP_TRY(collect_timing(ctx, b->st));
   if (b->need_sync) {
-    HIP_TRY(hipMemcpyAsync(b->scal_host, b->scal_dev, (size_t)b->plan.m * 8 * sizeof(double),
-                           hipMemcpyDeviceToHost, b->st));
     HIP_TRY(hipEventRecord(b->ev, b->st));
   }
   b->launched = true;
@@ -1168,7 +1168,7 @@ int batch_finish(pof_batch* b, int max_done, long long* done, int* n_done) {
   int rc = POF_OK;
   const int start_c = 0;
   if (!need.empty()) rc = plan_tables(b, need, b->hmaps, pc);
-  const int start_o = (int)b->hmaps.size();
+  const int start_o = ((int)b->hmaps.size() + 3) / 4 * 4;
   if (rc == POF_OK) rc = plan_tables(b, fin, b->hmaps, po);
   if (rc != POF_OK) return set_err(ctx, rc, "launch tables overflow");
   if (b->hmaps.size() > b->maps_cap) {

@@ -11,7 +11,7 @@
 namespace pof {
 
 constexpr int kMaxLevels = 40;
-constexpr int kChunk = 2048;  // time points per block of the stage-1 reduction
+constexpr int kChunk = 256;  // time points (threads) per block of the smoothed means and the stage-1 reduction
 
 // Optional per-kernel timing with HIP events (instrumented runs only).
 constexpr int kMaxTimed = 256;
@@ -59,9 +59,10 @@ struct Stage {
 };
 
 // Launch maps of one active set of a group (host view of a device int buffer):
-// the active IVP ids, then one prefix table per launch kind and level.
+// the active IVPs' records, then one prefix table per launch kind and level.
 struct LaunchPlan {
   const int* dev = nullptr;  // device buffer
+  IvpRec first{};            // the first active IVP's record
   int m = 0;                 // active IVPs
   int fl = 0, sl = 0;        // filter / smoother levels (maximum over the active IVPs)
   int leaf_off = 0, leaf_total = 0;    // per IVP: Ns work items
@@ -78,7 +79,9 @@ struct LaunchPlan {
   int sup_off[kMaxLevels] = {}, sup_total[kMaxLevels] = {};  // (Ns + 1) >> (l + 1)
   int sdn_off[kMaxLevels] = {}, sdn_total[kMaxLevels] = {};  // (((Ns + 1) >> l) + 1) / 2
   int fdn_ivps[kMaxLevels] = {}, sdn_ivps[kMaxLevels] = {};  // active IVPs that have level l
-  LaunchMap map(int off, int total) const { return LaunchMap{dev, dev + off, m, total}; }
+  LaunchMap map(int off, int total) const {
+    return LaunchMap{reinterpret_cast<const IvpRec*>(dev), dev + off, m, total, first};
+  }
 };
 
 // Kernel entry points per (D, d) instantiation, all over one group's active set.

@@ -53,12 +53,31 @@ __device__ __forceinline__ int find_seg(const int* pre, int m, int w) {
   return lo;
 }
 
-// IVP id j and local index i of work item w (false past the end).
-__device__ __forceinline__ bool locate(const LaunchMap& lm, int w, int& j, int& i) {
+// Work item w of a launch: its IVP's record and its index within that IVP's items (false past the end).
+struct Item {
+  int j, i, Ns;
+  long long base;
+};
+__device__ __forceinline__ bool locate(const LaunchMap& lm, int w, Item& it) {
   if (w >= lm.total) return false;
-  const int a = find_seg(lm.pre, lm.m, w);
-  j = lm.ivp[a];
-  i = w - lm.pre[a];
+  IvpRec rec = lm.one;
+  it.i = w;
+  if (lm.m > 1) {
+    const int a = find_seg(lm.pre, lm.m, w);
+    rec = lm.rec[a];
+    it.i = w - lm.pre[a];
+  }
+  it.j = rec.j;
+  it.Ns = rec.Ns;
+  it.base = rec.base;
+  return true;
+}
+// IVP id j and local index i of work item w.
+__device__ __forceinline__ bool locate(const LaunchMap& lm, int w, int& j, int& i) {
+  Item it;
+  if (!locate(lm, w, it)) return false;
+  j = it.j;
+  i = it.i;
   return true;
 }
 
@@ -188,11 +207,12 @@ __device__ __forceinline__ int stage_worker() { return ((threadIdx.x & 63) >> 4)
 template <int D, int DZ>
 __global__ __launch_bounds__(r16::kStageBlock, 2) void k_filter_up16(GroupArgs g, LaunchMap lm, int l0, int nlev) {
   if constexpr (DZ != D) l0 = 0, nlev = 1;
-  int j, b;
-  if (!locate(lm, blockIdx.x, j, b)) return;
-  const long long N = g.Ns[j];
+  Item it;
+  if (!locate(lm, blockIdx.x, it)) return;
+  const int b = it.i;
+  const long long N = it.Ns;
   const int r = threadIdx.x % r16::kRow, w = stage_worker();
-  long long off = g.base[j] + lev_off(N, l0);
+  long long off = it.base + lev_off(N, l0);
   StateArrays none{};
   for (int t = 0; t < nlev; ++t) {
     const int c = kStageWorkers >> t;
@@ -212,9 +232,10 @@ __global__ __launch_bounds__(r16::kStageBlock, 2) void k_filter_up16(GroupArgs g
 template <int D, int DZ>
 __global__ __launch_bounds__(r16::kStageBlock, 2) void k_filter_down16(GroupArgs g, LaunchMap lm, int l0, int nlev) {
   if constexpr (DZ != D) l0 = 0, nlev = 1;
-  int j, b;
-  if (!locate(lm, blockIdx.x, j, b)) return;
-  const long long N = g.Ns[j], base = g.base[j];
+  Item it;
+  if (!locate(lm, blockIdx.x, it)) return;
+  const int b = it.i;
+  const long long N = it.Ns, base = it.base;
   const int r = threadIdx.x % r16::kRow, w = stage_worker();
   for (int t = nlev - 1; t >= 0; --t) {
     const int l = l0 + t, c = kStageWorkers >> t;
@@ -251,9 +272,9 @@ __global__ __launch_bounds__(r16::kStageBlock, 2) void k_filter_down16(GroupArgs
 // Elements 0 .. Ns - 1, one row per lane, D <= 16.
 template <int D, int d, bool EK1>
 __global__ __launch_bounds__(r16::kBlock, 2) void k_filter_leaf16(GroupArgs g, LaunchMap lm) {
-  int j, k;
-  if (!locate(lm, blockIdx.x * r16::kPerBlock + threadIdx.x / r16::kRow, j, k)) return;
-  r16::filter_element<D, d, EK1>(threadIdx.x % r16::kRow, g, j, k, at(g.fel, g.base[j], D));
+  Item it;
+  if (!locate(lm, blockIdx.x * r16::kPerBlock + threadIdx.x / r16::kRow, it)) return;
+  r16::filter_element<D, d, EK1>(threadIdx.x % r16::kRow, g, it.j, it.base, it.i, at(g.fel, it.base, D));
 }
 
 // Per filtered state s = 0..Ns: smoother element (smoother.py:37-50) stored at
@@ -449,10 +470,10 @@ __global__ __launch_bounds__((Geo<D, kLdsPost>::BLOCK)) void k_filter_post(Group
 // The same with one row per lane, D <= 16.
 template <int D, int d, bool EK1>
 __global__ __launch_bounds__(r16::kBlock, 2) void k_filter_post16(GroupArgs g, LaunchMap lm, int mode) {
-  int j, s;
-  if (!locate(lm, blockIdx.x * r16::kPerBlock + threadIdx.x / r16::kRow, j, s)) return;
-  const long long base = g.base[j];
-  const int Ns = g.Ns[j];
+  Item it;
+  if (!locate(lm, blockIdx.x * r16::kPerBlock + threadIdx.x / r16::kRow, it)) return;
+  const long long base = it.base;
+  const int j = it.j, s = it.i, Ns = it.Ns;
   const StateArrays pre0 = at(g.fpre, base, D);
   const SmoArrays sel = at(g.sel, base, D);
   const int r = threadIdx.x % r16::kRow;
@@ -471,7 +492,7 @@ __global__ __launch_bounds__(r16::kBlock, 2) void k_filter_post16(GroupArgs g, L
     return;
   }
   const bool dm = mode == kPostDm;
-  r16::filter_post<D, d, EK1>(r, g, j, s, mp, Lp, mode == kPostFull, dm, dm || g.wchol[j] != 0, sel, ro, g.t_ssq + base,
+  r16::filter_post<D, d, EK1>(r, g, j, base, s, mp, Lp, mode == kPostFull, dm, dm || g.wchol[j] != 0, sel, ro, g.t_ssq + base,
                               g.t_nll + base);
 }
 
@@ -533,12 +554,13 @@ __global__ __launch_bounds__((Geo<D, kLdsSmooth>::BLOCK)) void k_smooth_down(Gro
 // The smoother's sweeps with one row per lane, D <= 16: stages as k_filter_up16 and k_filter_down16.
 template <int D>
 __global__ __launch_bounds__(r16::kStageBlock) void k_smooth_up16(GroupArgs g, LaunchMap lm, int l0, int nlev) {
-  int j, b;
-  if (!locate(lm, blockIdx.x, j, b)) return;
-  const long long n0 = (long long)g.Ns[j] + 1;
+  Item it;
+  if (!locate(lm, blockIdx.x, it)) return;
+  const int b = it.i;
+  const long long n0 = (long long)it.Ns + 1;
   const int r = threadIdx.x % r16::kRow, w = stage_worker();
-  const bool wc = g.wchol[j] != 0;
-  long long off = g.base[j] + lev_off(n0, l0);
+  const bool wc = g.wchol[it.j] != 0;
+  long long off = it.base + lev_off(n0, l0);
   StateArrays none{};
   for (int t = 0; t < nlev; ++t) {
     const int c = kStageWorkers >> t;
@@ -555,11 +577,12 @@ __global__ __launch_bounds__(r16::kStageBlock) void k_smooth_up16(GroupArgs g, L
 
 template <int D>
 __global__ __launch_bounds__(r16::kStageBlock) void k_smooth_down16(GroupArgs g, LaunchMap lm, int l0, int nlev) {
-  int j, b;
-  if (!locate(lm, blockIdx.x, j, b)) return;
-  const long long n0 = (long long)g.Ns[j] + 1, base = g.base[j];
+  Item it;
+  if (!locate(lm, blockIdx.x, it)) return;
+  const int b = it.i;
+  const long long n0 = (long long)it.Ns + 1, base = it.base;
   const int r = threadIdx.x % r16::kRow, w = stage_worker();
-  const bool wc = g.wchol[j] != 0;
+  const bool wc = g.wchol[it.j] != 0;
   for (int t = nlev - 1; t >= 0; --t) {
     const int l = l0 + t, c = kStageWorkers >> t;
     const long long i = (long long)b * c + w, n = n0 >> l;
@@ -596,116 +619,111 @@ __global__ __launch_bounds__(r16::kStageBlock) void k_smooth_down16(GroupArgs g,
   }
 }
 
-// Thread t: smoothed mean m_t (reversed prefix Ns - t) -> means_new[t];
-// obj_t = |LQ^-1 (m_t - F m_{t+1})|^2 (utils.py:97-101 with the argument order
-// of smoother.py:20); viol_t = 1 if any |m_old - m_new| > 1e-8 + 1e-13 |m_new|
-// (convergence_criteria.py:10, jnp.isclose).
-template <int D>
-__global__ void k_smooth_post(GroupArgs g, LaunchMap lm) {
-  int j, t;
-  if (!locate(lm, blockIdx.x * blockDim.x + threadIdx.x, j, t)) return;
-  const int Ns = g.Ns[j];
-  const long long base = g.base[j];
-  const StateArrays spre0 = at(g.spre, base, D);
-  const double* mold = (g.cur[j] ? g.means1 : g.means0) + (size_t)base * D;
-  double* mnew = (g.cur[j] ? g.means0 : g.means1) + (size_t)base * D;
-  double* t_obj = g.t_obj + base;
-  double* t_viol = g.t_viol + base;
-  const double* F = g.F;
-  const double* LQ = g.LQ;
-  const double* m = spre0.m + (size_t)(Ns - t) * D;
-  double mt[D];
-  load_row(mt, m);
-  store_row(mnew + (size_t)t * D, mt);
-  double v = 0.0;
+// Sum (or maximum) of a block's 256 values in a fixed order; the result is valid in thread 0.
+template <bool MAX>
+__device__ __forceinline__ double block_reduce(double v, double* sh) {
 #pragma unroll
-  for (int i = 0; i < D; ++i) {
-    const double o = mold[(size_t)t * D + i];
-    const bool close = fabs(o - mt[i]) <= 1e-8 + 1e-13 * fabs(mt[i]);
-    v = close ? v : 1.0;
+  for (int o = 32; o > 0; o >>= 1) {
+    const double x = __shfl_down(v, o);
+    v = MAX ? fmax(v, x) : v + x;
   }
-  t_viol[t] = v;
-  if (t < Ns) {
-    const double* mn = spre0.m + (size_t)(Ns - t - 1) * D;
-    double rr[D];
-#pragma unroll
-    for (int i = 0; i < D; ++i) {
-      double acc = mt[i];
-#pragma unroll
-      for (int j = 0; j < D; ++j) acc = fma(-F[i * D + j], mn[j], acc);
-      rr[i] = acc;
-    }
-    // forward substitution with LQ (lower)
-    double o = 0.0;
-#pragma unroll
-    for (int i = 0; i < D; ++i) {
-      double s = rr[i];
-#pragma unroll
-      for (int j = 0; j < i; ++j) s = fma(-LQ[i * D + j], rr[j], s);
-      rr[i] = s / LQ[i * D + i];
-      o = fma(rr[i], rr[i], o);
-    }
-    t_obj[t] = o;
-  }
-}
-
-// Fixed-order reduction of the per-step terms of each IVP, stage 1: block b
-// (chunk c of IVP j) sums the time points [c kChunk, (c + 1) kChunk) into
-// part[b * 4 + 0..3] (ssq, nll, obj: sums over t < Ns; violations: max over t <= Ns).
-static __global__ void k_reduce_part(GroupArgs g, LaunchMap lm) {
-  __shared__ double sh[4][256];
-  const int tid = threadIdx.x;
-  int j, c;
-  if (!locate(lm, blockIdx.x, j, c)) return;
-  const int Ns = g.Ns[j];
-  const long long base = g.base[j];
-  const int lo = c * kChunk;
-  const int hi = min(lo + kChunk, Ns + 1);
-  double s0 = 0.0, s1 = 0.0, s2 = 0.0, s3 = 0.0;
-  for (int i = lo + tid; i < hi; i += 256) {
-    if (i < Ns) {
-      s0 += g.t_ssq[base + i];
-      s1 += g.t_nll[base + i];
-      s2 += g.t_obj[base + i];
-    }
-    s3 = fmax(s3, g.t_viol[base + i]);
-  }
-  sh[0][tid] = s0;
-  sh[1][tid] = s1;
-  sh[2][tid] = s2;
-  sh[3][tid] = s3;
+  if ((threadIdx.x & 63) == 0) sh[threadIdx.x >> 6] = v;
   __syncthreads();
-  for (int w = 128; w > 0; w >>= 1) {
-    if (tid < w) {
-      sh[0][tid] += sh[0][tid + w];
-      sh[1][tid] += sh[1][tid + w];
-      sh[2][tid] += sh[2][tid + w];
-      sh[3][tid] = fmax(sh[3][tid], sh[3][tid + w]);
-    }
-    __syncthreads();
-  }
-  if (tid < 4) g.part[(size_t)blockIdx.x * 4 + tid] = sh[tid][0];
+  return MAX ? fmax(fmax(sh[0], sh[1]), fmax(sh[2], sh[3])) : (sh[0] + sh[1]) + (sh[2] + sh[3]);
 }
 
-// Stage 2, block a per active IVP: its chunks in order.  scal[a * 8 + k]:
-// 0 nll, 1 obj, 2 ssq (sum / (Ns d)), 3 = 1 if all means are close, 4 = NaN flag.
-static __global__ void k_reduce_final(GroupArgs g, LaunchMap lm, int d, double* scal) {
-  const int a = blockIdx.x;
-  if (a >= lm.m || threadIdx.x != 0) return;
-  const int Ns = g.Ns[lm.ivp[a]];
+// Block of an IVP's chunk of kChunk time points, thread t: smoothed mean m_t (reversed prefix Ns - t)
+// -> means_new[t]; obj_t = |LQ^-1 (m_t - F m_{t+1})|^2 (utils.py:97-101 with the argument order of
+// smoother.py:20); viol_t = 1 if any |m_old - m_new| > 1e-8 + 1e-13 |m_new| (convergence_criteria.py:10,
+// jnp.isclose).  The chunk's ssq, nll and obj sums (t < Ns) and largest violation go to part[4 block].
+template <int D>
+__global__ __launch_bounds__(kChunk) void k_smooth_post(GroupArgs g, LaunchMap lm) {
+  static_assert(kChunk == 256, "block_reduce adds four wavefronts");
+  __shared__ double sh[4][4];
+  Item it;
+  if (!locate(lm, blockIdx.x, it)) return;
+  const int Ns = it.Ns, t = it.i * kChunk + threadIdx.x;
+  const long long base = it.base;
   double s0 = 0.0, s1 = 0.0, s2 = 0.0, s3 = 0.0;
-  for (int b = lm.pre[a]; b < lm.pre[a + 1]; ++b) {
+  if (t <= Ns) {
+    const StateArrays spre0 = at(g.spre, base, D);
+    const int cur = g.cur[it.j];
+    const double* mold = (cur ? g.means1 : g.means0) + (size_t)base * D;
+    double* mnew = (cur ? g.means0 : g.means1) + (size_t)base * D;
+    const double* F = g.F;
+    const double* LQ = g.LQ;
+    const double* m = spre0.m + (size_t)(Ns - t) * D;
+    double mt[D];
+    load_row(mt, m);
+    store_row(mnew + (size_t)t * D, mt);
+#pragma unroll
+    for (int i = 0; i < D; ++i) {
+      const double o = mold[(size_t)t * D + i];
+      const bool close = fabs(o - mt[i]) <= 1e-8 + 1e-13 * fabs(mt[i]);
+      s3 = close ? s3 : 1.0;
+    }
+    if (t < Ns) {
+      s0 = g.t_ssq[base + t];
+      s1 = g.t_nll[base + t];
+      const double* mn = spre0.m + (size_t)(Ns - t - 1) * D;
+      double rr[D];
+#pragma unroll
+      for (int i = 0; i < D; ++i) {
+        double acc = mt[i];
+#pragma unroll
+        for (int j = 0; j < D; ++j) acc = fma(-F[i * D + j], mn[j], acc);
+        rr[i] = acc;
+      }
+      // forward substitution with LQ (lower)
+#pragma unroll
+      for (int i = 0; i < D; ++i) {
+        double s = rr[i];
+#pragma unroll
+        for (int j = 0; j < i; ++j) s = fma(-LQ[i * D + j], rr[j], s);
+        rr[i] = s / LQ[i * D + i];
+        s2 = fma(rr[i], rr[i], s2);
+      }
+    }
+  }
+  s0 = block_reduce<false>(s0, sh[0]);
+  s1 = block_reduce<false>(s1, sh[1]);
+  s2 = block_reduce<false>(s2, sh[2]);
+  s3 = block_reduce<true>(s3, sh[3]);
+  if (threadIdx.x == 0) {
+    double* o = g.part + (size_t)blockIdx.x * 4;
+    o[0] = s0;
+    o[1] = s1;
+    o[2] = s2;
+    o[3] = s3;
+  }
+}
+
+// Block a per active IVP: its chunks in a fixed order.  scal[a * 8 + k]: 0 nll, 1 obj,
+// 2 ssq (sum / (Ns d)), 3 = 1 if all means are close, 4 = NaN flag.  The IVP's result buffer becomes its
+// next linearisation point.
+static __global__ __launch_bounds__(256) void k_reduce_final(GroupArgs g, LaunchMap lm, int d, double* scal) {
+  __shared__ double sh[4][4];
+  const int a = blockIdx.x;
+  const IvpRec rec = (lm.m > 1) ? lm.rec[a] : lm.one;
+  double s0 = 0.0, s1 = 0.0, s2 = 0.0, s3 = 0.0;
+  for (int b = lm.pre[a] + threadIdx.x; b < lm.pre[a + 1]; b += 256) {
     s0 += g.part[(size_t)b * 4 + 0];
     s1 += g.part[(size_t)b * 4 + 1];
     s2 += g.part[(size_t)b * 4 + 2];
     s3 = fmax(s3, g.part[(size_t)b * 4 + 3]);
   }
+  s0 = block_reduce<false>(s0, sh[0]);
+  s1 = block_reduce<false>(s1, sh[1]);
+  s2 = block_reduce<false>(s2, sh[2]);
+  s3 = block_reduce<true>(s3, sh[3]);
+  if (threadIdx.x != 0) return;
   double* o = scal + (size_t)a * 8;
   o[0] = s1;
   o[1] = s2;
-  o[2] = s0 / Ns / d;
+  o[2] = s0 / rec.Ns / d;
   o[3] = (s3 == 0.0) ? 1.0 : 0.0;
   o[4] = (isnan(s1) || isnan(s2)) ? 1.0 : 0.0;
+  g.cur[rec.j] ^= 1;
 }
 
 // Output projection: means_out[t][i] = P_ii0 m_t[i0], chol_out[t][i][:] = scale * P_ii0 L_t[i0][:]
@@ -1140,6 +1158,17 @@ void filter_scan(const GroupArgs& g, const LaunchPlan& p, hipStream_t st, Rec& r
   }
 }
 
+// Smoothed means, objective, convergence partials, per-IVP reduction
+template <int D>
+hipError_t iteration_tail(const GroupArgs& g, const LaunchPlan& p, double* scal, int d, hipStream_t st, Rec& rec) {
+  const LaunchMap chunks = p.map(p.chunk_off, p.chunk_total);
+  hipLaunchKernelGGL((k_smooth_post<D>), dim3(p.chunk_total), dim3(kChunk), 0, st, g, chunks);
+  rec(kKSmoothPost, p.pts_total);
+  hipLaunchKernelGGL(k_reduce_final, dim3(p.m), dim3(256), 0, st, g, chunks, d, scal);
+  rec(kKReduce, p.leaf_total);
+  return hipGetLastError();
+}
+
 // k_filter_post of every filtered state
 template <int D, int d, bool EK1>
 void launch_post(const GroupArgs& g, const LaunchPlan& p, int mode, hipStream_t st) {
@@ -1194,13 +1223,7 @@ hipError_t run_iteration(const GroupArgs& g, const LaunchPlan& p, double* scal, 
   // ---- smoother scan (reversed order)
   smooth_scan<D>(g, p, st, rec);
   // ---- smoothed means, objective, convergence partials, per-IVP reduction
-  hipLaunchKernelGGL((k_smooth_post<D>), dim3((p.pts_total + 127) / 128), dim3(128), 0, st, g,
-                     p.map(p.pts_off, p.pts_total));
-  rec(kKSmoothPost, p.pts_total);
-  hipLaunchKernelGGL(k_reduce_part, dim3(p.chunk_total), dim3(256), 0, st, g, p.map(p.chunk_off, p.chunk_total));
-  hipLaunchKernelGGL(k_reduce_final, dim3(p.m), dim3(64), 0, st, g, p.map(p.chunk_off, p.chunk_total), d, scal);
-  rec(kKReduce, p.leaf_total);
-  return hipGetLastError();
+  return iteration_tail<D>(g, p, scal, d, st, rec);
 }
 
 // One sequential IEKS iteration (pof/step.py:33-45 with sequential=True) or,
@@ -1222,13 +1245,7 @@ hipError_t run_seq_iteration(const GroupArgs& g, const LaunchPlan& p, double* sc
   rec(kKFilterLeaf, p.leaf_total);
   POF_LAUNCH((k_seq_smooth<D>), kLdsSeq, p.one_total, st, g, one);
   rec(kKSmoothUp, p.leaf_total);
-  hipLaunchKernelGGL((k_smooth_post<D>), dim3((p.pts_total + 127) / 128), dim3(128), 0, st, g,
-                     p.map(p.pts_off, p.pts_total));
-  rec(kKSmoothPost, p.pts_total);
-  hipLaunchKernelGGL(k_reduce_part, dim3(p.chunk_total), dim3(256), 0, st, g, p.map(p.chunk_off, p.chunk_total));
-  hipLaunchKernelGGL(k_reduce_final, dim3(p.m), dim3(64), 0, st, g, p.map(p.chunk_off, p.chunk_total), d, scal);
-  rec(kKReduce, p.leaf_total);
-  return hipGetLastError();
+  return iteration_tail<D>(g, p, scal, d, st, rec);
 }
 
 // The smoother alone over filtered states already in the filter prefix arrays
@@ -1246,13 +1263,7 @@ hipError_t run_smooth_only(const GroupArgs& g, const LaunchPlan& p, double* scal
     rec(kKFilterPost, p.leaf_total);
     smooth_scan<D>(g, p, st, rec);
   }
-  hipLaunchKernelGGL((k_smooth_post<D>), dim3((p.pts_total + 127) / 128), dim3(128), 0, st, g,
-                     p.map(p.pts_off, p.pts_total));
-  rec(kKSmoothPost, p.pts_total);
-  hipLaunchKernelGGL(k_reduce_part, dim3(p.chunk_total), dim3(256), 0, st, g, p.map(p.chunk_off, p.chunk_total));
-  hipLaunchKernelGGL(k_reduce_final, dim3(p.m), dim3(64), 0, st, g, p.map(p.chunk_off, p.chunk_total), d, scal);
-  rec(kKReduce, p.leaf_total);
-  return hipGetLastError();
+  return iteration_tail<D>(g, p, scal, d, st, rec);
 }
 
 // Smoothed factors of the last sequential iteration (after means-only passes).

@@ -189,9 +189,6 @@ __device__ __forceinline__ void unroll_down(F&& f) {
 // x is formed here (not recomputed from its operands where it is used, which would hold all of them)
 __device__ __forceinline__ void keep(double& x) { asm volatile("" : "+v"(x)); }
 
-// End of a phase: later loads are not moved above it (they would hold registers through the phase).
-__device__ __forceinline__ void phase() { asm volatile("" ::: "memory"); }
-
 // ------------------------------------------------------------- products
 // y[c] += sum_k x[k] (row k of B)[c] over the columns c < min(N, k + LOW) of row k (LOW = 1: B lower
 // triangular; LOW >= N: full)
@@ -373,39 +370,73 @@ __device__ __forceinline__ void filter_combine(int r, const FiltArrays& x1, cons
   const bool act = r < D;
   const int rr = act ? r : 0;
   const double* U1 = (SO ? s1.L : x1.U) + i1 * DD;
+  const double* A1 = SO ? nullptr : x1.A + i1 * DD;
+  const double* Z1 = SO ? nullptr : x1.Z + i1 * DD;
   const double* A2 = x2.A + i2 * DD;
+  const double* U2 = x2.U + i2 * DD;
   const double* Z2 = x2.Z + i2 * DD;
+
+  // Reads are issued ahead of the phases that use them (the asm groups keep them in place), as far as the
+  // registers hold them: all of them here (D <= 8), or those of the first two phases here and the rest half
+  // way (D <= 12); beyond, each phase's at its head (more would spill).  A combine alone on its SIMD waits for
+  // memory at each such point, five times in the last form: at D = 12 reading ahead took the 10 iterations over
+  // 65,536 steps from 10.8 to 10.2 ms (with the shorter tail of an iteration), at D = 4 from 3.29 to 2.95 ms.
+  constexpr bool kAll = D <= 8, kTwo = D <= 12;
+  double u1t[D], z2[DZ], z2t[SO ? 1 : D], w[D], u1[D], u2[D], ar[SO ? 1 : D], a1t[SO ? 1 : D], z1[SO ? 1 : DZ];
+  auto load_z = [&](double (&z)[DZ], const double* Z) {
+    if constexpr (kLeaf) {
+#pragma unroll
+      for (int c = 0; c < DZ; ++c) z[c] = Z[rr * DZ + c];
+    } else {
+      load_row16<DZ>(z, Z + rr * D);
+    }
+  };
+  auto load_rest1 = [&] {
+    load_row16<D>(u2, U2 + rr * D);
+    if constexpr (!SO) load_row16<D>(ar, A1 + rr * D);
+  };
+  auto load_rest2 = [&] {
+    if constexpr (!SO) {
+      load_col16<D>(a1t, A1, rr);
+      load_z(z1, Z1);
+    }
+  };
   const double b1r = (SO ? s1.m : x1.b)[i1 * D + rr];
   const double eta2r = x2.eta[i2 * D + rr];
+  load_col16<D>(u1t, U1, rr);
+  load_z(z2, Z2);
+  if constexpr (!SO) {
+    if constexpr (kLeaf) {
+      const int rz = (r < DZ) ? r : 0;  // lanes past the last column hold no entry of Z2^T b1
+#pragma unroll
+      for (int k = 0; k < D; ++k) z2t[k] = Z2[k * DZ + rz];
+    } else {
+      load_col16<D>(z2t, Z2, rr);
+    }
+  }
+  if constexpr (kTwo) {
+    load_row16<D>(w, A2 + rr * D);
+    load_row16<D>(u1, U1 + rr * D);
+  }
+  const double b2r = x2.b[i2 * D + rr];
+  const double eta1r = SO ? 0.0 : x1.eta[i1 * D + rr];
+  if constexpr (kAll) {
+    load_rest1();
+    load_rest2();
+  }
 
-  double u, s2 = 0.0, uu = 0.0;
+  double s2 = 0.0, uu = 0.0;
   double a1[D], b1[D], b2[D], rd = 0.0;  // Xi11, Xi21, Xi22; rd: 1 / Xi11[r][r] in lane r
+  if constexpr (!SO) {
+    // s2 = eta2 - Z2 (Z2^T b1), uu = U1^T s2
+    const double t = dot_lanes<D>(z2t, b1r);
+    s2 = eta2r - dot_lanes<DZ>(z2, t);
+    uu = dot_lanes<D>(u1t, s2);
+  }
+  const double u = dot_lanes<D>(u1t, eta2r);
   {
     double a2[D];
     {
-      double u1t[D], z2[D];
-      load_col16<D>(u1t, U1, rr);
-      if constexpr (kLeaf) {
-#pragma unroll
-        for (int c = 0; c < DZ; ++c) z2[c] = Z2[rr * DZ + c];
-      } else {
-        load_row16<D>(z2, Z2 + rr * D);
-      }
-      if constexpr (!SO) {
-        // s2 = eta2 - Z2 (Z2^T b1), uu = U1^T s2
-        double z2t[D];
-        if constexpr (kLeaf) {
-          const int rz = (r < DZ) ? r : 0;  // lanes past the last column hold no entry of Z2^T b1
-#pragma unroll
-          for (int k = 0; k < D; ++k) z2t[k] = Z2[k * DZ + rz];
-        } else {
-          load_col16<D>(z2t, Z2, rr);
-        }
-        const double t = dot_lanes<D>(z2t, b1r);
-        s2 = eta2r - dot_lanes<DZ>(z2, t);
-        uu = dot_lanes<D>(u1t, s2);
-      }
-      u = dot_lanes<D>(u1t, eta2r);
       double x[DZ];
       zero(x);
       mul_rows<D, DZ, kLow>(x, u1t, z2);
@@ -454,18 +485,18 @@ __device__ __forceinline__ void filter_combine(int r, const FiltArrays& x1, cons
       b2[i] = -tb;
     });
   }
-
-  // MT = A2 U1 Xi11^-T, W = A2 - MT Xi21^T, b = W (b1 + U1 u) + b2
-  double mt[D], w[D];
-  zero(mt);
-  double sv;
-  {
-    double u1[D];
+  if constexpr (!kTwo) {
     load_row16<D>(w, A2 + rr * D);
     load_row16<D>(u1, U1 + rr * D);
-    mul_rows<D, D, 1>(mt, w, u1);
-    sv = dot_lanes<D>(u1, u, b1r);
+  } else if constexpr (!kAll) {
+    load_rest1();
   }
+
+  // MT = A2 U1 Xi11^-T, W = A2 - MT Xi21^T, b = W (b1 + U1 u) + b2
+  double mt[D];
+  zero(mt);
+  mul_rows<D, D, 1>(mt, w, u1);
+  const double sv = dot_lanes<D>(u1, u, b1r);
   unroll<0, D>([&](auto jc) {
     constexpr int j = decltype(jc)::value;
     mt[j] = mt[j] * bcast<j>(rd);
@@ -475,18 +506,9 @@ __device__ __forceinline__ void filter_combine(int r, const FiltArrays& x1, cons
     constexpr int j = decltype(jc)::value;
     fma_lanes<0, D>(w, b1[j], -mt[j]);
   });
-  const double bo = dot_lanes<D>(w, sv, x2.b[i2 * D + rr]);
+  const double bo = dot_lanes<D>(w, sv, b2r);
 
   if constexpr (!SO) {
-    // A = W A1
-    const double* A1 = x1.A + i1 * DD;
-    {
-      double ar[D], a[D];
-      load_row16<D>(ar, A1 + rr * D);
-      zero(a);
-      mul_rows<D, D, D>(a, w, ar);
-      if (act) store_row16<D>(y.A + (o * D + r) * D, a);
-    }
     // eta = A1^T (s2 - Xi21 Xi11^-1 U1^T s2) + eta1
     double w2 = 0.0;
     {
@@ -499,36 +521,29 @@ __device__ __forceinline__ void filter_combine(int r, const FiltArrays& x1, cons
       });
     }
     const double s3 = s2 - dot_lanes<D>(b1, w2);
+    if constexpr (kTwo && !kAll) load_rest2();
+    if constexpr (!kTwo) load_row16<D>(ar, A1 + rr * D);
+    // A = W A1
+    {
+      double a[D];
+      zero(a);
+      mul_rows<D, D, D>(a, w, ar);
+      if (act) store_row16<D>(y.A + (o * D + r) * D, a);
+    }
     // Xi22 triangular, then Z = tria([A1^T Xi22 | Z1])
     lq1<D, D, 0, 0>(b2, nullptr, r);
+    if constexpr (!kTwo) load_rest2();
     double z[D];
-    {
-      double a1t[D];
-      load_col16<D>(a1t, A1, rr);
-      const double eo = dot_lanes<D>(a1t, s3, x1.eta[i1 * D + rr]);
-      if (act) y.eta[o * D + r] = eo;
-      zero(z);
-      mul_rows<D, D, 1>(z, a1t, b2);
-    }
-    {
-      double z1[DZ];
-      const double* Z1 = x1.Z + i1 * DD;
-      if constexpr (kLeaf) {
-#pragma unroll
-        for (int c = 0; c < DZ; ++c) z1[c] = Z1[rr * DZ + c];
-      } else {
-        load_row16<DZ>(z1, Z1 + rr * D);
-      }
-      lq1<D, D, DZ, kLeaf ? DZ - 1 : 0>(z, z1, r);
-    }
+    const double eo = dot_lanes<D>(a1t, s3, eta1r);
+    if (act) y.eta[o * D + r] = eo;
+    zero(z);
+    mul_rows<D, D, 1>(z, a1t, b2);
+    lq1<D, D, DZ, kLeaf ? DZ - 1 : 0>(z, z1, r);
     if (act) store_lower16<D>(y.Z + (o * D + r) * D, z, r);
   }
   // U = tria([MT | U2])
-  {
-    double u2[D];
-    load_row16<D>(u2, x2.U + (i2 * D + rr) * D);
-    lq1<D, D, D, 0>(mt, u2, r);
-  }
+  if constexpr (!kTwo) load_row16<D>(u2, U2 + rr * D);
+  lq1<D, D, D, 0>(mt, u2, r);
   if (act) {
     (SO ? so.m : y.b)[o * D + r] = bo;
     store_lower16<D>((SO ? so.L : y.U) + (o * D + r) * D, mt, r);
@@ -546,14 +561,14 @@ __device__ __forceinline__ void smoother_combine(int r, const SmoArrays& x1, con
   constexpr size_t DD = (size_t)D * D;
   const bool act = r < D;
   const int rr = act ? r : 0;
-  double e2[D];
+  double e2[D], e1[SO ? 1 : D];
   load_row16<D>(e2, x2.E + i2 * DD + rr * D);
+  if constexpr (!SO) load_row16<D>(e1, x1.E + i1 * DD + rr * D);
   const double g1 = (SO ? s1.m : x1.g)[i1 * D + rr];
   const double g = x2.g[i2 * D + rr] + dot_lanes<D>(e2, g1);
   if (act) (SO ? so.m : y.g)[o * D + r] = g;
   if constexpr (!SO) {
-    double e1[D], e[D];
-    load_row16<D>(e1, x1.E + i1 * DD + rr * D);
+    double e[D];
     zero(e);
     mul_rows<D, D, D>(e, e2, e1);
     if (act) store_row16<D>(y.E + o * DD + r * D, e);
@@ -583,8 +598,8 @@ struct ObsRow<D, d, true> {
   Obs<D, d, true> o;
   double c[d];
   // (the parameters are read where they are: a local copy indexed by the field's cases would go through scratch)
-  __device__ __forceinline__ void load(const GroupArgs& g, int j, int k, int) {
-    const double* lin = (g.cur[j] ? g.means1 : g.means0) + (size_t)g.base[j] * D;
+  __device__ __forceinline__ void load(const GroupArgs& g, int j, long long base, int k, int) {
+    const double* lin = (g.cur[j] ? g.means1 : g.means0) + (size_t)base * D;
     o.load_at(g.kind[j], g.params + (size_t)j * kMaxParams, g.Pd + (size_t)j * D, lin + (size_t)(k + 1) * D);
 #pragma unroll
     for (int i = 0; i < d; ++i) c[i] = o.c[i];
@@ -656,7 +671,7 @@ template <int D, int d>
 struct ObsRow<D, d, false> {
   static constexpr int NR = d;
   double h[D], R[d], c[d];
-  __device__ __forceinline__ void load(const GroupArgs& g, int, int k, int r) {
+  __device__ __forceinline__ void load(const GroupArgs& g, int, long long, int k, int r) {
     const int i = (r < d) ? r : 0;
     const double* H = g.Hx + ((size_t)k * d + i) * D;
 #pragma unroll
@@ -734,14 +749,15 @@ struct Small {
 // in n.  The first d pivots leave Psi11 (t) and Psi21 (n's first d columns), the rest U = Psi22.
 // Without noise the last d columns are zero throughout and are left out.
 template <int D, int d, bool EK1>
-__device__ __forceinline__ void filter_element(int r, const GroupArgs& g, int j, int k, const FiltArrays& out) {
+__device__ __forceinline__ void filter_element(int r, const GroupArgs& g, int j, long long base, int k,
+                                               const FiltArrays& out) {
   using O = ObsRow<D, d, EK1>;
   constexpr int NR = O::NR, NC = D + NR;
   constexpr size_t DD = (size_t)D * D;
   const bool act = r < D;
   const int rr = act ? r : 0;
   O ob;
-  ob.load(g, j, k, r);
+  ob.load(g, j, base, k, r);
   double f[D];
   load_row16<D>(f, g.F + rr * D);
   double n[NC];
@@ -853,16 +869,16 @@ __device__ __forceinline__ void filter_element(int r, const GroupArgs& g, int j,
 //   Phi = tria([[F L, LQ], [L, 0]]), E = Phi21 Phi11^-1, g = m - E F m, D = Phi22,
 //   S = tria([H Phi11 | R]), yhat = H F m + c.
 // LOWL: L and LQ are lower triangular with LQ's diagonal nonzero (the solver's own model).
-// The observation model is read once the smoother element is stored, so that its values are not held
-// in registers through the factorisation.
 template <int D, int d, bool EK1>
-__device__ __forceinline__ void filter_post(int r, const GroupArgs& g, int j, int s, const double* mp, const double* Lp,
-                                            bool obs, bool dm_only, bool wc, const SmoArrays& sel, size_t ro,
+__device__ __forceinline__ void filter_post(int r, const GroupArgs& g, int j, long long base, int s, const double* mp,
+                                            const double* Lp, bool obs, bool dm_only, bool wc, const SmoArrays& sel, size_t ro,
                                             double* t_ssq, double* t_nll) {
   using O = ObsRow<D, d, EK1>;
   constexpr int NR = O::NR;
   const bool act = r < D;
   const int rr = act ? r : 0;
+  O ob;
+  if (D <= 12 && obs) ob.load(g, j, base, s, r);  // (beyond, its values would spill through the factorisation)
   double a1[D], b1[D], b2[D], fm, mr, rd = 0.0;
   {
     double a2[D], f[D];
@@ -899,7 +915,6 @@ __device__ __forceinline__ void filter_post(int r, const GroupArgs& g, int j, in
       fma_self<i, n2>(a2, -ta);
     });
   }
-  phase();
   if (wc) {
     lq1<D, D, 0, 0>(b2, nullptr, r);
     if (act) store_lower16<D>(sel.Dm + (ro * D + r) * D, b2, r);
@@ -923,9 +938,7 @@ __device__ __forceinline__ void filter_post(int r, const GroupArgs& g, int j, in
     }
     return;
   }
-  phase();
-  O ob;
-  ob.load(g, j, s, r);
+  if (D > 12) ob.load(g, j, base, s, r);
   double sr[D + NR];
   {
     double h[D];

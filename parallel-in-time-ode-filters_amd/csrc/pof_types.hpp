@@ -77,7 +77,7 @@ struct GroupArgs {
   const int* kind;            // [slots]
   const int* Ns;              // [slots]
   const long long* base;      // [slots] first entry of the IVP's range
-  const int* cur;             // [slots] means buffer holding the linearisation points
+  int* cur;                   // [slots] means buffer holding the linearisation points
   const int* wchol;           // [slots] 1: smoother scans also carry the factors
   double* means0;             // [entries, D]
   double* means1;             // [entries, D]
@@ -87,8 +87,6 @@ struct GroupArgs {
   StateArrays spre;           // smoother prefix states
   double* t_ssq;              // [entries] per-step partial terms
   double* t_nll;
-  double* t_obj;
-  double* t_viol;
   double* part;               // [chunks, 4] reduction partials
   double* const* out_means;   // [slots] caller-owned outputs (may hold null)
   double* const* out_chols;
@@ -104,13 +102,20 @@ struct GroupArgs {
   int lq_lower;  // 1: LQ's strict upper part is zero (the smoother-element factorisation skips it)
 };
 
-// Work list of one launch: active IVP a (id ivp[a]) owns the work items
-// [pre[a], pre[a + 1]); total = pre[m].
+// One active IVP of a launch: its slot, its steps and the first entry of its range.
+struct IvpRec {
+  int j, Ns;
+  long long base;
+};
+
+// Work list of one launch: active IVP a (rec[a]) owns the work items [pre[a], pre[a + 1]); total = pre[m].
+// A launch over one IVP carries its record itself (a kernel then starts without a dependent read).
 struct LaunchMap {
-  const int* ivp;
+  const IvpRec* rec;
   const int* pre;
   int m;
   int total;
+  IvpRec one;
 };
 
 }  // namespace pof
