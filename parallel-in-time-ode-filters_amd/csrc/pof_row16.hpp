@@ -11,7 +11,7 @@
 //
 // Against rows split over two lanes of a whole-wavefront worker, with each pivot row passed through
 // LDS and every lane repeating the pivot's scalar part: about 5,300 instructions per combine became
-// about 5,600 per four, and at D = 12 a level of 32,768 combines went from 364 to 107 us (up) and
+// about 4,300 per four (5,100 with a wait in front of every group and groups of at most eight), and at D = 12 a level of 32,768 combines went from 364 to 107 us (up) and
 // from 205 to 70 us (down), the latency of one combine from 19 to 14 us and from 13 to 9.7 us.  What
 // bounds it is FP64 issue: two waves per SIMD (248 registers), 2.5 ns per instruction.
 //
@@ -47,127 +47,232 @@ __device__ __forceinline__ double bcast(double v) {
 }
 
 // y += (lane l's p) * x.  A DPP operand must not have been written by the two instructions before
-// (the hardware does not wait for it and the compiler does not look into an asm statement), hence
-// the s_nop at the head of each group; within a group no source is a result.  Results are early
-// clobbers: an input that holds the same value as a result's initial one (two zeros) must not share
-// its register.
+// (the hardware does not wait for it and the compiler does not look into an asm statement): each group
+// begins with two instructions that write none of its DPP operands, or with s_nop 1, which costs a wavefront
+// as much as a multiply-add.  Within a group no source is a result.  Results are early clobbers: an input
+// that holds the same value as a result's initial one (two zeros) must not share its register.
 #define POF_FMAC(y, p, x, l) \
-  "v_fmac_f64_dpp %[" #y "], %[" #p "], %[" #x "] row_newbcast:%[" #l "] row_mask:0xf bank_mask:0xf\n"
+  "v_fmac_f64_dpp %[" #y "], %[" #p "], " x " row_newbcast:%[" #l "] row_mask:0xf bank_mask:0xf\n"
+
+// M(0) M(1) ... and M(0), M(1), ... of the group sizes
+#define POF_SEQ1(M) M(0)
+#define POF_SEQ2(M) POF_SEQ1(M) M(1)
+#define POF_SEQ3(M) POF_SEQ2(M) M(2)
+#define POF_SEQ4(M) POF_SEQ3(M) M(3)
+#define POF_SEQ5(M) POF_SEQ4(M) M(4)
+#define POF_SEQ6(M) POF_SEQ5(M) M(5)
+#define POF_SEQ7(M) POF_SEQ6(M) M(6)
+#define POF_SEQ8(M) POF_SEQ7(M) M(7)
+#define POF_SEQ9(M) POF_SEQ8(M) M(8)
+#define POF_SEQ10(M) POF_SEQ9(M) M(9)
+#define POF_SEQ11(M) POF_SEQ10(M) M(10)
+#define POF_SEQ12(M) POF_SEQ11(M) M(11)
+#define POF_SEQ13(M) POF_SEQ12(M) M(12)
+#define POF_SEQ14(M) POF_SEQ13(M) M(13)
+#define POF_SEQ15(M) POF_SEQ14(M) M(14)
+#define POF_SEQ16(M) POF_SEQ15(M) M(15)
+#define POF_CSV1(M) M(0)
+#define POF_CSV2(M) POF_CSV1(M), M(1)
+#define POF_CSV3(M) POF_CSV2(M), M(2)
+#define POF_CSV4(M) POF_CSV3(M), M(3)
+#define POF_CSV5(M) POF_CSV4(M), M(4)
+#define POF_CSV6(M) POF_CSV5(M), M(5)
+#define POF_CSV7(M) POF_CSV6(M), M(6)
+#define POF_CSV8(M) POF_CSV7(M), M(7)
+#define POF_CSV9(M) POF_CSV8(M), M(8)
+#define POF_CSV10(M) POF_CSV9(M), M(9)
+#define POF_CSV11(M) POF_CSV10(M), M(10)
+#define POF_CSV12(M) POF_CSV11(M), M(11)
+#define POF_CSV13(M) POF_CSV12(M), M(12)
+#define POF_CSV14(M) POF_CSV13(M), M(13)
+#define POF_CSV15(M) POF_CSV14(M), M(14)
+#define POF_CSV16(M) POF_CSV15(M), M(15)
+// CASE(n) for the group sizes
+#define POF_CASES(CASE)                                                                                            \
+  CASE(1) CASE(2) CASE(3) CASE(4) CASE(5) CASE(6) CASE(7) CASE(8) CASE(9) CASE(10) CASE(11) CASE(12) CASE(13) CASE(14) \
+      CASE(15) CASE(16)
+// the parity of a group's index
+#define POF_PAR0 "0"
+#define POF_PAR1 "1"
+#define POF_PAR2 "0"
+#define POF_PAR3 "1"
+#define POF_PAR4 "0"
+#define POF_PAR5 "1"
+#define POF_PAR6 "0"
+#define POF_PAR7 "1"
+#define POF_PAR8 "0"
+#define POF_PAR9 "1"
+#define POF_PAR10 "0"
+#define POF_PAR11 "1"
+#define POF_PAR12 "0"
+#define POF_PAR13 "1"
+#define POF_PAR14 "0"
+#define POF_PAR15 "1"
+#define POF_PAR(i) POF_PAR##i
+constexpr int kGroup = 16;  // largest group
+#define POF_Y(i) [y##i] "+&v"(y[i])
+#define POF_P(i) [p##i] "v"(p[i])
+#define POF_Q(i) [q##i] "v"(q[i])
+#define POF_L(i) [l##i] "n"(L + i)
 
 // y[c] += bcast_L(p[c]) x, c < N
 template <int L, int N>
 __device__ __forceinline__ void fma_rows(double* y, const double* p, double x) {
-  if constexpr (N >= 8) {
-    asm volatile("s_nop 1\n" POF_FMAC(y0, p0, x, l) POF_FMAC(y1, p1, x, l) POF_FMAC(y2, p2, x, l) POF_FMAC(y3, p3, x, l)
-            POF_FMAC(y4, p4, x, l) POF_FMAC(y5, p5, x, l) POF_FMAC(y6, p6, x, l) POF_FMAC(y7, p7, x, l)
-        : [y0] "+&v"(y[0]), [y1] "+&v"(y[1]), [y2] "+&v"(y[2]), [y3] "+&v"(y[3]), [y4] "+&v"(y[4]), [y5] "+&v"(y[5]),
-          [y6] "+&v"(y[6]), [y7] "+&v"(y[7])
-        : [p0] "v"(p[0]), [p1] "v"(p[1]), [p2] "v"(p[2]), [p3] "v"(p[3]), [p4] "v"(p[4]), [p5] "v"(p[5]),
-          [p6] "v"(p[6]), [p7] "v"(p[7]), [x] "v"(x), [l] "n"(L));
-    if constexpr (N > 8) fma_rows<L, N - 8>(y + 8, p + 8, x);
-  } else if constexpr (N >= 4) {
-    asm volatile("s_nop 1\n" POF_FMAC(y0, p0, x, l) POF_FMAC(y1, p1, x, l) POF_FMAC(y2, p2, x, l) POF_FMAC(y3, p3, x, l)
-        : [y0] "+&v"(y[0]), [y1] "+&v"(y[1]), [y2] "+&v"(y[2]), [y3] "+&v"(y[3])
-        : [p0] "v"(p[0]), [p1] "v"(p[1]), [p2] "v"(p[2]), [p3] "v"(p[3]), [x] "v"(x), [l] "n"(L));
-    if constexpr (N > 4) fma_rows<L, N - 4>(y + 4, p + 4, x);
-  } else if constexpr (N >= 2) {
-    asm volatile("s_nop 1\n" POF_FMAC(y0, p0, x, l) POF_FMAC(y1, p1, x, l)
-        : [y0] "+&v"(y[0]), [y1] "+&v"(y[1])
-        : [p0] "v"(p[0]), [p1] "v"(p[1]), [x] "v"(x), [l] "n"(L));
-    if constexpr (N > 2) fma_rows<L, N - 2>(y + 2, p + 2, x);
-  } else if constexpr (N == 1) {
-    asm volatile("s_nop 1\n" POF_FMAC(y0, p0, x, l) : [y0] "+&v"(y[0]) : [p0] "v"(p[0]), [x] "v"(x), [l] "n"(L));
+  if constexpr (N > kGroup) {
+    fma_rows<L, kGroup>(y, p, x);
+    fma_rows<L, N - kGroup>(y + kGroup, p + kGroup, x);
   }
-}
-
-// y[c] += bcast_L(y[c]) x, c < N (lane L's own values feed the products before they change)
-template <int L, int N>
-__device__ __forceinline__ void fma_self(double* y, double x) {
-  if constexpr (N >= 8) {
-    asm volatile("s_nop 1\n" POF_FMAC(y0, y0, x, l) POF_FMAC(y1, y1, x, l) POF_FMAC(y2, y2, x, l) POF_FMAC(y3, y3, x, l)
-            POF_FMAC(y4, y4, x, l) POF_FMAC(y5, y5, x, l) POF_FMAC(y6, y6, x, l) POF_FMAC(y7, y7, x, l)
-        : [y0] "+&v"(y[0]), [y1] "+&v"(y[1]), [y2] "+&v"(y[2]), [y3] "+&v"(y[3]), [y4] "+&v"(y[4]), [y5] "+&v"(y[5]),
-          [y6] "+&v"(y[6]), [y7] "+&v"(y[7])
-        : [x] "v"(x), [l] "n"(L));
-    if constexpr (N > 8) fma_self<L, N - 8>(y + 8, x);
-  } else if constexpr (N >= 4) {
-    asm volatile("s_nop 1\n" POF_FMAC(y0, y0, x, l) POF_FMAC(y1, y1, x, l) POF_FMAC(y2, y2, x, l) POF_FMAC(y3, y3, x, l)
-        : [y0] "+&v"(y[0]), [y1] "+&v"(y[1]), [y2] "+&v"(y[2]), [y3] "+&v"(y[3])
-        : [x] "v"(x), [l] "n"(L));
-    if constexpr (N > 4) fma_self<L, N - 4>(y + 4, x);
-  } else if constexpr (N >= 2) {
-    asm volatile("s_nop 1\n" POF_FMAC(y0, y0, x, l) POF_FMAC(y1, y1, x, l)
-        : [y0] "+&v"(y[0]), [y1] "+&v"(y[1])
-        : [x] "v"(x), [l] "n"(L));
-    if constexpr (N > 2) fma_self<L, N - 2>(y + 2, x);
-  } else if constexpr (N == 1) {
-    asm volatile("s_nop 1\n" POF_FMAC(y0, y0, x, l) : [y0] "+&v"(y[0]) : [x] "v"(x), [l] "n"(L));
-  }
+#define POF_OP(i) POF_FMAC(y##i, p##i, "%[x]", l)
+#define POF_CASE(n)      \
+  if constexpr (N == n)  \
+    asm volatile("s_nop 1\n" POF_SEQ##n(POF_OP) : POF_CSV##n(POF_Y) : POF_CSV##n(POF_P), [x] "v"(x), [l] "n"(L));
+  POF_CASES(POF_CASE)
+#undef POF_CASE
+#undef POF_OP
 }
 
 // y[c] += bcast_{L + c}(p) x, c < N
 template <int L, int N>
 __device__ __forceinline__ void fma_lanes(double* y, double p, double x) {
-  if constexpr (N >= 4) {
-    asm volatile("s_nop 1\n" POF_FMAC(y0, p, x, l0) POF_FMAC(y1, p, x, l1) POF_FMAC(y2, p, x, l2) POF_FMAC(y3, p, x, l3)
-        : [y0] "+&v"(y[0]), [y1] "+&v"(y[1]), [y2] "+&v"(y[2]), [y3] "+&v"(y[3])
-        : [p] "v"(p), [x] "v"(x), [l0] "n"(L), [l1] "n"(L + 1), [l2] "n"(L + 2), [l3] "n"(L + 3));
-    if constexpr (N > 4) fma_lanes<L + 4, N - 4>(y + 4, p, x);
-  } else if constexpr (N >= 2) {
-    asm volatile("s_nop 1\n" POF_FMAC(y0, p, x, l0) POF_FMAC(y1, p, x, l1)
-        : [y0] "+&v"(y[0]), [y1] "+&v"(y[1])
-        : [p] "v"(p), [x] "v"(x), [l0] "n"(L), [l1] "n"(L + 1));
-    if constexpr (N > 2) fma_lanes<L + 2, N - 2>(y + 2, p, x);
-  } else if constexpr (N == 1) {
-    asm volatile("s_nop 1\n" POF_FMAC(y0, p, x, l0) : [y0] "+&v"(y[0]) : [p] "v"(p), [x] "v"(x), [l0] "n"(L));
+#define POF_OP(i) POF_FMAC(y##i, p, "%[x]", l##i)
+#define POF_CASE(n)      \
+  if constexpr (N == n)  \
+    asm volatile("s_nop 1\n" POF_SEQ##n(POF_OP) : POF_CSV##n(POF_Y) : [p] "v"(p), [x] "v"(x), POF_CSV##n(POF_L));
+  POF_CASES(POF_CASE)
+#undef POF_CASE
+#undef POF_OP
+}
+
+// x *= d, then y[c] -= bcast_{L + c}(p) x, c < N
+template <int L, int N>
+__device__ __forceinline__ void scale_fma_lanes(double& x, double d, double* y, double p) {
+  if constexpr (N == 0) x *= d;
+#define POF_OP(i) POF_FMAC(y##i, p, "-%[x]", l##i)
+#define POF_CASE(n)                                                             \
+  if constexpr (N == n)                                                         \
+    asm volatile("v_mul_f64 %[x], %[x], %[d]\ns_nop 0\n" POF_SEQ##n(POF_OP)     \
+                 : [x] "+&v"(x), POF_CSV##n(POF_Y)                              \
+                 : [p] "v"(p), [d] "v"(d), POF_CSV##n(POF_L));
+  POF_CASES(POF_CASE)
+#undef POF_CASE
+#undef POF_OP
+}
+
+// sum_c bcast_L(p[c]) p[c], c < N: even and odd c in a sum each (the second sum's zero stands where a wait would)
+template <int L, int N>
+__device__ __forceinline__ double dot_self(const double* p) {
+  double s = 0.0, o;
+#define POF_OP(i)                                                                                       \
+  "v_fmac_f64_dpp %[s" POF_PAR(i) "], %[p" #i "], %[p" #i "] row_newbcast:%[l] row_mask:0xf bank_mask:0xf\n"
+#define POF_CASE(n)                                                                                            \
+  if constexpr (N == n)                                                                                        \
+    asm volatile("v_mov_b64 %[s0], 0\nv_mov_b64 %[s1], 0\n" POF_SEQ##n(POF_OP) "v_add_f64 %[s0], %[s0], %[s1]\n" \
+                 : [s0] "=&v"(s), [s1] "=&v"(o)                                                                \
+                 : POF_CSV##n(POF_P), [l] "n"(L));
+  POF_CASES(POF_CASE)
+#undef POF_CASE
+#undef POF_OP
+  if constexpr (N > kGroup) {
+    s = dot_self<L, kGroup>(p);
+    s += dot_self<L, N - kGroup>(p + kGroup);
+  }
+  return s;
+}
+
+// s = sum_c bcast_L(p[c]) p[c], t = sum_c bcast_L(p[c]) q[c], c < N
+template <int L, int N>
+__device__ __forceinline__ void dot_pair(double& s, double& t, const double* p, const double* q) {
+  if constexpr (N == 0) s = t = 0.0;
+#define POF_OP(i) POF_FMAC(s, p##i, "%[p" #i "]", l) POF_FMAC(t, p##i, "%[q" #i "]", l)
+#define POF_CASE(n)                                                             \
+  if constexpr (N == n)                                                         \
+    asm volatile("v_mov_b64 %[s], 0\nv_mov_b64 %[t], 0\n" POF_SEQ##n(POF_OP)    \
+                 : [s] "=&v"(s), [t] "=&v"(t)                                   \
+                 : POF_CSV##n(POF_P), POF_CSV##n(POF_Q), [l] "n"(L));
+  POF_CASES(POF_CASE)
+#undef POF_CASE
+#undef POF_OP
+  if constexpr (N > kGroup) {
+    double s2, t2;
+    dot_pair<L, kGroup>(s, t, p, q);
+    dot_pair<L, N - kGroup>(s2, t2, p + kGroup, q + kGroup);
+    s += s2;
+    t += t2;
   }
 }
 
-// s[c & 1] += bcast_L(p[c]) q[c], c = C .. C + N - 1: even and odd columns in a sum each
-template <int L, int N, int C = 0>
-__device__ __forceinline__ void dot_rows(double (&s)[2], const double* p, const double* q) {
-  double& e = s[C & 1];
-  double& o = s[(C + 1) & 1];
-  if constexpr (N >= 4) {
-    asm volatile("s_nop 1\n" POF_FMAC(e, p0, q0, l) POF_FMAC(o, p1, q1, l) POF_FMAC(e, p2, q2, l) POF_FMAC(o, p3, q3, l)
-        : [e] "+&v"(e), [o] "+&v"(o)
-        : [p0] "v"(p[C]), [p1] "v"(p[C + 1]), [p2] "v"(p[C + 2]), [p3] "v"(p[C + 3]), [q0] "v"(q[C]),
-          [q1] "v"(q[C + 1]), [q2] "v"(q[C + 2]), [q3] "v"(q[C + 3]), [l] "n"(L));
-    if constexpr (N > 4) dot_rows<L, N - 4, C + 4>(s, p, q);
-  } else if constexpr (N >= 2) {
-    asm volatile("s_nop 1\n" POF_FMAC(e, p0, q0, l) POF_FMAC(o, p1, q1, l)
-        : [e] "+&v"(e), [o] "+&v"(o)
-        : [p0] "v"(p[C]), [p1] "v"(p[C + 1]), [q0] "v"(q[C]), [q1] "v"(q[C + 1]), [l] "n"(L));
-    if constexpr (N > 2) dot_rows<L, N - 2, C + 2>(s, p, q);
-  } else if constexpr (N == 1) {
-    asm volatile("s_nop 1\n" POF_FMAC(e, p0, q0, l) : [e] "+&v"(e) : [p0] "v"(p[C]), [q0] "v"(q[C]), [l] "n"(L));
-  }
+// sum_c bcast_L(p[c]) q[c], c < N
+template <int L, int N>
+__device__ __forceinline__ double dot_rows(const double* p, const double* q) {
+  double s;
+#define POF_OP(i) POF_FMAC(s, p##i, "%[q" #i "]", l)
+#define POF_CASE(n)                                                \
+  if constexpr (N == n)                                            \
+    asm volatile("v_mov_b64 %[s], 0\ns_nop 0\n" POF_SEQ##n(POF_OP) \
+                 : [s] "=&v"(s)                                    \
+                 : POF_CSV##n(POF_P), POF_CSV##n(POF_Q), [l] "n"(L));
+  POF_CASES(POF_CASE)
+#undef POF_CASE
+#undef POF_OP
+  return s;
 }
 
-// sum_{k < N} bcast_k(v) x[k]: a row (or, of a transposed matrix, a column) times a vector whose
-// entry k sits in lane k; even and odd k in a sum each
-template <int N, int K = 0>
-__device__ __forceinline__ void dot_lanes_(double (&s)[2], const double* x, double v) {
-  if constexpr (N >= 4) {
-    asm volatile("s_nop 1\n" POF_FMAC(e, v, x0, l0) POF_FMAC(o, v, x1, l1) POF_FMAC(e, v, x2, l2) POF_FMAC(o, v, x3, l3)
-        : [e] "+&v"(s[0]), [o] "+&v"(s[1])
-        : [v] "v"(v), [x0] "v"(x[K]), [x1] "v"(x[K + 1]), [x2] "v"(x[K + 2]), [x3] "v"(x[K + 3]), [l0] "n"(K),
-          [l1] "n"(K + 1), [l2] "n"(K + 2), [l3] "n"(K + 3));
-    dot_lanes_<N - 4, K + 4>(s, x, v);
-  } else if constexpr (N >= 2) {
-    asm volatile("s_nop 1\n" POF_FMAC(e, v, x0, l0) POF_FMAC(o, v, x1, l1)
-        : [e] "+&v"(s[0]), [o] "+&v"(s[1])
-        : [v] "v"(v), [x0] "v"(x[K]), [x1] "v"(x[K + 1]), [l0] "n"(K), [l1] "n"(K + 1));
-    dot_lanes_<N - 2, K + 2>(s, x, v);
-  } else if constexpr (N == 1) {
-    asm volatile("s_nop 1\n" POF_FMAC(e, v, x0, l0) : [e] "+&v"(s[0]) : [v] "v"(v), [x0] "v"(x[K]), [l0] "n"(K));
-  }
+// t = rb (a + sc dot), y[c] -= bcast_L(p[c]) t, c < N: a reflector applied to the tail of other rows
+// (see Pivot).  Returns t.
+template <int L, int N>
+__device__ __forceinline__ double reflect_rows(double* y, const double* p, double rb, double sc, double dot, double a) {
+  double t;
+  if constexpr (N == 0 || N > kGroup) t = rb * fma(sc, dot, a);
+#define POF_OP(i) POF_FMAC(y##i, p##i, "-%[t]", l)
+#define POF_CASE(n)                                                                                           \
+  if constexpr (N == n)                                                                                       \
+    asm volatile("v_fma_f64 %[t], %[sc], %[dot], %[a]\nv_mul_f64 %[t], %[rb], %[t]\n" POF_SEQ##n(POF_OP)      \
+                 : [t] "=&v"(t), POF_CSV##n(POF_Y)                                                            \
+                 : POF_CSV##n(POF_P), [sc] "v"(sc), [dot] "v"(dot), [a] "v"(a), [rb] "v"(rb), [l] "n"(L));
+  POF_CASES(POF_CASE)
+#undef POF_CASE
+#undef POF_OP
+  if constexpr (N > kGroup) fma_rows<L, N>(y, p, -t);
+  return t;
 }
+
+// The same to the tails of the rows of lane L's own set (its values feed the products before they change)
+template <int L, int N>
+__device__ __forceinline__ double reflect_self(double* y, double rb, double sc, double dot, double a) {
+  double t;
+  if constexpr (N == 0) t = rb * fma(sc, dot, a);
+#define POF_OP(i) POF_FMAC(y##i, y##i, "-%[t]", l)
+#define POF_CASE(n)                                                                                           \
+  if constexpr (N == n)                                                                                       \
+    asm volatile("v_fma_f64 %[t], %[sc], %[dot], %[a]\nv_mul_f64 %[t], %[rb], %[t]\n" POF_SEQ##n(POF_OP)      \
+                 : [t] "=&v"(t), POF_CSV##n(POF_Y)                                                            \
+                 : [sc] "v"(sc), [dot] "v"(dot), [a] "v"(a), [rb] "v"(rb), [l] "n"(L));
+  POF_CASES(POF_CASE)
+#undef POF_CASE
+#undef POF_OP
+  if constexpr (N > kGroup) {
+    t = reflect_self<L, kGroup>(y, rb, sc, dot, a);
+    const double t2 = reflect_self<L, N - kGroup>(y + kGroup, rb, sc, dot, a);
+    (void)t2;  // the same value
+  }
+  return t;
+}
+
+// init + sum_{k < N} bcast_k(v) x[k]: a row (or, of a transposed matrix, a column) times a vector whose
+// entry k sits in lane k
 template <int N>
 __device__ __forceinline__ double dot_lanes(const double* x, double v, double init = 0.0) {
-  double s[2] = {init, 0.0};
-  dot_lanes_<N>(s, x, v);
-  return s[0] + s[1];
+  constexpr int L = 0;
+  const double* q = x;
+  double s = init;
+#define POF_OP(i) POF_FMAC(s, v, "%[q" #i "]", l##i)
+#define POF_CASE(n)      \
+  if constexpr (N == n)  \
+    asm volatile("s_nop 1\n" POF_SEQ##n(POF_OP) : [s] "+&v"(s) : [v] "v"(v), POF_CSV##n(POF_Q), POF_CSV##n(POF_L));
+  POF_CASES(POF_CASE)
+#undef POF_CASE
+#undef POF_OP
+  return s;
 }
 
 // ------------------------------------------------------------- compile-time loops
@@ -193,7 +298,7 @@ __device__ __forceinline__ void keep(double& x) { asm volatile("" : "+v"(x)); }
 // y[c] += sum_k x[k] (row k of B)[c] over the columns c < min(N, k + LOW) of row k (LOW = 1: B lower
 // triangular; LOW >= N: full)
 template <int K, int N, int LOW>
-__device__ __forceinline__ void mul_rows(double (&y)[N], const double* x, const double* B) {
+__device__ __forceinline__ void mul_rows(double* y, const double* x, const double* B) {
   unroll<0, K>([&](auto k) {
     constexpr int kk = decltype(k)::value;
     fma_rows<kk, (kk + LOW < N) ? kk + LOW : N>(y, B, x[kk]);
@@ -241,70 +346,38 @@ __device__ __forceinline__ Pivot pivot_nz(double alpha, double sig) {
   return p;
 }
 
-// Any pivot: a zero tail leaves the row (tau = 0, beta = alpha).
-__device__ __forceinline__ Pivot pivot(double alpha, double sig) {
-  const bool nz = sig != 0.0;
-  Pivot p = pivot_nz(nz ? alpha : 1.0, nz ? sig : 1.0);
-  p.beta = nz ? p.beta : alpha;
-  p.rb = nz ? p.rb : 0.0;
+// Any pivot: a zero tail leaves the rows as they are (rb = 0; beta = alpha).
+__device__ __forceinline__ Pivot pivot(double alpha, double sig, bool& nz) {
+  nz = sig != 0.0;
+  const double x = fma(alpha, alpha, sig);
+  Pivot p;
+  double n, rn;
+  norm_rnorm(nz ? x : 1.0, n, rn);
+  p.beta = -copysign(n, alpha);
+  p.den = alpha - p.beta;
+  p.sc = rcp3(p.den);
+  p.rb = nz ? copysign(rn, alpha) : 0.0;
   return p;
 }
 
 // ------------------------------------------------------------- LQ, one row set
-// LQ of a D-row matrix [B1 | B2] (B1 first-block columns a, B2 second-block columns b, rows in lanes
-// 0 .. D - 1): on return a holds the lower triangle of the factor in its columns <= row (entries
-// above are left over and not cleared).  Row r of the second block is zero beyond column
-// max(r, W2).  B1 >= D.
-template <int D, int B1, int B2, int W2>
-__device__ __forceinline__ void lq1(double (&a)[B1], double* b, int r) {
-  unroll<0, D>([&](auto ic) {
+// Pivots 0 .. K - 1 of the LQ of a matrix of N columns a (rows in lanes 0 .. K - 1): on return a holds the
+// lower triangle of the factor in its columns <= row (entries above are left over and not cleared).  The columns
+// from B1 on are a second block, whose row r is zero beyond its column max(r, W2) (W2 = N: a full block, or none);
+// so is the reflector of pivot r, and those columns are left out.
+template <int K, int N, int B1 = N, int W2 = N>
+__device__ __forceinline__ void lq1(double* a, int r) {
+  unroll<0, K>([&](auto ic) {
     constexpr int i = decltype(ic)::value;
-    constexpr int n1 = B1 - 1 - i;
-    constexpr int band = (i > W2 ? i : W2) + 1;
-    constexpr int n2 = (band < B2) ? band : B2;
-    if constexpr (n1 + n2 > 0) {
-      double s[2] = {0.0, 0.0};
-      dot_rows<i, n1, i + 1>(s, a, a);
-      dot_rows<i, n2, 0>(s, b, b);
-      const double dot = s[0] + s[1];
-      const Pivot p = pivot(bcast<i>(a[i]), bcast<i>(dot));
-      const double tws = p.rb * fma(p.sc, dot, a[i]);
-      a[i] = (r == i) ? p.beta : fma(-p.den, tws, a[i]);
-      fma_self<i, n1>(a + i + 1, -tws);
-      fma_self<i, n2>(b, -tws);
+    constexpr int band = B1 + (i > W2 ? i : W2) + 1;
+    constexpr int n = (band < N ? band : N) - 1 - i;
+    if constexpr (n > 0) {  // a length-1 tail: H = I
+      const double dot = dot_self<i, n>(a + i + 1);
+      bool nz;
+      const Pivot p = pivot(bcast<i>(a[i]), bcast<i>(dot), nz);
+      const double t = reflect_self<i, n>(a + i + 1, p.rb, p.sc, dot, a[i]);
+      a[i] = (r == i && nz) ? p.beta : fma(-p.den, t, a[i]);
     }
-  });
-}
-
-// The remaining pivots of a square factor whose rows r < D have N <= D columns that may be nonzero
-// (the rest zero): a zero column after a zero tail is left as it is.
-template <int D, int N>
-__device__ __forceinline__ void lq_rows(double (&a)[D], int r) {
-  unroll<0, N - 1>([&](auto ic) {
-    constexpr int i = decltype(ic)::value;
-    constexpr int n = N - 1 - i;
-    double s[2] = {0.0, 0.0};
-    dot_rows<i, n, i + 1>(s, a, a);
-    const double dot = s[0] + s[1];
-    const Pivot p = pivot(bcast<i>(a[i]), bcast<i>(dot));
-    const double tws = p.rb * fma(p.sc, dot, a[i]);
-    a[i] = (r == i) ? p.beta : fma(-p.den, tws, a[i]);
-    fma_self<i, n>(a + i + 1, -tws);
-  });
-}
-// LQ of a matrix of NR rows (lanes 0 .. NR - 1) and N > NR columns
-template <int NR, int N>
-__device__ __forceinline__ void lq_top(double (&a)[N], int r) {
-  unroll<0, NR>([&](auto ic) {
-    constexpr int i = decltype(ic)::value;
-    constexpr int n = N - 1 - i;
-    double s[2] = {0.0, 0.0};
-    dot_rows<i, n, i + 1>(s, a, a);
-    const double dot = s[0] + s[1];
-    const Pivot p = pivot(bcast<i>(a[i]), bcast<i>(dot));
-    const double tws = p.rb * fma(p.sc, dot, a[i]);
-    a[i] = (r == i) ? p.beta : fma(-p.den, tws, a[i]);
-    fma_self<i, n>(a + i + 1, -tws);
   });
 }
 
@@ -325,7 +398,7 @@ __device__ __forceinline__ void load_row16(double (&x)[N], const double* p) {
   }
 }
 template <int N>
-__device__ __forceinline__ void store_row16(double* p, const double (&x)[N]) {
+__device__ __forceinline__ void store_row16(double* p, const double* x) {
   if constexpr (N % 2 == 0) {
 #pragma unroll
     for (int i = 0; i < N; i += 2) *reinterpret_cast<double2*>(p + i) = make_double2(x[i], x[i + 1]);
@@ -342,10 +415,10 @@ __device__ __forceinline__ void load_col16(double (&x)[N], const double* M, int 
 }
 // the lower triangle of a factor, its strict upper part cleared
 template <int N>
-__device__ __forceinline__ void store_lower16(double* p, double (&x)[N], int r) {
+__device__ __forceinline__ void store_lower16(double* p, double* x, int r) {
 #pragma unroll
   for (int c = 1; c < N; ++c) x[c] = (c > r) ? 0.0 : x[c];
-  store_row16(p, x);
+  store_row16<N>(p, x);
 }
 
 // ------------------------------------------------------------- filter combine
@@ -426,7 +499,7 @@ __device__ __forceinline__ void filter_combine(int r, const FiltArrays& x1, cons
   }
 
   double s2 = 0.0, uu = 0.0;
-  double a1[D], b1[D], b2[D], rd = 0.0;  // Xi11, Xi21, Xi22; rd: 1 / Xi11[r][r] in lane r
+  double x11[D], x21[D], b[DZ + D], rd = 0.0;  // Xi11, Xi21; rd: 1 / Xi11[r][r] in lane r
   if constexpr (!SO) {
     // s2 = eta2 - Z2 (Z2^T b1), uu = U1^T s2
     const double t = dot_lanes<D>(z2t, b1r);
@@ -435,56 +508,45 @@ __device__ __forceinline__ void filter_combine(int r, const FiltArrays& x1, cons
   }
   const double u = dot_lanes<D>(u1t, eta2r);
   {
-    double a2[D];
-    {
-      double x[DZ];
-      zero(x);
-      mul_rows<D, DZ, kLow>(x, u1t, z2);
+    double a[DZ + D];
+    zero(a);
+    mul_rows<D, DZ, kLow>(a, u1t, z2);
 #pragma unroll
-      for (int c = 0; c < DZ; ++c) {
-        a1[c] = x[c];
-        b1[c] = z2[c];
-      }
-    }
+    for (int c = 0; c < DZ; ++c) b[c] = z2[c];
     unroll<0, D>([&](auto ic) {
       constexpr int i = decltype(ic)::value;
-      constexpr int n1 = (i < DZ) ? DZ - 1 - i : 0;
-      double sa[2] = {0.0, 0.0}, sb[2] = {0.0, 0.0};
-      dot_rows<i, n1, i + 1>(sa, a1, a1);
-      dot_rows<i, n1, i + 1>(sb, a1, b1);
-      dot_rows<i, i, 0>(sa, a2, a2);
-      dot_rows<i, i, 0>(sb, a2, b2);
-      const double da = sa[0] + sa[1], db = sb[0] + sb[1];
+      // the tail: columns i + 1 .. DZ - 1 of the first block, 0 .. i - 1 of the second
+      constexpr int c0 = (i < DZ) ? i + 1 : DZ, n = DZ + i - c0;
+      double da, db;
+      dot_pair<i, n>(da, db, a + c0, b + c0);
       const double sig = bcast<i>(da) + 1.0;
-      double ta, tb;
+      double ta, tb, rp;
       if constexpr (i < DZ) {
-        const Pivot p = pivot_nz(bcast<i>(a1[i]), sig);
-        ta = p.rb * fma(p.sc, da, a1[i]);
-        tb = p.rb * fma(p.sc, db, b1[i]);
-        a1[i] = fma(-p.den, ta, a1[i]);
-        b1[i] = fma(-p.den, tb, b1[i]);
-        rd = (r == i) ? -p.rb : rd;
-        keep(rd);
+        const Pivot p = pivot_nz(bcast<i>(a[i]), sig);
+        tb = reflect_rows<i, n>(b + c0, a + c0, p.rb, p.sc, db, b[i]);
+        ta = reflect_self<i, n>(a + c0, p.rb, p.sc, da, a[i]);
+        x11[i] = fma(-p.den, ta, a[i]);
+        x21[i] = fma(-p.den, tb, b[i]);
+        rp = -p.rb;
       } else {
         // column i of the first block is zero: alpha = 0, den = norm, beta = -norm
-        double n, rn;
-        norm_rnorm(sig, n, rn);
-        const double wa = rn * da, wb = rn * db;
-        ta = rn * wa;
-        tb = rn * wb;
-        a1[i] = -wa;
-        b1[i] = -wb;
-        rd = (r == i) ? -rn : rd;
-        keep(rd);
+        double nr, rn;
+        norm_rnorm(sig, nr, rn);
+        tb = reflect_rows<i, n>(b + c0, a + c0, rn, rn, db, 0.0);
+        ta = reflect_self<i, n>(a + c0, rn, rn, da, 0.0);
+        x11[i] = -rn * da;
+        x21[i] = -rn * db;
+        rp = -rn;
       }
-      fma_rows<i, n1>(b1 + i + 1, a1 + i + 1, -tb);
-      fma_rows<i, i>(b2, a2, -tb);
-      fma_self<i, n1>(a1 + i + 1, -ta);
-      fma_self<i, i>(a2, -ta);
-      a2[i] = -ta;
-      b2[i] = -tb;
+      rd = (r == i) ? rp : rd;
+      keep(rd);
+      keep(x11[i]);
+      keep(x21[i]);
+      a[DZ + i] = -ta;
+      b[DZ + i] = -tb;
     });
   }
+  double* x22 = b + DZ;
   if constexpr (!kTwo) {
     load_row16<D>(w, A2 + rr * D);
     load_row16<D>(u1, U1 + rr * D);
@@ -493,18 +555,17 @@ __device__ __forceinline__ void filter_combine(int r, const FiltArrays& x1, cons
   }
 
   // MT = A2 U1 Xi11^-T, W = A2 - MT Xi21^T, b = W (b1 + U1 u) + b2
-  double mt[D];
+  double mt[2 * D];
   zero(mt);
   mul_rows<D, D, 1>(mt, w, u1);
   const double sv = dot_lanes<D>(u1, u, b1r);
   unroll<0, D>([&](auto jc) {
     constexpr int j = decltype(jc)::value;
-    mt[j] = mt[j] * bcast<j>(rd);
-    fma_lanes<j + 1, D - 1 - j>(mt + j + 1, a1[j], -mt[j]);
+    scale_fma_lanes<j + 1, D - 1 - j>(mt[j], bcast<j>(rd), mt + j + 1, x11[j]);
   });
   unroll<0, D>([&](auto jc) {
     constexpr int j = decltype(jc)::value;
-    fma_lanes<0, D>(w, b1[j], -mt[j]);
+    fma_lanes<0, D>(w, x21[j], -mt[j]);
   });
   const double bo = dot_lanes<D>(w, sv, b2r);
 
@@ -517,10 +578,10 @@ __device__ __forceinline__ void filter_combine(int r, const FiltArrays& x1, cons
         constexpr int j = decltype(jc)::value;
         const double wj = bcast<j>(x * rd);
         w2 = (r == j) ? wj : w2;
-        x = fma(-a1[j], wj, x);
+        x = fma(-x11[j], wj, x);
       });
     }
-    const double s3 = s2 - dot_lanes<D>(b1, w2);
+    const double s3 = s2 - dot_lanes<D>(x21, w2);
     if constexpr (kTwo && !kAll) load_rest2();
     if constexpr (!kTwo) load_row16<D>(ar, A1 + rr * D);
     // A = W A1
@@ -531,19 +592,23 @@ __device__ __forceinline__ void filter_combine(int r, const FiltArrays& x1, cons
       if (act) store_row16<D>(y.A + (o * D + r) * D, a);
     }
     // Xi22 triangular, then Z = tria([A1^T Xi22 | Z1])
-    lq1<D, D, 0, 0>(b2, nullptr, r);
+    lq1<D, D>(x22, r);
     if constexpr (!kTwo) load_rest2();
-    double z[D];
+    double z[D + DZ];
     const double eo = dot_lanes<D>(a1t, s3, eta1r);
     if (act) y.eta[o * D + r] = eo;
     zero(z);
-    mul_rows<D, D, 1>(z, a1t, b2);
-    lq1<D, D, DZ, kLeaf ? DZ - 1 : 0>(z, z1, r);
+    mul_rows<D, D, 1>(z, a1t, x22);
+#pragma unroll
+    for (int c = 0; c < DZ; ++c) z[D + c] = z1[c];
+    lq1<D, D + DZ, D, kLeaf ? DZ - 1 : 0>(z, r);
     if (act) store_lower16<D>(y.Z + (o * D + r) * D, z, r);
   }
   // U = tria([MT | U2])
   if constexpr (!kTwo) load_row16<D>(u2, U2 + rr * D);
-  lq1<D, D, D, 0>(mt, u2, r);
+#pragma unroll
+  for (int c = 0; c < D; ++c) mt[D + c] = u2[c];
+  lq1<D, 2 * D, D, 0>(mt, r);
   if (act) {
     (SO ? so.m : y.b)[o * D + r] = bo;
     store_lower16<D>((SO ? so.L : y.U) + (o * D + r) * D, mt, r);
@@ -574,12 +639,14 @@ __device__ __forceinline__ void smoother_combine(int r, const SmoArrays& x1, con
     if (act) store_row16<D>(y.E + o * DD + r * D, e);
   }
   if (wc) {
-    double d1[D], d2[D], t[D];
+    double d1[D], d2[D], t[2 * D];
     load_row16<D>(d1, (SO ? s1.L : x1.Dm) + i1 * DD + rr * D);
     load_row16<D>(d2, x2.Dm + i2 * DD + rr * D);
     zero(t);
     mul_rows<D, D, D>(t, e2, d1);  // the first aggregate's D may be a caller's factor, not triangular
-    lq1<D, D, D, 0>(t, d2, r);
+#pragma unroll
+    for (int c = 0; c < D; ++c) t[D + c] = d2[c];
+    lq1<D, 2 * D, D, 0>(t, r);
     if (act) store_lower16<D>((SO ? so.L : y.Dm) + o * DD + r * D, t, r);
   }
 }
@@ -693,11 +760,7 @@ struct ObsRow<D, d, false> {
   __device__ __forceinline__ void times_col(const double* F, int r, double (&y)[d]) const {
     double f[D];
     load_col16<D>(f, F, r);
-    unroll<0, d>([&](auto ic) {
-      double s[2] = {0.0, 0.0};
-      dot_rows<decltype(ic)::value, D>(s, h, f);
-      y[decltype(ic)::value] = s[0] + s[1];
-    });
+    unroll<0, d>([&](auto ic) { y[decltype(ic)::value] = dot_rows<decltype(ic)::value, D>(h, f); });
   }
   __device__ __forceinline__ void sub_gain(const double (&K)[d], const double (&M)[D], double (&x)[D]) const {
     double kh[D];
@@ -774,13 +837,15 @@ __device__ __forceinline__ void filter_element(int r, const GroupArgs& g, int j,
       for (int c = 0; c < D; ++c) nz = nz || l0[c] != 0.0;
       // N1 = tria([F L0 | LQ]); of a zero L0 it is N1z
       if ((__ballot(nz) >> ((threadIdx.x & 63) & ~(kRow - 1))) & 0xffffull) {
-        double lq[D];
+        double lq[D], m[2 * D];
         load_row16<D>(lq, g.LQ + rr * D);
-        zero(n1);
-        mul_rows<D, D, D>(n1, f, l0);
-        lq1<D, D, D, D>(n1, lq, r);
+        zero(m);
+        mul_rows<D, D, D>(m, f, l0);
 #pragma unroll
-        for (int c = 1; c < D; ++c) n1[c] = (c > r) ? 0.0 : n1[c];
+        for (int c = 0; c < D; ++c) m[D + c] = lq[c];
+        lq1<D, 2 * D>(m, r);
+#pragma unroll
+        for (int c = 0; c < D; ++c) n1[c] = (c > r) ? 0.0 : m[c];
       }
     }
 #pragma unroll
@@ -804,16 +869,14 @@ __device__ __forceinline__ void filter_element(int r, const GroupArgs& g, int j,
   unroll<0, d>([&](auto ic) {
     constexpr int i = decltype(ic)::value;
     constexpr int nt = NC - 1 - i;
-    double st[2] = {0.0, 0.0}, sn[2] = {0.0, 0.0};
-    dot_rows<i, nt, i + 1>(st, t, t);
-    dot_rows<i, nt, i + 1>(sn, t, n);
-    const double dt = st[0] + st[1], dn = sn[0] + sn[1];
-    const Pivot p = pivot(bcast<i>(t[i]), bcast<i>(dt));
-    const double tt = p.rb * fma(p.sc, dt, t[i]), tn = p.rb * fma(p.sc, dn, n[i]);
-    t[i] = (r == i) ? p.beta : fma(-p.den, tt, t[i]);
+    double dt, dn;
+    dot_pair<i, nt>(dt, dn, t + i + 1, n + i + 1);
+    bool nz;
+    const Pivot p = pivot(bcast<i>(t[i]), bcast<i>(dt), nz);
+    const double tn = reflect_rows<i, nt>(n + i + 1, t + i + 1, p.rb, p.sc, dn, n[i]);
+    const double tt = reflect_self<i, nt>(t + i + 1, p.rb, p.sc, dt, t[i]);
+    t[i] = (r == i && nz) ? p.beta : fma(-p.den, tt, t[i]);
     n[i] = fma(-p.den, tn, n[i]);
-    fma_rows<i, nt>(n + i + 1, t + i + 1, -tn);
-    fma_self<i, nt>(t + i + 1, -tt);
   });
   Small<d> p11;
   p11.load(t);
@@ -858,7 +921,7 @@ __device__ __forceinline__ void filter_element(int r, const GroupArgs& g, int j,
     double u[D];
 #pragma unroll
     for (int c = 0; c < D; ++c) u[c] = (d + c < NC) ? n[(d + c < NC) ? d + c : 0] : 0.0;
-    lq_rows<D, NC - d>(u, r);
+    lq1<NC - d, NC - d>(u, r);  // the last pivot has no tail
     if (act) store_lower16<D>(out.U + o * D, u, r);
   }
 }
@@ -879,56 +942,56 @@ __device__ __forceinline__ void filter_post(int r, const GroupArgs& g, int j, lo
   const int rr = act ? r : 0;
   O ob;
   if (D <= 12 && obs) ob.load(g, j, base, s, r);  // (beyond, its values would spill through the factorisation)
-  double a1[D], b1[D], b2[D], fm, mr, rd = 0.0;
+  double x11[D], b[2 * D], fm, mr, rd = 0.0;
   {
-    double a2[D], f[D];
+    double a[2 * D], f[D], l0[D], lq[D];
     mr = mp[rr];
-    load_row16<D>(b1, Lp + rr * D);
+    load_row16<D>(l0, Lp + rr * D);
     load_row16<D>(f, g.F + rr * D);
-    load_row16<D>(a2, g.LQ + rr * D);
+    load_row16<D>(lq, g.LQ + rr * D);
     fm = dot_lanes<D>(f, mr);
-    zero(a1);
-    mul_rows<D, D, EK1 ? 1 : D>(a1, f, b1);
-    zero(b2);
+    zero(a);
+    mul_rows<D, D, EK1 ? 1 : D>(a, f, l0);
+#pragma unroll
+    for (int c = 0; c < D; ++c) {
+      a[D + c] = lq[c];
+      b[c] = l0[c];
+      b[D + c] = 0.0;
+    }
     unroll<0, D>([&](auto ic) {
       constexpr int i = decltype(ic)::value;
-      constexpr int n1 = D - 1 - i, n2 = EK1 ? i + 1 : D;
-      double sa[2] = {0.0, 0.0}, sb[2] = {0.0, 0.0};
-      dot_rows<i, n1, i + 1>(sa, a1, a1);
-      dot_rows<i, n1, i + 1>(sb, a1, b1);
-      dot_rows<i, n2, 0>(sa, a2, a2);
-      dot_rows<i, (EK1 ? i : D), 0>(sb, a2, b2);
-      const double da = sa[0] + sa[1], db = sb[0] + sb[1];
-      const double alpha = bcast<i>(a1[i]), sig = bcast<i>(da);
-      const Pivot p = EK1 ? pivot_nz(alpha, sig) : pivot(alpha, sig);
-      const double ta = p.rb * fma(p.sc, da, a1[i]), tb = p.rb * fma(p.sc, db, b1[i]);
-      a1[i] = (r == i) ? p.beta : fma(-p.den, ta, a1[i]);
-      b1[i] = fma(-p.den, tb, b1[i]);
-      const double rp = EK1 ? -p.rb : 1.0 / p.beta;
+      constexpr int n = EK1 ? D : 2 * D - 1 - i;  // LQ lower triangular: second-block columns 0 .. i
+      double da, db;
+      dot_pair<i, n>(da, db, a + i + 1, b + i + 1);
+      const double alpha = bcast<i>(a[i]), sig = bcast<i>(da);
+      bool nz = true;
+      const Pivot p = EK1 ? pivot_nz(alpha, sig) : pivot(alpha, sig, nz);
+      const double tb = reflect_rows<i, n>(b + i + 1, a + i + 1, p.rb, p.sc, db, b[i]);
+      const double ta = reflect_self<i, n>(a + i + 1, p.rb, p.sc, da, a[i]);
+      const double beta = nz ? p.beta : alpha;
+      x11[i] = (r == i) ? beta : fma(-p.den, ta, a[i]);
+      b[i] = fma(-p.den, tb, b[i]);
+      const double rp = EK1 ? -p.rb : 1.0 / beta;
       rd = (r == i) ? rp : rd;
       keep(rd);
-      keep(a1[i]);
-      keep(b1[i]);
-      fma_rows<i, n1>(b1 + i + 1, a1 + i + 1, -tb);
-      fma_rows<i, n2>(b2, a2, -tb);
-      fma_self<i, n1>(a1 + i + 1, -ta);
-      fma_self<i, n2>(a2, -ta);
+      keep(x11[i]);
+      keep(b[i]);
     });
   }
   if (wc) {
-    lq1<D, D, 0, 0>(b2, nullptr, r);
-    if (act) store_lower16<D>(sel.Dm + (ro * D + r) * D, b2, r);
+    lq1<D, D>(b + D, r);
+    if (act) store_lower16<D>(sel.Dm + (ro * D + r) * D, b + D, r);
   }
   if (dm_only) return;
   // E = Phi21 Phi11^-1
   unroll_down<D - 1, 0>([&](auto jc) {
     constexpr int j = decltype(jc)::value;
-    b1[j] = b1[j] * bcast<j>(rd);
-    fma_rows<j, j>(b1, a1, -b1[j]);
+    b[j] = b[j] * bcast<j>(rd);
+    fma_rows<j, j>(b, x11, -b[j]);
   });
-  const double gr = mr - dot_lanes<D>(b1, fm);
+  const double gr = mr - dot_lanes<D>(b, fm);
   if (act) {
-    store_row16<D>(sel.E + (ro * D + r) * D, b1);
+    store_row16<D>(sel.E + (ro * D + r) * D, b);
     sel.g[ro * D + r] = gr;
   }
   if (!obs) {
@@ -943,13 +1006,13 @@ __device__ __forceinline__ void filter_post(int r, const GroupArgs& g, int j, lo
   {
     double h[D];
     zero(h);
-    ob.template times_rows<1>(r, a1, h);
+    ob.template times_rows<1>(r, x11, h);
 #pragma unroll
     for (int c = 0; c < D; ++c) sr[c] = h[c];
 #pragma unroll
     for (int c = D; c < D + NR; ++c) sr[c] = ob.r_at(c - D);
   }
-  lq_top<d, D + NR>(sr, r);
+  lq1<d, D + NR>(sr, r);
   Small<d> S;
   S.load(sr);
   double yh[d], w[d];
