@@ -1009,9 +1009,16 @@ struct Obs<D, d, true> {
   // linearise at the (preconditioned) state mean m
   __device__ __forceinline__ void load_at(const ModelArgs& a, const double* m) { load_at(a.kind, a.params, a.Pd, m); }
   __device__ __forceinline__ void load_at(int kind, const double* params, const double* Pd, const double* m) {
+    double mi[d];
+#pragma unroll
+    for (int i = 0; i < d; ++i) mi[i] = m[i * q1];
+    load_entries(kind, params, Pd, mi);
+  }
+  // the same of the mean's entries i q1, the ones that the field reads
+  __device__ __forceinline__ void load_entries(int kind, const double* params, const double* Pd, const double (&mi)[d]) {
     double y[d];
 #pragma unroll
-    for (int i = 0; i < d; ++i) y[i] = Pd[i * q1] * m[i * q1];
+    for (int i = 0; i < d; ++i) y[i] = Pd[i * q1] * mi[i];
     double f[d];
     double J[d][d];
     field_and_jacobian<d>(kind, params, y, f, J);

@@ -286,8 +286,9 @@ __global__ __launch_bounds__(r16::kBlock, 2) void k_filter_leaf16(GroupArgs g, L
 // factorisation and is formed only when the IVP's smoothed factors are wanted
 // this iteration (wchol).  mode kPostDm recomputes just D, for the factor pass
 // of an IVP whose last iteration carried means only; kPostNoObs forms the
-// smoother elements without observation statistics (smoother on its own).
-enum PostMode : int { kPostFull = 0, kPostDm = 1, kPostNoObs = 2 };
+// smoother elements without observation statistics (smoother on its own);
+// kPostGain (D <= 16) does so beside statistics that the sequential filter wrote.
+enum PostMode : int { kPostFull = 0, kPostDm = 1, kPostNoObs = 2, kPostGain = 3 };
 template <int D, int d, bool EK1>
 __global__ __launch_bounds__((Geo<D, kLdsPost>::BLOCK)) void k_filter_post(GroupArgs g, LaunchMap lm, int mode) {
   extern __shared__ double smem[];
@@ -492,8 +493,8 @@ __global__ __launch_bounds__(r16::kBlock, 2) void k_filter_post16(GroupArgs g, L
     return;
   }
   const bool dm = mode == kPostDm;
-  r16::filter_post<D, d, EK1>(r, g, j, base, s, mp, Lp, mode == kPostFull, dm, dm || g.wchol[j] != 0, sel, ro, g.t_ssq + base,
-                              g.t_nll + base);
+  r16::filter_post<D, d, EK1>(r, g, j, base, s, mp, Lp, mode == kPostFull, dm, dm || g.wchol[j] != 0, sel, ro,
+                              (mode == kPostGain) ? nullptr : g.t_ssq + base, g.t_nll + base);
 }
 
 // Smoother up-sweep, D > 16
@@ -1057,6 +1058,25 @@ __global__ __launch_bounds__((Geo<D, kLdsSeq>::BLOCK)) void k_seq_smooth(GroupAr
   }
 }
 
+// k_seq_filter with one IVP per row, D <= 16
+template <int D, int d, bool EK1, bool AT_PRED>
+__global__ __launch_bounds__(r16::kBlock, 1) void k_seq_filter16(GroupArgs g, LaunchMap lm) {
+  __shared__ double sh[r16::kPerBlock][D + kMaxParams];
+  Item it;
+  const int w = threadIdx.x / r16::kRow;
+  if (!locate(lm, blockIdx.x * r16::kPerBlock + w, it)) return;
+  r16::seq_filter<D, d, EK1, AT_PRED>(threadIdx.x % r16::kRow, g, it.j, it.base, it.Ns, at(g.fpre, it.base, D), sh[w]);
+}
+
+// k_seq_smooth over smoother elements, D <= 16
+template <int D>
+__global__ __launch_bounds__(r16::kBlock, 1) void k_seq_smooth16(GroupArgs g, LaunchMap lm) {
+  Item it;
+  if (!locate(lm, blockIdx.x * r16::kPerBlock + threadIdx.x / r16::kRow, it)) return;
+  r16::seq_smooth<D>(threadIdx.x % r16::kRow, g, it.j, it.Ns, at(g.fpre, it.base, D), at(g.spre, it.base, D),
+                     at(g.sel, it.base, D));
+}
+
 // ------------------------------------------------------------ launch logic
 template <int D, int K>
 inline unsigned grid_workers(size_t nworkers) {
@@ -1226,6 +1246,31 @@ hipError_t run_iteration(const GroupArgs& g, const LaunchPlan& p, double* scal, 
   return iteration_tail<D>(g, p, scal, d, st, rec);
 }
 
+// The sequential filter of every active IVP
+template <int D, int d, bool EK1, bool AT_PRED>
+void launch_seq_filter(const GroupArgs& g, const LaunchPlan& p, hipStream_t st) {
+  const LaunchMap one = p.map(p.one_off, p.one_total);
+  if constexpr (D <= r16::kRow)
+    POF_LAUNCH16((k_seq_filter16<D, d, EK1, AT_PRED>), p.one_total, st, g, one);
+  else
+    POF_LAUNCH((k_seq_filter<D, d, EK1, AT_PRED>), kLdsSeq, p.one_total, st, g, one);
+}
+
+// The sequential smoother of every active IVP.  D <= 16: mode says what of the smoother elements it needs
+// formed (kPostDm: their gains are there).
+template <int D, int d, bool EK1>
+void launch_seq_smooth(const GroupArgs& g, const LaunchPlan& p, int mode, hipStream_t st, Rec& rec) {
+  const LaunchMap one = p.map(p.one_off, p.one_total);
+  if constexpr (D <= r16::kRow) {
+    launch_post<D, d, EK1>(g, p, mode, st);
+    rec(kKFilterPost, p.leaf_total);
+    POF_LAUNCH16((k_seq_smooth16<D>), p.one_total, st, g, one);
+  } else {
+    POF_LAUNCH((k_seq_smooth<D>), kLdsSeq, p.one_total, st, g, one);
+  }
+  rec(kKSmoothUp, p.leaf_total);
+}
+
 // One sequential IEKS iteration (pof/step.py:33-45 with sequential=True) or,
 // with at_pred, the single pass of sequential_eks_solve (pof/solver.py:76-96):
 // sequential filter and smoother, then the smoothed means, objective,
@@ -1234,17 +1279,17 @@ template <int D, int d>
 hipError_t run_seq_iteration(const GroupArgs& g, const LaunchPlan& p, double* scal, int at_pred, hipStream_t st,
                              KernelTimer* t) {
   Rec rec(t, st);
-  const LaunchMap one = p.map(p.one_off, p.one_total);
-  if (g.affine) {
-    POF_LAUNCH((k_seq_filter<D, d, false, false>), kLdsSeq, p.one_total, st, g, one);
-  } else if (at_pred) {
-    POF_LAUNCH((k_seq_filter<D, d, true, true>), kLdsSeq, p.one_total, st, g, one);
-  } else {
-    POF_LAUNCH((k_seq_filter<D, d, true, false>), kLdsSeq, p.one_total, st, g, one);
-  }
+  if (g.affine)
+    launch_seq_filter<D, d, false, false>(g, p, st);
+  else if (at_pred)
+    launch_seq_filter<D, d, true, true>(g, p, st);
+  else
+    launch_seq_filter<D, d, true, false>(g, p, st);
   rec(kKFilterLeaf, p.leaf_total);
-  POF_LAUNCH((k_seq_smooth<D>), kLdsSeq, p.one_total, st, g, one);
-  rec(kKSmoothUp, p.leaf_total);
+  if (g.affine)
+    launch_seq_smooth<D, d, false>(g, p, kPostGain, st, rec);
+  else
+    launch_seq_smooth<D, d, true>(g, p, kPostGain, st, rec);
   return iteration_tail<D>(g, p, scal, d, st, rec);
 }
 
@@ -1256,8 +1301,7 @@ hipError_t run_smooth_only(const GroupArgs& g, const LaunchPlan& p, double* scal
                            KernelTimer* t) {
   Rec rec(t, st);
   if (sequential) {
-    POF_LAUNCH((k_seq_smooth<D>), kLdsSeq, p.one_total, st, g, p.map(p.one_off, p.one_total));
-    rec(kKSmoothUp, p.leaf_total);
+    launch_seq_smooth<D, d, false>(g, p, kPostNoObs, st, rec);
   } else {
     launch_post<D, d, false>(g, p, kPostNoObs, st);
     rec(kKFilterPost, p.leaf_total);
@@ -1270,8 +1314,10 @@ hipError_t run_smooth_only(const GroupArgs& g, const LaunchPlan& p, double* scal
 template <int D, int d>
 hipError_t run_seq_smooth_chol(const GroupArgs& g, const LaunchPlan& p, hipStream_t st, KernelTimer* t) {
   Rec rec(t, st);
-  POF_LAUNCH((k_seq_smooth<D>), kLdsSeq, p.one_total, st, g, p.map(p.one_off, p.one_total));
-  rec(kKSmoothUp, p.leaf_total);
+  if (g.affine)
+    launch_seq_smooth<D, d, false>(g, p, kPostDm, st, rec);
+  else
+    launch_seq_smooth<D, d, true>(g, p, kPostDm, st, rec);
   return hipGetLastError();
 }
 

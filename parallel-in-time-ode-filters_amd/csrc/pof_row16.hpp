@@ -671,6 +671,12 @@ struct ObsRow<D, d, true> {
 #pragma unroll
     for (int i = 0; i < d; ++i) c[i] = o.c[i];
   }
+  // at the mean's entries i q1
+  __device__ __forceinline__ void load_entries(int kind, const double* params, const double* Pd, const double (&mi)[d]) {
+    o.load_entries(kind, params, Pd, mi);
+#pragma unroll
+    for (int i = 0; i < d; ++i) c[i] = o.c[i];
+  }
   __device__ __forceinline__ double r_at(int) const { return 0.0; }
   // out[c] += (H M)[r][c] for r < d, M's row j (columns < j + LOW) in lane j
   template <int LOW>
@@ -803,6 +809,24 @@ struct Small {
   }
 };
 
+// The first d pivots of the LQ of [[t], [n]]: d rows t (lanes 0 .. d - 1) and D rows n of NC columns each.  Leaves the
+// factor of the first block row in t and its columns of the second in n[0 .. d - 1].
+template <int d, int NC>
+__device__ __forceinline__ void lq_obs(double (&t)[NC], double (&n)[NC], int r) {
+  unroll<0, d>([&](auto ic) {
+    constexpr int i = decltype(ic)::value;
+    constexpr int nt = NC - 1 - i;
+    double dt, dn;
+    dot_pair<i, nt>(dt, dn, t + i + 1, n + i + 1);
+    bool nz;
+    const Pivot p = pivot(bcast<i>(t[i]), bcast<i>(dt), nz);
+    const double tn = reflect_rows<i, nt>(n + i + 1, t + i + 1, p.rb, p.sc, dn, n[i]);
+    const double tt = reflect_self<i, nt>(t + i + 1, p.rb, p.sc, dt, t[i]);
+    t[i] = (r == i && nz) ? p.beta : fma(-p.den, tt, t[i]);
+    n[i] = fma(-p.den, tn, n[i]);
+  });
+}
+
 // ------------------------------------------------------------- filter element
 // _get_element (pof/parallel_filtsmooth/filter.py:50-81) for element k, as filter_element() of
 // pof_core.hpp; element 0 carries the prior (x0m, x0L), the others a zero one.  The element's
@@ -866,18 +890,7 @@ __device__ __forceinline__ void filter_element(int r, const GroupArgs& g, int j,
   }
 #pragma unroll
   for (int c = D; c < NC; ++c) t[c] = ob.r_at(c - D);
-  unroll<0, d>([&](auto ic) {
-    constexpr int i = decltype(ic)::value;
-    constexpr int nt = NC - 1 - i;
-    double dt, dn;
-    dot_pair<i, nt>(dt, dn, t + i + 1, n + i + 1);
-    bool nz;
-    const Pivot p = pivot(bcast<i>(t[i]), bcast<i>(dt), nz);
-    const double tn = reflect_rows<i, nt>(n + i + 1, t + i + 1, p.rb, p.sc, dn, n[i]);
-    const double tt = reflect_self<i, nt>(t + i + 1, p.rb, p.sc, dt, t[i]);
-    t[i] = (r == i && nz) ? p.beta : fma(-p.den, tt, t[i]);
-    n[i] = fma(-p.den, tn, n[i]);
-  });
+  lq_obs<d, NC>(t, n, r);
   Small<d> p11;
   p11.load(t);
   // gain K = Psi21 Psi11^-1; A = F - K H F, b = m1 - K (H m1 + c)
@@ -995,7 +1008,7 @@ __device__ __forceinline__ void filter_post(int r, const GroupArgs& g, int j, lo
     sel.g[ro * D + r] = gr;
   }
   if (!obs) {
-    if (r == 0) {
+    if (r == 0 && t_ssq) {
       t_ssq[s] = 0.0;
       t_nll[s] = 0.0;
     }
@@ -1037,6 +1050,195 @@ __device__ __forceinline__ void filter_post(int r, const GroupArgs& g, int j, lo
     t_ssq[s] = ss;
     // -loglik = 0.5 |S^-1 y|^2 + sum log|S_ii| + d log(2 pi) / 2
     t_nll[s] = 0.5 * nn + (ld + d * log(2.0 * M_PI) / 2.0);
+  }
+}
+
+// ------------------------------------------------------------- sequential filter and smoother
+// k_seq_filter of one IVP (pof/sequential_filtsmooth/filter.py:9-92), state and model in the registers of one row.
+// A step is a serial chain of about 2 D + d pivots and its one wavefront issues an FP64 instruction every 8.5
+// cycles, so it is the instructions of a step that count: the predicted factor never leaves the registers, the
+// model's values are read a step ahead, and the step's logarithms wait for sixteen steps, a step per lane.
+// Against a whole wavefront per IVP with its tiles in LDS, filter and smoother of 513 points: 8.6 -> 2.1 ms at
+// D = 8, 16.1 -> 3.6 ms at D = 12, 22.4 -> 5.4 ms at D = 15 (17.4, 31 and 44 us per step before).
+template <int D, int d, bool EK1, bool AT_PRED>
+__device__ __forceinline__ void seq_filter(int r, const GroupArgs& g, int j, long long base, int Ns,
+                                           const StateArrays& fp, double* shared) {
+  using O = ObsRow<D, d, EK1>;
+  constexpr int NR = O::NR, NC = D + NR, q1 = D / d;
+  const bool act = r < D;
+  const int rr = act ? r : 0;
+  double* t_ssq = g.t_ssq + base;
+  double* t_nll = g.t_nll + base;
+  const double* lin = (g.cur[j] ? g.means1 : g.means0) + (size_t)base * D;
+  const int kind = EK1 ? g.kind[j] : 0;
+  double* Pd = shared;  // [D], then the field's parameters
+  double* params = shared + D;
+  if constexpr (EK1) {
+    if (act) Pd[r] = g.Pd[(size_t)j * D + r];
+    if (r < kMaxParams) params[r] = g.params[(size_t)j * kMaxParams + r];
+    wsync();
+  }
+  double f[D], lq[D], l[D];
+  load_row16<D>(f, g.F + rr * D);
+  load_row16<D>(lq, g.LQ + rr * D);
+  load_row16<D>(l, g.x0L + (size_t)j * D * D + rr * D);
+  double m = g.x0m[(size_t)j * D + rr];
+  O ob, next;      // (affine) the model of this step and of the next
+  double y1[d];    // (EK1 at given means) the next step's
+  auto fetch = [&](int k) {
+    if constexpr (!EK1) {
+      next.load(g, j, base, k, r);
+    } else if constexpr (!AT_PRED) {
+#pragma unroll
+      for (int i = 0; i < d; ++i) y1[i] = lin[(size_t)(k + 1) * D + i * q1];
+    }
+  };
+  if (Ns > 0) fetch(0);
+  double dg[d], nn = 0.0, ss = 0.0;  // lane k % 16: step k's diagonal of I, |I^-1 y|^2, |I^-T y|^2
+#pragma unroll
+  for (int i = 0; i < d; ++i) dg[i] = 1.0;
+  for (int k = 0; k < Ns; ++k) {
+    if constexpr (!EK1) {
+      ob = next;
+    } else if constexpr (!AT_PRED) {
+      ob.load_entries(kind, params, Pd, y1);
+    }
+    if (k + 1 < Ns) fetch(k + 1);
+    // predict: mp = F m, N1 = tria([F L | LQ])
+    const double mp = dot_lanes<D>(f, m);
+    double n[NC];
+    {
+      double a[2 * D];
+      zero(a);
+      mul_rows<D, D, EK1 ? 1 : D>(a, f, l);  // an affine model's first factor is the caller's, not triangular
+#pragma unroll
+      for (int c = 0; c < D; ++c) a[D + c] = lq[c];
+      lq1<D, 2 * D, D, EK1 ? 0 : D>(a, r);
+#pragma unroll
+      for (int c = 0; c < D; ++c) n[c] = (c > r) ? 0.0 : a[c];
+#pragma unroll
+      for (int c = D; c < NC; ++c) n[c] = 0.0;
+    }
+    if constexpr (EK1 && AT_PRED) {
+      double mi[d];
+      unroll<0, d>([&](auto ic) { mi[decltype(ic)::value] = bcast<decltype(ic)::value * q1>(mp); });
+      ob.load_entries(kind, params, Pd, mi);
+    }
+    // update: tria([[H N1, R], [N1, 0]]) = [[I, 0], [G, L]]
+    double t[NC];
+    {
+      double hn[D], n1[D];
+      zero(hn);
+#pragma unroll
+      for (int c = 0; c < D; ++c) n1[c] = n[c];
+      ob.template times_rows<1>(r, n1, hn);
+#pragma unroll
+      for (int c = 0; c < D; ++c) t[c] = hn[c];
+#pragma unroll
+      for (int c = D; c < NC; ++c) t[c] = ob.r_at(c - D);
+    }
+    lq_obs<d, NC>(t, n, r);
+    Small<d> S;
+    S.load(t);
+    double z[d], w[d];
+    ob.predict(mp, z);
+#pragma unroll
+    for (int i = 0; i < d; ++i) w[i] = z[i] = -z[i];
+    S.solve(z);    // I z = y
+    S.solve_t(w);  // I^T w = y (whiten)
+    m = mp;
+#pragma unroll
+    for (int i = 0; i < d; ++i) m = fma(n[i], z[i], m);
+#pragma unroll
+    for (int c = 0; c < D; ++c) l[c] = (d + c < NC) ? n[(d + c < NC) ? d + c : 0] : 0.0;
+    lq1<NC - d, NC - d>(l, r);  // the last pivot has no tail
+#pragma unroll
+    for (int c = 1; c < D; ++c) l[c] = (c > r) ? 0.0 : l[c];
+    if (act) {
+      fp.m[(size_t)k * D + r] = m;
+      store_row16<D>(fp.L + ((size_t)k * D + r) * D, l);
+    }
+    double sn = 0.0, sw = 0.0;
+#pragma unroll
+    for (int i = 0; i < d; ++i) {
+      sn = fma(z[i], z[i], sn);
+      sw = fma(w[i], w[i], sw);
+    }
+    const int e = k % kRow;
+    const bool mine = r == e;
+    nn = mine ? sn : nn;
+    ss = mine ? sw : ss;
+#pragma unroll
+    for (int i = 0; i < d; ++i) dg[i] = mine ? S.l[i][i] : dg[i];
+    if (e == kRow - 1 || k + 1 == Ns) {
+      double ld = 0.0;
+#pragma unroll
+      for (int i = 0; i < d; ++i) ld += log(fabs(dg[i]));
+      if (r <= e) {
+        t_ssq[k - e + r] = ss;
+        // mvn_loglikelihood (utils.py:22-30): -|I^-1 y|^2 / 2 - sum log|I_ii| - d log(2 pi) / 2
+        t_nll[k - e + r] = -0.5 * nn - (ld + d * log(2.0 * M_PI) / 2.0);
+      }
+    }
+  }
+}
+
+// The RTS recursion (pof/sequential_filtsmooth/smoother.py:8-48) over gains E and factors Phi22 = D formed beforehand
+// for all steps at once (filter_post; its other half is what a step would otherwise spend most of its time on):
+//   mean = mf + E (mean - F mf), L = tria([D | E L]),
+// state Ns - s of the smoother arrays as k_seq_smooth.  A step's reads are issued a step ahead.
+template <int D>
+__device__ __forceinline__ void seq_smooth(int r, const GroupArgs& g, int j, int Ns, const StateArrays& fp,
+                                           const StateArrays& sp, const SmoArrays& sel) {
+  const bool act = r < D;
+  const int rr = act ? r : 0;
+  const bool wc = g.wchol[j] != 0;
+  const double* x0m = g.x0m + (size_t)j * D;
+  double f[D], l[D];
+  load_row16<D>(f, g.F + rr * D);
+  load_row16<D>(l, (Ns == 0 ? g.x0L + (size_t)j * D * D : fp.L + (size_t)(Ns - 1) * D * D) + rr * D);
+  double m = (Ns == 0 ? x0m : fp.m + (size_t)(Ns - 1) * D)[rr];
+  if (act) {
+    sp.m[r] = m;
+    if (wc) store_row16<D>(sp.L + r * D, l);
+  }
+  double e1[D], d1[D], mf1 = 0.0;  // the next step's
+  zero(d1);
+  auto fetch = [&](int s) {  // s = Ns - k
+    const int k = Ns - s;
+    mf1 = ((k == 0) ? x0m : fp.m + (size_t)(k - 1) * D)[rr];
+    load_row16<D>(e1, sel.E + ((size_t)s * D + rr) * D);
+    if (wc) load_row16<D>(d1, sel.Dm + ((size_t)s * D + rr) * D);
+  };
+  if (Ns > 0) fetch(1);
+  for (int s = 1; s <= Ns; ++s) {
+    double e[D], a[D];
+    const double mf = mf1;
+#pragma unroll
+    for (int c = 0; c < D; ++c) {
+      e[c] = e1[c];
+      a[c] = d1[c];
+    }
+    if (s < Ns) fetch(s + 1);
+    m = dot_lanes<D>(e, m - dot_lanes<D>(f, mf), mf);
+    if (act) sp.m[(size_t)s * D + r] = m;
+    if (wc) {
+      double t[D];
+      zero(t);
+      mul_rows<D, D, D>(t, e, l);  // the last state's factor may be a caller's, not triangular
+      // D's row i ends at column i, and so does what the reflectors before pivot i leave of it
+      unroll<0, D>([&](auto ic) {
+        constexpr int i = decltype(ic)::value;
+        const double dot = dot_self<i, D>(t);
+        bool nz;
+        const Pivot p = pivot(bcast<i>(a[i]), bcast<i>(dot), nz);
+        const double x = reflect_self<i, D>(t, p.rb, p.sc, dot, a[i]);
+        a[i] = (r == i && nz) ? p.beta : fma(-p.den, x, a[i]);
+      });
+#pragma unroll
+      for (int c = 0; c < D; ++c) l[c] = (c > r) ? 0.0 : a[c];
+      if (act) store_row16<D>(sp.L + ((size_t)s * D + r) * D, l);
+    }
   }
 }
 

@@ -64,3 +64,43 @@ def test_linear_model_against_oracle(gpu, d, q):
             assert rel(a, b) <= t
         # the filtered factors are lower triangular, their strict upper part stored as zeros
         assert not np.triu(filt.chol.cpu().numpy()[1:], 1).any()
+
+
+@pytest.mark.parametrize("d,q", PAIRS)
+def test_sequential_linear_model_against_oracle(gpu, d, q):
+    """The sequential filter and smoother, one problem per row: one step, and the sixteen steps between two writes of the
+    scalar terms less, exactly and more, with a prior factor that is not triangular.  Tolerances as above."""
+    import torch
+
+    import pof.sequential_filtsmooth as sfs
+    from oracle import model as om
+    from oracle import sequential as oseq
+    from pof.observations import AffineModel
+    from pof.transitions import TransitionModel
+    from pof.utils import MVNSqrt
+
+    D = d * (q + 1)
+    F, QL = om.preconditioned_discretize(om.IWP(d, q))
+    for n in [1, 2, 15, 16, 17, 33]:
+        rng = np.random.default_rng(2000 * D + n)
+        H, c = rng.standard_normal((n, d, D)), rng.standard_normal((n, d))
+        R = np.tril(rng.standard_normal((n, d, d))) * 0.3 + 0.5 * np.eye(d)
+        m0, L0 = rng.standard_normal(D), rng.standard_normal((D, D))
+        print(f"D={D} d={d} steps={n}", flush=True)
+        t = [torch.as_tensor(x, device="cuda") for x in (H, c, R)]
+        out, nll, obj, ssq = sfs.linear_filtsmooth(MVNSqrt(m0, L0), TransitionModel(F, QL), AffineModel(*t))
+        filt, _, _ = sfs.linear_noiseless_filter(MVNSqrt(m0, L0), TransitionModel(F, QL), AffineModel(*t))
+        torch.cuda.synchronize()
+
+        def oracle(e=0.0):
+            x0, mod = om.MVNSqrt(m0, L0 * (1 + e)), om.AffineModel(H * (1 - e), c, R)
+            sm, nll, obj, _ = oseq.linear_filtsmooth(x0, F, QL, mod)
+            fi, _, _ = oseq.linear_noiseless_filter(x0, F, QL, mod)
+            return [sm.mean, gram(sm.chol), fi.mean, gram(fi.chol), np.array(nll), np.array(obj)]
+
+        ref = oracle()
+        tol = [max(1e-12, 20 * max(rel(a, b) for a in x)) for *x, b in zip(*(oracle(e) for e in (1e-15, -1e-15, 3e-15)), ref)]
+        got = [out.mean.cpu().numpy(), gram(out.chol.cpu().numpy()), filt.mean.cpu().numpy(),
+               gram(filt.chol.cpu().numpy()), np.array(nll), np.array(obj)]
+        for a, b, t in zip(got, ref, tol):
+            assert rel(a, b) <= t
