@@ -395,6 +395,9 @@ struct pof_ctx {
   std::vector<pof_batch*> cache;
   // small batches for the coarse initial trajectory (EKS on 100 points), one per (D, d)
   std::vector<pof_batch*> aux;
+  // batches kept for the next call of pof_linear_filtsmooth / pof_smoothing / pof_ekf, the last used at the end
+  std::vector<pof_batch*> kept;
+  std::mutex kept_mu;
   // large-state engine (batched primitives), created on first use
   pof::large::Engine* large = nullptr;
   // replay unchanged iterations from a HIP graph (pof_graphs_enable)
@@ -407,6 +410,16 @@ struct pof_ctx {
   // tune_version counts changes, so that batches rebuild plans and graphs
   std::map<int, pof::Tuning> tuning;
   int tune_version = 0;
+};
+
+// A host table of a batch in its pinned block (see pof_batch::arena).
+template <class T>
+struct HostTable {
+  T* p = nullptr;
+  size_t n = 0;
+  T& operator[](size_t i) { return p[i]; }
+  T* begin() { return p; }
+  T* end() { return p + n; }
 };
 
 // A group of IVPs with one (D, d) sharing one device workspace.  IVP slots are
@@ -452,18 +465,32 @@ struct pof_batch {
   long long* base = nullptr;
   double** outp = nullptr;  // [4, slots]: means, chols, full means, full chols
   int* maps_dev = nullptr;
+  int *maps_host = nullptr, *maps_map = nullptr;  // pinned source of maps_dev, its device address
   size_t maps_cap = 0;
-  // host mirrors
-  std::vector<double> hPd, hx0m, hx0L, hparams, hscale, hcvec;
-  std::vector<int> hkind, hNs, hcur, hwchol;  // hcur: 0, uploaded at admission (the device flips it)
-  std::vector<int> hpfull;
-  std::vector<long long> hbase;
-  std::vector<double*> hout;
+  // The device tables above and the transition model stand in one block each of device memory (arena_dev) and of
+  // pinned host memory (arena_host; device address arena_map) with the same layout: the host mirrors.  One
+  // kernel brings every part that an admission or a retirement changed to the device (see upload()).
+  char *arena_host = nullptr, *arena_map = nullptr, *arena_dev = nullptr;
+  HostTable<double> hPd, hx0m, hx0L, hparams, hscale, hcvec, hF, hLQ, hN1z;
+  HostTable<int> hkind, hNs, hcur_up, hwchol;
+  HostTable<int> hpfull;
+  HostTable<long long> hbase;
+  HostTable<double*> hout;
+  HostTable<double> stage;  // initial means of small IVPs
+  size_t stage_used = 0;
+  std::vector<int> hcur;  // mirror of cur (0 at admission, flipped with each launch); an upload reads its copy hcur_up
   std::vector<int> hmaps;
+  hipEvent_t up_ev = nullptr;  // the last upload has read its sources
+  bool model_dirty = false;    // F, LQ, N1z to upload
   std::vector<Slot> sl;
   std::map<long long, long long> free_;  // free entry ranges: start -> length
   std::vector<int> dirty_slots;          // per-slot tables to upload before the next launch
-  std::vector<std::pair<long long, std::vector<double>>> init_host;  // initial means to upload
+  struct Staged {
+    long long start;
+    size_t at, n;  // in stage
+  };
+  std::vector<Staged> init_stage;                                    // initial means to upload from stage
+  std::vector<std::pair<long long, std::vector<double>>> init_host;  // ... or, larger ones, from a vector
   std::vector<std::pair<long long, const double*>> init_dev;         // ... or to copy on the device
   std::vector<long long> init_zero;                                  // ... or to clear (entries, count D each)
   std::vector<long long> init_zero_n;
@@ -531,10 +558,93 @@ int n_levels_host(long long n0) {
 
 long long entries_for(long long n_times) { return 2 * n_times; }
 
-// A constant initial trajectory: rows 0 .. n - 1 of m (D each) = v.
-__global__ void k_fill_rows(double* m, const double* v, long long n, int D) {
-  const long long e = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (e < n * D) m[e] = v[e % D];
+// Parts of host tables to bring to the device, in 4-byte words.
+struct Upload {
+  const unsigned* src;  // pinned host memory, by its device address
+  unsigned* dst;
+  size_t n;
+};
+constexpr int kUploads = 24;
+struct Uploads {
+  Upload u[kUploads];
+};
+// An admission changes some twenty small tables.  One launch that reads pinned memory over the bus takes the place of
+// a copy call each, whose sources the host had to wait for (96 problems in one call: 14.0 -> 12.7 ms, with one fill
+// of their initial trajectories; one of 63 steps: 0.89 -> 0.85 ms).
+__global__ void k_upload(Uploads a) {
+  const Upload u = a.u[blockIdx.y];
+  for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < u.n; i += (size_t)gridDim.x * blockDim.x)
+    u.dst[i] = u.src[i];
+}
+
+// Constant initial trajectories: rows 0 .. Ns of the means of the slots in `a` repeat their cvec row.
+constexpr int kFills = 64;
+struct Fills {
+  int j[kFills];
+};
+__global__ void k_fill_rows(Fills a, double* means, const double* cvec, const int* Ns, const long long* base, int D) {
+  const int j = a.j[blockIdx.y];
+  const size_t n = ((size_t)Ns[j] + 1) * D;
+  double* m = means + (size_t)base[j] * D;
+  const double* v = cvec + (size_t)j * D;
+  for (size_t e = (size_t)blockIdx.x * blockDim.x + threadIdx.x; e < n; e += (size_t)gridDim.x * blockDim.x)
+    m[e] = v[e % D];
+}
+
+// Collects uploads of a batch and launches them on its stream.
+struct Uploader {
+  pof_batch* b;
+  Uploads a;
+  int n = 0;
+  size_t most = 0;
+  hipError_t status = hipSuccess;
+  explicit Uploader(pof_batch* b_) : b(b_) {}
+  void add(const void* src, void* dst, size_t bytes) {
+    if (bytes == 0) return;
+    if (n == kUploads) flush();
+    a.u[n++] = Upload{static_cast<const unsigned*>(src), static_cast<unsigned*>(dst), bytes / 4};
+    most = std::max(most, bytes / 4);
+  }
+  // entries [at, at + count) of a table of the arena
+  template <class T>
+  void table(const HostTable<T>& t, size_t at, size_t count) {
+    const size_t off = (size_t)((const char*)(t.p + at) - b->arena_host);
+    add(b->arena_map + off, b->arena_dev + off, count * sizeof(T));
+  }
+  void maps() { add(b->maps_map, b->maps_dev, b->hmaps.size() * sizeof(int)); }
+  void flush() {
+    if (n == 0 || status != hipSuccess) return;
+    const unsigned blocks = (unsigned)std::min<size_t>((most + 255) / 256, 256);
+    hipLaunchKernelGGL(k_upload, dim3(blocks, n), dim3(256), 0, b->st, a);
+    status = hipGetLastError();
+    if (status == hipSuccess) status = hipEventRecord(b->up_ev, b->st);
+    n = 0;
+    most = 0;
+  }
+};
+
+// The launch tables in hmaps to their pinned block, which grows (with the device's) where it is too small.
+// The batch's stream has been drained or holds nothing that reads them.
+hipError_t stage_maps(pof_batch* b) {
+  const size_t n = b->hmaps.size();
+  if (n > b->maps_cap) {
+    hipError_t e = hipStreamSynchronize(b->st);
+    if (e == hipSuccess && b->maps_dev) e = hipFree(b->maps_dev);
+    if (e == hipSuccess && b->maps_host) e = hipHostFree(b->maps_host);
+    if (e != hipSuccess) return e;
+    b->maps_dev = nullptr;
+    b->maps_host = nullptr;
+    b->maps_cap = 0;
+    const size_t cap = std::max<size_t>(n * 2, 4096);
+    e = hipMalloc((void**)&b->maps_dev, cap * sizeof(int));
+    if (e == hipSuccess)
+      e = hipHostMalloc((void**)&b->maps_host, cap * sizeof(int), hipHostMallocMapped | hipHostMallocCoherent);
+    if (e == hipSuccess) e = hipHostGetDevicePointer((void**)&b->maps_map, b->maps_host, 0);
+    if (e != hipSuccess) return e;
+    b->maps_cap = cap;
+  }
+  std::copy(b->hmaps.begin(), b->hmaps.end(), b->maps_host);
+  return hipSuccess;
 }
 
 // after an instrumented run: accumulate event intervals per kernel class
@@ -576,7 +686,10 @@ void batch_free(pof_batch* b) {
   for (void* p : b->allocs) (void)hipFree(p);
   if (b->scal_host) (void)hipHostFree(b->scal_host);
   if (b->maps_dev) (void)hipFree(b->maps_dev);
+  if (b->maps_host) (void)hipHostFree(b->maps_host);
+  if (b->arena_host) (void)hipHostFree(b->arena_host);
   if (b->ev) (void)hipEventDestroy(b->ev);
+  if (b->up_ev) (void)hipEventDestroy(b->up_ev);
   if (b->join_ev) (void)hipEventDestroy(b->join_ev);
   if (b->own_st) (void)hipStreamDestroy(b->own_st);
   delete b;
@@ -592,6 +705,9 @@ hipError_t dalloc(pof_batch* b, size_t n, T** out) {
   return hipSuccess;
 }
 
+// Doubles of a batch's stage: initial means up to this size go to the device with the tables.
+constexpr size_t kStageDoubles = 8192;
+
 // Device bytes of a batch of `entries` entries and `slots` IVPs with state dimension D.
 size_t batch_bytes(int D, long long entries, int slots) {
   const size_t DD = (size_t)D * D;
@@ -600,7 +716,13 @@ size_t batch_bytes(int D, long long entries, int slots) {
   return per_entry * (size_t)entries + per_slot * (size_t)slots + 8 * 4 * ((size_t)entries / kChunk + slots + 1);
 }
 
-int batch_new(pof_ctx* ctx, int D, int d, long long entries, int slots, bool affine, pof_batch** out) {
+void drop_kept(pof_ctx* ctx) {
+  std::lock_guard<std::mutex> lk(ctx->kept_mu);
+  for (pof_batch* b : ctx->kept) batch_free(b);
+  ctx->kept.clear();
+}
+
+int batch_try(pof_ctx* ctx, int D, int d, long long entries, int slots, bool affine, pof_batch** out) {
   *out = nullptr;
   const EngineFns* e = engine_or_err(ctx, D, d);
   if (!e) return POF_E_UNSUPPORTED;
@@ -631,11 +753,45 @@ int batch_new(pof_ctx* ctx, int D, int d, long long entries, int slots, bool aff
   POF_A(sg, n * D) POF_A(sE, n * DD) POF_A(sD, n * DD) POF_A(qm, n * D) POF_A(qL, n * DD)
   POF_A(m0, n * D) POF_A(m1, n * D) POF_A(ts, n) POF_A(tn, n)
   POF_A(part, 4 * (n / kChunk + S + 1))
-  POF_A(b->F, DD) POF_A(b->LQ, DD) POF_A(b->N1z, DD) POF_A(b->Pd, S * D) POF_A(b->x0m, S * D)
-  POF_A(b->x0L, S * DD) POF_A(b->params, S * kMaxParams) POF_A(b->scale, S)
-  POF_A(b->kind, S) POF_A(b->Ns, S) POF_A(b->cur, S) POF_A(b->wchol, S) POF_A(b->base, S) POF_A(b->outp, 4 * S)
-  POF_A(b->pfull, S) POF_A(b->cvec, S * D)
+  // the tables: offsets first (nullptr base), then the two blocks and everyone's address in them
+  size_t arena = 0;
+  auto place = [&](auto& t, size_t count, auto*& dev) {
+    using T = std::remove_reference_t<decltype(t[0])>;
+    const size_t at = (arena + 255) / 256 * 256;
+    arena = at + count * sizeof(T);
+    t.n = count;
+    t.p = reinterpret_cast<T*>(b->arena_host + at);
+    dev = reinterpret_cast<std::remove_reference_t<decltype(dev)>>(b->arena_dev + at);
+  };
+  double* stage_dev = nullptr;  // (the stage's own place on the device is not used)
+  auto tables = [&] {
+    arena = 0;
+    place(b->hF, DD, b->F);
+    place(b->hLQ, DD, b->LQ);
+    place(b->hN1z, DD, b->N1z);
+    place(b->hPd, S * D, b->Pd);
+    place(b->hx0m, S * D, b->x0m);
+    place(b->hx0L, S * DD, b->x0L);
+    place(b->hparams, S * kMaxParams, b->params);
+    place(b->hscale, S, b->scale);
+    place(b->hcvec, S * D, b->cvec);
+    place(b->hkind, S, b->kind);
+    place(b->hNs, S, b->Ns);
+    place(b->hcur_up, S, b->cur);
+    place(b->hwchol, S, b->wchol);
+    place(b->hpfull, S, b->pfull);
+    place(b->hbase, S, b->base);
+    place(b->hout, 4 * S, b->outp);
+    place(b->stage, kStageDoubles, stage_dev);
+  };
+  tables();
+  const size_t arena_bytes = arena, arena_dev_bytes = arena - kStageDoubles * sizeof(double);
+  POF_A(b->arena_dev, arena_dev_bytes)
 #undef POF_A
+  if (he == hipSuccess)
+    he = hipHostMalloc((void**)&b->arena_host, arena_bytes, hipHostMallocMapped | hipHostMallocCoherent);
+  if (he == hipSuccess) he = hipHostGetDevicePointer((void**)&b->arena_map, b->arena_host, 0);
+  if (he == hipSuccess) tables();
   // the iteration's scalars go straight to host memory: no copy behind the last kernel
   if (he == hipSuccess)
     he = hipHostMalloc((void**)&b->scal_host, S * 8 * sizeof(double), hipHostMallocMapped | hipHostMallocCoherent);
@@ -643,6 +799,7 @@ int batch_new(pof_ctx* ctx, int D, int d, long long entries, int slots, bool aff
   if (he == hipSuccess) he = hipStreamCreateWithFlags(&b->own_st, hipStreamNonBlocking);
   if (he == hipSuccess) he = hipEventCreateWithFlags(&b->ev, hipEventDisableTiming);
   if (he == hipSuccess) he = hipEventCreateWithFlags(&b->join_ev, hipEventDisableTiming);
+  if (he == hipSuccess) he = hipEventCreateWithFlags(&b->up_ev, hipEventDisableTiming);
   if (he != hipSuccess) {
     batch_free(b);
     return set_err(ctx, POF_E_HIP, "batch allocation failed: %s", hipGetErrorString(he));
@@ -680,19 +837,10 @@ int batch_new(pof_ctx* ctx, int D, int d, long long entries, int slots, bool aff
   g.q = b->q;
   g.affine = affine ? 1 : 0;
   g.lq_lower = 0;
-  b->hPd.assign(S * D, 0.0);
-  b->hx0m.assign(S * D, 0.0);
-  b->hcvec.assign(S * D, 0.0);
-  b->hx0L.assign(S * DD, 0.0);
-  b->hparams.assign(S * kMaxParams, 0.0);
-  b->hscale.assign(S, 1.0);
-  b->hkind.assign(S, 0);
-  b->hNs.assign(S, 1);
+  std::fill(b->arena_host, b->arena_host + arena_bytes, 0);  // (zero bits: 0.0, null)
   b->hcur.assign(S, 0);
-  b->hwchol.assign(S, 0);
-  b->hpfull.assign(S, 0);
-  b->hbase.assign(S, 0);
-  b->hout.assign(4 * S, nullptr);
+  std::fill(b->hscale.begin(), b->hscale.end(), 1.0);
+  std::fill(b->hNs.begin(), b->hNs.end(), 1);
   b->sl.assign(S, pof_batch::Slot{});
   b->free_[0] = entries;
   // the transition model of the group (pof/transitions.py:37-50) and N1 of a zero prior
@@ -704,18 +852,76 @@ int batch_new(pof_ctx* ctx, int D, int d, long long entries, int slots, bool aff
     for (int r = 0; r < D; ++r)
       for (int c = 0; c < D; ++c) M[(size_t)r * 2 * D + D + c] = LQm[(size_t)r * D + c];
     tria_host(M, D, 2 * D, N1);
-    he = hipMemcpy(b->F, Fm.data(), DD * 8, hipMemcpyHostToDevice);
-    if (he == hipSuccess) he = hipMemcpy(b->LQ, LQm.data(), DD * 8, hipMemcpyHostToDevice);
+    std::copy(Fm.begin(), Fm.end(), b->hF.p);
+    std::copy(LQm.begin(), LQm.end(), b->hLQ.p);
+    std::copy(N1.begin(), N1.end(), b->hN1z.p);
     b->g.lq_lower = strictly_upper_zero(LQm.data(), D) ? 1 : 0;
-    if (he == hipSuccess) he = hipMemcpy(b->N1z, N1.data(), DD * 8, hipMemcpyHostToDevice);
-    if (he != hipSuccess) {
-      batch_free(b);
-      return set_err(ctx, POF_E_HIP, "batch set-up copy failed: %s", hipGetErrorString(he));
-    }
+    b->model_dirty = true;
   }
   *out = b;
   return POF_OK;
 }
+
+int batch_new(pof_ctx* ctx, int D, int d, long long entries, int slots, bool affine, pof_batch** out) {
+  int rc = batch_try(ctx, D, d, entries, slots, affine, out);
+  if (rc != POF_E_HIP) return rc;
+  {
+    std::lock_guard<std::mutex> lk(ctx->kept_mu);
+    if (ctx->kept.empty()) return rc;
+  }
+  // out of memory with workspaces kept: without them
+  (void)hipGetLastError();
+  drop_kept(ctx);
+  return batch_try(ctx, D, d, entries, slots, affine, out);
+}
+
+// The workspace of one call of pof_linear_filtsmooth, pof_smoothing or pof_ekf.  Its 26 allocations and their
+// releases cost 3.1 of the 3.9 ms of a call over 16,384 steps at D = 12, so a finished call's is kept for the next
+// one of its (D, d) that fits, at most kKeptBatches of them and kKeptBytes together per context (and none where
+// another allocation of the library needs the memory).  A call takes it out of the list, so that calls
+// from several threads have one each; it is put back only idle: its work done, its slots free.
+constexpr size_t kKeptBatches = 4;
+constexpr size_t kKeptBytes = size_t(1) << 30;
+struct CallBatch {
+  pof_ctx* ctx;
+  pof_batch* b = nullptr;
+  bool done = false;  // the call ended well
+  explicit CallBatch(pof_ctx* c) : ctx(c) {}
+  int open(int D, int d, long long entries, bool affine) {
+    {
+      std::lock_guard<std::mutex> lk(ctx->kept_mu);
+      for (size_t i = ctx->kept.size(); i-- > 0;) {
+        pof_batch* x = ctx->kept[i];
+        if (x->D != D || x->d != d || x->affine != affine || x->entries < entries) continue;
+        b = x;
+        ctx->kept.erase(ctx->kept.begin() + i);
+        break;
+      }
+    }
+    if (!b) return batch_new(ctx, D, d, entries, 1, affine, &b);
+    HIP_TRY(hipSetDevice(ctx->device));
+    return POF_OK;
+  }
+  ~CallBatch() {
+    if (!b) return;
+    const size_t bytes = batch_bytes(b->D, b->entries, b->slots);
+    if (!done || bytes > kKeptBytes) {
+      batch_free(b);
+      return;
+    }
+    b->g.Hx = b->g.cx = b->g.Rx = nullptr;
+    std::lock_guard<std::mutex> lk(ctx->kept_mu);
+    ctx->kept.push_back(b);
+    size_t total = 0;
+    for (pof_batch* x : ctx->kept) total += batch_bytes(x->D, x->entries, x->slots);
+    while (ctx->kept.size() > kKeptBatches || total > kKeptBytes) {
+      pof_batch* x = ctx->kept.front();
+      total -= batch_bytes(x->D, x->entries, x->slots);
+      ctx->kept.erase(ctx->kept.begin());
+      batch_free(x);
+    }
+  }
+};
 
 // first-fit range allocator over the batch's entries
 bool range_alloc(pof_batch* b, long long len, long long* start) {
@@ -903,7 +1109,14 @@ int admit_raw(pof_batch* b, int Nsteps, const double* Pd, const double* x0m, con
     std::copy(m_const, m_const + D, &b->hcvec[(size_t)j * D]);
     b->init_const.push_back(j);
   } else if (m_host) {
-    b->init_host.emplace_back(start, std::move(*m_host));
+    if (b->init_stage.empty()) b->stage_used = 0;  // everything in it has been read (settle)
+    if (m_host->size() <= kStageDoubles - b->stage_used) {
+      std::copy(m_host->begin(), m_host->end(), b->stage.p + b->stage_used);
+      b->init_stage.push_back({start, b->stage_used, m_host->size()});
+      b->stage_used += m_host->size();
+    } else {
+      b->init_host.emplace_back(start, std::move(*m_host));
+    }
   } else if (m_dev) {
     b->init_dev.emplace_back(start, m_dev);
   } else {
@@ -965,6 +1178,7 @@ int batch_launch(pof_batch* b) {
   if (b->launched) return set_err(ctx, POF_E_ARG, "pof_batch_launch called twice without pof_batch_finish");
   HIP_TRY(hipSetDevice(ctx->device));
   if (b->tune_version != ctx->tune_version) b->plan_dirty = true;  // other kernel forms: new plan and graph
+  Uploader up(b);
   if (b->plan_dirty) {
     if (settle(b) != POF_OK) return POF_E_HIP;
     drop_graph(b);
@@ -981,53 +1195,51 @@ int batch_launch(pof_batch* b) {
     int rc = plan_tables(b, b->active, b->hmaps, b->plan);
     if (rc != POF_OK) return set_err(ctx, rc, "launch tables overflow");
     b->tune_version = ctx->tune_version;
-    if (b->hmaps.size() > b->maps_cap) {
-      HIP_TRY(hipStreamSynchronize(b->st));
-      if (b->maps_dev) HIP_TRY(hipFree(b->maps_dev));
-      b->maps_dev = nullptr;
-      b->maps_cap = 0;
-      const size_t cap = std::max<size_t>(b->hmaps.size() * 2, 4096);
-      HIP_TRY(hipMalloc((void**)&b->maps_dev, cap * sizeof(int)));
-      b->maps_cap = cap;
-    }
-    HIP_TRY(hipMemcpyAsync(b->maps_dev, b->hmaps.data(), b->hmaps.size() * sizeof(int), hipMemcpyHostToDevice,
-                           b->st));
+    HIP_TRY(stage_maps(b));
+    up.maps();
     b->plan.dev = b->maps_dev;
     b->plan_dirty = false;
   }
   if (b->plan.m == 0) return POF_OK;
   // newly admitted IVPs: per-slot tables and initial means
-  if (!b->dirty_slots.empty() || !b->init_host.empty() || !b->init_dev.empty() || !b->init_zero.empty() ||
-      !b->init_const.empty()) {
-    const int D = b->D;
-    const size_t DD = (size_t)D * D, S = (size_t)b->slots;
-    if (!b->dirty_slots.empty()) {
-      // one copy per table over the slot range of the new IVPs: the host
-      // tables mirror the device ones for every slot (cur through the flips
-      // of each launch), so the slots in between are rewritten unchanged
-      int lo = b->slots, hi = -1;
-      for (int j : b->dirty_slots) {
-        lo = std::min(lo, j);
-        hi = std::max(hi, j);
-      }
-      const size_t n = (size_t)(hi - lo + 1), l = (size_t)lo;
-      HIP_TRY(hipMemcpyAsync(b->Pd + l * D, &b->hPd[l * D], n * D * 8, hipMemcpyHostToDevice, b->st));
-      HIP_TRY(hipMemcpyAsync(b->x0m + l * D, &b->hx0m[l * D], n * D * 8, hipMemcpyHostToDevice, b->st));
-      HIP_TRY(hipMemcpyAsync(b->x0L + l * DD, &b->hx0L[l * DD], n * DD * 8, hipMemcpyHostToDevice, b->st));
-      HIP_TRY(hipMemcpyAsync(b->params + l * kMaxParams, &b->hparams[l * kMaxParams], n * kMaxParams * 8,
-                             hipMemcpyHostToDevice, b->st));
-      for (int t = 0; t < 4; ++t)
-        HIP_TRY(hipMemcpyAsync(b->outp + t * S + l, &b->hout[t * S + l], n * sizeof(double*), hipMemcpyHostToDevice,
-                               b->st));
-      HIP_TRY(hipMemcpyAsync(b->cur + l, &b->hcur[l], n * sizeof(int), hipMemcpyHostToDevice, b->st));
-      HIP_TRY(hipMemcpyAsync(b->wchol + l, &b->hwchol[l], n * sizeof(int), hipMemcpyHostToDevice, b->st));
-      HIP_TRY(hipMemcpyAsync(b->pfull + l, &b->hpfull[l], n * sizeof(int), hipMemcpyHostToDevice, b->st));
-      HIP_TRY(hipMemcpyAsync(b->cvec + l * D, &b->hcvec[l * D], n * D * 8, hipMemcpyHostToDevice, b->st));
+  const int D = b->D;
+  const size_t DD = (size_t)D * D, S = (size_t)b->slots;
+  if (b->model_dirty) {
+    up.table(b->hF, 0, DD);
+    up.table(b->hLQ, 0, DD);
+    up.table(b->hN1z, 0, DD);
+  }
+  if (!b->dirty_slots.empty()) {
+    // the slot range of the new IVPs: the host tables mirror the device ones for every slot (cur
+    // through the flips of each launch), so the slots in between are rewritten unchanged
+    int lo = b->slots, hi = -1;
+    for (int j : b->dirty_slots) {
+      lo = std::min(lo, j);
+      hi = std::max(hi, j);
     }
-    b->dirty_slots.clear();
-    HIP_TRY(hipMemcpyAsync(b->kind, b->hkind.data(), S * sizeof(int), hipMemcpyHostToDevice, b->st));
-    HIP_TRY(hipMemcpyAsync(b->Ns, b->hNs.data(), S * sizeof(int), hipMemcpyHostToDevice, b->st));
-    HIP_TRY(hipMemcpyAsync(b->base, b->hbase.data(), S * sizeof(long long), hipMemcpyHostToDevice, b->st));
+    const size_t n = (size_t)(hi - lo + 1), l = (size_t)lo;
+    up.table(b->hPd, l * D, n * D);
+    up.table(b->hx0m, l * D, n * D);
+    up.table(b->hx0L, l * DD, n * DD);
+    up.table(b->hparams, l * kMaxParams, n * kMaxParams);
+    up.table(b->hcvec, l * D, n * D);
+    for (int t = 0; t < 4; ++t) up.table(b->hout, t * S + l, n);
+    up.table(b->hkind, l, n);
+    up.table(b->hNs, l, n);
+    std::copy(b->hcur.begin() + lo, b->hcur.begin() + hi + 1, b->hcur_up.p + l);
+    up.table(b->hcur_up, l, n);
+    up.table(b->hwchol, l, n);
+    up.table(b->hpfull, l, n);
+    up.table(b->hbase, l, n);
+  }
+  for (const auto& t : b->init_stage)
+    up.add(b->arena_map + ((const char*)(b->stage.p + t.at) - b->arena_host), b->g.means0 + (size_t)t.start * D, t.n * 8);
+  up.flush();
+  HIP_TRY(up.status);
+  b->model_dirty = false;
+  b->dirty_slots.clear();
+  b->init_stage.clear();
+  if (!b->init_host.empty() || !b->init_dev.empty() || !b->init_zero.empty() || !b->init_const.empty()) {
     for (auto& pr : b->init_host)
       HIP_TRY(hipMemcpyAsync(b->g.means0 + (size_t)pr.first * D, pr.second.data(), pr.second.size() * 8,
                              hipMemcpyHostToDevice, b->st));
@@ -1038,18 +1250,23 @@ int batch_launch(pof_batch* b) {
       HIP_TRY(hipMemcpyAsync(b->g.means0 + (size_t)pr.first * D, pr.second, (size_t)n * D * 8,
                              hipMemcpyDeviceToDevice, b->st));
     }
-    for (int j : b->init_const) {
-      const long long rows = (long long)b->hNs[j] + 1;
-      const long long e = rows * D;
-      hipLaunchKernelGGL(k_fill_rows, dim3((unsigned)((e + 255) / 256)), dim3(256), 0, b->st,
-                         b->g.means0 + (size_t)b->hbase[j] * D, (const double*)(b->cvec + (size_t)j * D), rows, D);
+    for (size_t i0 = 0; i0 < b->init_const.size(); i0 += kFills) {
+      const size_t m = std::min<size_t>(b->init_const.size() - i0, kFills);
+      Fills f;
+      long long most = 0;
+      for (size_t i = 0; i < m; ++i) {
+        f.j[i] = b->init_const[i0 + i];
+        most = std::max(most, ((long long)b->hNs[f.j[i]] + 1) * D);
+      }
+      hipLaunchKernelGGL(k_fill_rows, dim3((unsigned)std::min<long long>((most + 255) / 256, 1024), (unsigned)m), dim3(256),
+                         0, b->st, f, b->g.means0, (const double*)b->cvec, (const int*)b->Ns, (const long long*)b->base, D);
       HIP_TRY(hipGetLastError());
     }
     for (size_t i = 0; i < b->init_zero.size(); ++i)
       HIP_TRY(hipMemsetAsync(b->g.means0 + (size_t)b->init_zero[i] * D, 0, (size_t)b->init_zero_n[i] * D * 8,
                              b->st));
-    // host sources must outlive the copies: wait here (admission only)
-    HIP_TRY(hipStreamSynchronize(b->st));
+    // the vectors must outlive their copies: wait here
+    if (!b->init_host.empty()) HIP_TRY(hipStreamSynchronize(b->st));
     b->init_host.clear();
     b->init_dev.clear();
     b->init_zero.clear();
@@ -1068,12 +1285,14 @@ int batch_launch(pof_batch* b) {
     if (!fixed || s.k + 1 >= s.opts.fixed_iters) b->need_sync = true;
   }
   if (wchange) {
-    if (settle(b) != POF_OK) return POF_E_HIP;
+    HIP_TRY(hipEventSynchronize(b->up_ev));  // no upload may still be reading the table
     for (int j : b->active) {
       const pof_batch::Slot& s = b->sl[j];
       b->hwchol[j] = (s.opts.fixed_iters > 0 && s.k + 1 == s.opts.fixed_iters) ? 1 : 0;
     }
-    HIP_TRY(hipMemcpyAsync(b->wchol, b->hwchol.data(), (size_t)b->slots * sizeof(int), hipMemcpyHostToDevice, b->st));
+    up.table(b->hwchol, 0, S);
+    up.flush();
+    HIP_TRY(up.status);
   }
   KernelTimer* tm = ctx->profiling ? &ctx->timer : nullptr;
   // an instrumented run times every launch from the host: no replay then
@@ -1171,21 +1390,15 @@ int batch_finish(pof_batch* b, int max_done, long long* done, int* n_done) {
   const int start_o = ((int)b->hmaps.size() + 3) / 4 * 4;
   if (rc == POF_OK) rc = plan_tables(b, fin, b->hmaps, po);
   if (rc != POF_OK) return set_err(ctx, rc, "launch tables overflow");
-  if (b->hmaps.size() > b->maps_cap) {
-    HIP_TRY(hipStreamSynchronize(b->st));
-    if (b->maps_dev) HIP_TRY(hipFree(b->maps_dev));
-    b->maps_dev = nullptr;
-    b->maps_cap = 0;
-    const size_t cap = std::max<size_t>(b->hmaps.size() * 2, 4096);
-    HIP_TRY(hipMalloc((void**)&b->maps_dev, cap * sizeof(int)));
-    b->maps_cap = cap;
-  }
-  HIP_TRY(hipMemcpyAsync(b->maps_dev, b->hmaps.data(), b->hmaps.size() * sizeof(int), hipMemcpyHostToDevice,
-                         b->st));
+  HIP_TRY(stage_maps(b));
+  Uploader up(b);
+  up.maps();
+  up.table(b->hwchol, 0, S);
+  up.table(b->hscale, 0, S);
+  up.flush();
+  HIP_TRY(up.status);
   pc.dev = b->maps_dev + start_c;
   po.dev = b->maps_dev + start_o;
-  HIP_TRY(hipMemcpyAsync(b->wchol, b->hwchol.data(), S * sizeof(int), hipMemcpyHostToDevice, b->st));
-  HIP_TRY(hipMemcpyAsync(b->scale, b->hscale.data(), S * sizeof(double), hipMemcpyHostToDevice, b->st));
   KernelTimer* tm = ctx->profiling ? &ctx->timer : nullptr;
   if (!need.empty()) {
     if (b->mode == 1 || b->mode == 2 || b->mode == 4) {
@@ -1308,6 +1521,7 @@ void batch_abort(pof_batch* b) {
   b->free_.clear();
   b->free_[0] = b->entries;
   b->dirty_slots.clear();
+  b->init_stage.clear();
   b->init_host.clear();
   b->init_dev.clear();
   b->init_zero.clear();
@@ -1479,6 +1693,7 @@ void pof_ctx_destroy(pof_ctx* ctx) {
   ctx->cache.clear();
   for (pof_batch* b : ctx->aux) batch_free(b);
   ctx->aux.clear();
+  drop_kept(ctx);
   pof::large::engine_destroy(ctx->large);
   ctx->large = nullptr;
   if (ctx->timer.ready)
@@ -1836,7 +2051,7 @@ namespace {
 // A caller's transition model (F, QL) for an affine batch: F, QL, N1 = tria([0 | QL]),
 // and whether QL is lower triangular (its strict upper part exactly zero), which
 // lets the smoother-element factorisation skip QL's upper columns.
-hipError_t upload_transition(pof_batch* b, const double* F_host, const double* QL_host) {
+void set_transition(pof_batch* b, const double* F_host, const double* QL_host) {
   const int D = b->D;
   const size_t DD = (size_t)D * D;
   std::vector<double> M(DD * 2, 0.0), N1z;
@@ -1844,10 +2059,10 @@ hipError_t upload_transition(pof_batch* b, const double* F_host, const double* Q
     for (int c = 0; c < D; ++c) M[(size_t)r * 2 * D + D + c] = QL_host[(size_t)r * D + c];
   pof::tria_host(M, D, 2 * D, N1z);
   b->g.lq_lower = pof::strictly_upper_zero(QL_host, D) ? 1 : 0;
-  hipError_t e = hipMemcpy(b->F, F_host, DD * 8, hipMemcpyHostToDevice);
-  if (e == hipSuccess) e = hipMemcpy(b->LQ, QL_host, DD * 8, hipMemcpyHostToDevice);
-  if (e == hipSuccess) e = hipMemcpy(b->N1z, N1z.data(), DD * 8, hipMemcpyHostToDevice);
-  return e;
+  std::copy(F_host, F_host + DD, b->hF.p);
+  std::copy(QL_host, QL_host + DD, b->hLQ.p);
+  std::copy(N1z.begin(), N1z.end(), b->hN1z.p);
+  b->model_dirty = true;
 }
 }  // namespace
 
@@ -1864,17 +2079,14 @@ int pof_smoothing(pof_ctx* ctx, int D, int64_t Ns, const double* F_host, const d
     if (D % dd == 0 && (e = pof::find_engine(D, dd)) != nullptr) d = dd;
   if (!e) return set_err(ctx, POF_E_UNSUPPORTED, "no kernels for state dimension %d", D);
   HIP_TRY(hipSetDevice(ctx->device));
-  pof_batch* b = nullptr;
-  int rc = batch_new(ctx, D, d, entries_for(Ns + 1), 1, true, &b);
+  CallBatch call(ctx);
+  int rc = call.open(D, d, entries_for(Ns + 1), true);
   if (rc != POF_OK) return rc;
-  struct Guard {
-    pof_batch* b;
-    ~Guard() { batch_free(b); }
-  } guard{b};
+  pof_batch* b = call.b;
   StreamScope scope(b, stream);
   HIP_TRY(scope.status);
   const size_t DD = (size_t)D * D;
-  HIP_TRY(upload_transition(b, F_host, QL_host));
+  set_transition(b, F_host, QL_host);
   // state 0 enters as the prior of the slot, states 1..Ns as the level-0 filter prefixes
   std::vector<double> m0(D), L0(DD);
   HIP_TRY(hipMemcpy(m0.data(), filt_mean_dev, D * 8, hipMemcpyDeviceToHost));
@@ -1897,6 +2109,7 @@ int pof_smoothing(pof_ctx* ctx, int D, int64_t Ns, const double* F_host, const d
   rc = run_to_completion(b);
   if (rc != POF_OK) return rc;
   if (obj) *obj = po.obj;
+  call.done = true;
   return POF_OK;
 }
 
@@ -1910,18 +2123,15 @@ int pof_ekf(pof_ctx* ctx, const pof_problem* prob, const double* x0_mean_host, c
   if (rc != POF_OK) return rc;
   if (!engine_or_err(ctx, s.D, s.d)) return POF_E_UNSUPPORTED;
   HIP_TRY(hipSetDevice(ctx->device));
-  pof_batch* b = nullptr;
-  rc = batch_new(ctx, s.D, s.d, entries_for(prob->n_times), 1, false, &b);
+  CallBatch call(ctx);
+  rc = call.open(s.D, s.d, entries_for(prob->n_times), false);
   if (rc != POF_OK) return rc;
-  struct Guard {
-    pof_batch* b;
-    ~Guard() { batch_free(b); }
-  } guard{b};
+  pof_batch* b = call.b;
   StreamScope scope(b, stream);
   HIP_TRY(scope.status);
   const int D = s.D;
   const size_t DD = (size_t)D * D;
-  HIP_TRY(upload_transition(b, F_host, QL_host));
+  set_transition(b, F_host, QL_host);
   pof_opts o{};
   o.maxiters = 1;
   o.fixed_iters = 1;
@@ -1938,6 +2148,7 @@ int pof_ekf(pof_ctx* ctx, const pof_problem* prob, const double* x0_mean_host, c
   if (rc != POF_OK) return rc;
   if (nll) *nll = po.nll;
   if (ssq) *ssq = po.sigma_squared;
+  call.done = true;
   return POF_OK;
 }
 
@@ -1952,18 +2163,15 @@ int pof_linear_filtsmooth(pof_ctx* ctx, int D, int d, int64_t Ns, const double* 
       !H_dev || !c_dev)
     return set_err(ctx, POF_E_ARG, "invalid linear_filtsmooth arguments");
   if (!engine_or_err(ctx, D, d)) return POF_E_UNSUPPORTED;
-  pof_batch* b = nullptr;
-  int rc = batch_new(ctx, D, d, entries_for(Ns + 1), 1, true, &b);
+  CallBatch call(ctx);
+  int rc = call.open(D, d, entries_for(Ns + 1), true);
   if (rc != POF_OK) return rc;
-  struct Guard {
-    pof_batch* b;
-    ~Guard() { batch_free(b); }
-  } guard{b};
+  pof_batch* b = call.b;
   StreamScope scope(b, stream);
   HIP_TRY(scope.status);
   // the caller's model: F, QL, N1 = tria([0 | QL]), x0; no preconditioning (P = 1)
   const size_t DD = (size_t)D * D;
-  HIP_TRY(upload_transition(b, F_host, QL_host));
+  set_transition(b, F_host, QL_host);
   b->g.Hx = H_dev;
   b->g.cx = c_dev;
   b->g.Rx = R_dev;
@@ -1990,6 +2198,7 @@ int pof_linear_filtsmooth(pof_ctx* ctx, int D, int d, int64_t Ns, const double* 
   if (nll) *nll = po.nll;
   if (obj) *obj = po.obj;
   if (ssq) *ssq = po.sigma_squared;
+  call.done = true;
   return POF_OK;
 }
 
