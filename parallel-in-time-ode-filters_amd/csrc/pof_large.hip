@@ -17,6 +17,7 @@
 #include "pof_large.hpp"
 
 #include "pof_problems.hpp"
+#include "pof_row16.hpp"
 #include "pof_wave.hpp"
 
 #include <algorithm>
@@ -51,335 +52,495 @@ __device__ inline double wave_sum(double v) {
   return v;
 }
 
-constexpr int kLqThreads = 256;
-constexpr int kLqMaxN = 512;
-
-// In-place Householder LQ of the m x n matrix of item blockIdx.x: afterwards its
-// first min(m, n) columns hold tria(A) = qr(A^T).R^T (utils.py:33-41) with
-// LAPACK's reflectors (beta = -sign(alpha) ||x||, tau = (beta - alpha) / beta,
-// v = x / (alpha - beta), no reflector for a zero tail).  Pivot row i's tail is
-// reduced by the whole block; every later row is updated by one wave.
-__global__ __launch_bounds__(kLqThreads) void k_lq(double* A, long long stride, int m, int n, int ld) {
-  __shared__ double v[kLqMaxN];
-  __shared__ double red[kLqThreads / 64];
-  double* a = A + (long long)blockIdx.x * stride;
-  const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
-  constexpr int NW = kLqThreads / 64;
-  const int K = m < n ? m : n;
-  for (int i = 0; i < K && i < n - 1; ++i) {
-    double* pr = a + (size_t)i * ld;
-    double s = 0.0;
-    for (int j = i + 1 + tid; j < n; j += kLqThreads) s = fma(pr[j], pr[j], s);
-    s = wave_sum(s);
-    if (lane == 0) red[wv] = s;
-    __syncthreads();
-    const double sig = (red[0] + red[1]) + (red[2] + red[3]);
-    const double alpha = pr[i];
-    double tau = 0.0, beta = alpha, scal = 0.0;
-    if (sig != 0.0) {
-      const double nrm = sqrt(fma(alpha, alpha, sig));
-      beta = -copysign(nrm, alpha);
-      tau = (beta - alpha) / beta;
-      scal = 1.0 / (alpha - beta);
-    }
-    for (int j = i + 1 + tid; j < n; j += kLqThreads) v[j] = pr[j] * scal;
-    __syncthreads();
-    if (tau != 0.0) {
-      for (int r = i + 1 + wv; r < m; r += NW) {
-        double* rr = a + (size_t)r * ld;
-        double w = 0.0;
-        for (int j = i + 1 + lane; j < n; j += 64) w = fma(rr[j], v[j], w);
-        w = wave_sum(w) + rr[i];
-        const double tw = tau * w;
-        for (int j = i + 1 + lane; j < n; j += 64) rr[j] = fma(-tw, v[j], rr[j]);
-        if (lane == 0) rr[i] -= tw;
-      }
-    }
-    if (tid == 0) pr[i] = beta;
-    for (int j = i + 1 + tid; j < n; j += kLqThreads) pr[j] = 0.0;
-    __syncthreads();
-  }
-}
-
-constexpr int kNB = 16;  // rows per panel of the blocked LQ
-
-// f(integral_constant<int, K>) for K = 0, 1, ... in order: a loop whose index
-// is a compile-time constant in every step
-template <typename F, int... K>
-__device__ __forceinline__ void unroll_steps(F& f, std::integer_sequence<int, K...>) {
-  (f(std::integral_constant<int, K>()), ...);
-}
-
-// One panel of the blocked LQ (LAPACK dgelqf: dgelq2 on the panel, dlarft
-// forward / rowwise): rows i0 .. i0 + np - 1 of item blockIdx.x, columns
-// i0 .. n - 1, factored by one wave with the panel in registers (lane holds
-// columns lane + 64 q) and the reflectors of k_lq.  Writes the panel's rows of
-// L back, the reflectors V (np x (n - i0), leading 1, zeros before it) and the
-// triangular factor T (np x np) with H_1 ... H_np = I - V^T T V.  Pivot column
-// k < kNB < 64 lives in slot 0 of lane k, so only slot 0 needs the test c > k;
-// columns c >= n - i0 are loaded as zeros and stay zero (every update adds a
-// multiple of the pivot row, zero there too), so they need no test.  Rows
-// np .. kNB - 1 are zeros too: their updates leave them so and they are never
-// written, so the steps need no row test either.
+// ------------------------------------------------------------------ LQ
+// tria(A) = qr(A^T).R^T (utils.py:33-41) of a batch of m x n matrices in place, LAPACK's reflectors (beta =
+// -sign(alpha) ||x||, tau = (beta - alpha) / beta, v = x / (alpha - beta), no reflector for a zero tail), blocked by
+// strips of 16 rows: strip s first takes the block reflectors I - V^T T V of the strips before it, in order, and is
+// then factored itself (dgelq2 with dlarft, forward / rowwise).  One wave does this for a whole matrix, two strips at a
+// time; the rows below the pivots, which only take block reflectors, go to waves of their own (k_lq_below).
 //
-// Step k sums 16 - k values over the wave at once (the squared tail of pivot
-// row k and the products of rows k + 1 .. kNB - 1 with it) in registers: a
-// transposed wave sum leaves each total in a group of lanes, and scalar reads
-// of one lane broadcast it, so a step has no LDS round trip and no barrier.
-typedef double lq_panel_d4 __attribute__((ext_vector_type(4)));
-// Three waves per SIMD at four column slots: the Gram matrix accumulates in
-// ordinary VGPRs then, and the panel fits in 156 registers.
-template <int NQ>
-__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(3))) void k_lq_panel(
-    double* A, long long sA, int n, int ld, int i0, int np, double* Vb, long long sV, int ldV, double* Tb,
-    long long sT, int ldT) {
-  __shared__ double G[kNB][kNB + 1];
-  __shared__ double taus[kNB];
-  const int lane = threadIdx.x;
-  double* a = A + (long long)blockIdx.x * sA + (size_t)i0 * ld + i0;
-  double* Vo = Vb + (long long)blockIdx.x * sV;
-  const int nc = n - i0;
-  double P[kNB][NQ];
-#pragma unroll
-  for (int r = 0; r < kNB; ++r) {
-#pragma unroll
-    for (int q = 0; q < NQ; ++q) {
-      const int c = lane + 64 * q;
-      P[r][q] = (r < np && c < nc) ? a[(size_t)r * ld + c] : 0.0;
-    }
-  }
-  // Householder step k (a compile-time constant); NV, a power of two >= kNB - k,
-  // values per wave sum
-  auto step = [&](auto kc) __attribute__((always_inline)) {
-    constexpr int k = decltype(kc)::value;
-    constexpr int NV = k < 8 ? 16 : (k < 12 ? 8 : (k < 14 ? 4 : (k < 15 ? 2 : 1)));
-    constexpr int G1 = 64 / NV;  // lanes per total after the wave sum
-    if (k >= np) return;
-    // value 0: the squared tail of pivot row k; value j >= 1: row k + j . tail of row k.
-    // Slot 0 holds a tail column only in lanes beyond k: masked once, here.
-    const double pk0 = (lane > k) ? P[k][0] : 0.0;
-    double x[NV];
-    {
-      double sq = pk0 * pk0;
-#pragma unroll
-      for (int q = 1; q < NQ; ++q) sq = fma(P[k][q], P[k][q], sq);
-      x[0] = sq;
-    }
-#pragma unroll
-    for (int j = 1; j < NV; ++j) {
-      const int r = k + j;
-      double w = 0.0;
-      if (r < kNB) {
-        w = P[r][0] * pk0;
-#pragma unroll
-        for (int q = 1; q < NQ; ++q) w = fma(P[r][q], P[k][q], w);
-      }
-      x[j] = w;
-    }
-    wave::sum_scatter<NV>(x, lane);
-    const double sig = wave::lane_value(x[0], 0);
-    const double alpha = wave::lane_value(P[k][0], k);
-    double tau = 0.0, beta = alpha, scal = 0.0;
-    if (sig != 0.0) {
-      const double nrm = sqrt(fma(alpha, alpha, sig));
-      beta = -copysign(nrm, alpha);
-      tau = (beta - alpha) / beta;
-      scal = 1.0 / (alpha - beta);
-    }
-    // the reflector in slot 0: 1 in the pivot lane, the scaled tail beyond it, 0 before
-    const double v0 = (lane > k) ? P[k][0] * scal : ((lane == k) ? 1.0 : 0.0);
-    P[k][0] = (lane > k) ? v0 : P[k][0];
-#pragma unroll
-    for (int q = 1; q < NQ; ++q) P[k][q] *= scal;
-    // row k is final: L row k back to A, V row k out (slots q >= 1 hold columns
-    // 64 q + lane > k: zero in L, tail in V)
-    if (lane < nc) {
-      a[(size_t)k * ld + lane] = (lane < k) ? P[k][0] : ((lane == k) ? beta : 0.0);
-      Vo[(size_t)k * ldV + lane] = (lane < k) ? 0.0 : ((lane == k) ? 1.0 : P[k][0]);
-    }
-#pragma unroll
-    for (int q = 1; q < NQ; ++q) {
-      const int c = lane + 64 * q;
-      if (c < nc) {
-        a[(size_t)k * ld + c] = 0.0;
-        Vo[(size_t)k * ldV + c] = P[k][q];
-      }
-    }
-    if (lane == 0) taus[k] = tau;
-    if (tau != 0.0) {
-#pragma unroll
-      for (int r = k + 1; r < kNB; ++r) {
-        // row r . v with v = [1, scal * tail]; the pivot column of row r sits in lane k
-        const double tr = wave::lane_value(x[0], (r - k) * G1);
-        const double ck = wave::lane_value(P[r][0], k);
-        const double tw = tau * fma(scal, tr, ck);
-        P[r][0] = fma(-tw, v0, P[r][0]);
-#pragma unroll
-        for (int q = 1; q < NQ; ++q) P[r][q] = fma(-tw, P[k][q], P[r][q]);
-      }
-    }
-  };
-  unroll_steps(step, std::make_integer_sequence<int, kNB>());
-  // T (dlarft, forward / rowwise): G = V V^T on the matrix cores, with V read back from the
-  // rows just stored (L2; the panel's registers are free by then), 64 columns per batch of
-  // loads and four accumulation chains (a Gram matrix sums over every column, so the order
-  // of the columns is free); then lane j forms row j of T:
-  // T[j][k] = -tau_k sum_{l = j}^{k - 1} T[j][l] G[l][k], T[k][k] = tau_k
-  __threadfence_block();
-  __syncthreads();
-  const int gj = lane & 15, gg = lane >> 4;
-  const double* vr = Vo + (size_t)gj * ldV;
-  lq_panel_d4 ga[4] = {{0.0, 0.0, 0.0, 0.0}, {0.0, 0.0, 0.0, 0.0}, {0.0, 0.0, 0.0, 0.0}, {0.0, 0.0, 0.0, 0.0}};
-#pragma unroll
-  for (int q = 0; q < NQ; ++q) {
-    if (64 * q < nc) {
-      double x[16];
-#pragma unroll
-      for (int e = 0; e < 16; ++e) {
-        const int c = 64 * q + 16 * (e >> 2) + 4 * gg + (e & 3);
-        x[e] = (gj < np && c < nc) ? vr[c] : 0.0;
-      }
-#pragma unroll
-      for (int e = 0; e < 16; ++e) ga[e & 3] = __builtin_amdgcn_mfma_f64_16x16x4f64(x[e], x[e], ga[e & 3], 0, 0, 0);
-    }
-  }
-  // the FP64 accumulator holds element (l / 16 + 4 v, l % 16) in value v of lane l
-#pragma unroll
-  for (int v = 0; v < 4; ++v) G[gg + 4 * v][gj] = (ga[0][v] + ga[1][v]) + (ga[2][v] + ga[3][v]);
-  __syncthreads();
-  if (lane < np) {
-    double trow[kNB];
-#pragma unroll
-    for (int k = 0; k < kNB; ++k) {
-      double acc = 0.0;
-#pragma unroll
-      for (int l = 0; l < k; ++l) acc = fma(trow[l], -taus[k] * G[l][k], acc);  // trow[l] = 0 for l < lane
-      trow[k] = (k < np) ? ((lane < k) ? acc : ((lane == k) ? taus[k] : 0.0)) : 0.0;
-    }
-    double* T = Tb + (long long)blockIdx.x * sT + (size_t)lane * ldT;
-#pragma unroll
-    for (int k = 0; k < kNB; ++k)
-      if (k < np) T[k] = trow[k];
-  }
-}
-
+// Why left-looking: a panel kernel and an update kernel over all matrices per 16 pivots read and wrote every row below the
+// panel each time (6 MB per combine at D = 128), and a panel, one wave with its columns over the lanes, summed over the
+// wave for every pivot.  Here a strip is read and written once and stays in registers; the reflectors of the strips
+// before it are read once per two strips; a matrix's waits are another's work.  Two iterations of 8,192 steps at
+// D = 128: 138 -> 83 ms in these kernels, and no copies put [B1 | B2] together or take the factor out (22 ms); at
+// D = 24 an LQ of 24 rows 38 -> 13 us.  Bound by the two waves' FP64 issue (a pivot: 173 instructions, of which 72
+// products) and, at D = 128, by the reflectors' traffic: 0.7 MB per matrix, 2,048 of which take 0.4 ms.
+//
+// Layout of a strip: tile t holds columns 16 t .. 16 t + 15 from the window's first on, lane j + 16 g value v holds
+// (row j, column 16 t + 4 g + v).  These registers are at once
+//  - rows of lanes of a DPP row for the factorisation: lane j of each of the wave's four DPP rows holds row j, a
+//    quarter of its columns, and takes row k's as a broadcast operand (pof_row16.hpp);
+//  - the B operand of K-step v of W^T = V A_s^T (summation index 4 v + g standing for column 4 g + v);
+//  - the accumulator of A_s^T -= V^T W2^T, W2^T = T^T W^T, when tile row i stands for column 4 (i % 4) + i / 4 (the FP64
+//    accumulator holds element (l / 16 + 4 v, l % 16) in value v of lane l).
+// W^T's accumulator value v is likewise the B operand of K-step v of the next product.
+//
+// The window of panel p is its columns 16 p .. lq_end(p) - 1: a banded second block's columns beyond it are zero in the
+// pivot rows.  Before the next panel a strip stores its first tile, which is final, and shifts by one.
+// The matrix's blocks are read from where they are and the factor is written to where it is wanted (LqArgs): no copy
+// puts [B1 | B2] together or takes the factor out.
+constexpr int kLqSlots = 2048;  // matrices factored at a time (two waves per SIMD); scratch is kept for as many
+constexpr int kLqBelowWaves = 4;
 typedef double lq_d4 __attribute__((ext_vector_type(4)));
 
-// Trailing update of one panel of the blocked LQ, in one pass over the rows
-// below the panel: A_t <- A_t (I - V^T T V) for A_t = rows i0 + np .. i0 + np
-// + mr - 1 and columns i0 .. i0 + nc - 1 of an item, with V (np x nc) and T
-// (np x np) from k_lq_panel.  Per strip of 16 rows, on the FP64 matrix cores
-// (v_mfma_f64_16x16x4f64): W^T = V A_s^T, W2^T = T^T W^T, A_s^T -= V^T W2^T.
-// The strip stays in registers between the three products, so A_t is read
-// and written once per panel.
-//
-// Register layout of a strip: tile t holds columns 16 t .. 16 t + 15, lane
-// j + 16 g value v holds (row j, column 16 t + 4 g + v).  These registers are
-// at once the B operand of K-step v of W^T = V A_s^T (summation index 4 v + g
-// standing for column 4 g + v) and the accumulator of A_s^T's tile when its
-// row i stands for column 4 (i % 4) + i / 4 (the FP64 accumulator holds
-// element (l / 16 + 4 v, l % 16) in value v of lane l).  W^T's accumulator
-// value v is likewise the B operand of K-step v of the next product.
-//
-// Four waves per block, one strip each; V (zero-padded to 16 rows and 16 NT
-// columns) and T are staged in LDS.  Blocks are numbered so that the blocks of
-// one item run on one XCD (work-groups go round-robin over the 8 XCDs) and
-// share V through its L2.
-constexpr int kLqUpdWaves = 4;
-template <int NT, bool VEC>
-__global__ __launch_bounds__(64 * kLqUpdWaves, 2) void k_lq_update(double* A, long long sA, int ld, int i0, int np,
-                                                                    int mr, int nc, const double* Vb, long long sV,
-                                                                    int ldV, const double* Tb, long long sT, int ldT,
-                                                                    int cnt, int sbk) {
-  constexpr int LDV = 16 * NT + 1;
-  __shared__ double Vs[16 * LDV];
-  __shared__ double Ts[16 * 17];
-  const int L = blockIdx.x;
-  const int rr = L / 8;
-  const long long item = (long long)(rr / sbk) * 8 + (L % 8);
-  const int sb = rr % sbk;
-  if (item >= cnt) return;  // uniform over the block
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const double* vsrc = Vb + item * sV;
-  for (int e = tid; e < 16 * 16 * NT; e += 64 * kLqUpdWaves) {
-    const int p = e / (16 * NT), c = e % (16 * NT);
-    Vs[p * LDV + c] = (p < np && c < nc) ? vsrc[(size_t)p * ldV + c] : 0.0;
-  }
-  {
-    const int p = tid / 16, c = tid % 16;
-    Ts[p * 17 + c] = (p < np && c < np) ? Tb[item * sT + (size_t)p * ldT + c] : 0.0;
-  }
-  __syncthreads();
-  const int r0 = 16 * (sb * kLqUpdWaves + wave);
-  if (r0 >= mr) return;  // no barrier follows
-  const int j = lane & 15, g = lane >> 4;
-  const int ntr = (nc + 15) / 16;
-  const int nfull = nc / 16;  // tiles without a column beyond nc
-  const bool rowok = r0 + j < mr;
-  // a row past the trailing block reads the block's last row: every product below keeps
-  // the strip's rows apart (row j of the strip only meets column j of W^T), and it is not stored
-  double* arow = A + item * sA + (size_t)(i0 + np + min(r0 + j, mr - 1)) * ld + i0 + 4 * g;
-  lq_d4 X[NT];
-#pragma unroll
-  for (int t = 0; t < NT; ++t) {
-    if (t < nfull) {
-      if constexpr (VEC) {
-        const double2 lo = *(const double2*)(arow + 16 * t);
-        const double2 hi = *(const double2*)(arow + 16 * t + 2);
-        X[t] = lq_d4{lo.x, lo.y, hi.x, hi.y};
-      } else {
-#pragma unroll
-        for (int v = 0; v < 4; ++v) X[t][v] = arow[16 * t + v];
-      }
-    } else if (t < ntr) {
-#pragma unroll
-      for (int v = 0; v < 4; ++v) X[t][v] = (16 * t + 4 * g + v < nc) ? arow[16 * t + v] : 0.0;
-    } else {
-      X[t] = lq_d4{0.0, 0.0, 0.0, 0.0};
+enum LqSecond : int { kLqNone = 0, kLqGiven = 1, kLqIdentity = 2 };
+struct LqArgs {
+  // columns < ca of rows < rs, and of rows >= rs
+  const double *a, *a2;
+  long long sa, sa2;
+  int lda, lda2, rs, ca;
+  // columns >= ca: none, the matrix b (zero from row rs on) or [I; 0]
+  int second;
+  const double *b, *b_;
+  long long sb, sb_;
+  int ldb;
+  // the result, columns < no (rows of pivots: columns < min(no, ca), the strict upper part zero)
+  double *o, *o_;
+  long long so, so_;
+  int ldo, no;
+  int half;   // items from half on: b_ and o_, counted from there
+  int item0;  // item of block 0
+  int m, n;
+  int npiv;    // pivots 0 .. npiv - 1
+  int b1, w2;  // b1 > 0: in columns b1 .. n - 1 row r < rs is zero beyond column b1 + max(r, w2)
+  double* scr;  // per matrix and panel: V [NT * 256], T [256]
+  long long sS;
+};
+__host__ __device__ inline int lq_np(int npiv, int p) { return npiv - 16 * p < 16 ? npiv - 16 * p : 16; }
+// end (exclusive) of the columns that panel p's reflectors reach
+__host__ __device__ inline int lq_end(int n, int npiv, int b1, int w2, int p) {
+  const int last = 16 * p + lq_np(npiv, p) - 1;
+  if (b1 <= 0 || last >= b1) return n;
+  const int e = b1 + (last > w2 ? last : w2) + 1;
+  return e < n ? e : n;
+}
+__host__ __device__ constexpr int lq_panel_doubles(int nt) { return nt * 256 + 256; }
+
+// tiles of the widest panel, and the tiles that the kernels are compiled for: registers and scratch scale with them
+// (the banded panels of the D = 128 combines have 9 or 10, those of D = 24 and 32 three)
+inline int lq_tiles(int n, int npiv, int b1, int w2) {
+  int nt = 1;
+  for (int p = 0; 16 * p < npiv; ++p) nt = std::max(nt, (lq_end(n, npiv, b1, w2, p) - 16 * p + 15) / 16);
+  for (int t : {3, 5, 8, 9, 10})
+    if (nt <= t) return t;
+  return 16;
+}
+// Pivots of the first factorisation of an m x n matrix (Ops::lq)
+inline int lq_first(int m, int n, int b1) {
+  const int kmax = std::min(std::min(m, n), n - 1);
+  return (b1 > 0 && kmax > b1) ? b1 : kmax;
+}
+// Scratch doubles per matrix
+inline size_t lq_need(int m, int n, int b1, int w2) {
+  const int npiv = lq_first(m, n, b1);
+  if (npiv <= 0) return 0;
+  const size_t need = (size_t)((npiv + 15) / 16) * lq_panel_doubles(lq_tiles(n, npiv, b1, w2));
+  return (npiv == b1 && m > b1 && n - b1 > 1) ? std::max(need, lq_need(m - b1, n - b1, 0, 0)) : need;
+}
+
+// Row r of item it: where its two blocks are read (b from column ca on) and where it is written; columns from end on are
+// not read (zeros, or the identity's)
+struct LqRow {
+  const double *a, *b;
+  double* o;
+  int r, end;
+  bool ok;
+};
+__device__ __forceinline__ LqRow lq_row(const LqArgs& q, long long it, int r, bool ok) {
+  LqRow w;
+  w.r = r;
+  w.ok = ok;
+  const int rr = ok ? r : 0, h = it >= q.half ? 1 : 0;
+  const long long ih = it - (h ? q.half : 0);
+  w.a = (rr < q.rs) ? q.a + it * q.sa + (size_t)rr * q.lda : q.a2 + it * q.sa2 + (size_t)(rr - q.rs) * q.lda2;
+  const bool given = q.second == kLqGiven && rr < q.rs;
+  const double* b = h ? q.b_ : q.b;
+  w.b = given ? b + ih * (h ? q.sb_ : q.sb) + (size_t)rr * q.ldb - q.ca : w.a;
+  const int band = q.ca + (rr > q.w2 ? rr : q.w2) + 1;
+  w.end = !ok ? 0 : (!given ? q.ca : (band < q.n ? band : q.n));
+  double* o = h ? q.o_ : q.o;
+  w.o = o + ih * (h ? q.so_ : q.so) + (size_t)rr * q.ldo;
+  return w;
+}
+// x is formed here and now: not moved out of the loop or block that it is in, which would hold it in a register for long
+template <class T>
+__device__ __forceinline__ void lq_here(T& x) {
+  asm volatile("" : "+v"(x));
+}
+// Columns c .. c + 3.  VEC: 16-byte accesses, every row starts on a 16-byte boundary and ca, n and no are multiples of 4.
+// (Loads without a branch, of some valid address where there is nothing to read, and selects afterwards took 10 % longer.)
+template <bool VEC>
+__device__ __forceinline__ lq_d4 lq_load(const LqArgs& q, const LqRow& w, int c) {
+  lq_here(c);
+  lq_d4 x = {0.0, 0.0, 0.0, 0.0};
+  if constexpr (VEC) {
+    if (c < w.end) {
+      const double* src = (c < q.ca ? w.a : w.b) + c;
+      const double2 lo = *(const double2*)src, hi = *(const double2*)(src + 2);
+      x = lq_d4{lo.x, lo.y, hi.x, hi.y};
     }
+  } else {
+#pragma unroll
+    for (int v = 0; v < 4; ++v)
+      if (c + v < w.end) x[v] = (c + v < q.ca ? w.a : w.b)[c + v];
   }
-  // W^T (rows: panel rows p, columns: strip rows j) = V A_s^T
-  lq_d4 wt = {0.0, 0.0, 0.0, 0.0};
+  if (q.second == kLqIdentity && w.ok) {
+#pragma unroll
+    for (int v = 0; v < 4; ++v) x[v] = (c + v - q.ca == w.r) ? 1.0 : x[v];
+  }
+  return x;
+}
+template <bool VEC>
+__device__ __forceinline__ void lq_store(const LqRow& w, int c, int lim, lq_d4 x) {
+  if (!w.ok) return;
+  if constexpr (VEC) {
+    lq_here(c);
+    if (c < lim) {
+      *(double2*)(w.o + c) = double2{x[0], x[1]};
+      *(double2*)(w.o + c + 2) = double2{x[2], x[3]};
+    }
+  } else {
+#pragma unroll
+    for (int v = 0; v < 4; ++v)
+      if (c + v < lim) w.o[c + v] = x[v];
+  }
+}
+
+// V of a panel in LDS, as in the scratch: 16 bytes (h, 4 j + g) of tile t are V[j][16 t + 4 g + 2 h ..], so that lane
+// (j, g) finds its operand of the first product there and the transposed one of the last without bank conflicts.
+// Chunks first, first + step, ... of 1 KB go from the scratch straight into LDS (no registers); the caller waits.
+template <int NT>
+__device__ __forceinline__ void lq_stage(const double* vp, double* sh, int nt, int lane, int first, int step) {
+#pragma unroll
+  for (int c = 0; c < 2 * NT; ++c)
+    if (c % step == first && c < 2 * nt)
+      __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)(vp + c * 128 + 2 * lane),
+                                       (__attribute__((address_space(3))) void*)(sh + c * 128), 16, 0, 0);
+}
+__device__ __forceinline__ void lq_wait() { asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory"); }
+__device__ __forceinline__ void lq_wait_lds() { asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory"); }
+
+// T as the second product's A operand: value s is T[4 s + g][j]
+__device__ __forceinline__ void lq_load_t(double (&T)[4], const double* t, int j, int g) {
+#pragma unroll
+  for (int s = 0; s < 4; ++s) T[s] = t[64 * s + 16 * g + j];
+}
+
+// The block reflector (V in LDS) to the first nt tiles of S strips
+template <int NT, int S>
+__device__ __forceinline__ void lq_apply(lq_d4 (*X)[NT], const double* sh, const double (&T)[4], int nt, int j, int g) {
+  const double2* v1 = reinterpret_cast<const double2*>(sh) + 4 * j + g;
+  // V[4 s + g][16 t + 4 (j % 4) + j / 4]
+  const double* v2 = sh + (j / 8) * 128 + 8 * g + 2 * (j % 4) + (j / 4) % 2;
+  lq_d4 wt[S];
+#pragma unroll
+  for (int i = 0; i < S; ++i) wt[i] = lq_d4{0.0, 0.0, 0.0, 0.0};
 #pragma unroll
   for (int t = 0; t < NT; ++t) {
-    if (t < ntr) {
+    if (t < nt) {
+      const double2 a0 = v1[t * 128], a1 = v1[t * 128 + 64];
+      const double av[4] = {a0.x, a0.y, a1.x, a1.y};
 #pragma unroll
       for (int s = 0; s < 4; ++s)
-        wt = __builtin_amdgcn_mfma_f64_16x16x4f64(Vs[j * LDV + 16 * t + 4 * g + s], X[t][s], wt, 0, 0, 0);
+#pragma unroll
+        for (int i = 0; i < S; ++i) wt[i] = __builtin_amdgcn_mfma_f64_16x16x4f64(av[s], X[i][t][s], wt[i], 0, 0, 0);
     }
   }
-  // W2^T = T^T W^T
-  lq_d4 w2t = {0.0, 0.0, 0.0, 0.0};
+  lq_d4 w2[S];
 #pragma unroll
-  for (int s = 0; s < 4; ++s) w2t = __builtin_amdgcn_mfma_f64_16x16x4f64(Ts[(4 * s + g) * 17 + j], wt[s], w2t, 0, 0, 0);
-  // A_s^T -= V^T W2^T: accumulator row i of tile t stands for column 16 t + 4 (i % 4) + i / 4
-  const int ci = 4 * (j & 3) + (j >> 2);
+  for (int i = 0; i < S; ++i) w2[i] = lq_d4{0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+  for (int s = 0; s < 4; ++s)
+#pragma unroll
+    for (int i = 0; i < S; ++i) w2[i] = __builtin_amdgcn_mfma_f64_16x16x4f64(T[s], wt[i][s], w2[i], 0, 0, 0);
+#pragma unroll
+  for (int i = 0; i < S; ++i) w2[i] = -w2[i];
 #pragma unroll
   for (int t = 0; t < NT; ++t) {
-    if (t < ntr) {
+    if (t < nt) {
 #pragma unroll
       for (int s = 0; s < 4; ++s)
-        X[t] = __builtin_amdgcn_mfma_f64_16x16x4f64(-Vs[(4 * s + g) * LDV + 16 * t + ci], w2t[s], X[t], 0, 0, 0);
+#pragma unroll
+        for (int i = 0; i < S; ++i)
+          X[i][t] = __builtin_amdgcn_mfma_f64_16x16x4f64(v2[t * 256 + 32 * s], w2[i][s], X[i][t], 0, 0, 0);
     }
   }
-  if (rowok) {
+}
+
+// A strip's first tile is final and taken out, and the window moves on by one tile (last, read before)
+template <int NT>
+__device__ __forceinline__ lq_d4 lq_shift(lq_d4 (&X)[NT], lq_d4 last) {
+  const lq_d4 first = X[0];
+#pragma unroll
+  for (int t = 0; t + 1 < NT; ++t) X[t] = X[t + 1];
+  X[NT - 1] = last;
+  return first;
+}
+
+// The sums over the wave's four DPP rows of a and of b, in every lane
+__device__ __forceinline__ void lq_row_sums(double& a, double& b) {
+  wave::swap_halves(a, b);
+  double y = a + b, y2 = y;  // lanes < 32: a's, the others b's
+  wave::swap_rows(y, y2);
+  a = y + y2;
+  b = a;
+  wave::swap_halves(a, b);
+}
+
+// Pivots 0 .. np - 1 of a strip: on return x holds the reflectors' tails in rows < np (to be scaled by sc; zeros before them)
+// and the updated columns of the others, lt the finished columns of the strip's first tile, tr row j of T in lane j.  The
+// product of row k's tail with every row gives, besides the update, V's Gram matrix for T: no pass of its own.
+template <int NT>
+__device__ __forceinline__ void lq_factor(double (&x)[4 * NT], double (&lt)[4], double (&tr)[16], double& sc, int np, int j,
+                                          int g) {
+  sc = 1.0;  // 1 / (alpha - beta) of row j's pivot
+#pragma unroll
+  for (int v = 0; v < 4; ++v) lt[v] = 0.0;
+#pragma unroll
+  for (int k = 0; k < 16; ++k) tr[k] = 0.0;
+  r16::unroll<0, 16>([&](auto kc) {
+    constexpr int k = decltype(kc)::value, gk = k / 4, vk = k % 4;
+    if (k >= np) return;  // uniform
+    const bool own = g == gk;
+    // the pivot column leaves the strip: what remains of row k is its tail
+    double ac = own ? x[vk] : 0.0;
+    x[vk] = own ? 0.0 : x[vk];
+    const double xk = ac;
+    double dot = r16::dot_self<k, 4 * NT>(x);
+    lq_row_sums(dot, ac);
+    const double alpha = r16::bcast<k>(ac);
+    bool nz;
+    const r16::Pivot p = r16::pivot(alpha, r16::bcast<k>(dot), nz);
+    const double w = fma(p.sc, dot, ac);  // row j . v
+    const double t = (j > k) ? p.rb * w : 0.0;
+    r16::fnma_self<k, 4 * NT>(x, t);
+    const double fin = (j > k) ? fma(-p.den, t, ac) : ((j == k) ? (nz ? p.beta : alpha) : 0.0);
+    lt[vk] = own ? fin : lt[vk];
+    x[vk] = (own && j < k) ? xk : x[vk];
+    // T[j][k] = -tau_k sum_{j <= l < k} T[j][l] v_l . v_k, T[k][k] = tau_k
+    const double acc = r16::dot_lanes<k>(tr, sc * w);
+    const double tau = p.den * p.rb;
+    tr[k] = (j < k) ? -tau * acc : ((j == k) ? tau : 0.0);
+    sc = (j == k) ? p.sc : sc;
+  });
+}
+
+// Whether a wave's second strip waits in LDS (V's place) while the first is factored: the registers would not hold both ...
+template <int NT, int S>
+constexpr bool kLqPark = S == 2 && NT >= 5;
+// ... and whether it stays there until V has left the registers too, so that V comes back from the scratch
+template <int NT, int S>
+constexpr bool kLqBack = S == 2 && NT >= 9;
+// doubles of LDS of k_lq_rows: V, and T where it does not come back from the scratch (eight blocks per CU up to ten tiles)
+template <int NT, int S>
+constexpr int kLqLds = NT * 256 + (kLqBack<NT, S> ? 0 : 256);
+
+// Factors strip X[0] (panel p), stores its rows and, with keep, V and T in the scratch.  With next, V is in LDS afterwards and
+// T in registers, for the other strip.
+template <int NT, int S, bool VEC>
+__device__ __forceinline__ void lq_strip(const LqArgs& q, lq_d4 (&X)[S][NT], const LqRow& w, int p, int j, int g,
+                                         double* sh, double (&T)[4], double* vp, bool keep, bool next) {
+  constexpr bool kPark = kLqPark<NT, S>, kBack = kLqBack<NT, S>;
+  const int np = lq_np(q.npiv, p), nt = (lq_end(q.n, q.npiv, q.b1, q.w2, p) - 16 * p + 15) / 16;
+  const int lane = j + 16 * g;
+  double2* park = reinterpret_cast<double2*>(sh) + lane;
+  if constexpr (kPark) {
 #pragma unroll
     for (int t = 0; t < NT; ++t) {
-      if (t < nfull) {
-        if constexpr (VEC) {
-          *(double2*)(arow + 16 * t) = double2{X[t][0], X[t][1]};
-          *(double2*)(arow + 16 * t + 2) = double2{X[t][2], X[t][3]};
-        } else {
+      park[128 * t] = double2{X[S - 1][t][0], X[S - 1][t][1]};
+      park[128 * t + 64] = double2{X[S - 1][t][2], X[S - 1][t][3]};
+    }
+  }
+  keep = keep || (kBack && next);
+  auto unpark = [&] {  // (also without next: else it would be taken to live on in registers)
+    lq_wait_lds();
 #pragma unroll
-          for (int v = 0; v < 4; ++v) arow[16 * t + v] = X[t][v];
-        }
-      } else if (t < ntr) {
+    for (int t = 0; t < NT; ++t) {
+      const double2 lo = park[128 * t], hi = park[128 * t + 64];
+      X[S - 1][t] = lq_d4{lo.x, lo.y, hi.x, hi.y};
+    }
+    lq_wait_lds();
+  };
+  double x[4 * NT], lt[4], sc;
+  {
+    double tr[16];
 #pragma unroll
-        for (int v = 0; v < 4; ++v)
-          if (16 * t + 4 * g + v < nc) arow[16 * t + v] = X[t][v];
+    for (int t = 0; t < NT; ++t)
+#pragma unroll
+      for (int v = 0; v < 4; ++v) x[4 * t + v] = X[0][t][v];
+    lq_factor<NT>(x, lt, tr, sc, np, j, g);
+    if (g == 0) {
+      if constexpr (!kBack && S == 2) {
+        double2* t = reinterpret_cast<double2*>(sh + NT * 256) + 8 * j;
+#pragma unroll
+        for (int k = 0; k < 8; ++k) t[k] = double2{tr[2 * k], tr[2 * k + 1]};
+      }
+      if (keep) {
+        double2* t = reinterpret_cast<double2*>(vp + NT * 256) + 8 * j;
+#pragma unroll
+        for (int k = 0; k < 8; ++k) t[k] = double2{tr[2 * k], tr[2 * k + 1]};
       }
     }
   }
+  if constexpr (kPark && !kBack) unpark();
+  const bool piv = j < np;
+  const int lim = piv ? (q.no < q.ca ? q.no : q.ca) : q.no;
+#pragma unroll
+  for (int t = 0; t < NT; ++t) {
+    if (t < nt) {
+      lq_d4 y;
+      double v[4];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        double z = x[4 * t + e];
+        lq_here(z);
+        v[e] = piv ? z * sc : 0.0;
+        y[e] = piv ? 0.0 : z;
+        if (t == 0) {
+          v[e] = (piv && 4 * g + e == j) ? 1.0 : v[e];
+          y[e] = (4 * g + e < np) ? lt[e] : y[e];
+        }
+      }
+      lq_store<VEC>(w, 16 * (p + t) + 4 * g, lim, y);
+      const int at = t * 128 + 4 * j + g;
+      if constexpr (!kBack && S == 2) {
+        double2* l = reinterpret_cast<double2*>(sh) + at;
+        l[0] = double2{v[0], v[1]};
+        l[64] = double2{v[2], v[3]};
+      }
+      if (keep) {
+        double2* l = reinterpret_cast<double2*>(vp) + at;
+        l[0] = double2{v[0], v[1]};
+        l[64] = double2{v[2], v[3]};
+      }
+    }
+  }
+  if constexpr (kBack) unpark();
+  if (!next) return;
+  if constexpr (kBack) {
+    lq_wait();
+    lq_stage<NT>(vp, sh, nt, lane, 0, 1);
+    lq_load_t(T, vp + NT * 256, j, g);
+    lq_wait();
+  } else {
+    lq_wait_lds();
+    lq_load_t(T, sh + NT * 256, j, g);
+  }
+}
+
+// Rows 0 .. 16 ceil(npiv / 16) - 1 of a matrix, S strips at a time
+template <int NT, int S, bool VEC>
+__global__ __launch_bounds__(64, 2) void k_lq_rows(LqArgs q) {
+  static_assert(S <= 2, "strips");
+  __shared__ __align__(16) double sh[kLqLds<NT, S>];
+  const int lane = threadIdx.x, j = lane & 15, g = lane >> 4;
+  double* scr = q.scr + (long long)blockIdx.x * q.sS;
+  const int P = (q.npiv + 15) / 16;
+  for (int s0 = 0; s0 < P; s0 += S) {
+    lq_d4 X[S][NT];
+    LqRow w[S];
+#pragma unroll
+    for (int i = 0; i < S; ++i) {
+      const int r = 16 * (s0 + i) + j;
+      w[i] = lq_row(q, q.item0 + (long long)blockIdx.x, r, r < q.m && s0 + i < P);
+#pragma unroll
+      for (int t = 0; t < NT; ++t) X[i][t] = lq_load<VEC>(q, w[i], 16 * t + 4 * g);
+    }
+    lq_wait();  // ... and for the strips before to be in the scratch
+    // a tile taken out is stored beside the next panel's products: a store just before a wait would be waited for
+    lq_d4 last[S], fin[S];
+    for (int p = 0; p < s0; ++p) {
+      const int nt = (lq_end(q.n, q.npiv, q.b1, q.w2, p) - 16 * p + 15) / 16;
+      const double* vp = scr + (size_t)p * lq_panel_doubles(NT);
+      double T[4];
+      lq_stage<NT>(vp, sh, nt, lane, 0, 1);
+      lq_load_t(T, vp + NT * 256, j, g);
+#pragma unroll
+      for (int i = 0; i < S; ++i) last[i] = lq_load<VEC>(q, w[i], 16 * (p + NT) + 4 * g);
+      lq_wait();
+      if (p > 0) {
+#pragma unroll
+        for (int i = 0; i < S; ++i) lq_store<VEC>(w[i], 16 * (p - 1) + 4 * g, q.no, fin[i]);
+      }
+      lq_apply<NT, S>(X, sh, T, nt, j, g);
+      lq_wait_lds();
+#pragma unroll
+      for (int i = 0; i < S; ++i) fin[i] = lq_shift<NT>(X[i], last[i]);
+    }
+    if (s0 > 0) {
+#pragma unroll
+      for (int i = 0; i < S; ++i) lq_store<VEC>(w[i], 16 * (s0 - 1) + 4 * g, q.no, fin[i]);
+    }
+    // the strips in turn at X[0]
+#pragma unroll 1
+    for (int p = s0; p < s0 + S && p < P; ++p) {
+      // later strips and the rows below read it from the scratch
+      double T[4];
+      lq_strip<NT, S, VEC>(q, X, w[0], p, j, g, sh, T, scr + (size_t)p * lq_panel_doubles(NT), s0 + S < P || q.m > 16 * P,
+                           S > 1 && p == s0 && p + 1 < P);
+      if (S > 1 && p == s0 && p + 1 < P) {
+        const int nt = (lq_end(q.n, q.npiv, q.b1, q.w2, p) - 16 * p + 15) / 16;
+        const lq_d4 nx = lq_load<VEC>(q, w[S - 1], 16 * (p + NT) + 4 * g);
+        lq_apply<NT, 1>(&X[S - 1], sh, T, nt, j, g);
+        lq_wait_lds();
+        const lq_d4 f = lq_shift<NT>(X[S - 1], nx);
+        lq_store<VEC>(w[S - 1], 16 * p + 4 * g, q.no, f);
+#pragma unroll
+        for (int t = 0; t < NT; ++t) X[0][t] = X[S - 1][t];
+        w[0] = w[S - 1];
+      }
+    }
+  }
+}
+
+// The rows below, r0 .. m - 1, take every panel's block reflector: S strips per wave, V and T shared by the block's waves
+template <int NT, int S, bool VEC>
+__global__ __launch_bounds__(64 * kLqBelowWaves, 2) void k_lq_below(LqArgs q, int r0) {
+  __shared__ __align__(16) double sh[NT * 256];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, j = lane & 15, g = lane >> 4;
+  const int s0 = (blockIdx.y * kLqBelowWaves + wave) * S;
+  const bool act = r0 + 16 * s0 < q.m;  // uniform per wave
+  const double* scr = q.scr + (long long)blockIdx.x * q.sS;
+  const int P = (q.npiv + 15) / 16;
+  lq_d4 X[S][NT];
+  LqRow w[S];
+#pragma unroll
+  for (int i = 0; i < S; ++i) {
+    const int r = r0 + 16 * (s0 + i) + j;
+    w[i] = lq_row(q, q.item0 + (long long)blockIdx.x, r, r < q.m);
+#pragma unroll
+    for (int t = 0; t < NT; ++t) X[i][t] = lq_load<VEC>(q, w[i], 16 * t + 4 * g);
+  }
+  lq_d4 last[S], fin[S];
+  for (int p = 0; p < P; ++p) {
+    const int nt = (lq_end(q.n, q.npiv, q.b1, q.w2, p) - 16 * p + 15) / 16;
+    const double* vp = scr + (size_t)p * lq_panel_doubles(NT);
+    double T[4];
+    lq_stage<NT>(vp, sh, nt, lane, wave, kLqBelowWaves);
+    lq_load_t(T, vp + NT * 256, j, g);
+#pragma unroll
+    for (int i = 0; i < S; ++i) last[i] = lq_load<VEC>(q, w[i], 16 * (p + NT) + 4 * g);
+    lq_wait();
+    __syncthreads();
+    if (act) {
+      if (p > 0) {
+#pragma unroll
+        for (int i = 0; i < S; ++i) lq_store<VEC>(w[i], 16 * (p - 1) + 4 * g, q.no, fin[i]);
+      }
+      lq_apply<NT, S>(X, sh, T, nt, j, g);
+      if (p + 1 < P) {
+#pragma unroll
+        for (int i = 0; i < S; ++i) fin[i] = lq_shift<NT>(X[i], last[i]);
+      }
+    }
+    __syncthreads();
+  }
+  if (!act) return;
+#pragma unroll
+  for (int i = 0; i < S; ++i)
+#pragma unroll
+    for (int t = 0; t < NT; ++t) lq_store<VEC>(w[i], 16 * (P - 1 + t) + 4 * g, q.no, X[i][t]);
 }
 
 constexpr int kTrsmMaxN = 128;  // order of the triangular matrix at most (D <= 128)
@@ -1069,97 +1230,122 @@ struct Ops {
                          alpha, A.p, A.s, A.ld, B.p, B.s, B.ld, beta, C.p, C.s, C.ld);
     }
   }
-  // tria in place: the blocked LQ (panels of kNB rows, trailing rows updated in one
-  // pass per panel), or k_lq for matrices of at most one panel.  b1 > 0 declares a
-  // banded second block: in columns b1 .. n - 1, row r is zero beyond column
-  // b1 + max(r, w2).  Pivot i's reflector is then zero beyond column b1 + max(i, w2)
-  // (the reflectors before it only reach that far), so a panel of first-block pivots
-  // leaves the columns beyond its last pivot's band as they are and skips them: the
-  // same factor, with the panel and its trailing update over fewer columns.
-  void lq(V A, int m, int n, int cnt, int b1 = 0, int w2 = 0) {
+  // tria in place of m x n matrices
+  void lq(V A, int m, int n, int cnt) {
+    LqBlocks q{};
+    q.a = A;
+    q.rs = m;
+    q.o[0] = A;
+    q.no = n;
+    lq(q, m, n, cnt, 0, 0);
+  }
+  // Where the matrices of an LQ and their factors are.  The second block (columns from b1 on) is banded: row r < rs is zero
+  // beyond column b1 + max(r, w2).  Pivot i's reflector is then zero beyond column b1 + max(i, w2) (the reflectors before it
+  // only reach that far), so a panel of first-block pivots leaves the columns beyond its last pivot's band as they
+  // are and skips them: the same factor over fewer columns.
+  struct LqBlocks {
+    V a;               // first block of rows < rs
+    V a2;              // ... of the rows from rs on
+    int rs;
+    int second;        // second block of rows < rs: none (everything is in a), given by b, or the identity; then zero
+    V b[2];
+    V o[2];            // result: columns < no
+    int no;
+    int half;          // with a second set, b[1] and o[1] are those of the items from half on (0: one set)
+  };
+  // tria; b1 columns in the first block (0: all).  Pivots of the second block (m > b1) are a factorisation of their own,
+  // of what the first leaves in the result: to o2 if given, else in place.
+  void lq(const LqBlocks& q, int m, int n, int cnt, int b1, int w2, const V* o2 = nullptr) {
     if (err || cnt <= 0) return;
     if (n > 256) {
       fail("lq: more than 256 columns", -1);
       return;
     }
-    const int K = m < n ? m : n;
-    const int kmax = K < n - 1 ? K : n - 1;
-    if (m <= kNB || kmax <= 0) {
-      hipLaunchKernelGGL(k_lq, dim3(cnt), dim3(kLqThreads), 0, st, A.p, A.s, m, n, A.ld);
-      check("k_lq");
-      return;
+    const int npiv = lq_first(m, n, b1);
+    if (npiv <= 0) return;
+    switch (lq_tiles(n, npiv, b1, w2)) {
+      case 3: launch_lq<3, 2>(q, m, n, cnt, npiv, b1, w2); break;
+      case 5: launch_lq<5, 2>(q, m, n, cnt, npiv, b1, w2); break;
+      case 8: launch_lq<8, 2>(q, m, n, cnt, npiv, b1, w2); break;
+      case 9: launch_lq<9, 2>(q, m, n, cnt, npiv, b1, w2); break;
+      case 10: launch_lq<10, 2>(q, m, n, cnt, npiv, b1, w2); break;
+      default: launch_lq<16, 1>(q, m, n, cnt, npiv, b1, w2);  // two strips would not fit the registers
     }
+    if (m <= b1 || n <= b1 || b1 <= 0) return;
+    LqBlocks r{};
+    r.a = q.o[0].at(b1, b1);
+    r.rs = m - b1;
+    r.o[0] = o2 ? *o2 : r.a;
+    r.no = n - b1;
+    lq(r, m - b1, n - b1, cnt, 0, 0);
+  }
+  template <int NT, int S>
+  void launch_lq(const LqBlocks& q, int m, int n, int cnt, int npiv, int b1, int w2) {
+    const int P = (npiv + 15) / 16;
     const size_t mark = arena_mark(ar);
-    V Vb{arena_take(ar, (size_t)cnt * kNB * n), (long long)kNB * n, n};
-    V Tb{arena_take(ar, (size_t)cnt * kNB * kNB), (long long)kNB * kNB, kNB};
-    if (!Vb.p || !Tb.p) {
+    const long long sS = (long long)P * lq_panel_doubles(NT);
+    LqArgs a{};
+    a.a = q.a.p;
+    a.sa = q.a.s;
+    a.lda = q.a.ld;
+    a.a2 = q.a2.p;
+    a.sa2 = q.a2.s;
+    a.lda2 = q.a2.ld;
+    a.rs = q.rs;
+    a.ca = q.second == kLqNone ? n : b1;
+    a.second = q.second;
+    bool vec = a.ca % 4 == 0 && n % 4 == 0 && q.no % 4 == 0;
+    auto even = [&](const V& v) {
+      if (v.p) vec = vec && (uintptr_t)v.p % 16 == 0 && v.s % 2 == 0 && v.ld % 2 == 0;
+    };
+    even(q.a);
+    even(q.a2);
+    for (int h = 0; h < 2; ++h) {
+      even(q.b[h]);
+      even(q.o[h]);
+    }
+    a.b = q.b[0].p;
+    a.b_ = q.b[1].p;
+    a.sb = q.b[0].s;
+    a.sb_ = q.b[1].s;
+    a.o = q.o[0].p;
+    a.o_ = q.o[1].p;
+    a.so = q.o[0].s;
+    a.so_ = q.o[1].s;
+    a.ldb = q.b[0].ld;
+    a.ldo = q.o[0].ld;
+    a.no = q.no;
+    a.half = q.half > 0 ? q.half : cnt;
+    a.m = m;
+    a.n = n;
+    a.npiv = npiv;
+    a.b1 = b1;
+    a.w2 = w2;
+    a.scr = arena_take(ar, (size_t)std::min(cnt, kLqSlots) * sS);
+    a.sS = sS;
+    if (!a.scr) {
       fail("workspace (lq)", -2);
       return;
     }
-    for (int i0 = 0; i0 < kmax && !err; i0 += kNB) {
-      const int np = (kmax - i0) < kNB ? (kmax - i0) : kNB;
-      int ce = n;  // end (exclusive) of the columns this panel's reflectors reach
-      if (b1 > 0 && i0 + np <= b1) {
-        const int last = i0 + np - 1;
-        ce = std::min(n, b1 + std::max(last, w2) + 1);
-      }
-      const int nc = ce - i0;
-      // column slots for this panel's own width: later panels are narrower
-      const int nq = (nc + 63) / 64;
-      if (nq <= 1) {
-        hipLaunchKernelGGL(k_lq_panel<1>, dim3(cnt), dim3(64), 0, st, A.p, A.s, ce, A.ld, i0, np, Vb.p, Vb.s, Vb.ld,
-                           Tb.p, Tb.s, Tb.ld);
-      } else if (nq == 2) {
-        hipLaunchKernelGGL(k_lq_panel<2>, dim3(cnt), dim3(64), 0, st, A.p, A.s, ce, A.ld, i0, np, Vb.p, Vb.s, Vb.ld,
-                           Tb.p, Tb.s, Tb.ld);
-      } else if (nq == 3) {
-        hipLaunchKernelGGL(k_lq_panel<3>, dim3(cnt), dim3(64), 0, st, A.p, A.s, ce, A.ld, i0, np, Vb.p, Vb.s, Vb.ld,
-                           Tb.p, Tb.s, Tb.ld);
-      } else {
-        hipLaunchKernelGGL(k_lq_panel<4>, dim3(cnt), dim3(64), 0, st, A.p, A.s, ce, A.ld, i0, np, Vb.p, Vb.s, Vb.ld,
-                           Tb.p, Tb.s, Tb.ld);
-      }
-      check("k_lq_panel");
-      const int mr = m - (i0 + np);
-      if (mr <= 0) continue;
-      // A_trail (I - V^T T V) in one pass (FP64, as the rest of the factorisation)
-      lq_update(A, i0, np, mr, nc, Vb, Tb, cnt);
+    for (int c0 = 0; c0 < cnt; c0 += kLqSlots) {
+      const int c = std::min(cnt - c0, kLqSlots);
+      a.item0 = c0;
+      if (vec)
+        launch_lq_part<NT, S, true>(a, c, P);
+      else
+        launch_lq_part<NT, S, false>(a, c, P);
     }
     arena_release(ar, mark);
   }
-  void lq_update(V A, int i0, int np, int mr, int nc, V Vb, V Tb, int cnt) {
-    const int strips = (mr + 15) / 16;
-    const int sbk = (strips + kLqUpdWaves - 1) / kLqUpdWaves;
-    const dim3 grid((unsigned)(((cnt + 7) / 8) * 8 * sbk));
-    const dim3 block(64 * kLqUpdWaves);
-    // 16-byte loads and stores when every row of the block starts on a 16-byte boundary
-    const bool vec = ((uintptr_t)A.p % 16 == 0) && (A.s % 2 == 0) && (A.ld % 2 == 0) && (i0 % 2 == 0);
-    // tiles of 16 columns: the fewest that cover nc (registers and LDS scale with them; the banded
-    // panels of the D = 128 combines have 144 or 160 columns)
-    if (nc <= 64) {
-      launch_update<4>(vec, grid, block, A, i0, np, mr, nc, Vb, Tb, cnt, sbk);
-    } else if (nc <= 128) {
-      launch_update<8>(vec, grid, block, A, i0, np, mr, nc, Vb, Tb, cnt, sbk);
-    } else if (nc <= 144) {
-      launch_update<9>(vec, grid, block, A, i0, np, mr, nc, Vb, Tb, cnt, sbk);
-    } else if (nc <= 160) {
-      launch_update<10>(vec, grid, block, A, i0, np, mr, nc, Vb, Tb, cnt, sbk);
-    } else if (nc <= 192) {
-      launch_update<12>(vec, grid, block, A, i0, np, mr, nc, Vb, Tb, cnt, sbk);
-    } else {
-      launch_update<16>(vec, grid, block, A, i0, np, mr, nc, Vb, Tb, cnt, sbk);
-    }
-    check("k_lq_update");
-  }
-  template <int NT>
-  void launch_update(bool vec, dim3 grid, dim3 block, V A, int i0, int np, int mr, int nc, V Vb, V Tb, int cnt,
-                     int sbk) {
-    if (vec) {
-      hipLaunchKernelGGL((k_lq_update<NT, true>), grid, block, 0, st, A.p, A.s, A.ld, i0, np, mr, nc, Vb.p, Vb.s,
-                         Vb.ld, Tb.p, Tb.s, Tb.ld, cnt, sbk);
-    } else {
-      hipLaunchKernelGGL((k_lq_update<NT, false>), grid, block, 0, st, A.p, A.s, A.ld, i0, np, mr, nc, Vb.p, Vb.s,
-                         Vb.ld, Tb.p, Tb.s, Tb.ld, cnt, sbk);
+  template <int NT, int S, bool VEC>
+  void launch_lq_part(const LqArgs& a, int cnt, int P) {
+    hipLaunchKernelGGL((k_lq_rows<NT, S, VEC>), dim3(cnt), dim3(64), 0, st, a);
+    check("k_lq_rows");
+    if (a.m > 16 * P) {
+      const int per = 16 * S * kLqBelowWaves;
+      hipLaunchKernelGGL((k_lq_below<NT, S, VEC>), dim3(cnt, (a.m - 16 * P + per - 1) / per), dim3(64 * kLqBelowWaves), 0,
+                         st, a, 16 * P);
+      check("k_lq_below");
     }
   }
   // op(L) X = R (L lower n x n, X n x m): R is X itself (in place), or the separate R when given
@@ -1297,9 +1483,9 @@ void filter_fn(Ops& o, Arena& ar, int D, const FE& e1, const FE& e2, const FE& o
   const size_t mark = ar.off;
   const long long DD = (long long)D * D;
   V X{ar.take((size_t)cnt * 4 * DD), 4 * DD, 2 * D};
-  // [M^T | U2] for items 0 .. cnt - 1 and [A1^T Xi22 | Z1] for items cnt .. 2 cnt - 1: both are
+  // M^T for items 0 .. cnt - 1 and A1^T Xi22 for items cnt .. 2 cnt - 1: [M^T | U2] and [A1^T Xi22 | Z1] are
   // factored by one LQ call over 2 cnt items
-  V Y{ar.take((size_t)cnt * 4 * DD), 2 * DD, 2 * D};
+  V Y{ar.take((size_t)cnt * 2 * DD), DD, D};
   const V YZ = Y.item(cnt);
   V T2{ar.take((size_t)cnt * DD), DD, D};
   V T3{ar.take((size_t)cnt * DD), DD, D}, T4{ar.take((size_t)cnt * DD), DD, D};
@@ -1309,9 +1495,16 @@ void filter_fn(Ops& o, Arena& ar, int D, const FE& e1, const FE& e2, const FE& o
   }
   // Xi = tria([[U1^T Z2, I], [Z2, 0]])
   o.gemm(true, false, D, D, D, 1.0, e1.U, e2.Z, 0.0, X.at(0, 0), cnt);
-  o.copies({{X.at(0, D), V{}, D, D, 1.0}, {X.at(D, 0), e2.Z, D, D, 0.0}, {X.at(D, D), V{}, D, D, 0.0}}, cnt);
-  // second block [I; 0]: row r is zero beyond column D + r
-  o.lq(X, 2 * D, 2 * D, cnt, D, 0);
+  {
+    Ops::LqBlocks q{};
+    q.a = X;
+    q.a2 = e2.Z;
+    q.rs = D;
+    q.second = kLqIdentity;
+    q.o[0] = X;
+    q.no = 2 * D;
+    o.lq(q, 2 * D, 2 * D, cnt, D, 0);
+  }
   const V Xi11 = X.at(0, 0), Xi21 = X.at(D, 0), Xi22 = X.at(D, D);
   // m_ = Xi11^-1 U1^T -> T3; M^T = (m_ A2^T)^T = A2 m_^T, formed in place as the left
   // block of [M^T | U2] (Y)
@@ -1327,12 +1520,22 @@ void filter_fn(Ops& o, Arena& ar, int D, const FE& e1, const FE& e2, const FE& o
   o.trsm(true, D, D, Xi11, T4, cnt, Xi21, true);
   o.vec_chain(D, e2.Z, true, e2.Z, false, e1.U, true, T4, true, e1.A, true, e1.b, e2.eta, -1.0, e1.eta, out.eta,
               cnt);
-  // A1^T Xi22 and the right blocks U2, Z1; then U = tria([M^T | U2]) and Z = tria([A1^T Xi22 | Z1]) in one call
+  // A1^T Xi22; then U = tria([M^T | U2]) and Z = tria([A1^T Xi22 | Z1]) in one call
   o.gemm(true, false, D, D, D, 1.0, e1.A, Xi22, 0.0, YZ.at(0, 0), cnt);
-  o.copies({{Y.at(0, D), e2.U, D, D, 0.0}, {YZ.at(0, D), e1.Z, D, D, 0.0}}, cnt);
   // second blocks U2 (lower triangular) and Z1 (lower triangular, or [Zr | 0] at the leaves)
-  o.lq(Y, D, 2 * D, 2 * cnt, D, o.zw2);
-  o.copies({{out.U, Y.at(0, 0), D, D, 0.0}, {out.Z, YZ.at(0, 0), D, D, 0.0}}, cnt);
+  {
+    Ops::LqBlocks q{};
+    q.a = Y;
+    q.rs = D;
+    q.second = kLqGiven;
+    q.b[0] = e2.U;
+    q.b[1] = e1.Z;
+    q.o[0] = out.U;
+    q.o[1] = out.Z;
+    q.no = D;
+    q.half = cnt;
+    o.lq(q, D, 2 * D, 2 * cnt, D, o.zw2);
+  }
   ar.off = mark;
 }
 
@@ -1346,15 +1549,20 @@ void smoother_fn(Ops& o, Arena& ar, int D, const SE& e1, const SE& e2, const SE&
   o.gemm(false, false, D, D, D, 1.0, e2.E, e1.E, 0.0, out.E, cnt);
   if (with_chol) {
     const long long DD = (long long)D * D;
-    V Y{ar.take((size_t)cnt * 2 * DD), 2 * DD, 2 * D};
+    V Y{ar.take((size_t)cnt * DD), DD, D};
     if (!Y.p) {
       o.fail("workspace", -2);
       return;
     }
-    o.gemm(false, false, D, D, D, 1.0, e2.E, e1.Dm, 0.0, Y.at(0, 0), cnt);
-    o.copy(Y.at(0, D), e2.Dm, D, D, cnt);
-    o.lq(Y, D, 2 * D, cnt, D, 0);  // second block D2: lower triangular
-    o.copy(out.Dm, Y.at(0, 0), D, D, cnt);
+    o.gemm(false, false, D, D, D, 1.0, e2.E, e1.Dm, 0.0, Y, cnt);
+    Ops::LqBlocks q{};
+    q.a = Y;
+    q.rs = D;
+    q.second = kLqGiven;
+    q.b[0] = e2.Dm;
+    q.o[0] = out.Dm;
+    q.no = D;
+    o.lq(q, D, 2 * D, cnt, D, 0);  // second block D2: lower triangular
   }
   ar.off = mark;
 }
@@ -1428,7 +1636,7 @@ bool supports(int kind, int D, int d) {
 namespace {
 
 // workspace doubles for one solve
-size_t workspace_doubles(int D, int d, long long Ns, bool f32) {
+size_t workspace_doubles(int D, int d, long long Ns, bool f32, bool ql_lower) {
   const size_t DD = (size_t)D * D;
   const size_t n1 = (size_t)Ns + 1;
   size_t w = 0;
@@ -1442,12 +1650,16 @@ size_t workspace_doubles(int D, int d, long long Ns, bool f32) {
   // per-call temporaries at the widest level (the filter combine), and the post step
   const size_t h = (size_t)(Ns / 2 + 1);
   w += h * (4 * DD + 4 * DD + 5 * DD) + 4096;
-  w += (size_t)(Ns + 1) * (2 * D * kNB + kNB * kNB) + 4096;  // blocked-LQ panels (V, T)
+  // the reflectors of the matrices that are factored at a time
+  const int qw = ql_lower ? 0 : D - 1;
+  const size_t lq = std::max({lq_need(d + D, D, 0, 0), lq_need(2 * D, 2 * D, D, 0), lq_need(D, 2 * D, D, d - 1),
+                              lq_need(2 * D, 2 * D, D, qw), lq_need(D, 2 * D, D, qw)});
+  w += std::min<size_t>(n1 + 1, kLqSlots) * lq + 4096;
   w += (size_t)Ns * (5 * DD + (size_t)d * D + 2 * D + 3 * d + 4) + 4096;
   w += 8 * n1 + 64 * 1024;
   // FP32 staging of one GEMM (both operands and the product; at most n1 items of D x D)
   if (f32) w += n1 * 2 * DD + 3 * 4096;
-  return w + w / 10;
+  return w + w / 20;
 }
 
 }  // namespace
@@ -1475,7 +1687,11 @@ int solve(Engine* e, const Problem& p, const pof_opts& opts, pof_out* out, const
   }
   // workspace
   const bool f32 = opts.products == POF_PRODUCTS_F32;
-  const size_t need = workspace_doubles(D, d, Ns, f32) * sizeof(double);
+  // a lower-triangular QL makes the second blocks [QL] and [QL; 0] banded (the LQs skip past the band)
+  bool ql_lower = true;
+  for (int i = 0; i < D; ++i)
+    for (int j = i + 1; j < D; ++j) ql_lower = ql_lower && p.QL[(size_t)i * D + j] == 0.0;
+  const size_t need = workspace_doubles(D, d, Ns, f32, ql_lower) * sizeof(double);
   if (e->cap < need) {
     if (e->buf) (void)hipFree(e->buf);
     e->buf = nullptr;
@@ -1536,11 +1752,7 @@ int solve(Engine* e, const Problem& p, const pof_opts& opts, pof_out* out, const
       qli[(size_t)i * D + j] = v / p.QL[(size_t)i * D + i];
     }
   up(dQLi, qli.data(), DD);
-  // a lower-triangular QL makes the second blocks [QL] and [QL; 0] banded (the LQs skip past the band)
-  bool ql_lower = true;
-  for (int i = 0; i < D; ++i)
-    for (int j = i + 1; j < D; ++j) ql_lower = ql_lower && p.QL[(size_t)i * D + j] == 0.0;
-  const int ql_band = ql_lower ? D : 0;
+  const int ql_w2 = ql_lower ? 0 : D - 1;
   up(dm0, p.x0m, D);
   up(mA, p.m0, (size_t)(Ns + 1) * D);
   if (he != hipSuccess) {
@@ -1592,8 +1804,16 @@ int solve(Engine* e, const Problem& p, const pof_opts& opts, pof_out* out, const
       // element 0: m1 = F m0, N1 = tria([F L0 | QL]); elements k >= 1: m1 = 0, N1 = tria([0 | QL])
       o.gemm(false, false, D, 1, D, 1.0, Fv, V{dm0, 0, 1}, 0.0, m1, 1);
       o.gemm(false, false, D, D, D, 1.0, Fv, V{dL0, 0, D}, 0.0, N10.at(0, 0), 1);
-      o.copy(N10.at(0, D), QLv, D, D, 1);
-      o.lq(N10, D, 2 * D, 1, ql_band, 0);
+      {
+        Ops::LqBlocks q{};
+        q.a = N10;
+        q.rs = D;
+        q.second = kLqGiven;
+        q.b[0] = QLv;
+        q.o[0] = N10;
+        q.no = D;
+        o.lq(q, D, 2 * D, 1, D, ql_w2);
+      }
       for (int part = 0; part < 2; ++part) {
         const int k0 = part == 0 ? 0 : 1;
         const int cnt = part == 0 ? 1 : n - 1;
@@ -1661,13 +1881,21 @@ int solve(Engine* e, const Problem& p, const pof_opts& opts, pof_out* out, const
       if (!Phi.p || !Fm.p || !Sb.p || !yv.p || !Phin.p) o.fail("workspace", -2);
       const V fmv{fm, D, 1}, fLv{fL, DD, D};
       o.gemm(false, false, D, D, D, 1.0, Fv, fLv, 0.0, Phi.at(0, 0), n);
-      o.copies({{Phi.at(0, D), QLv, D, D, 0.0}, {Phi.at(D, 0), fLv, D, D, 0.0}, {Phi.at(D, D), V{}, D, D, 0.0}}, n);
-      o.lq(Phi, 2 * D, 2 * D, n, ql_band, 0);  // second block [QL; 0]
+      {
+        Ops::LqBlocks q{};
+        q.a = Phi;
+        q.a2 = fLv;
+        q.rs = D;
+        q.second = kLqGiven;  // [QL; 0]
+        q.b[0] = QLv;
+        q.o[0] = Phi;
+        q.no = 2 * D;
+        o.lq(q, 2 * D, 2 * D, n, D, ql_w2, &snat.Dm);
+      }
       // E = Phi21 Phi11^-1, D = Phi22, g = m - E F m
       // E^T = Phi11^-T Phi21^T
       o.trsm(true, D, D, Phi.at(0, 0), Phin, n, Phi.at(D, 0), true);
       o.copy(snat.E, Phin, D, D, n, true);
-      o.copy(snat.Dm, Phi.at(D, D), D, D, n);
       o.gemm(false, false, D, 1, D, 1.0, Fv, fmv, 0.0, Fm, n);
       o.copy(snat.g, fmv, D, 1, n);
       o.gemm(false, false, D, 1, D, -1.0, snat.E, Fm, 1.0, snat.g, n);

@@ -258,6 +258,22 @@ __device__ __forceinline__ double reflect_self(double* y, double rb, double sc, 
   return t;
 }
 
+// y[c] -= bcast_L(y[c]) t, c < N (lane L's own values feed the products before they change)
+template <int L, int N>
+__device__ __forceinline__ void fnma_self(double* y, double t) {
+#define POF_OP(i) POF_FMAC(y##i, y##i, "-%[t]", l)
+#define POF_CASE(n)     \
+  if constexpr (N == n) \
+    asm volatile("s_nop 1\n" POF_SEQ##n(POF_OP) : POF_CSV##n(POF_Y) : [t] "v"(t), [l] "n"(L));
+  POF_CASES(POF_CASE)
+#undef POF_CASE
+#undef POF_OP
+  if constexpr (N > kGroup) {
+    fnma_self<L, kGroup>(y, t);
+    fnma_self<L, N - kGroup>(y + kGroup, t);
+  }
+}
+
 // init + sum_{k < N} bcast_k(v) x[k]: a row (or, of a transposed matrix, a column) times a vector whose
 // entry k sits in lane k
 template <int N>

@@ -159,3 +159,43 @@ def test_lorenz96_fp32_combine_products_fenced(gpu):
     err = rel(means.cpu().numpy(), ref.mean)
     print(f"fp32 combine products: means vs the FP64 oracle {err:.2e}", flush=True)
     assert err < 1e-5
+
+
+@pytest.mark.parametrize("d,q", [(4, 1), (5, 2), (6, 2), (6, 4), (8, 3), (16, 2), (16, 3), (16, 4), (32, 2), (32, 3)])
+def test_lorenz96_shapes_match_oracle(gpu, d, q):
+    """The factorisations' shapes: strips of 16 rows whole and in part (D = 8, 15, 18, 30, 32, 48, 64, 80, 96, 128), rows and
+    block boundaries off the 16-byte grid (D = 15, 18, 30), every number of column tiles that the kernels are compiled for,
+    one strip per matrix and several pairs; one step, odd and even levels.  Tolerances as above."""
+    import torch
+
+    import pof.solver
+    from oracle import solver as osolver
+
+    ivp, oivp = _pair("lorenz96", d=d)
+    for N in (2, 3, 4, 8):
+        ts = np.linspace(0.0, (N - 1) * 5.0 / 8192, N)
+        print(f"lorenz96 shapes d={d} q={q} N={N}", flush=True)
+        ys, info = pof.solver.solve(f=ivp.f, y0=ivp.y0, ts=ts, order=q, init="constant", fixed_iters=2, engine="large")
+        torch.cuda.synchronize()
+        ref, rinfo = osolver.solve(oivp, ts, q, init="constant", fixed_iters=2)
+        assert rel(ys.mean.cpu().numpy(), ref.mean) < 1e-8
+        s_gpu, s_ref = info["sigma_squared"], rinfo["sigma_squared"]
+        assert rel(cov(ys.chol.cpu().numpy()) / s_gpu**2, cov(ref.chol) / s_ref**2) < 1e-6
+        assert abs(info["obj"] - rinfo["obj"]) <= 1e-6 * abs(rinfo["obj"]) + 1e-12
+
+
+def test_more_matrices_than_are_factored_at_a_time(gpu):
+    """4,499 steps: levels of more than twice 2,048 matrices, in part, against the per-worker engine."""
+    import torch
+
+    import pof.solver
+
+    ivp, oivp = _pair("rigid_body")
+    ts = np.linspace(oivp.t0, oivp.tmax, 4500)
+    kw = dict(f=ivp.f, y0=ivp.y0, ts=ts, order=2, init="constant", fixed_iters=3)
+    ys, info = pof.solver.solve(engine="large", **kw)
+    yr, rinfo = pof.solver.solve(**kw)
+    torch.cuda.synchronize()
+    assert rel(ys.mean.cpu().numpy(), yr.mean.cpu().numpy()) < 1e-9
+    s1, s2 = info["sigma_squared"], rinfo["sigma_squared"]
+    assert rel(cov(ys.chol.cpu().numpy()) / s1**2, cov(yr.chol.cpu().numpy()) / s2**2) < 1e-6
