@@ -564,11 +564,9 @@ constexpr int kTrsmBS = 16 * 17;  // one padded 16 x 16 block
 __host__ __device__ constexpr int trsm_tri(int K, int J) { return K * (K + 1) / 2 + J; }
 // Four waves per SIMD (128 VGPRs): two blocks per CU, 2 x 78 KiB of LDS.
 template <bool TRANS>
-__global__ __launch_bounds__(64 * kTrsmWaves) __attribute__((amdgpu_waves_per_eu(4))) void k_trsm(
-    const double* L, long long sL, int ldL, double* B, long long sB, int ldB, int n, int m, const double* R,
-    long long sR, int ldR, int RT) {
+__device__ __forceinline__ void trsm_block(double* Lt, const double* L, long long sL, int ldL, double* B, long long sB,
+                                           int ldB, int n, int m, const double* R, long long sR, int ldR, int RT) {
   constexpr int NB = kTrsmNB;
-  __shared__ double Lt[trsm_tri(NB, 0) * kTrsmBS];
   const double* l = L + (long long)blockIdx.x * sL;
   double* b = B + (long long)blockIdx.x * sB;
   const double* rb = R + (long long)blockIdx.x * sR;
@@ -658,6 +656,24 @@ __global__ __launch_bounds__(64 * kTrsmWaves) __attribute__((amdgpu_waves_per_eu
       if (r < n && cok) b[(size_t)r * ldB + c] = x[v];
     }
   }
+}
+
+template <bool TRANS>
+__global__ __launch_bounds__(64 * kTrsmWaves) __attribute__((amdgpu_waves_per_eu(4))) void k_trsm(
+    const double* L, long long sL, int ldL, double* B, long long sB, int ldB, int n, int m, const double* R,
+    long long sR, int ldR, int RT) {
+  __shared__ double Lt[trsm_tri(kTrsmNB, 0) * kTrsmBS];
+  trsm_block<TRANS>(Lt, L, sL, ldL, B, sB, ldB, n, m, R, sR, ldR, RT);
+}
+// Two solves with one matrix: L X = R^T (blocks with y = 0) and L^T X_ = R_^T (y = 1)
+__global__ __launch_bounds__(64 * kTrsmWaves) __attribute__((amdgpu_waves_per_eu(4))) void k_trsm_pair(
+    const double* L, long long sL, int ldL, double* B, long long sB, int ldB, const double* R, long long sR, int ldR,
+    double* B_, long long sB_, int ldB_, const double* R_, long long sR_, int ldR_, int n) {
+  __shared__ double Lt[trsm_tri(kTrsmNB, 0) * kTrsmBS];
+  if (blockIdx.y == 0)
+    trsm_block<false>(Lt, L, sL, ldL, B, sB, ldB, n, n, R, sR, ldR, 1);
+  else
+    trsm_block<true>(Lt, L, sL, ldL, B_, sB_, ldB_, n, n, R_, sR_, ldR_, 1);
 }
 
 // dst item b (rows x cols) = alpha * src item b' (r, c), or src (c, r) when trans;
@@ -875,10 +891,14 @@ __global__ void k_project(const double* m, const double* L, const double* P, int
 }
 
 // ------------------------------------------------------------------ GEMM
-// C = alpha op(A) op(B) + beta C for item blockIdx.x of a strided batch
-// (row-major, op = transpose when tA / tB; a stride of 0 shares a matrix over
-// the batch; beta = 0 does not read C).  A workgroup of four waves computes a
-// BM x BN tile of C (blockIdx.y, blockIdx.z); the waves form a WM x WN grid,
+// C = alpha op(A) op(B) + beta C for the items of a strided batch (row-major,
+// op = transpose when tA / tB; a stride of 0 shares a matrix over the batch;
+// beta = 0 does not read C), up to kGemmOps independent products of one shape in
+// a launch: a launch of one took 5.1 us at D = 24 whatever it multiplied.
+// Work-groups go round the 8 XCDs in turn: an item's tiles and products are
+// numbered 8 apart, so that they run together on one XCD and share their operands in
+// its L2.  A workgroup of four waves computes a
+// BM x BN tile of C; the waves form a WM x WN grid,
 // each computing (BM / WM) x (BN / WN) as 16 x 16 tiles on the matrix cores.
 // K advances in chunks of 16 staged through LDS (zero-padded at the edges),
 // loaded along whichever index is contiguous in memory; the next chunk is
@@ -896,10 +916,20 @@ typedef float gemm_f4 __attribute__((ext_vector_type(4)));
 
 constexpr int kGemmKc = 16;
 
+struct GemmOp {
+  int tA, tB, lda, ldb, ldc;
+  double alpha, beta;
+  const double *A, *B;
+  double* C;
+  long long sA, sB, sC;
+};
+constexpr int kGemmOps = 3;
+struct GemmOps {
+  GemmOp op[kGemmOps];
+};
+
 template <bool F32, int BM, int BN, int WM, int WN>
-__global__ __launch_bounds__(256, 3) void k_gemm(int tA, int tB, int M, int N, int K, double alpha, const double* A,
-                                              long long sA, int lda, const double* B, long long sB, int ldb,
-                                              double beta, double* C, long long sC, int ldc) {
+__global__ __launch_bounds__(256, 3) void k_gemm(GemmOps ops, int nops, int M, int N, int K, int mb, int nb, int cnt) {
   static_assert(WM * WN == 4, "four waves");
   using T = typename std::conditional<F32, float, double>::type;
   using V4 = typename std::conditional<F32, gemm_f4, gemm_d4>::type;
@@ -908,11 +938,21 @@ __global__ __launch_bounds__(256, 3) void k_gemm(int tA, int tB, int M, int N, i
   static_assert(LA >= 1 && LB >= 1 && TM >= 1 && TN >= 1, "tile shape");
   __shared__ T As[BM][kGemmKc + 1];
   __shared__ T Bs[kGemmKc][BN + 1];
-  const long long z = blockIdx.x;
-  const double* Az = A + z * sA;
-  const double* Bz = B + z * sB;
-  double* Cz = C + z * sC;
-  const int m0 = blockIdx.y * BM, n0 = blockIdx.z * BN;
+  const int r8 = blockIdx.x / 8, per = nops * mb * nb, sub = r8 % per;
+  const long long z = (long long)(r8 / per) * 8 + blockIdx.x % 8;
+  if (z >= cnt) return;  // uniform over the block
+  const int oi = sub / (mb * nb), blk = sub % (mb * nb);
+  // the product by compile-time indices (uniform selects; no dynamic index into the arguments)
+  GemmOp op = ops.op[0];
+#pragma unroll
+  for (int q = 1; q < kGemmOps; ++q)
+    if (oi == q) op = ops.op[q];
+  const int tA = op.tA, tB = op.tB, lda = op.lda, ldb = op.ldb, ldc = op.ldc;
+  const double alpha = op.alpha, beta = op.beta;
+  const double* Az = op.A + z * op.sA;
+  const double* Bz = op.B + z * op.sB;
+  double* Cz = op.C + z * op.sC;
+  const int m0 = (blk / nb) * BM, n0 = (blk % nb) * BN;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int wr = wave / WN, wc = wave % WN;
   // element e (0 .. BM * 16 - 1) of the A chunk -> (i, k): along i when A is stored K x M (tA)
@@ -1035,7 +1075,8 @@ constexpr int kGemvRowWaves = 4;
 __global__ __launch_bounds__(64 * kGemvRowWaves) void k_gemv_rows(int tB, int M, int K, double alpha, const double* A,
                                                                   long long sA, int lda, const double* B,
                                                                   long long sB, int ldb, double beta, double* C,
-                                                                  long long sC, int ldc) {
+                                                                  long long sC, int ldc, const double* C0,
+                                                                  long long sC0, int ldc0) {
   const int lane = threadIdx.x & 63;
   const int i = blockIdx.y * kGemvRowWaves + (threadIdx.x >> 6);
   if (i >= M) return;  // uniform per wave; no barrier follows
@@ -1046,9 +1087,8 @@ __global__ __launch_bounds__(64 * kGemvRowWaves) void k_gemv_rows(int tB, int M,
   for (int k = lane; k < K; k += 64) acc = fma(ar[k], tB ? Bz[k] : Bz[(size_t)k * ldb], acc);
   acc = wave_sum(acc);
   if (lane == 0) {
-    double* c = C + z * sC + (size_t)i * ldc;
     const double prod = alpha * acc;
-    *c = (beta == 0.0) ? prod : fma(beta, *c, prod);
+    C[z * sC + (size_t)i * ldc] = (beta == 0.0) ? prod : fma(beta, C0[z * sC0 + (size_t)i * ldc0], prod);
   }
 }
 
@@ -1110,10 +1150,15 @@ __device__ __forceinline__ void chain_mv(const double* M, int ld, int trans, con
   }
   __syncthreads();
 }
-__global__ __launch_bounds__(256) void k_vec_chain(ChainArgs a) {
+struct ChainPair {
+  ChainArgs c[2];
+};
+__global__ __launch_bounds__(256) void k_vec_chain(ChainPair p) {
   __shared__ double v0[kChainMaxD], v1[kChainMaxD], v2[kChainMaxD], v3[kChainMaxD];
   __shared__ double red[256];
   const long long it = blockIdx.x;
+  ChainArgs a = p.c[0];
+  if (blockIdx.y == 1) a = p.c[1];
   const int tid = threadIdx.x, D = a.D;
   const double* M[5];
 #pragma unroll
@@ -1164,13 +1209,8 @@ struct Ops {
     gemm_impl(false, tA, tB, M, N, K, alpha, A, B, beta, C, cnt);
   }
   // out = z + op5(M5) (t2 - op4(M4) op3(M3) t2), t2 = y + s2 op2(M2) op1(M1) x, per item (k_vec_chain)
-  void vec_chain(int D, V m1, bool t1, V m2, bool t2, V m3, bool t3, V m4, bool t4, V m5, bool t5, V x, V y,
-                 double s2, V z, V out, int cnt) {
-    if (err || cnt <= 0) return;
-    if (D > kChainMaxD) {
-      fail("vector chain: D beyond 128", -1);
-      return;
-    }
+  static ChainArgs chain(int D, V m1, bool t1, V m2, bool t2, V m3, bool t3, V m4, bool t4, V m5, bool t5, V x, V y,
+                         double s2, V z, V out) {
     ChainArgs a{};
     const V mm[5] = {m1, m2, m3, m4, m5};
     const bool tt[5] = {t1, t2, t3, t4, t5};
@@ -1190,8 +1230,40 @@ struct Ops {
     a.out = out.p;
     a.outs = out.s;
     a.D = D;
-    hipLaunchKernelGGL(k_vec_chain, dim3(cnt), dim3(256), 0, st, a);
+    return a;
+  }
+  // two independent chains in a launch
+  void vec_chains(const ChainArgs& a, const ChainArgs& b, int cnt) {
+    if (err || cnt <= 0) return;
+    if (a.D > kChainMaxD) {
+      fail("vector chain: D beyond 128", -1);
+      return;
+    }
+    hipLaunchKernelGGL(k_vec_chain, dim3(cnt, 2), dim3(256), 0, st, ChainPair{{a, b}});
     check("k_vec_chain");
+  }
+  // y = C0 + A b (D x D, N = 1)
+  void gemv_add(int D, V A, V b, V C0, V C, int cnt) {
+    if (err || cnt <= 0) return;
+    hipLaunchKernelGGL(k_gemv_rows, dim3(cnt, (D + kGemvRowWaves - 1) / kGemvRowWaves), dim3(64 * kGemvRowWaves), 0, st, 0,
+                       D, D, 1.0, A.p, A.s, A.ld, b.p, b.s, b.ld, 1.0, C.p, C.s, C.ld, C0.p, C0.s, C0.ld);
+    check("k_gemv");
+  }
+  struct Product {
+    bool tA, tB;
+    double alpha;
+    V A, B;
+    double beta;
+    V C;
+  };
+  // up to kGemmOps independent products of one shape in a launch (precision as gemm())
+  void gemms(int M, int N, int K, std::initializer_list<Product> ps, int cnt) {
+    if (err || cnt <= 0 || M <= 0 || N <= 0) return;
+    if (ps.size() > (size_t)kGemmOps) {
+      fail("gemms: too many products", -1);
+      return;
+    }
+    gemm_ops(f32 && M > 1 && N > 1 && K > 1, M, N, K, ps, cnt);
   }
   void gemm_impl(bool use32, bool tA, bool tB, int M, int N, int K, double alpha, V A, V B, double beta, V C,
                  int cnt) {
@@ -1202,33 +1274,39 @@ struct Ops {
                            A.s, A.ld, B.p, B.s, B.ld, beta, C.p, C.s, C.ld);
       } else {
         hipLaunchKernelGGL(k_gemv_rows, dim3(cnt, (M + kGemvRowWaves - 1) / kGemvRowWaves), dim3(64 * kGemvRowWaves),
-                           0, st, tB ? 1 : 0, M, K, alpha, A.p, A.s, A.ld, B.p, B.s, B.ld, beta, C.p, C.s, C.ld);
+                           0, st, tB ? 1 : 0, M, K, alpha, A.p, A.s, A.ld, B.p, B.s, B.ld, beta, C.p, C.s, C.ld, C.p,
+                           C.s, C.ld);
       }
       check("k_gemv");
       return;
     }
+    gemm_ops(use32, M, N, K, {Product{tA, tB, alpha, A, B, beta, C}}, cnt);
+  }
+  void gemm_ops(bool use32, int M, int N, int K, std::initializer_list<Product> ps, int cnt) {
+    GemmOps o{};
+    int n = 0;
+    for (const Product& p : ps)
+      o.op[n++] = GemmOp{p.tA ? 1 : 0, p.tB ? 1 : 0, p.A.ld, p.B.ld, p.C.ld, p.alpha, p.beta,
+                         p.A.p,        p.B.p,        p.C.p,  p.A.s,  p.B.s,  p.C.s};
     // tile shape by the product's shape: 128 x 16 for the skinny panel products (N <= 16),
     // 128 x 64 for the large ones, 64 x 64 otherwise
     if (N <= 16) {
-      launch_gemm<128, 16, 4, 1>(use32, tA, tB, M, N, K, alpha, A, B, beta, C, cnt);
+      launch_gemm<128, 16, 4, 1>(use32, o, n, M, N, K, cnt);
     } else if (M >= 128 && N >= 64) {
-      launch_gemm<128, 64, 2, 2>(use32, tA, tB, M, N, K, alpha, A, B, beta, C, cnt);
+      launch_gemm<128, 64, 2, 2>(use32, o, n, M, N, K, cnt);
     } else {
-      launch_gemm<64, 64, 2, 2>(use32, tA, tB, M, N, K, alpha, A, B, beta, C, cnt);
+      launch_gemm<64, 64, 2, 2>(use32, o, n, M, N, K, cnt);
     }
     check("k_gemm");
   }
   template <int BM, int BN, int WM, int WN>
-  void launch_gemm(bool use32, bool tA, bool tB, int M, int N, int K, double alpha, V A, V B, double beta, V C,
-                   int cnt) {
-    const dim3 grid(cnt, (M + BM - 1) / BM, (N + BN - 1) / BN);
-    if (use32) {
-      hipLaunchKernelGGL((k_gemm<true, BM, BN, WM, WN>), grid, dim3(256), 0, st, tA ? 1 : 0, tB ? 1 : 0, M, N, K,
-                         alpha, A.p, A.s, A.ld, B.p, B.s, B.ld, beta, C.p, C.s, C.ld);
-    } else {
-      hipLaunchKernelGGL((k_gemm<false, BM, BN, WM, WN>), grid, dim3(256), 0, st, tA ? 1 : 0, tB ? 1 : 0, M, N, K,
-                         alpha, A.p, A.s, A.ld, B.p, B.s, B.ld, beta, C.p, C.s, C.ld);
-    }
+  void launch_gemm(bool use32, const GemmOps& o, int n, int M, int N, int K, int cnt) {
+    const int mb = (M + BM - 1) / BM, nb = (N + BN - 1) / BN;
+    const dim3 grid((unsigned)((cnt + 7) / 8 * 8) * (unsigned)(n * mb * nb));
+    if (use32)
+      hipLaunchKernelGGL((k_gemm<true, BM, BN, WM, WN>), grid, dim3(256), 0, st, o, n, M, N, K, mb, nb, cnt);
+    else
+      hipLaunchKernelGGL((k_gemm<false, BM, BN, WM, WN>), grid, dim3(256), 0, st, o, n, M, N, K, mb, nb, cnt);
   }
   // tria in place of m x n matrices
   void lq(V A, int m, int n, int cnt) {
@@ -1369,6 +1447,17 @@ struct Ops {
                          rt ? 1 : 0);
     check("k_trsm");
   }
+  // L X = R^T and L^T X_ = R_^T, n right-hand sides each
+  void trsm_pair(int n, V L, V X, V R, V X_, V R_, int cnt) {
+    if (err || cnt <= 0) return;
+    if (n > kTrsmMaxN) {
+      fail("trsm: order beyond 128", -1);
+      return;
+    }
+    hipLaunchKernelGGL(k_trsm_pair, dim3(cnt, 2), dim3(64 * kTrsmWaves), 0, st, L.p, L.s, L.ld, X.p, X.s, X.ld, R.p, R.s,
+                       R.ld, X_.p, X_.s, X_.ld, R_.p, R_.s, R_.ld, n);
+    check("k_trsm_pair");
+  }
   void copy(V dst, V src, int rows, int cols, int cnt, bool trans = false, bool rev = false, double alpha = 1.0) {
     if (err || cnt <= 0) return;
     if (trans && rows > 1 && cols > 1) {
@@ -1506,22 +1595,23 @@ void filter_fn(Ops& o, Arena& ar, int D, const FE& e1, const FE& e2, const FE& o
     o.lq(q, 2 * D, 2 * D, cnt, D, 0);
   }
   const V Xi11 = X.at(0, 0), Xi21 = X.at(D, 0), Xi22 = X.at(D, D);
-  // m_ = Xi11^-1 U1^T -> T3; M^T = (m_ A2^T)^T = A2 m_^T, formed in place as the left
-  // block of [M^T | U2] (Y)
-  o.trsm(false, D, D, Xi11, T3, cnt, e1.U, true);
-  o.gemm(false, true, D, D, D, 1.0, e2.A, T3, 0.0, Y.at(0, 0), cnt);
-  // A = A2 A1 - M^T (Xi21^T A1)
-  o.gemm(true, false, D, D, D, 1.0, Xi21, e1.A, 0.0, T2, cnt);
-  o.gemm(false, false, D, D, D, 1.0, e2.A, e1.A, 0.0, out.A, cnt);
-  o.gemm(false, false, D, D, D, -1.0, Y.at(0, 0), T2, 1.0, out.A, cnt);
-  // b = A2 (v2 - m_^T Xi21^T v2) + b2, v2 = b1 + U1 (U1^T eta2)
-  o.vec_chain(D, e1.U, true, e1.U, false, Xi21, true, T3, true, e2.A, false, e2.eta, e1.b, 1.0, e2.b, out.b, cnt);
-  // _e = Xi11^-T Xi21^T -> T4; eta = A1^T (w2 - _e^T U1^T w2) + eta1, w2 = eta2 - Z2 (Z2^T b1)
-  o.trsm(true, D, D, Xi11, T4, cnt, Xi21, true);
-  o.vec_chain(D, e2.Z, true, e2.Z, false, e1.U, true, T4, true, e1.A, true, e1.b, e2.eta, -1.0, e1.eta, out.eta,
-              cnt);
-  // A1^T Xi22; then U = tria([M^T | U2]) and Z = tria([A1^T Xi22 | Z1]) in one call
-  o.gemm(true, false, D, D, D, 1.0, e1.A, Xi22, 0.0, YZ.at(0, 0), cnt);
+  // m_ = Xi11^-1 U1^T -> T3, _e = Xi11^-T Xi21^T -> T4
+  o.trsm_pair(D, Xi11, T3, e1.U, T4, Xi21, cnt);
+  // T2 = Xi21^T A1, A2 A1 and A1^T Xi22 (the left block of [A1^T Xi22 | Z1])
+  o.gemms(D, D, D,
+          {{true, false, 1.0, Xi21, e1.A, 0.0, T2},
+           {false, false, 1.0, e2.A, e1.A, 0.0, out.A},
+           {true, false, 1.0, e1.A, Xi22, 0.0, YZ}},
+          cnt);
+  // M^T = (m_ A2^T)^T = A2 m_^T, the left block of [M^T | U2]; A = A2 A1 - M^T (Xi21^T A1)
+  o.gemm(false, true, D, D, D, 1.0, e2.A, T3, 0.0, Y, cnt);
+  o.gemm(false, false, D, D, D, -1.0, Y, T2, 1.0, out.A, cnt);
+  // b = A2 (v2 - m_^T Xi21^T v2) + b2, v2 = b1 + U1 (U1^T eta2);
+  // eta = A1^T (w2 - _e^T U1^T w2) + eta1, w2 = eta2 - Z2 (Z2^T b1)
+  o.vec_chains(Ops::chain(D, e1.U, true, e1.U, false, Xi21, true, T3, true, e2.A, false, e2.eta, e1.b, 1.0, e2.b, out.b),
+               Ops::chain(D, e2.Z, true, e2.Z, false, e1.U, true, T4, true, e1.A, true, e1.b, e2.eta, -1.0, e1.eta, out.eta),
+               cnt);
+  // U = tria([M^T | U2]) and Z = tria([A1^T Xi22 | Z1]) in one call:
   // second blocks U2 (lower triangular) and Z1 (lower triangular, or [Zr | 0] at the leaves)
   {
     Ops::LqBlocks q{};
@@ -1544,9 +1634,8 @@ void smoother_fn(Ops& o, Arena& ar, int D, const SE& e1, const SE& e2, const SE&
   if (cnt <= 0 || o.err) return;
   CombineProducts prec(o);
   const size_t mark = ar.off;
-  o.copy(out.g, e2.g, D, 1, cnt);
-  o.gemm(false, false, D, 1, D, 1.0, e2.E, e1.g, 1.0, out.g, cnt);
-  o.gemm(false, false, D, D, D, 1.0, e2.E, e1.E, 0.0, out.E, cnt);
+  o.gemv_add(D, e2.E, e1.g, e2.g, out.g, cnt);
+  if (!with_chol) o.gemm(false, false, D, D, D, 1.0, e2.E, e1.E, 0.0, out.E, cnt);
   if (with_chol) {
     const long long DD = (long long)D * D;
     V Y{ar.take((size_t)cnt * DD), DD, D};
@@ -1554,7 +1643,7 @@ void smoother_fn(Ops& o, Arena& ar, int D, const SE& e1, const SE& e2, const SE&
       o.fail("workspace", -2);
       return;
     }
-    o.gemm(false, false, D, D, D, 1.0, e2.E, e1.Dm, 0.0, Y, cnt);
+    o.gemms(D, D, D, {{false, false, 1.0, e2.E, e1.E, 0.0, out.E}, {false, false, 1.0, e2.E, e1.Dm, 0.0, Y}}, cnt);
     Ops::LqBlocks q{};
     q.a = Y;
     q.rs = D;
