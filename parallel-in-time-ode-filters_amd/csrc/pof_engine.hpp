@@ -51,6 +51,9 @@ struct Tuning {
 // [b c, (b + 1) c) of each level, c = kStageWorkers >> (level - l0): in the up-sweep their inputs, in the
 // down-sweep their prefixes, are the block's own (but for one prefix, that of everything before the block).
 constexpr int kStageWorkers = 16;
+// Blocks of an up-sweep stage up to which two workers share a combine (k_filter_up16): one block per CU, whose eight
+// wavefronts are two per SIMD.
+constexpr int kTwoBlocks = 256;
 constexpr int kStageLevels = 5;  // kStageWorkers >> (kStageLevels - 1) = 1
 struct Stage {
   int l0 = 0, nlev = 0;

@@ -202,10 +202,16 @@ __global__ __launch_bounds__((Geo<D, kLdsState>::BLOCK)) void k_filter_down(Grou
 // and its first wavefronts start cold; at D = 3 a level's combine takes about as long.
 // DZ: columns of the elements' Z: d at level 0, which is a stage of its own (with a second combine for the
 // levels above, the kernel's registers would spill at D = 15 and 16), D above.
-__device__ __forceinline__ int stage_worker() { return ((threadIdx.x & 63) >> 4) * 4 + (threadIdx.x >> 6); }
+// TWO: two workers per combine, w of the first four wavefronts and w of the others, of an Xi that both factor: one forms U, b
+// and A, the other eta and Z.  The second is put two SIMDs on, where a level of one or two combines leaves nobody else
+// (beside the first one on its SIMD, both took longer than one worker for everything).
+__device__ __forceinline__ int stage_worker() {
+  return ((threadIdx.x & 63) >> 4) * 4 + ((threadIdx.x >> 6) + (threadIdx.x >> 8) * 2) % 4;
+}
 
-template <int D, int DZ>
-__global__ __launch_bounds__(r16::kStageBlock, 2) void k_filter_up16(GroupArgs g, LaunchMap lm, int l0, int nlev) {
+template <int D, int DZ, bool TWO>
+__global__ __launch_bounds__(r16::kStageBlock * (TWO ? 2 : 1), 2) void k_filter_up16(GroupArgs g, LaunchMap lm, int l0,
+                                                                                       int nlev) {
   if constexpr (DZ != D) l0 = 0, nlev = 1;
   Item it;
   if (!locate(lm, blockIdx.x, it)) return;
@@ -219,7 +225,15 @@ __global__ __launch_bounds__(r16::kStageBlock, 2) void k_filter_up16(GroupArgs g
     const long long i = (long long)b * c + w, next = off + (N >> (l0 + t));
     if (w < c && i < N >> (l0 + t + 1)) {
       const FiltArrays in = at(g.fel, off, D), out = at(g.fel, next, D);
-      r16::filter_combine<D, DZ, false>(r, in, none, 2 * (size_t)i, in, 2 * (size_t)i + 1, out, none, (size_t)i);
+      constexpr int kUA = r16::kPartU | r16::kPartA;
+      if (!TWO)
+        r16::filter_combine<D, DZ, false, kUA | r16::kPartZ>(r, in, none, 2 * (size_t)i, in, 2 * (size_t)i + 1, out, none,
+                                                             (size_t)i);
+      else if (threadIdx.x < r16::kStageBlock)
+        r16::filter_combine<D, DZ, false, kUA>(r, in, none, 2 * (size_t)i, in, 2 * (size_t)i + 1, out, none, (size_t)i);
+      else
+        r16::filter_combine<D, DZ, false, r16::kPartZ>(r, in, none, 2 * (size_t)i, in, 2 * (size_t)i + 1, out, none,
+                                                       (size_t)i);
     }
     off = next;
     if (t + 1 < nlev) __syncthreads();
@@ -262,7 +276,8 @@ __global__ __launch_bounds__(r16::kStageBlock, 2) void k_filter_down16(GroupArgs
         const StateArrays s = first ? at(g.fpre, base + lev_off(N, l0 + nlev), D) : up;
         const size_t is = (size_t)(first ? (long long)b * (kStageWorkers >> (nlev - 1)) - 1 : i - 1);
         FiltArrays none{};
-        r16::filter_combine<D, DZ, true>(r, none, s, is, el, 2 * (size_t)i, none, p, 2 * (size_t)i);
+        r16::filter_combine<D, DZ, true, r16::kPartU | r16::kPartA>(r, none, s, is, el, 2 * (size_t)i, none, p,
+                                                                    2 * (size_t)i);
       }
     }
     if (t > 0) __syncthreads();
@@ -1111,20 +1126,20 @@ struct Rec {
 }  // namespace
 
 // One launch per stage of a sweep
-#define POF_LAUNCH_STAGE(kernel, sg, ...) \
-  hipLaunchKernelGGL(kernel, dim3((sg).blocks), dim3(r16::kStageBlock), 0, __VA_ARGS__, (sg).l0, (sg).nlev)
+#define POF_LAUNCH_STAGE(kernel, sg, threads, ...) \
+  hipLaunchKernelGGL(kernel, dim3((sg).blocks), dim3(threads), 0, __VA_ARGS__, (sg).l0, (sg).nlev)
 
 template <int D>
 void smooth_scan(const GroupArgs& g, const LaunchPlan& p, hipStream_t st, Rec& rec) {
   if constexpr (D <= r16::kRow) {
     for (int k = 0; k < p.n_sup; ++k) {
       const Stage& s = p.sup[k];
-      POF_LAUNCH_STAGE(k_smooth_up16<D>, s, st, g, p.map(s.off, s.blocks));
+      POF_LAUNCH_STAGE(k_smooth_up16<D>, s, r16::kStageBlock, st, g, p.map(s.off, s.blocks));
       rec(kKSmoothUp, s.work);
     }
     for (int k = 0; k < p.n_sdn; ++k) {
       const Stage& s = p.sdn[k];
-      POF_LAUNCH_STAGE(k_smooth_down16<D>, s, st, g, p.map(s.off, s.blocks));
+      POF_LAUNCH_STAGE(k_smooth_down16<D>, s, r16::kStageBlock, st, g, p.map(s.off, s.blocks));
       rec(kKSmoothDown, s.work);
     }
   } else {
@@ -1143,23 +1158,38 @@ void smooth_scan(const GroupArgs& g, const LaunchPlan& p, hipStream_t st, Rec& r
   }
 }
 
+// A stage of the filter's up-sweep.  Two workers per combine where the launch leaves every CU to one block, D <= 8 (a launch of
+// five levels of 299 steps at D = 8: 25.3 -> 20.6 us; beyond, two paths through the combine's code cost what they
+// save: 46.8 and 44.7 us at D = 12, 1,000 steps, and more at 16,384; so does splitting the down-sweep's, where
+// the mean alone can be left to the other: 32.5 and 35 us).
+template <int D, int DZ>
+void filter_up_stage(const GroupArgs& g, const LaunchPlan& p, const Stage& s, hipStream_t st) {
+  if constexpr (D <= 8) {
+    if (s.blocks <= kTwoBlocks) {
+      POF_LAUNCH_STAGE((k_filter_up16<D, DZ, true>), s, 2 * r16::kStageBlock, st, g, p.map(s.off, s.blocks));
+      return;
+    }
+  }
+  POF_LAUNCH_STAGE((k_filter_up16<D, DZ, false>), s, r16::kStageBlock, st, g, p.map(s.off, s.blocks));
+}
+
 template <int D, int d>
 void filter_scan(const GroupArgs& g, const LaunchPlan& p, hipStream_t st, Rec& rec) {
   if constexpr (D <= r16::kRow) {
     for (int k = 0; k < p.n_fup; ++k) {
       const Stage& s = p.fup[k];
       if (s.l0 == 0)
-        POF_LAUNCH_STAGE((k_filter_up16<D, d>), s, st, g, p.map(s.off, s.blocks));
+        filter_up_stage<D, d>(g, p, s, st);
       else
-        POF_LAUNCH_STAGE((k_filter_up16<D, D>), s, st, g, p.map(s.off, s.blocks));
+        filter_up_stage<D, D>(g, p, s, st);
       rec(kKFilterUp, s.work);
     }
     for (int k = 0; k < p.n_fdn; ++k) {
       const Stage& s = p.fdn[k];
       if (s.l0 == 0)
-        POF_LAUNCH_STAGE((k_filter_down16<D, d>), s, st, g, p.map(s.off, s.blocks));
+        POF_LAUNCH_STAGE((k_filter_down16<D, d>), s, r16::kStageBlock, st, g, p.map(s.off, s.blocks));
       else
-        POF_LAUNCH_STAGE((k_filter_down16<D, D>), s, st, g, p.map(s.off, s.blocks));
+        POF_LAUNCH_STAGE((k_filter_down16<D, D>), s, r16::kStageBlock, st, g, p.map(s.off, s.blocks));
       rec(kKFilterDown, s.work);
     }
   } else {

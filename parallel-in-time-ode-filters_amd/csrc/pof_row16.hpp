@@ -449,12 +449,17 @@ __device__ __forceinline__ void store_lower16(double* p, double* x, int r) {
 // Xi = [[U1^T Z2, I], [Z2, 0]], rows 0 .. D - 1 (a) and D .. 2D - 1 (b) of a lane's two row sets.
 // Column i of the second block is still the identity's when pivot i comes: it adds 1 to the pivot
 // row's squared tail (so no tail vanishes) and its update is -tau w v_i without a product.
-template <int D, int DZ, bool SO>
+//
+// PARTS: the results that this worker forms: U, (b, A), (eta, Z).  A second worker can form the rest at the same time
+// from the same Xi, which both factor; the instructions of a result are the same either way.
+constexpr int kPartU = 1, kPartA = 2, kPartZ = 4;
+template <int D, int DZ, bool SO, int PARTS>
 __device__ __forceinline__ void filter_combine(int r, const FiltArrays& x1, const StateArrays& s1, size_t i1,
                                                const FiltArrays& x2, size_t i2, const FiltArrays& y,
                                                const StateArrays& so, size_t o) {
   constexpr size_t DD = (size_t)D * D;
   constexpr bool kLeaf = DZ < D;
+  constexpr bool pU = PARTS & kPartU, pA = PARTS & kPartA, pZ = !SO && (PARTS & kPartZ), pM = pU || pA;
   constexpr int kLow = kLeaf ? D : 1;  // Z2's row k holds columns < min(DZ, k + kLow)
   const bool act = r < D;
   const int rr = act ? r : 0;
@@ -481,11 +486,11 @@ __device__ __forceinline__ void filter_combine(int r, const FiltArrays& x1, cons
     }
   };
   auto load_rest1 = [&] {
-    load_row16<D>(u2, U2 + rr * D);
-    if constexpr (!SO) load_row16<D>(ar, A1 + rr * D);
+    if constexpr (pU) load_row16<D>(u2, U2 + rr * D);
+    if constexpr (pA && !SO) load_row16<D>(ar, A1 + rr * D);
   };
   auto load_rest2 = [&] {
-    if constexpr (!SO) {
+    if constexpr (pZ) {
       load_col16<D>(a1t, A1, rr);
       load_z(z1, Z1);
     }
@@ -494,7 +499,7 @@ __device__ __forceinline__ void filter_combine(int r, const FiltArrays& x1, cons
   const double eta2r = x2.eta[i2 * D + rr];
   load_col16<D>(u1t, U1, rr);
   load_z(z2, Z2);
-  if constexpr (!SO) {
+  if constexpr (pZ) {
     if constexpr (kLeaf) {
       const int rz = (r < DZ) ? r : 0;  // lanes past the last column hold no entry of Z2^T b1
 #pragma unroll
@@ -503,12 +508,12 @@ __device__ __forceinline__ void filter_combine(int r, const FiltArrays& x1, cons
       load_col16<D>(z2t, Z2, rr);
     }
   }
-  if constexpr (kTwo) {
+  if constexpr (kTwo && pM) {
     load_row16<D>(w, A2 + rr * D);
     load_row16<D>(u1, U1 + rr * D);
   }
-  const double b2r = x2.b[i2 * D + rr];
-  const double eta1r = SO ? 0.0 : x1.eta[i1 * D + rr];
+  const double b2r = pA ? x2.b[i2 * D + rr] : 0.0;
+  const double eta1r = pZ ? x1.eta[i1 * D + rr] : 0.0;
   if constexpr (kAll) {
     load_rest1();
     load_rest2();
@@ -516,13 +521,13 @@ __device__ __forceinline__ void filter_combine(int r, const FiltArrays& x1, cons
 
   double s2 = 0.0, uu = 0.0;
   double x11[D], x21[D], b[DZ + D], rd = 0.0;  // Xi11, Xi21; rd: 1 / Xi11[r][r] in lane r
-  if constexpr (!SO) {
+  if constexpr (pZ) {
     // s2 = eta2 - Z2 (Z2^T b1), uu = U1^T s2
     const double t = dot_lanes<D>(z2t, b1r);
     s2 = eta2r - dot_lanes<DZ>(z2, t);
     uu = dot_lanes<D>(u1t, s2);
   }
-  const double u = dot_lanes<D>(u1t, eta2r);
+  const double u = pA ? dot_lanes<D>(u1t, eta2r) : 0.0;
   {
     double a[DZ + D];
     zero(a);
@@ -563,29 +568,35 @@ __device__ __forceinline__ void filter_combine(int r, const FiltArrays& x1, cons
     });
   }
   double* x22 = b + DZ;
-  if constexpr (!kTwo) {
+  if constexpr (!kTwo && pM) {
     load_row16<D>(w, A2 + rr * D);
     load_row16<D>(u1, U1 + rr * D);
-  } else if constexpr (!kAll) {
+  } else if constexpr (kTwo && !kAll) {
     load_rest1();
   }
 
   // MT = A2 U1 Xi11^-T, W = A2 - MT Xi21^T, b = W (b1 + U1 u) + b2
-  double mt[2 * D];
-  zero(mt);
-  mul_rows<D, D, 1>(mt, w, u1);
-  const double sv = dot_lanes<D>(u1, u, b1r);
-  unroll<0, D>([&](auto jc) {
-    constexpr int j = decltype(jc)::value;
-    scale_fma_lanes<j + 1, D - 1 - j>(mt[j], bcast<j>(rd), mt + j + 1, x11[j]);
-  });
-  unroll<0, D>([&](auto jc) {
-    constexpr int j = decltype(jc)::value;
-    fma_lanes<0, D>(w, x21[j], -mt[j]);
-  });
-  const double bo = dot_lanes<D>(w, sv, b2r);
+  double mt[2 * D], bo = 0.0;
+  if constexpr (pM) {
+    zero(mt);
+    mul_rows<D, D, 1>(mt, w, u1);
+    double sv = 0.0;
+    if constexpr (pA) sv = dot_lanes<D>(u1, u, b1r);
+    unroll<0, D>([&](auto jc) {
+      constexpr int j = decltype(jc)::value;
+      scale_fma_lanes<j + 1, D - 1 - j>(mt[j], bcast<j>(rd), mt + j + 1, x11[j]);
+    });
+    if constexpr (pA) {
+      unroll<0, D>([&](auto jc) {
+        constexpr int j = decltype(jc)::value;
+        fma_lanes<0, D>(w, x21[j], -mt[j]);
+      });
+      bo = dot_lanes<D>(w, sv, b2r);
+    }
+  }
 
-  if constexpr (!SO) {
+  double s3 = 0.0;
+  if constexpr (pZ) {
     // eta = A1^T (s2 - Xi21 Xi11^-1 U1^T s2) + eta1
     double w2 = 0.0;
     {
@@ -597,16 +608,18 @@ __device__ __forceinline__ void filter_combine(int r, const FiltArrays& x1, cons
         x = fma(-x11[j], wj, x);
       });
     }
-    const double s3 = s2 - dot_lanes<D>(x21, w2);
-    if constexpr (kTwo && !kAll) load_rest2();
+    s3 = s2 - dot_lanes<D>(x21, w2);
+  }
+  if constexpr (kTwo && !kAll) load_rest2();
+  if constexpr (pA && !SO) {
     if constexpr (!kTwo) load_row16<D>(ar, A1 + rr * D);
     // A = W A1
-    {
-      double a[D];
-      zero(a);
-      mul_rows<D, D, D>(a, w, ar);
-      if (act) store_row16<D>(y.A + (o * D + r) * D, a);
-    }
+    double a[D];
+    zero(a);
+    mul_rows<D, D, D>(a, w, ar);
+    if (act) store_row16<D>(y.A + (o * D + r) * D, a);
+  }
+  if constexpr (pZ) {
     // Xi22 triangular, then Z = tria([A1^T Xi22 | Z1])
     lq1<D, D>(x22, r);
     if constexpr (!kTwo) load_rest2();
@@ -620,14 +633,16 @@ __device__ __forceinline__ void filter_combine(int r, const FiltArrays& x1, cons
     lq1<D, D + DZ, D, kLeaf ? DZ - 1 : 0>(z, r);
     if (act) store_lower16<D>(y.Z + (o * D + r) * D, z, r);
   }
+  if constexpr (pA) {
+    if (act) (SO ? so.m : y.b)[o * D + r] = bo;
+  }
   // U = tria([MT | U2])
-  if constexpr (!kTwo) load_row16<D>(u2, U2 + rr * D);
+  if constexpr (pU) {
+    if constexpr (!kTwo) load_row16<D>(u2, U2 + rr * D);
 #pragma unroll
-  for (int c = 0; c < D; ++c) mt[D + c] = u2[c];
-  lq1<D, 2 * D, D, 0>(mt, r);
-  if (act) {
-    (SO ? so.m : y.b)[o * D + r] = bo;
-    store_lower16<D>((SO ? so.L : y.U) + (o * D + r) * D, mt, r);
+    for (int c = 0; c < D; ++c) mt[D + c] = u2[c];
+    lq1<D, 2 * D, D, 0>(mt, r);
+    if (act) store_lower16<D>((SO ? so.L : y.U) + (o * D + r) * D, mt, r);
   }
 }
 

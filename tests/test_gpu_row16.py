@@ -104,3 +104,38 @@ def test_sequential_linear_model_against_oracle(gpu, d, q):
                gram(filt.chol.cpu().numpy()), np.array(nll), np.array(obj)]
         for a, b, t in zip(got, ref, tol):
             assert rel(a, b) <= t
+
+
+@pytest.mark.parametrize("d,q", [(1, 2), (2, 3)])
+def test_one_and_two_workers_per_combine(gpu, d, q):
+    """D <= 8: the up-sweep's widest launch with 256 blocks of 16 combines (two workers each) and with 257 (one each), against
+    the oracle's parallel filter.  Tolerances as above."""
+    import torch
+
+    import pof.parallel_filtsmooth as pfs
+    from oracle import model as om
+    from oracle import parallel as opar
+    from pof.observations import AffineModel
+    from pof.transitions import TransitionModel
+    from pof.utils import MVNSqrt
+
+    D = d * (q + 1)
+    F, QL = om.preconditioned_discretize(om.IWP(d, q))
+    for n in (8193, 8194):
+        rng = np.random.default_rng(3000 * D + n)
+        H, c = rng.standard_normal((n, d, D)), rng.standard_normal((n, d))
+        R = np.tril(rng.standard_normal((n, d, d))) * 0.3 + 0.5 * np.eye(d)
+        m0, L0 = rng.standard_normal(D), np.tril(rng.standard_normal((D, D)))
+        print(f"D={D} d={d} steps={n}", flush=True)
+        t = [torch.as_tensor(x, device="cuda") for x in (H, c, R)]
+        filt, _, _, _ = pfs.linear_noiseless_filtering(MVNSqrt(m0, L0), TransitionModel(F, QL), AffineModel(*t))
+        torch.cuda.synchronize()
+
+        def oracle(e=0.0):
+            fi, _, _, _ = opar.linear_noiseless_filtering(om.MVNSqrt(m0, L0 * (1 + e)), F, QL, om.AffineModel(H * (1 - e), c, R))
+            return [fi.mean, gram(fi.chol)]
+
+        ref = oracle()
+        tol = [max(1e-12, 20 * max(rel(a, b) for a in x)) for *x, b in zip(*(oracle(e) for e in (1e-15, -1e-15, 3e-15)), ref)]
+        for a, b, t in zip([filt.mean.cpu().numpy(), gram(filt.chol.cpu().numpy())], ref, tol):
+            assert rel(a, b) <= t
