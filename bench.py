@@ -40,7 +40,7 @@ METRIC = "ODE solves/s + p50/p99 latency, batched vs plain GPU scan at 1e-6 rel 
 NS = 65536
 Q = 3
 ITERS = 10
-TRAFFIC_SUMMARY = ROOT / "profiles" / "ieks_lorenz63_Ns65536_q3_f64_hbm_traffic.md"
+TRAFFIC_SUMMARY = ROOT / "profiles" / "ieks_lorenz63_Ns65536_q3_f64_row16_hbm_traffic.md"
 
 
 def gpu_run(steps, warmup):
@@ -110,7 +110,8 @@ def gpu_run(steps, warmup):
     # FETCH_SIZE / WRITE_SIZE summary of this workload (null if absent)
     from pof.profiling import read_traffic
 
-    traffic = read_traffic(str(TRAFFIC_SUMMARY), f"k_{dom}<{D}")
+    # (state dimensions up to 16: the kernels with one row per lane, one instantiation for the leaf level, one above)
+    traffic = read_traffic(str(TRAFFIC_SUMMARY), f"k_{dom}16<{D}" if D <= 16 else f"k_{dom}<{D}")
     iter_flops = roofline.iteration_flops(NS, D, d)
     iter_bytes = roofline.iteration_bytes(NS, D)
     t_it = float(np.median(step_s)) / ITERS
@@ -150,8 +151,7 @@ def gpu_run(steps, warmup):
             * work[roofline.KERNEL_CLASSES.index(dom)] / c["launches"],
             "traffic_source": TRAFFIC_SUMMARY.name if traffic is not None else None,
             "peak_note": "MI355X's FP64 peak (78.6 TFLOP/s) is the same on the matrix cores and the vector ALUs; "
-                         "the D = 12 combines form their tile products on the matrix cores and the Householder "
-                         "pivots on the vector ALUs",
+                         "the D = 12 combines run on the vector ALUs",
         },
         "instrumented_iteration_ms": total_ms / ITERS,
         "iteration_tflops_algorithmic": iter_flops / (total_ms / ITERS * 1e-3) / 1e12,
@@ -406,7 +406,7 @@ def batched_run(n_ivps, maxiters, plain_sample, seed=4, cpu=True):
     res = pof.batch.solve_batch(probs, maxiters=maxiters)
     torch.cuda.synchronize()
     t_batch = time.perf_counter() - t0
-    # the same batch with every scan level in the latency form (the kernels' forms before tuning)
+    # the same batch with the tuning off: every scan level shares launches
     from pof import autotune
 
     tuned = autotune.read_cache()
@@ -442,8 +442,8 @@ def batched_run(n_ivps, maxiters, plain_sample, seed=4, cpu=True):
         "solves_per_s": n_ivps / t_batch,
         "seconds": t_batch,
         "autotuned": {
-            "what": "scan kernel forms from the autotuner's cache (pof/tuning_gfx950.json) against every level in "
-                    "the latency form",
+            "what": "scan levels' launches by the autotuner's cache (pof/tuning_gfx950.json) against launches "
+                    "shared by all levels",
             "tuned_seconds": t_batch,
             "default_seconds": t_default,
             "speedup": (t_default / t_batch) if t_default else None,

@@ -278,16 +278,18 @@ def issue_markdown(busy_csv, insts_csv, command="", levels=()):
 
 
 def read_traffic(md_path, kernel):
-    """Bytes per launch of the first kernel whose name contains ``kernel``, or None."""
+    """Mean bytes per launch over the kernels whose names contain ``kernel``, or None."""
     try:
         text = open(md_path).read()
     except OSError:
         return None
+    n = total = 0.0
     for line in text.splitlines():
         m = re.match(r"\| `([^`]*)` \| (\d+) \| [\d.]+ \| [\d.]+ \| (\d+) \|", line)
         if m and kernel in m.group(1):
-            return float(m.group(3))
-    return None
+            n += float(m.group(2))
+            total += float(m.group(2)) * float(m.group(3))
+    return total / n if n else None
 
 
 def main(argv=None):
