@@ -11,9 +11,10 @@
 //
 // Against rows split over two lanes of a whole-wavefront worker, with each pivot row passed through
 // LDS and every lane repeating the pivot's scalar part: about 5,300 instructions per combine became
-// about 4,300 per four (5,100 with a wait in front of every group and groups of at most eight), and at D = 12 a level of 32,768 combines went from 364 to 107 us (up) and
-// from 205 to 70 us (down), the latency of one combine from 19 to 14 us and from 13 to 9.7 us.  What
-// bounds it is FP64 issue: two waves per SIMD (248 registers), 2.5 ns per instruction.
+// about 4,300 per four (5,100 with a wait in front of every group and groups of at most eight), and at
+// D = 12 a level of 32,768 combines went from 364 to 91 us (up) and from 205 to 61 us (down), the latency
+// of one combine from 19 to 13 us and from 13 to 9.5 us.  What bounds it is FP64 issue: two waves per SIMD
+// (221 registers), 2.5 ns per instruction.
 //
 // Lanes r >= D of a row repeat row 0; only lanes r < D are ever the source of a broadcast or store.
 // A whole row is active or not (a worker past the end returns as a whole), so a broadcast never
@@ -985,7 +986,9 @@ __device__ __forceinline__ void filter_post(int r, const GroupArgs& g, int j, lo
   const bool act = r < D;
   const int rr = act ? r : 0;
   O ob;
-  if (D <= 12 && obs) ob.load(g, j, base, s, r);  // (beyond, its values would spill through the factorisation)
+  // early, so that the reads are over when they are needed; beyond D = 8 its values cost more as registers held through the
+  // factorisation (D = 12, 65,536 points: 107 us early, 97 us late; at 1,000 points no difference)
+  if (D <= 8 && obs) ob.load(g, j, base, s, r);
   double x11[D], b[2 * D], fm, mr, rd = 0.0;
   {
     double a[2 * D], f[D], l0[D], lq[D];
@@ -1045,7 +1048,7 @@ __device__ __forceinline__ void filter_post(int r, const GroupArgs& g, int j, lo
     }
     return;
   }
-  if (D > 12) ob.load(g, j, base, s, r);
+  if (D > 8) ob.load(g, j, base, s, r);
   double sr[D + NR];
   {
     double h[D];
