@@ -890,6 +890,7 @@ struct CallBatch {
   int open(int D, int d, long long entries, bool affine) {
     {
       std::lock_guard<std::mutex> lk(ctx->kept_mu);
+      ctx->kept.reserve(kKeptBatches + 1);  // the destructor's push_back allocates nothing
       for (size_t i = ctx->kept.size(); i-- > 0;) {
         pof_batch* x = ctx->kept[i];
         if (x->D != D || x->d != d || x->affine != affine || x->entries < entries) continue;

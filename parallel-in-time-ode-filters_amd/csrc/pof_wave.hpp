@@ -117,13 +117,5 @@ __device__ __forceinline__ void sum_scatter(double (&x)[NV], int lane) {
   x[0] += dpp<kQuadSwap2>(x[0]);
 }
 
-// The value of v in lane L (a compile-time lane): two scalar reads.
-__device__ __forceinline__ double lane_value(double v, int L) {
-  const unsigned long long x = __builtin_bit_cast(unsigned long long, v);
-  const unsigned lo = (unsigned)__builtin_amdgcn_readlane((int)(unsigned)x, L);
-  const unsigned hi = (unsigned)__builtin_amdgcn_readlane((int)(unsigned)(x >> 32), L);
-  return from_bits(lo, hi);
-}
-
 }  // namespace wave
 }  // namespace pof
