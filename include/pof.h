@@ -266,8 +266,8 @@ int pof_smoothing(pof_ctx* ctx, int D, int64_t Ns, const double* F_host, const d
                   double* smooth_chol_dev, double* obj, void* stream);
 
 /* Square-root EKF of the problem's residual model, linearised at each predicted
- * mean, with the caller's prior x0 and constant transition (F, QL) (host), for
- * n_times - 1 steps.  Replaces pof.sequential_filtsmooth.extended_kalman_filter
+ * mean, with the caller's prior x0 and constant transition (F, QL) (host; x0_chol
+ * and QL: any square roots, triangular or not), for n_times - 1 steps.  Replaces pof.sequential_filtsmooth.extended_kalman_filter
  * (sequential_filtsmooth/filter.py:9-30): filtered states [Ns+1, ...] on the
  * device (may be NULL), nll = summed log-likelihood, ssq. */
 int pof_ekf(pof_ctx* ctx, const pof_problem* prob, const double* x0_mean_host, const double* x0_chol_host,

@@ -837,6 +837,7 @@ int batch_try(pof_ctx* ctx, int D, int d, long long entries, int slots, bool aff
   g.q = b->q;
   g.affine = affine ? 1 : 0;
   g.lq_lower = 0;
+  g.own_factors = 1;
   std::fill(b->arena_host, b->arena_host + arena_bytes, 0);  // (zero bits: 0.0, null)
   b->hcur.assign(S, 0);
   std::fill(b->hscale.begin(), b->hscale.end(), 1.0);
@@ -2133,6 +2134,9 @@ int pof_ekf(pof_ctx* ctx, const pof_problem* prob, const double* x0_mean_host, c
   const int D = s.D;
   const size_t DD = (size_t)D * D;
   set_transition(b, F_host, QL_host);
+  bool own = b->g.lq_lower && pof::strictly_upper_zero(x0_chol_host, D);
+  for (int i = 0; i < D; ++i) own = own && QL_host[(size_t)i * D + i] != 0.0;
+  b->g.own_factors = own ? 1 : 0;
   pof_opts o{};
   o.maxiters = 1;
   o.fixed_iters = 1;

@@ -1074,13 +1074,14 @@ __global__ __launch_bounds__((Geo<D, kLdsSeq>::BLOCK)) void k_seq_smooth(GroupAr
 }
 
 // k_seq_filter with one IVP per row, D <= 16
-template <int D, int d, bool EK1, bool AT_PRED>
+template <int D, int d, bool EK1, bool AT_PRED, bool LOW>
 __global__ __launch_bounds__(r16::kBlock, 1) void k_seq_filter16(GroupArgs g, LaunchMap lm) {
   __shared__ double sh[r16::kPerBlock][D + kMaxParams];
   Item it;
   const int w = threadIdx.x / r16::kRow;
   if (!locate(lm, blockIdx.x * r16::kPerBlock + w, it)) return;
-  r16::seq_filter<D, d, EK1, AT_PRED>(threadIdx.x % r16::kRow, g, it.j, it.base, it.Ns, at(g.fpre, it.base, D), sh[w]);
+  r16::seq_filter<D, d, EK1, AT_PRED, LOW>(threadIdx.x % r16::kRow, g, it.j, it.base, it.Ns, at(g.fpre, it.base, D),
+                                           sh[w]);
 }
 
 // k_seq_smooth over smoother elements, D <= 16
@@ -1276,12 +1277,12 @@ hipError_t run_iteration(const GroupArgs& g, const LaunchPlan& p, double* scal, 
   return iteration_tail<D>(g, p, scal, d, st, rec);
 }
 
-// The sequential filter of every active IVP
-template <int D, int d, bool EK1, bool AT_PRED>
+// The sequential filter of every active IVP (LOW: see r16::seq_filter)
+template <int D, int d, bool EK1, bool AT_PRED, bool LOW>
 void launch_seq_filter(const GroupArgs& g, const LaunchPlan& p, hipStream_t st) {
   const LaunchMap one = p.map(p.one_off, p.one_total);
   if constexpr (D <= r16::kRow)
-    POF_LAUNCH16((k_seq_filter16<D, d, EK1, AT_PRED>), p.one_total, st, g, one);
+    POF_LAUNCH16((k_seq_filter16<D, d, EK1, AT_PRED, LOW>), p.one_total, st, g, one);
   else
     POF_LAUNCH((k_seq_filter<D, d, EK1, AT_PRED>), kLdsSeq, p.one_total, st, g, one);
 }
@@ -1309,14 +1310,18 @@ template <int D, int d>
 hipError_t run_seq_iteration(const GroupArgs& g, const LaunchPlan& p, double* scal, int at_pred, hipStream_t st,
                              KernelTimer* t) {
   Rec rec(t, st);
+  // (a filter over a caller's factors is always one that linearises at the predicted means)
   if (g.affine)
-    launch_seq_filter<D, d, false, false>(g, p, st);
+    launch_seq_filter<D, d, false, false, false>(g, p, st);
+  else if (at_pred && !g.own_factors)
+    launch_seq_filter<D, d, true, true, false>(g, p, st);
   else if (at_pred)
-    launch_seq_filter<D, d, true, true>(g, p, st);
+    launch_seq_filter<D, d, true, true, true>(g, p, st);
   else
-    launch_seq_filter<D, d, true, false>(g, p, st);
+    launch_seq_filter<D, d, true, false, true>(g, p, st);
   rec(kKFilterLeaf, p.leaf_total);
-  if (g.affine)
+  // (the gains need no observation model: the affine form serves any factors)
+  if (g.affine || !g.own_factors)
     launch_seq_smooth<D, d, false>(g, p, kPostGain, st, rec);
   else
     launch_seq_smooth<D, d, true>(g, p, kPostGain, st, rec);
@@ -1344,7 +1349,7 @@ hipError_t run_smooth_only(const GroupArgs& g, const LaunchPlan& p, double* scal
 template <int D, int d>
 hipError_t run_seq_smooth_chol(const GroupArgs& g, const LaunchPlan& p, hipStream_t st, KernelTimer* t) {
   Rec rec(t, st);
-  if (g.affine)
+  if (g.affine || !g.own_factors)
     launch_seq_smooth<D, d, false>(g, p, kPostDm, st, rec);
   else
     launch_seq_smooth<D, d, true>(g, p, kPostDm, st, rec);

@@ -976,7 +976,7 @@ __device__ __forceinline__ void filter_element(int r, const GroupArgs& g, int j,
 // OBS, the predicted observation's statistics (filter.py:84-114): see k_filter_post.
 //   Phi = tria([[F L, LQ], [L, 0]]), E = Phi21 Phi11^-1, g = m - E F m, D = Phi22,
 //   S = tria([H Phi11 | R]), yhat = H F m + c.
-// LOWL: L and LQ are lower triangular with LQ's diagonal nonzero (the solver's own model).
+// EK1: L and LQ are lower triangular with LQ's diagonal nonzero (GroupArgs::own_factors).
 template <int D, int d, bool EK1>
 __device__ __forceinline__ void filter_post(int r, const GroupArgs& g, int j, long long base, int s, const double* mp,
                                             const double* Lp, bool obs, bool dm_only, bool wc, const SmoArrays& sel, size_t ro,
@@ -1094,7 +1094,8 @@ __device__ __forceinline__ void filter_post(int r, const GroupArgs& g, int j, lo
 // model's values are read a step ahead, and the step's logarithms wait for sixteen steps, a step per lane.
 // Against a whole wavefront per IVP with its tiles in LDS, filter and smoother of 513 points: 8.6 -> 2.1 ms at
 // D = 8, 16.1 -> 3.6 ms at D = 12, 22.4 -> 5.4 ms at D = 15 (17.4, 31 and 44 us per step before).
-template <int D, int d, bool EK1, bool AT_PRED>
+// LOW: LQ and the prior's factor are lower triangular (GroupArgs::own_factors): a caller's need not be.
+template <int D, int d, bool EK1, bool AT_PRED, bool LOW>
 __device__ __forceinline__ void seq_filter(int r, const GroupArgs& g, int j, long long base, int Ns,
                                            const StateArrays& fp, double* shared) {
   using O = ObsRow<D, d, EK1>;
@@ -1144,10 +1145,10 @@ __device__ __forceinline__ void seq_filter(int r, const GroupArgs& g, int j, lon
     {
       double a[2 * D];
       zero(a);
-      mul_rows<D, D, EK1 ? 1 : D>(a, f, l);  // an affine model's first factor is the caller's, not triangular
+      mul_rows<D, D, LOW ? 1 : D>(a, f, l);
 #pragma unroll
       for (int c = 0; c < D; ++c) a[D + c] = lq[c];
-      lq1<D, 2 * D, D, EK1 ? 0 : D>(a, r);
+      lq1<D, 2 * D, D, LOW ? 0 : D>(a, r);
 #pragma unroll
       for (int c = 0; c < D; ++c) n[c] = (c > r) ? 0.0 : a[c];
 #pragma unroll

@@ -100,6 +100,9 @@ struct GroupArgs {
   int q;
   int affine;
   int lq_lower;  // 1: LQ's strict upper part is zero (the smoother-element factorisation skips it)
+  // 1: LQ and every x0L are lower triangular and LQ's diagonal has no zero, as the solver's own model is.  0 for an
+  // extended filter over a caller's factors of any other form (any L with the right L L^T is one).
+  int own_factors;
 };
 
 // One active IVP of a launch: its slot, its steps and the first entry of its range.
