@@ -113,6 +113,14 @@ int pof_ctx_create(int device, pof_ctx** out);
 void pof_ctx_destroy(pof_ctx* ctx);
 const char* pof_last_error(const pof_ctx* ctx);
 
+/* Gives back the device memory that finished calls of pof_linear_filtsmooth,
+ * pof_smoothing and pof_ekf left for the next one (at most 1 GiB per device over
+ * all contexts; no reference counterpart).  The library does so by itself where
+ * one of its own allocations finds no room; a program that is about to
+ * allocate elsewhere, or reads the device's free memory, calls it first.
+ * Returns the bytes. */
+int64_t pof_trim(void);
+
 /* 1 if a kernel instantiation exists for state dimension D = d (q + 1) and ODE dimension d. */
 int pof_supported(int D, int d);
 

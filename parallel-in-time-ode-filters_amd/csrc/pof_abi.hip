@@ -14,6 +14,7 @@
 #include <cstdarg>
 #include <cstdio>
 #include <cstring>
+#include <list>
 #include <map>
 #include <mutex>
 #include <string>
@@ -395,9 +396,6 @@ struct pof_ctx {
   std::vector<pof_batch*> cache;
   // small batches for the coarse initial trajectory (EKS on 100 points), one per (D, d)
   std::vector<pof_batch*> aux;
-  // batches kept for the next call of pof_linear_filtsmooth / pof_smoothing / pof_ekf, the last used at the end
-  std::vector<pof_batch*> kept;
-  std::mutex kept_mu;
   // large-state engine (batched primitives), created on first use
   pof::large::Engine* large = nullptr;
   // replay unchanged iterations from a HIP graph (pof_graphs_enable)
@@ -441,6 +439,7 @@ struct pof_batch {
   };
 
   pof_ctx* ctx = nullptr;
+  int device = 0;  // ctx's
   int D = 0, d = 0, q = 0;
   bool affine = false;
   bool cached = false;
@@ -636,7 +635,7 @@ hipError_t stage_maps(pof_batch* b) {
     b->maps_host = nullptr;
     b->maps_cap = 0;
     const size_t cap = std::max<size_t>(n * 2, 4096);
-    e = hipMalloc((void**)&b->maps_dev, cap * sizeof(int));
+    e = device_malloc((void**)&b->maps_dev, cap * sizeof(int));
     if (e == hipSuccess)
       e = hipHostMalloc((void**)&b->maps_host, cap * sizeof(int), hipHostMallocMapped | hipHostMallocCoherent);
     if (e == hipSuccess) e = hipHostGetDevicePointer((void**)&b->maps_map, b->maps_host, 0);
@@ -680,7 +679,7 @@ bool isclose(double a, double b, double rtol, double atol) {
 // ------------------------------------------------------------ batch memory
 void batch_free(pof_batch* b) {
   if (!b) return;
-  (void)hipSetDevice(b->ctx->device);
+  (void)hipSetDevice(b->device);
   if (b->st) (void)hipStreamSynchronize(b->st);
   if (b->gexec) (void)hipGraphExecDestroy(b->gexec);
   for (void* p : b->allocs) (void)hipFree(p);
@@ -698,7 +697,7 @@ void batch_free(pof_batch* b) {
 template <class T>
 hipError_t dalloc(pof_batch* b, size_t n, T** out) {
   void* p = nullptr;
-  hipError_t e = hipMalloc(&p, std::max<size_t>(n * sizeof(T), 256));
+  hipError_t e = device_malloc(&p, std::max<size_t>(n * sizeof(T), 256));
   if (e != hipSuccess) return e;
   b->allocs.push_back(p);
   *out = static_cast<T*>(p);
@@ -716,13 +715,99 @@ size_t batch_bytes(int D, long long entries, int slots) {
   return per_entry * (size_t)entries + per_slot * (size_t)slots + 8 * 4 * ((size_t)entries / kChunk + slots + 1);
 }
 
-void drop_kept(pof_ctx* ctx) {
-  std::lock_guard<std::mutex> lk(ctx->kept_mu);
-  for (pof_batch* b : ctx->kept) batch_free(b);
-  ctx->kept.clear();
+// The workspaces that finished calls left for the next (see CallBatch), the last used at the end.  One list for the
+// process: contexts belong to threads, and what they keep on a device has one bound; a call takes only its own
+// context's.  They are given back where an allocation of the library finds no room on their device (device_malloc),
+// with their context, and by pof_trim.  Never destroyed: contexts may live as long as the process.
+constexpr size_t kKeptBatches = 4;
+constexpr size_t kKeptBytes = size_t(1) << 30;
+using Kept = std::list<pof_batch*>;  // (moved between lists by splice: the end of a call allocates nothing)
+struct KeptList {
+  std::mutex mu;
+  Kept list;
+};
+KeptList& kept_list() {
+  static KeptList* const k = new KeptList;
+  return *k;
 }
 
-int batch_try(pof_ctx* ctx, int D, int d, long long entries, int slots, bool affine, pof_batch** out) {
+size_t kept_bytes(const pof_batch* b) { return batch_bytes(b->D, b->entries, b->slots); }
+
+// Frees the workspaces of a list; returns their bytes.
+size_t kept_free(const Kept& out) {
+  if (out.empty()) return 0;
+  int device = 0;
+  const bool back = hipGetDevice(&device) == hipSuccess;
+  size_t bytes = 0;
+  for (pof_batch* b : out) {
+    bytes += kept_bytes(b);
+    batch_free(b);
+  }
+  if (back) (void)hipSetDevice(device);
+  return bytes;
+}
+
+// Frees the kept workspaces that `which` picks; returns their bytes.
+template <class F>
+size_t kept_drop(F which) {
+  KeptList& k = kept_list();
+  Kept out;
+  {
+    std::lock_guard<std::mutex> lk(k.mu);
+    for (auto it = k.list.begin(); it != k.list.end();) {
+      const auto next = std::next(it);
+      if (which(*it)) out.splice(out.end(), k.list, it);
+      it = next;
+    }
+  }
+  return kept_free(out);
+}
+
+// A kept workspace of ctx that serves a call over `entries` entries, the last used one, or an empty list
+Kept kept_take(const pof_ctx* ctx, int D, int d, long long entries, bool affine) {
+  KeptList& k = kept_list();
+  Kept one;
+  std::lock_guard<std::mutex> lk(k.mu);
+  for (auto it = k.list.end(); it != k.list.begin();) {
+    --it;
+    const pof_batch* x = *it;
+    if (x->ctx != ctx || x->D != D || x->d != d || x->affine != affine || x->entries < entries) continue;
+    one.splice(one.end(), k.list, it);
+    break;
+  }
+  return one;
+}
+
+// Keeps the workspace in `one`, and frees the longest unused ones beyond the bounds (it, if it is beyond them alone)
+void kept_put(Kept& one) {
+  const pof_batch* b = one.front();
+  KeptList& k = kept_list();
+  Kept out;
+  {
+    std::lock_guard<std::mutex> lk(k.mu);
+    k.list.splice(k.list.end(), one);
+    size_t total = 0, own = 0;
+    for (const pof_batch* x : k.list) {
+      if (x->device != b->device) continue;
+      total += kept_bytes(x);
+      own += (x->ctx == b->ctx) ? 1 : 0;
+    }
+    for (auto it = k.list.begin(); it != k.list.end();) {
+      const auto next = std::next(it);
+      const pof_batch* x = *it;
+      const bool mine = x->ctx == b->ctx;
+      if (x->device == b->device && (total > kKeptBytes || (mine && own > kKeptBatches))) {
+        total -= kept_bytes(x);
+        own -= mine ? 1 : 0;
+        out.splice(out.end(), k.list, it);
+      }
+      it = next;
+    }
+  }
+  kept_free(out);
+}
+
+int batch_new(pof_ctx* ctx, int D, int d, long long entries, int slots, bool affine, pof_batch** out) {
   *out = nullptr;
   const EngineFns* e = engine_or_err(ctx, D, d);
   if (!e) return POF_E_UNSUPPORTED;
@@ -731,10 +816,13 @@ int batch_try(pof_ctx* ctx, int D, int d, long long entries, int slots, bool aff
   size_t free_b = 0, total_b = 0;
   HIP_TRY(hipMemGetInfo(&free_b, &total_b));
   const size_t need = batch_bytes(D, entries, slots);
+  if (need > free_b && kept_drop([&](const pof_batch* x) { return x->device == ctx->device; }) > 0)
+    HIP_TRY(hipMemGetInfo(&free_b, &total_b));
   if (need > free_b)
     return set_err(ctx, POF_E_HIP, "batch needs %zu bytes of device memory, %zu free", need, free_b);
   pof_batch* b = new pof_batch();
   b->ctx = ctx;
+  b->device = ctx->device;
   b->D = D;
   b->d = d;
   b->q = D / d - 1;
@@ -863,65 +951,36 @@ int batch_try(pof_ctx* ctx, int D, int d, long long entries, int slots, bool aff
   return POF_OK;
 }
 
-int batch_new(pof_ctx* ctx, int D, int d, long long entries, int slots, bool affine, pof_batch** out) {
-  int rc = batch_try(ctx, D, d, entries, slots, affine, out);
-  if (rc != POF_E_HIP) return rc;
-  {
-    std::lock_guard<std::mutex> lk(ctx->kept_mu);
-    if (ctx->kept.empty()) return rc;
-  }
-  // out of memory with workspaces kept: without them
-  (void)hipGetLastError();
-  drop_kept(ctx);
-  return batch_try(ctx, D, d, entries, slots, affine, out);
-}
-
 // The workspace of one call of pof_linear_filtsmooth, pof_smoothing or pof_ekf.  Its 26 allocations and their
 // releases cost 3.1 of the 3.9 ms of a call over 16,384 steps at D = 12, so a finished call's is kept for the next
-// one of its (D, d) that fits, at most kKeptBatches of them and kKeptBytes together per context (and none where
-// another allocation of the library needs the memory).  A call takes it out of the list, so that calls
-// from several threads have one each; it is put back only idle: its work done, its slots free.
-constexpr size_t kKeptBatches = 4;
-constexpr size_t kKeptBytes = size_t(1) << 30;
+// one of its context and (D, d) that fits: at most kKeptBatches of a context, and of all contexts on a device
+// kKeptBytes together (see KeptList).  A call takes it out of the list, so that calls from several threads
+// have one each; it is put back only idle: its work done, its slots free.
 struct CallBatch {
   pof_ctx* ctx;
   pof_batch* b = nullptr;
+  Kept own;           // holds b
   bool done = false;  // the call ended well
   explicit CallBatch(pof_ctx* c) : ctx(c) {}
   int open(int D, int d, long long entries, bool affine) {
-    {
-      std::lock_guard<std::mutex> lk(ctx->kept_mu);
-      ctx->kept.reserve(kKeptBatches + 1);  // the destructor's push_back allocates nothing
-      for (size_t i = ctx->kept.size(); i-- > 0;) {
-        pof_batch* x = ctx->kept[i];
-        if (x->D != D || x->d != d || x->affine != affine || x->entries < entries) continue;
-        b = x;
-        ctx->kept.erase(ctx->kept.begin() + i);
-        break;
-      }
+    own = kept_take(ctx, D, d, entries, affine);
+    if (!own.empty()) {
+      b = own.front();
+      HIP_TRY(hipSetDevice(ctx->device));
+      return POF_OK;
     }
-    if (!b) return batch_new(ctx, D, d, entries, 1, affine, &b);
-    HIP_TRY(hipSetDevice(ctx->device));
-    return POF_OK;
+    own.push_back(nullptr);
+    const int rc = batch_new(ctx, D, d, entries, 1, affine, &b);
+    own.front() = b;
+    return rc;
   }
   ~CallBatch() {
     if (!b) return;
-    const size_t bytes = batch_bytes(b->D, b->entries, b->slots);
-    if (!done || bytes > kKeptBytes) {
-      batch_free(b);
-      return;
-    }
     b->g.Hx = b->g.cx = b->g.Rx = nullptr;
-    std::lock_guard<std::mutex> lk(ctx->kept_mu);
-    ctx->kept.push_back(b);
-    size_t total = 0;
-    for (pof_batch* x : ctx->kept) total += batch_bytes(x->D, x->entries, x->slots);
-    while (ctx->kept.size() > kKeptBatches || total > kKeptBytes) {
-      pof_batch* x = ctx->kept.front();
-      total -= batch_bytes(x->D, x->entries, x->slots);
-      ctx->kept.erase(ctx->kept.begin());
-      batch_free(x);
-    }
+    if (done)
+      kept_put(own);
+    else
+      batch_free(b);
   }
 };
 
@@ -1595,7 +1654,7 @@ int coarse_means(pof_ctx* ctx, const pof_problem* prob, const Setup& fine, std::
   if (rc != POF_OK) return rc;
   double* full = nullptr;
   HIP_TRY(hipSetDevice(ctx->device));
-  HIP_TRY(hipMalloc((void**)&full, (size_t)kCoarse * D * sizeof(double)));
+  HIP_TRY(device_malloc((void**)&full, (size_t)kCoarse * D * sizeof(double)));
   pof_out po{};
   po.full_means_dev = full;
   rc = eks_run(b, &cp, cs, 1, &po);
@@ -1668,7 +1727,23 @@ size_t lin_buffer_doubles(int D, int d, int method, long long n) {
 
 }  // namespace
 
+namespace pof {
+hipError_t device_malloc(void** p, size_t bytes) {
+  hipError_t e = hipMalloc(p, bytes);
+  if (e != hipErrorOutOfMemory) return e;
+  int device = 0;
+  if (hipGetDevice(&device) != hipSuccess) return e;
+  if (kept_drop([&](const pof_batch* x) { return x->device == device; }) == 0) return e;
+  (void)hipGetLastError();
+  return hipMalloc(p, bytes);
+}
+}  // namespace pof
+
 extern "C" {
+
+int64_t pof_trim(void) {
+  return (int64_t)kept_drop([](const pof_batch*) { return true; });
+}
 
 int pof_ctx_create(int device, pof_ctx** out) {
   if (!out) return POF_E_ARG;
@@ -1695,7 +1770,7 @@ void pof_ctx_destroy(pof_ctx* ctx) {
   ctx->cache.clear();
   for (pof_batch* b : ctx->aux) batch_free(b);
   ctx->aux.clear();
-  drop_kept(ctx);
+  kept_drop([&](const pof_batch* x) { return x->ctx == ctx; });
   pof::large::engine_destroy(ctx->large);
   ctx->large = nullptr;
   if (ctx->timer.ready)
@@ -1828,7 +1903,7 @@ int pof_linearize(pof_ctx* ctx, const pof_problem* prob, const double* m_dev, in
   hipStream_t st = (hipStream_t)stream;
   HIP_TRY(hipSetDevice(ctx->device));
   double* Pd = nullptr;
-  HIP_TRY(hipMalloc((void**)&Pd, s.D * sizeof(double)));
+  HIP_TRY(pof::device_malloc((void**)&Pd, s.D * sizeof(double)));
   hipError_t he = hipMemcpyAsync(Pd, s.P.data(), s.D * sizeof(double), hipMemcpyHostToDevice, st);
   pof::ModelArgs a{};
   a.Pd = Pd;
@@ -1880,7 +1955,7 @@ int linearize_model(pof_ctx* ctx, const pof_problem* prob, int method, const dou
   hipStream_t st = (hipStream_t)stream;
   HIP_TRY(hipSetDevice(ctx->device));
   const bool own = buf == nullptr;
-  if (own) HIP_TRY(hipMalloc((void**)&buf, need * sizeof(double)));
+  if (own) HIP_TRY(pof::device_malloc((void**)&buf, need * sizeof(double)));
   // P, then the per-state work slices (uncertain / unscented); each slice is
   // written before it is read, so nothing needs clearing
   const size_t head = lin_buffer_doubles(s.D, s.d, POF_LIN_EK1, 0);

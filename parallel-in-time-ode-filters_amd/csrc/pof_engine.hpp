@@ -10,6 +10,11 @@
 
 namespace pof {
 
+// hipMalloc on the current device.  Where it has no room, the workspaces that finished calls left there for the next
+// (pof_linear_filtsmooth, pof_smoothing, pof_ekf; of every context of the process) are given back first.
+// Every allocation of device memory goes through it.
+hipError_t device_malloc(void** p, size_t bytes);
+
 constexpr int kMaxLevels = 40;
 constexpr int kChunk = 256;  // time points (threads) per block of the smoothed means and the stage-1 reduction
 

@@ -1785,7 +1785,7 @@ int solve(Engine* e, const Problem& p, const pof_opts& opts, pof_out* out, const
     if (e->buf) (void)hipFree(e->buf);
     e->buf = nullptr;
     e->cap = 0;
-    if (hipMalloc((void**)&e->buf, need) != hipSuccess) {
+    if (device_malloc((void**)&e->buf, need) != hipSuccess) {
       err = "large-state engine: workspace allocation failed";
       return POF_E_HIP;
     }

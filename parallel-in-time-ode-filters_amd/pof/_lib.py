@@ -92,6 +92,7 @@ SIGNATURES = {
     "pof_ctx_create": (ctypes.c_int, [ctypes.c_int, _P(_vp)]),
     "pof_ctx_destroy": (None, [_vp]),
     "pof_last_error": (ctypes.c_char_p, [_vp]),
+    "pof_trim": (ctypes.c_int64, []),
     "pof_supported": (ctypes.c_int, [ctypes.c_int, ctypes.c_int]),
     "pof_profile_enable": (ctypes.c_int, [_vp, ctypes.c_int]),
     "pof_profile_read": (ctypes.c_int, [_vp, ctypes.c_int, _dp, _P(ctypes.c_longlong), _P(ctypes.c_longlong)]),
@@ -200,6 +201,11 @@ def context(device=None):
 
         autotune.apply_cache(c)
     return c
+
+
+def trim():
+    """Give back the device memory that finished linear filter / smoother calls left for the next one; returns the bytes."""
+    return int(_lib.pof_trim()) if _lib is not None else 0
 
 
 def set_graphs(on, device=None):

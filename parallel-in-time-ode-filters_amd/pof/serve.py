@@ -30,6 +30,7 @@ import time
 
 import numpy as np
 
+from . import _lib
 from . import batch as _batch
 
 
@@ -87,8 +88,14 @@ class Server:
         D = d * (order + 1)
         first = not self.groups.get(key)
         free = torch.cuda.mem_get_info()[0]
+        trimmed = False
         for entries in (max(self._target_entries(D), need), max(self.MIN_ENTRIES, need)):
             nbytes = _batch.bytes_for(D, entries, self.slots)
+            if nbytes + self.reserve > free and not trimmed:
+                # what finished calls left for the next one is free too
+                trimmed = True
+                if _lib.trim() > 0:
+                    free = torch.cuda.mem_get_info()[0]
             if nbytes + self.reserve > free:
                 continue
             if not first and self.used + nbytes > self.budget:

@@ -1,0 +1,145 @@
+// Host-only checks of the library against a stand-in of the HIP runtime (runtime_stand_in.cpp): what its host code does with
+// memory, streams and failed calls.  No kernel runs, so no result is looked at.  The argument picks a check.
+#include <cstdio>
+#include <cstring>
+#include <string>
+#include <vector>
+
+#include "../../include/pof.h"
+#include "runtime_stand_in.hpp"
+
+static int failures = 0;
+#define CHECK(cond)                                                          \
+  do {                                                                       \
+    if (!(cond)) {                                                           \
+      std::fprintf(stderr, "check failed: %s (line %d)\n", #cond, __LINE__); \
+      ++failures;                                                            \
+    }                                                                        \
+  } while (0)
+
+// A linear filter and smoother call of D = 12, d = 3 over n steps (device arrays: any addresses, nothing reads them)
+static int filtsmooth(pof_ctx* ctx, long n, void* stream = nullptr) {
+  constexpr int D = 12, d = 3;
+  std::vector<double> m(D), L(D * D), F(D * D), Q(D * D);
+  static double dev[1];
+  double nll, obj, ssq;
+  return pof_linear_filtsmooth(ctx, D, d, n, m.data(), L.data(), F.data(), Q.data(), dev, dev, nullptr, 0, nullptr, nullptr,
+                               nullptr, nullptr, &nll, &obj, &ssq, stream);
+}
+// Steps of which a call's workspace takes about `bytes`
+static long steps_for(double bytes) { return (long)(bytes / (2.0 * 8 * (7 * 144 + 7 * 12 + 2))); }
+
+static pof_problem problem(int kind, int d, int q, std::vector<double>& ts, std::vector<double>& y0) {
+  pof_problem p{};
+  p.kind = kind;
+  p.d = d;
+  p.q = q;
+  p.init = POF_INIT_CONSTANT;
+  p.n_times = (int64_t)ts.size();
+  p.ts_host = ts.data();
+  p.y0_host = y0.data();
+  p.params[0] = 8.0;
+  return p;
+}
+static std::vector<double> grid(int n) {
+  std::vector<double> ts(n);
+  for (int k = 0; k < n; ++k) ts[k] = 1e-3 * k;
+  return ts;
+}
+
+static int solve_large(pof_ctx* ctx, int d, int q, int n) {
+  std::vector<double> ts = grid(n + 1), y0(d, 8.0);
+  const pof_problem p = problem(POF_LORENZ96, d, q, ts, y0);
+  pof_opts o{};
+  o.maxiters = o.fixed_iters = 1;
+  pof_out out{};
+  return pof_solve_large(ctx, &p, &o, &out, nullptr);
+}
+
+// What calls leave for the next is given back to every other allocation of the library, of any context
+static void kept_memory() {
+  const double MiB = 1 << 20;
+  pof_ctx *a = nullptr, *b = nullptr;
+  CHECK(pof_ctx_create(0, &a) == POF_OK);
+  CHECK(pof_ctx_create(0, &b) == POF_OK);
+  const size_t before = stand_in::live;
+  CHECK(filtsmooth(a, steps_for(400 * MiB)) == POF_OK);
+  const size_t kept = stand_in::live - before;
+  CHECK(kept > (size_t)(350 * MiB));
+  // the next call of the context takes it
+  CHECK(filtsmooth(a, steps_for(300 * MiB)) == POF_OK);
+  CHECK(stand_in::live - before == kept);
+  // a batch, of the other context, where nothing else is left
+  stand_in::limit = stand_in::live + (size_t)(50 * MiB);
+  pof_batch* batch = nullptr;
+  CHECK(pof_batch_create(b, 12, 3, 2 * steps_for(200 * MiB), 1, &batch) == POF_OK);
+  pof_batch_destroy(batch);
+  CHECK(stand_in::live == before);
+  // the large-state engine, of the other context
+  stand_in::limit = ~size_t(0);
+  CHECK(filtsmooth(a, steps_for(400 * MiB)) == POF_OK);
+  stand_in::limit = stand_in::live + (size_t)(20 * MiB);
+  CHECK(solve_large(b, 8, 2, 600) == POF_OK);
+  // the linearisation's work slices
+  stand_in::limit = ~size_t(0);
+  CHECK(filtsmooth(a, steps_for(400 * MiB)) == POF_OK);
+  stand_in::limit = stand_in::live + (size_t)(20 * MiB);
+  {
+    std::vector<double> ts = grid(3), y0(3, 1.0);
+    const pof_problem p = problem(POF_RIGID_BODY, 3, 3, ts, y0);
+    static double dev[1];
+    const double par[4] = {1.0, 1.0, 0.0, 0.0};
+    CHECK(pof_linearize_model(b, &p, POF_LIN_UNSCENTED, par, dev, dev, 60000, dev, dev, dev, nullptr) == POF_OK);
+  }
+  // a batch's launch tables and the coarse start's buffer are too small to be the ones that fail alone: that they ask
+  // in the same way is in the sources (test_host_runtime.py)
+  stand_in::limit = ~size_t(0);
+  // an allocation that fails with nothing kept fails
+  CHECK(pof_trim() >= 0 && pof_trim() == 0);
+  stand_in::limit = stand_in::live + (size_t)(1 * MiB);
+  CHECK(pof_batch_create(b, 12, 3, 2 * steps_for(200 * MiB), 1, &batch) == POF_E_HIP);
+  stand_in::limit = ~size_t(0);
+  // by hand
+  const size_t base = stand_in::live;
+  CHECK(filtsmooth(a, steps_for(100 * MiB)) == POF_OK);
+  CHECK(filtsmooth(b, steps_for(100 * MiB)) == POF_OK);
+  CHECK(stand_in::live > base + (size_t)(150 * MiB));
+  CHECK(pof_trim() > (int64_t)(150 * MiB));
+  CHECK(stand_in::live == base);
+  pof_ctx_destroy(a);
+  pof_ctx_destroy(b);
+  CHECK(stand_in::live == 0);
+}
+
+// Contexts belong to threads: what all of them keep has one bound
+static void kept_bound() {
+  const double MiB = 1 << 20;
+  std::vector<pof_ctx*> ctx(5, nullptr);
+  for (auto& c : ctx) CHECK(pof_ctx_create(0, &c) == POF_OK);
+  for (auto& c : ctx) {
+    CHECK(filtsmooth(c, steps_for(300 * MiB)) == POF_OK);
+    CHECK(filtsmooth(c, steps_for(310 * MiB)) == POF_OK);
+    CHECK(stand_in::live <= (size_t)(1100 * MiB));
+  }
+  // one beyond the bound by itself is not kept, and takes nothing of the others'
+  pof_trim();
+  CHECK(filtsmooth(ctx[0], steps_for(200 * MiB)) == POF_OK);
+  const size_t live = stand_in::live;
+  CHECK(filtsmooth(ctx[1], steps_for(1200 * MiB)) == POF_OK);
+  CHECK(stand_in::live <= live);
+  // a context takes its own with it, the others' stay
+  CHECK(filtsmooth(ctx[1], steps_for(200 * MiB)) == POF_OK);
+  pof_ctx_destroy(ctx[0]);
+  CHECK(stand_in::live > (size_t)(150 * MiB) && stand_in::live < (size_t)(250 * MiB));
+  for (size_t i = 1; i < ctx.size(); ++i) pof_ctx_destroy(ctx[i]);
+  CHECK(stand_in::live == 0);
+}
+
+int main(int argc, char** argv) {
+  const std::string what = argc > 1 ? argv[1] : "";
+  if (what == "kept_memory") kept_memory();
+  else if (what == "kept_bound") kept_bound();
+  else CHECK(!"a known check");
+  std::printf("%s: %d failures\n", what.c_str(), failures);
+  return failures == 0 ? 0 : 1;
+}

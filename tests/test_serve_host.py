@@ -140,3 +140,20 @@ def test_admission_respects_free_memory(monkeypatch):
                        reserve_bytes=2_000_000)
     recs = srv.run([(_F(), np.zeros(1), np.zeros(3000), 2, "constant")], np.zeros(1))
     assert recs[0].status == "rejected" and srv.batches_created == 0
+
+
+def test_admission_counts_kept_workspaces_as_free(monkeypatch):
+    """Memory that finished linear smoother calls left for the next one is given back before a request is turned away."""
+    import torch
+
+    srv = _fake_server(monkeypatch, free_bytes=5_000_000, budget_bytes=1 << 40, n_groups=1, slots=8, reserve_bytes=0)
+    trims = []
+
+    def trim():
+        trims.append(1)
+        monkeypatch.setattr(torch.cuda, "mem_get_info", lambda *a: (7_000_000, 1 << 40))
+        return 2_000_000
+
+    monkeypatch.setattr(serve._lib, "trim", trim)
+    recs = srv.run([(_F(), np.zeros(1), np.zeros(3000), 2, "constant")], np.zeros(1))  # 6000 entries of 1000 bytes
+    assert recs[0].status == "converged" and len(trims) == 1
