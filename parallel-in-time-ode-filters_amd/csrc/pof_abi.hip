@@ -1259,9 +1259,10 @@ int batch_launch(pof_batch* b) {
     HIP_TRY(stage_maps(b));
     up.maps();
     b->plan.dev = b->maps_dev;
-    b->plan_dirty = false;
   }
   if (b->plan.m == 0) return POF_OK;
+  // work that reads the host tables is enqueued from here on, also where a later call fails
+  b->unsynced = true;
   // newly admitted IVPs: per-slot tables and initial means
   const int D = b->D;
   const size_t DD = (size_t)D * D, S = (size_t)b->slots;
@@ -1297,6 +1298,7 @@ int batch_launch(pof_batch* b) {
     up.add(b->arena_map + ((const char*)(b->stage.p + t.at) - b->arena_host), b->g.means0 + (size_t)t.start * D, t.n * 8);
   up.flush();
   HIP_TRY(up.status);
+  b->plan_dirty = false;
   b->model_dirty = false;
   b->dirty_slots.clear();
   b->init_stage.clear();
@@ -1376,7 +1378,6 @@ int batch_launch(pof_batch* b) {
     HIP_TRY(hipEventRecord(b->ev, b->st));
   }
   b->launched = true;
-  b->unsynced = true;
   return POF_OK;
 }
 
@@ -1451,7 +1452,9 @@ int batch_finish(pof_batch* b, int max_done, long long* done, int* n_done) {
   const int start_o = ((int)b->hmaps.size() + 3) / 4 * 4;
   if (rc == POF_OK) rc = plan_tables(b, fin, b->hmaps, po);
   if (rc != POF_OK) return set_err(ctx, rc, "launch tables overflow");
+  b->plan_dirty = true;  // (also where a call below fails: the launch tables are overwritten now)
   HIP_TRY(stage_maps(b));
+  b->unsynced = true;
   Uploader up(b);
   up.maps();
   up.table(b->hwchol, 0, S);
@@ -1471,6 +1474,7 @@ int batch_finish(pof_batch* b, int max_done, long long* done, int* n_done) {
   }
   HIP_TRY(b->e->output(b->g, po, b->st));
   HIP_TRY(hipStreamSynchronize(b->st));
+  b->unsynced = false;
   int nd = 0;
   for (int j : fin) {
     pof_batch::Slot& s = b->sl[j];
@@ -1488,7 +1492,6 @@ int batch_finish(pof_batch* b, int max_done, long long* done, int* n_done) {
     s.used = false;
     b->hwchol[j] = 0;
   }
-  b->plan_dirty = true;
   if (n_done) *n_done = nd;
   return POF_OK;
 }

@@ -135,10 +135,69 @@ static void kept_bound() {
   CHECK(stand_in::live == 0);
 }
 
+// The words that launches of k_upload bring to the device (its argument: {source, destination, words} per grid row)
+static size_t g_words = 0;
+static void count_words(const std::string& name, unsigned rows, void** args) {
+  struct Part {
+    const unsigned* src;
+    unsigned* dst;
+    size_t n;
+  };
+  if (name.find("k_upload") == std::string::npos) return;
+  const Part* p = static_cast<const Part*>(args[0]);
+  for (unsigned i = 0; i < rows; ++i) g_words += p[i].n;
+}
+
+// A batch after a call that failed part way: its tables are not taken to be on the device, and the host's are not
+// written while an upload may still be reading them
+static void failed_launch() {
+  pof_ctx* ctx = nullptr;
+  CHECK(pof_ctx_create(0, &ctx) == POF_OK);
+  pof_batch* b = nullptr;
+  CHECK(pof_batch_create(ctx, 12, 3, 4096, 4, &b) == POF_OK);
+  stand_in::on_launch = count_words;
+  std::vector<double> ts = grid(65), y0(3, 1.0);
+  const pof_problem p = problem(POF_RIGID_BODY, 3, 3, ts, y0);
+  pof_opts o{};
+  o.maxiters = o.fixed_iters = 2;
+  pof_out out[4] = {};
+  for (int i = 0; i < 2; ++i) CHECK(pof_batch_admit(b, &p, &o, &out[i], nullptr) == POF_OK);
+  // the upload of an admission
+  stand_in::fail_launch = "k_upload";
+  g_words = 0;
+  CHECK(pof_batch_launch(b) == POF_E_HIP);
+  const size_t first = g_words;
+  g_words = 0;
+  // ... and, once it has gone, a launch behind it
+  stand_in::fail_launch = "k_filter_leaf16";
+  CHECK(pof_batch_launch(b) == POF_E_HIP);
+  CHECK(first > 0 && g_words == first);
+  const long syncs = stand_in::syncs;
+  CHECK(pof_batch_admit(b, &p, &o, &out[2], nullptr) == POF_OK);
+  CHECK(stand_in::syncs > syncs);
+  // two iterations, and a retirement that fails
+  CHECK(pof_batch_launch(b) == POF_OK);
+  int n = 0;
+  CHECK(pof_batch_finish(b, 0, nullptr, &n) == POF_OK && n == 0);
+  g_words = 0;
+  CHECK(pof_batch_launch(b) == POF_OK);
+  CHECK(g_words == 4);  // the factor flags of the last iteration alone
+  stand_in::fail_launch = "k_output";
+  CHECK(pof_batch_finish(b, 0, nullptr, &n) == POF_E_HIP);
+  g_words = 0;
+  CHECK(pof_batch_launch(b) == POF_OK);
+  CHECK(g_words >= 3 * 4);  // the launch tables (records of three IVPs, ...), which the retirement's have overwritten
+  stand_in::on_launch = nullptr;
+  pof_batch_destroy(b);
+  pof_ctx_destroy(ctx);
+  CHECK(stand_in::live == 0);
+}
+
 int main(int argc, char** argv) {
   const std::string what = argc > 1 ? argv[1] : "";
   if (what == "kept_memory") kept_memory();
   else if (what == "kept_bound") kept_bound();
+  else if (what == "failed_launch") failed_launch();
   else CHECK(!"a known check");
   std::printf("%s: %d failures\n", what.c_str(), failures);
   return failures == 0 ? 0 : 1;

@@ -17,6 +17,7 @@ long syncs = 0;
 std::string fail_launch;
 void* capturing = nullptr;
 std::map<std::string, long> launches;
+std::function<void(const std::string&, unsigned, void**)> on_launch;
 static std::mutex mu;
 static std::map<void*, size_t> sizes;
 static std::map<const void*, std::string> names;
@@ -161,9 +162,10 @@ int hipEventElapsedTime(float* ms, void*, void*) {
   *ms = 0.0f;
   return 0;
 }
-int hipLaunchKernel(const void* f, Dim3, Dim3, void**, size_t, void*) {
+int hipLaunchKernel(const void* f, Dim3 grid, Dim3, void** args, size_t, void*) {
   std::lock_guard<std::mutex> lk(mu);
   const std::string& name = names[f];
+  if (on_launch) on_launch(name, grid.y, args);
   if (!fail_launch.empty() && name.find(fail_launch) != std::string::npos) {
     fail_launch.clear();  // once
     return set(kLaunchFailure);
