@@ -1566,6 +1566,17 @@ struct StreamScope {
   }
 };
 
+// A call on a stream that the caller is capturing is refused before it enqueues or takes anything: it waits for its
+// results, and what it had enqueued by then would stay in the caller's graph, over workspaces that a failed call frees.
+int check_stream(pof_ctx* ctx, void* stream) {
+  if (!stream) return POF_OK;
+  hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+  HIP_TRY(hipStreamIsCapturing((hipStream_t)stream, &cs));
+  if (cs != hipStreamCaptureStatusNone)
+    return set_err(ctx, POF_E_HIP, "the stream is being captured: a call waits for its results");
+  return POF_OK;
+}
+
 // Drop every IVP of b after a failed call (the cached batches of pof_solve,
 // pof_eks_solve, pof_ieks_step and pof_solve_batch serve one call at a time):
 // wait for its stream, errors ignored, then free every slot and entry range,
@@ -2056,6 +2067,8 @@ int pof_solve(pof_ctx* ctx, const pof_problem* prob, const pof_opts* opts, pof_o
       (!pof::find_engine(s.D, s.d) && pof::large::supports(prob->kind, s.D, s.d)))
     return solve_large(ctx, prob, opts, out, stream);
   if (!engine_or_err(ctx, s.D, s.d)) return POF_E_UNSUPPORTED;
+  rc = check_stream(ctx, stream);
+  if (rc != POF_OK) return rc;
   pof_batch* b = nullptr;
   rc = cached_batch(ctx, s.D, s.d, entries_for(prob->n_times), 1, &b);
   if (rc != POF_OK) return rc;
@@ -2086,6 +2099,8 @@ int pof_eks_solve(pof_ctx* ctx, const pof_problem* prob, int calibrate, pof_out*
   int rc = pof::build_setup(prob, s, ctx->err);
   if (rc != POF_OK) return rc;
   if (!engine_or_err(ctx, s.D, s.d)) return POF_E_UNSUPPORTED;
+  rc = check_stream(ctx, stream);
+  if (rc != POF_OK) return rc;
   pof_batch* b = nullptr;
   rc = cached_batch(ctx, s.D, s.d, entries_for(prob->n_times), 1, &b);
   if (rc != POF_OK) return rc;
@@ -2101,6 +2116,8 @@ int pof_ieks_step(pof_ctx* ctx, const pof_problem* prob, const double* states_me
   int rc = pof::build_setup(prob, s, ctx->err);
   if (rc != POF_OK) return rc;
   if (!engine_or_err(ctx, s.D, s.d)) return POF_E_UNSUPPORTED;
+  rc = check_stream(ctx, stream);
+  if (rc != POF_OK) return rc;
   pof_batch* b = nullptr;
   rc = cached_batch(ctx, s.D, s.d, entries_for(prob->n_times), 1, &b);
   if (rc != POF_OK) return rc;
@@ -2159,8 +2176,10 @@ int pof_smoothing(pof_ctx* ctx, int D, int64_t Ns, const double* F_host, const d
     if (D % dd == 0 && (e = pof::find_engine(D, dd)) != nullptr) d = dd;
   if (!e) return set_err(ctx, POF_E_UNSUPPORTED, "no kernels for state dimension %d", D);
   HIP_TRY(hipSetDevice(ctx->device));
+  int rc = check_stream(ctx, stream);
+  if (rc != POF_OK) return rc;
   CallBatch call(ctx);
-  int rc = call.open(D, d, entries_for(Ns + 1), true);
+  rc = call.open(D, d, entries_for(Ns + 1), true);
   if (rc != POF_OK) return rc;
   pof_batch* b = call.b;
   StreamScope scope(b, stream);
@@ -2203,6 +2222,8 @@ int pof_ekf(pof_ctx* ctx, const pof_problem* prob, const double* x0_mean_host, c
   if (rc != POF_OK) return rc;
   if (!engine_or_err(ctx, s.D, s.d)) return POF_E_UNSUPPORTED;
   HIP_TRY(hipSetDevice(ctx->device));
+  rc = check_stream(ctx, stream);
+  if (rc != POF_OK) return rc;
   CallBatch call(ctx);
   rc = call.open(s.D, s.d, entries_for(prob->n_times), false);
   if (rc != POF_OK) return rc;
@@ -2246,8 +2267,10 @@ int pof_linear_filtsmooth(pof_ctx* ctx, int D, int d, int64_t Ns, const double* 
       !H_dev || !c_dev)
     return set_err(ctx, POF_E_ARG, "invalid linear_filtsmooth arguments");
   if (!engine_or_err(ctx, D, d)) return POF_E_UNSUPPORTED;
+  int rc = check_stream(ctx, stream);
+  if (rc != POF_OK) return rc;
   CallBatch call(ctx);
-  int rc = call.open(D, d, entries_for(Ns + 1), true);
+  rc = call.open(D, d, entries_for(Ns + 1), true);
   if (rc != POF_OK) return rc;
   pof_batch* b = call.b;
   StreamScope scope(b, stream);

@@ -193,11 +193,54 @@ static void failed_launch() {
   CHECK(stand_in::live == 0);
 }
 
+// A call on a stream that its caller is capturing is refused before anything is enqueued: what it enqueued would
+// stay in the caller's graph, over memory that the refused call gives back
+static void captured_stream() {
+  pof_ctx* ctx = nullptr;
+  CHECK(pof_ctx_create(0, &ctx) == POF_OK);
+  int handle = 0;
+  void* stream = &handle;
+  std::vector<double> ts = grid(65), y0(3, 1.0), m(12), L(144), F(144), Q(144);
+  const pof_problem p = problem(POF_RIGID_BODY, 3, 3, ts, y0);
+  pof_opts o{};
+  o.maxiters = o.fixed_iters = 2;
+  pof_out out{};
+  std::vector<double> dev(64 * 1024);
+  double nll, obj, ssq;
+  auto call = [&](int k) {
+    switch (k) {
+      case 0: return filtsmooth(ctx, 64, stream);
+      case 1: return pof_solve(ctx, &p, &o, &out, stream);
+      case 2: return pof_eks_solve(ctx, &p, 1, &out, stream);
+      case 3: return pof_ieks_step(ctx, &p, dev.data(), 0, nullptr, nullptr, &nll, &obj, &ssq, stream);
+      case 4: return pof_smoothing(ctx, 12, 64, F.data(), Q.data(), dev.data(), dev.data(), 0, nullptr, nullptr, &obj, stream);
+      default: return pof_ekf(ctx, &p, m.data(), L.data(), F.data(), Q.data(), nullptr, nullptr, &nll, &ssq, stream);
+    }
+  };
+  for (int warm = 0; warm < 2; ++warm) {  // without and with workspaces of calls before
+    for (int k = 0; k < 6; ++k) {
+      const long n = stand_in::launched("");
+      const size_t live = stand_in::live;
+      stand_in::capturing = stream;
+      CHECK(call(k) == POF_E_HIP);
+      CHECK(std::strlen(pof_last_error(ctx)) > 0);
+      stand_in::capturing = nullptr;
+      CHECK(stand_in::launched("") == n);
+      CHECK(stand_in::live == live);
+      CHECK(call(k) == POF_OK);
+      CHECK(stand_in::launched("") > n);
+    }
+  }
+  pof_ctx_destroy(ctx);
+  CHECK(stand_in::live == 0);
+}
+
 int main(int argc, char** argv) {
   const std::string what = argc > 1 ? argv[1] : "";
   if (what == "kept_memory") kept_memory();
   else if (what == "kept_bound") kept_bound();
   else if (what == "failed_launch") failed_launch();
+  else if (what == "captured_stream") captured_stream();
   else CHECK(!"a known check");
   std::printf("%s: %d failures\n", what.c_str(), failures);
   return failures == 0 ? 0 : 1;
