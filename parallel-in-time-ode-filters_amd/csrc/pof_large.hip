@@ -118,13 +118,15 @@ __host__ __device__ inline int lq_end(int n, int npiv, int b1, int w2, int p) {
 __host__ __device__ constexpr int lq_panel_doubles(int nt) { return nt * 256 + 256; }
 
 // tiles of the widest panel, and the tiles that the kernels are compiled for: registers and scratch scale with them
-// (the banded panels of the D = 128 combines have 9 or 10, those of D = 24 and 32 three)
+// (the banded panels of the D = 128 combines have 9 or 10, those of D = 24 and 32 three).  A panel reaches at most
+// D + max(16, d) columns: 160 for D <= 128 and the fields' d <= 32.
+constexpr int kLqMaxTiles = 10;
 inline int lq_tiles(int n, int npiv, int b1, int w2) {
   int nt = 1;
   for (int p = 0; 16 * p < npiv; ++p) nt = std::max(nt, (lq_end(n, npiv, b1, w2, p) - 16 * p + 15) / 16);
-  for (int t : {3, 5, 8, 9, 10})
+  for (int t : {3, 5, 8, 9, kLqMaxTiles})
     if (nt <= t) return t;
-  return 16;
+  return nt;
 }
 // Pivots of the first factorisation of an m x n matrix (Ops::lq)
 inline int lq_first(int m, int n, int b1) {
@@ -1347,8 +1349,9 @@ struct Ops {
       case 8: launch_lq<8, 2>(q, m, n, cnt, npiv, b1, w2); break;
       case 9: launch_lq<9, 2>(q, m, n, cnt, npiv, b1, w2); break;
       case 10: launch_lq<10, 2>(q, m, n, cnt, npiv, b1, w2); break;
-      default: launch_lq<16, 1>(q, m, n, cnt, npiv, b1, w2);  // two strips would not fit the registers
+      default: fail("lq: panels of more than 160 columns", -1);
     }
+    if (err) return;
     if (m <= b1 || n <= b1 || b1 <= 0) return;
     LqBlocks r{};
     r.a = q.o[0].at(b1, b1);
@@ -1410,8 +1413,10 @@ struct Ops {
       a.item0 = c0;
       if (vec)
         launch_lq_part<NT, S, true>(a, c, P);
-      else
+      else if constexpr (NT <= 8)
         launch_lq_part<NT, S, false>(a, c, P);
+      else
+        fail("lq: rows off the 16-byte grid in panels of more than 128 columns", -1);  // (D = 128 alone has such)
     }
     arena_release(ar, mark);
   }
@@ -1419,11 +1424,14 @@ struct Ops {
   void launch_lq_part(const LqArgs& a, int cnt, int P) {
     hipLaunchKernelGGL((k_lq_rows<NT, S, VEC>), dim3(cnt), dim3(64), 0, st, a);
     check("k_lq_rows");
-    if (a.m > 16 * P) {
+    if (a.m <= 16 * P) return;
+    if constexpr (NT < kLqMaxTiles) {
       const int per = 16 * S * kLqBelowWaves;
       hipLaunchKernelGGL((k_lq_below<NT, S, VEC>), dim3(cnt, (a.m - 16 * P + per - 1) / per), dim3(64 * kLqBelowWaves), 0,
                          st, a, 16 * P);
       check("k_lq_below");
+    } else {
+      fail("lq: rows below the pivots of panels of more than 144 columns", -1);  // ([A1^T Xi22 | Z1] of D = 128, without)
     }
   }
   // op(L) X = R (L lower n x n, X n x m): R is X itself (in place), or the separate R when given

@@ -235,12 +235,58 @@ static void captured_stream() {
   CHECK(stand_in::live == 0);
 }
 
+// The large-state engine over every shape that it takes (a grid of the longest there is among them): its workspace is large
+// enough, and every kernel of the factorisation that the library holds is one that some shape runs
+static void large_shapes() {
+  int shapes = 0;
+  for (int d = 1; d <= 4; ++d)  // fields of the per-worker kernels, whose states the engine takes too
+    for (int q = 1; q <= 5; ++q) {
+      if (!pof_supported(d * (q + 1), d)) continue;
+      const int kinds[] = {POF_LOGISTIC, POF_FHN_CLASSIC, POF_RIGID_BODY, POF_HENONHEILES};
+      for (int n : {1, 2, 3, 7, 64, 1025, 4099}) {
+        std::vector<double> ts = grid(n + 1), y0(d, 0.5);
+        const pof_problem p = problem(kinds[d - 1], d, q, ts, y0);
+        pof_opts o{};
+        o.maxiters = o.fixed_iters = 1;
+        pof_out out{};
+        pof_ctx* c = nullptr;
+        CHECK(pof_ctx_create(0, &c) == POF_OK);
+        CHECK(pof_solve_large(c, &p, &o, &out, nullptr) == POF_OK);
+        pof_ctx_destroy(c);
+      }
+    }
+  for (int d = 4; d <= 64; ++d)
+    for (int q = 1; d * (q + 1) <= 128; ++q) {
+      std::vector<double> ts = grid(3), y0(d, 8.0);
+      const pof_problem p = problem(POF_LORENZ96, d, q, ts, y0);
+      if (pof_setup(&p, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr) != POF_OK) continue;
+      ++shapes;
+      for (int n : {1, 2, 3, 5, 6, 7, 11, 64, 65, 200, 1025, 2047, 2048, 4099, 65534}) {
+        if (n > 5000 && q > 3) continue;
+        // a fresh context for each: the engine's buffer grows and is not given back
+        pof_ctx* c = nullptr;
+        CHECK(pof_ctx_create(0, &c) == POF_OK);
+        const int rc = solve_large(c, d, q, n);
+        if (rc != POF_OK) std::fprintf(stderr, "d=%d q=%d n=%d: %s\n", d, q, n, pof_last_error(c));
+        CHECK(rc == POF_OK);
+        pof_ctx_destroy(c);
+      }
+    }
+  CHECK(shapes > 40);
+  for (const std::string& k : stand_in::kernels("k_lq_")) {
+    if (stand_in::launched(k) == 0) std::fprintf(stderr, "not reached: %s\n", k.c_str());
+    CHECK(stand_in::launched(k) > 0);
+  }
+  CHECK(stand_in::live == 0);
+}
+
 int main(int argc, char** argv) {
   const std::string what = argc > 1 ? argv[1] : "";
   if (what == "kept_memory") kept_memory();
   else if (what == "kept_bound") kept_bound();
   else if (what == "failed_launch") failed_launch();
   else if (what == "captured_stream") captured_stream();
+  else if (what == "large_shapes") large_shapes();
   else CHECK(!"a known check");
   std::printf("%s: %d failures\n", what.c_str(), failures);
   return failures == 0 ? 0 : 1;

@@ -3,12 +3,15 @@
 // linked with it in place of the runtime.  The knobs and counters are declared in runtime_stand_in.hpp.
 #include "runtime_stand_in.hpp"
 
+#include <sys/mman.h>
+
 #include <cstdint>
 #include <cstdlib>
 #include <cstring>
 #include <map>
 #include <mutex>
 #include <string>
+#include <vector>
 
 namespace stand_in {
 size_t limit = ~size_t(0);
@@ -23,6 +26,12 @@ static std::map<void*, size_t> sizes;
 static std::map<const void*, std::string> names;
 static int last_error = 0;
 
+std::vector<std::string> kernels(const std::string& part) {
+  std::vector<std::string> out;
+  for (const auto& kv : names)
+    if (kv.second.find(part) != std::string::npos) out.push_back(kv.second);
+  return out;
+}
 long launched(const std::string& part) {
   long n = 0;
   for (const auto& kv : launches)
@@ -59,7 +68,12 @@ int hipMalloc(void** p, size_t n) {
   std::lock_guard<std::mutex> lk(mu);
   *p = nullptr;
   if (live + n > limit) return set(kOutOfMemory);
-  *p = std::malloc(n);
+  // address space alone until it is touched
+  *p = mmap(nullptr, n, PROT_READ | PROT_WRITE, MAP_PRIVATE | MAP_ANONYMOUS | MAP_NORESERVE, -1, 0);
+  if (*p == MAP_FAILED) {
+    *p = nullptr;
+    return set(kOutOfMemory);
+  }
   sizes[*p] = n;
   live += n;
   if (live > peak) peak = live;
@@ -71,8 +85,8 @@ int hipFree(void* p) {
   const auto it = sizes.find(p);
   if (it == sizes.end()) std::abort();  // not from hipMalloc, or freed before
   live -= it->second;
+  munmap(p, it->second);
   sizes.erase(it);
-  std::free(p);
   return 0;
 }
 int hipHostMalloc(void** p, size_t n, unsigned) {

@@ -5,6 +5,7 @@
 #include <functional>
 #include <map>
 #include <string>
+#include <vector>
 
 namespace stand_in {
 extern size_t limit;             // bytes of device memory
@@ -16,4 +17,5 @@ extern std::map<std::string, long> launches;
 // called at each launch that is to succeed or fail: the kernel's name, its grid's y and its arguments
 extern std::function<void(const std::string&, unsigned, void**)> on_launch;
 long launched(const std::string& part);  // launches of the kernels whose names contain part
+std::vector<std::string> kernels(const std::string& part);  // the library's kernels whose names contain part
 }  // namespace stand_in

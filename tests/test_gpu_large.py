@@ -199,3 +199,46 @@ def test_more_matrices_than_are_factored_at_a_time(gpu):
     assert rel(ys.mean.cpu().numpy(), yr.mean.cpu().numpy()) < 1e-9
     s1, s2 = info["sigma_squared"], rinfo["sigma_squared"]
     assert rel(cov(ys.chol.cpu().numpy()) / s1**2, cov(yr.chol.cpu().numpy()) / s2**2) < 1e-6
+
+
+@pytest.mark.parametrize("d,q", [(5, 6), (6, 6), (8, 6), (6, 10), (16, 7), (32, 1)])
+def test_lorenz96_high_orders_match_oracle(gpu, monkeypatch, d, q):
+    """Rows off the 16-byte grid with five and eight column tiles (D = 35, 42, 66), and nine tiles with eight equations a
+    panel (D = 128, q = 7).  The Cholesky factor QL of the order's Hilbert matrix is determined to 1e-10 (q = 6) to 1e-3
+    (q = 10) only, so the oracle takes the library's.  Tolerances as above, and 20 times the oracle's own change when y0
+    moves by 1e-15 relative where that is more."""
+    import torch
+
+    import pof.solver
+    from oracle import model as om
+    from oracle import problems as op
+    from oracle import solver as osolver
+    from pof import _lib
+
+    lib = _lib.load()
+
+    def discretize(iwp):
+        D = d * (q + 1)
+        F, QL = np.empty((D, D)), np.empty((D, D))
+        assert lib.pof_transitions(d, q, 1.0, _lib.hptr(F), _lib.hptr(QL), None, None) == _lib.POF_OK
+        return F, QL
+
+    monkeypatch.setattr(om, "preconditioned_discretize", discretize)
+    ivp, oivp = _pair("lorenz96", d=d)
+    for N in (2, 3, 4):
+        ts = np.linspace(0.0, (N - 1) * 5.0 / 8192, N)
+        print(f"lorenz96 high orders d={d} q={q} N={N}", flush=True)
+
+        def oracle(e=0.0):
+            p = op.Problem(oivp.name, oivp.params, oivp.y0 * (1 + e), oivp.t0, oivp.tmax)
+            r, i = osolver.solve(p, ts, q, init="constant", fixed_iters=2)
+            return [r.mean, cov(r.chol) / i["sigma_squared"] ** 2, np.array(i["obj"])]
+
+        ref = oracle()
+        spread = [max(rel(a, b) for a in x) for *x, b in zip(*(oracle(e) for e in (1e-15, -1e-15, 3e-15)), ref)]
+        ys, info = pof.solver.solve(f=ivp.f, y0=ivp.y0, ts=ts, order=q, init="constant", fixed_iters=2, engine="large")
+        torch.cuda.synchronize()
+        got = [ys.mean.cpu().numpy(), cov(ys.chol.cpu().numpy()) / info["sigma_squared"] ** 2, np.array(info["obj"])]
+        for k, (a, b, t, s) in enumerate(zip(got, ref, (1e-8, 1e-6, 1e-6), spread)):
+            print(f"  result {k}: {rel(a, b):.1e} of {max(t, 20 * s):.1e}", flush=True)
+            assert rel(a, b) <= max(t, 20 * s), k
