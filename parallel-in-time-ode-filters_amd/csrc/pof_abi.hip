@@ -954,8 +954,8 @@ int batch_new(pof_ctx* ctx, int D, int d, long long entries, int slots, bool aff
 // The workspace of one call of pof_linear_filtsmooth, pof_smoothing or pof_ekf.  Its 26 allocations and their
 // releases cost 3.1 of the 3.9 ms of a call over 16,384 steps at D = 12, so a finished call's is kept for the next
 // one of its context and (D, d) that fits: at most kKeptBatches of a context, and of all contexts on a device
-// kKeptBytes together (see KeptList).  A call takes it out of the list, so that calls from several threads
-// have one each; it is put back only idle: its work done, its slots free.
+// kKeptBytes together (see KeptList).  A call takes it out of the list and puts it back only idle: its work done, its
+// slots free.
 struct CallBatch {
   pof_ctx* ctx;
   pof_batch* b = nullptr;

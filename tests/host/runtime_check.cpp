@@ -135,6 +135,25 @@ static void kept_bound() {
   CHECK(stand_in::live == 0);
 }
 
+// A call that fails once its workspace is open gives it back, and the next call has one of its own
+static void failed_call() {
+  pof_ctx* ctx = nullptr;
+  CHECK(pof_ctx_create(0, &ctx) == POF_OK);
+  const size_t before = stand_in::live;
+  for (const char* kernel : {"k_upload", "k_filter_leaf16", "k_filter_up16", "k_reduce_final", "k_output"}) {
+    CHECK(filtsmooth(ctx, 100) == POF_OK);
+    CHECK(stand_in::live > before);
+    stand_in::fail_launch = kernel;
+    CHECK(filtsmooth(ctx, 90) == POF_E_HIP);
+    CHECK(stand_in::fail_launch.empty());
+    CHECK(stand_in::live == before);
+    CHECK(filtsmooth(ctx, 90) == POF_OK);
+    pof_trim();
+  }
+  pof_ctx_destroy(ctx);
+  CHECK(stand_in::live == 0);
+}
+
 // The words that launches of k_upload bring to the device (its argument: {source, destination, words} per grid row)
 static size_t g_words = 0;
 static void count_words(const std::string& name, unsigned rows, void** args) {
@@ -287,6 +306,7 @@ int main(int argc, char** argv) {
   else if (what == "failed_launch") failed_launch();
   else if (what == "captured_stream") captured_stream();
   else if (what == "large_shapes") large_shapes();
+  else if (what == "failed_call") failed_call();
   else CHECK(!"a known check");
   std::printf("%s: %d failures\n", what.c_str(), failures);
   return failures == 0 ? 0 : 1;

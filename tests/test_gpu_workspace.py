@@ -97,3 +97,104 @@ def test_threads_have_a_workspace_each(gpu):
     for t in ts:
         t.join()
     assert not bad
+
+
+def _filters_and_smoothers():
+    """Calls that share workspaces of one (D, d): extended filters of other fields, parameters, priors and transition models,
+    smoothers over given filtered states, both forms, and linear models in between."""
+    import torch
+
+    import pof.convenience as pc
+    import pof.ivp
+    import pof.parallel_filtsmooth as pfs
+    import pof.sequential_filtsmooth as sfs
+    from pof.observations import AffineModel
+    from pof.transitions import TransitionModel
+    from pof.utils import MVNSqrt
+
+    def arrays(*xs):
+        torch.cuda.synchronize()
+        return [x.cpu().numpy() if hasattr(x, "cpu") else np.array(x) for x in xs]
+
+    out = []
+    for q, ivps in [(3, [pof.ivp.fitzhughnagumo(), pof.ivp.vanderpol(), pof.ivp.fhn_classic(a=0.3, b=0.1, c=2.0)]),
+                    (3, [pof.ivp.rigid_body(), pof.ivp.lorenz63(), pof.ivp.rigid_body(y0=[0.9, 0.1, 1.1])])]:
+        for k, (ivp, n) in enumerate(zip(ivps, (60, 23, 41))):
+            s = pc.set_up_solver(f=ivp.f, y0=ivp.y0, ts=np.linspace(0.0, 0.5, n + 1), order=q)
+            F, QL = np.asarray(s["dtm"].F)[0], np.asarray(s["dtm"].QL)[0]
+            D = F.shape[0]
+            d = D // (q + 1)
+            rng = np.random.default_rng(100 * D + k)
+            rot, _ = np.linalg.qr(rng.standard_normal((D, D)))
+
+            def model(QL_, F_=F, n_=n, D_=D):
+                return TransitionModel(np.broadcast_to(F_, (n_, D_, D_)), np.broadcast_to(QL_, (n_, D_, D_)))
+
+            def ekf(x0=s["x0"], dtm=s["dtm"], om=s["om"]):
+                f, nll, ssq = sfs.extended_kalman_filter(x0, dtm, om)
+                return arrays(f.mean, f.chol, nll, ssq)
+
+            x1 = MVNSqrt(np.asarray(s["x0"].mean), 0.1 * rng.standard_normal((D, D)))
+            fm = torch.as_tensor(rng.standard_normal((n + 1, D)), device="cuda")
+            fL = torch.as_tensor(rng.standard_normal((n + 1, D, D)), device="cuda")
+
+            def smooth(fn, dtm, m=fm, L=fL):
+                o, obj = fn(dtm, MVNSqrt(m, L))
+                return arrays(o.mean, o.chol, obj)
+
+            H, c = rng.standard_normal((n, d, D)), rng.standard_normal((n, d))
+
+            def linear(fs, dtm, H_=H, c_=c, x0=x1):
+                t = [torch.as_tensor(x, device="cuda") for x in (H_, c_)]
+                o, nll, obj, ssq = fs.linear_filtsmooth(x0, dtm, AffineModel(*t, None))
+                return arrays(o.mean, o.chol, nll, obj, ssq)
+
+            out += [ekf, lambda e=ekf, x=x1, m=model(QL @ rot): e(x0=x, dtm=m), lambda f=smooth, m=model(QL): f(pfs.smoothing, m),
+                    lambda f=linear, m=model(1.5 * QL): f(pfs, m), lambda f=smooth, m=model(QL @ rot): f(sfs.smoothing, m),
+                    lambda f=linear, m=model(QL @ rot): f(sfs, m)]
+    return out
+
+
+def test_filters_and_smoothers_in_turn_equal_calls_alone(gpu):
+    """As above for every call that takes a kept workspace: what one leaves in it (model, field, parameters, flags) is not
+    what the next one uses."""
+    from pof import _lib
+
+    calls = _filters_and_smoothers()
+
+    def alone(call):
+        res = []
+
+        def work():
+            for key in [k for k in _lib._ctx if k[0] == threading.get_ident()]:
+                del _lib._ctx[key]
+            res.append(call())
+
+        t = threading.Thread(target=work)
+        t.start()
+        t.join()
+        return res[0]
+
+    want = [alone(c) for c in calls]
+    order = np.random.default_rng(5).permutation(np.repeat(np.arange(len(calls)), 2))
+    for i in order:
+        print(f"call {i}", flush=True)
+        for a, b in zip(calls[i](), want[i]):
+            np.testing.assert_array_equal(a, b)
+
+
+def test_trim_gives_the_memory_back(gpu):
+    import torch
+
+    from pof import _lib
+
+    _lib.context()
+    _lib.trim()
+    free = torch.cuda.mem_get_info()[0]
+    call = _calls()[0]
+    first = _run(call)
+    assert torch.cuda.mem_get_info()[0] <= free
+    assert _lib.trim() > 0
+    assert _lib.trim() == 0
+    for a, b in zip(_run(call), first):
+        np.testing.assert_array_equal(a, b)
