@@ -404,7 +404,7 @@ struct pof_ctx {
   // scratch_err saying why its address could not be taken
   double* scratch = nullptr;
   std::string scratch_err;
-  // scan-level widths of the throughput kernel forms per state dimension (pof_tuning_set);
+  // widths from which a scan level has a launch of its own, per state dimension (pof_tuning_set);
   // tune_version counts changes, so that batches rebuild plans and graphs
   std::map<int, pof::Tuning> tuning;
   int tune_version = 0;
@@ -1238,7 +1238,7 @@ int batch_launch(pof_batch* b) {
   pof_ctx* ctx = b->ctx;
   if (b->launched) return set_err(ctx, POF_E_ARG, "pof_batch_launch called twice without pof_batch_finish");
   HIP_TRY(hipSetDevice(ctx->device));
-  if (b->tune_version != ctx->tune_version) b->plan_dirty = true;  // other kernel forms: new plan and graph
+  if (b->tune_version != ctx->tune_version) b->plan_dirty = true;  // other stages: new plan and graph
   Uploader up(b);
   if (b->plan_dirty) {
     if (settle(b) != POF_OK) return POF_E_HIP;

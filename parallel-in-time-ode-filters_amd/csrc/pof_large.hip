@@ -65,7 +65,12 @@ __device__ inline double wave_sum(double v) {
 // before it are read once per two strips; a matrix's waits are another's work.  Two iterations of 8,192 steps at
 // D = 128: 138 -> 83 ms in these kernels, and no copies put [B1 | B2] together or take the factor out (22 ms); at
 // D = 24 an LQ of 24 rows 38 -> 13 us.  Bound by the two waves' FP64 issue (a pivot: 173 instructions, of which 72
-// products) and, at D = 128, by the reflectors' traffic: 0.7 MB per matrix, 2,048 of which take 0.4 ms.
+// products) and, at D = 128, by the reflectors' traffic: 0.7 MB per matrix, 2,048 of which take 0.4 ms.  A level of one matrix
+// takes 170 to 190 us at D = 128, half of a level of 2,048: its one wave does all of it.
+//
+// Registers: two strips, the row of T and a pivot's sums do not fit 256 from five tiles on.  What the compiler keeps in scratch
+// memory then, per lane: 36 to 52 B at 5 tiles (8 to 12 registers), 304 to 312 B at 8, 348 B at 9 and 476 B at 10 (75 to
+// 132 registers).  k_lq_rows<3> and every k_lq_below keep everything in registers.
 //
 // Layout of a strip: tile t holds columns 16 t .. 16 t + 15 from the window's first on, lane j + 16 g value v holds
 // (row j, column 16 t + 4 g + v).  These registers are at once
@@ -1725,8 +1730,8 @@ void engine_destroy(Engine* e) {
 }
 
 bool supports(int kind, int D, int d) {
-  // the LQ panel kernel holds up to 256 columns (2 D) in registers and the triangular solves
-  // take orders up to 128: D <= 128
+  // the factorisations take matrices of up to 256 columns (2 D), in panels of at most 160, and the triangular solves
+  // orders up to 128: D <= 128
   return kind == kLorenz96 && d >= 4 && D % d == 0 && D / d >= 2 && D <= 128;
 }
 

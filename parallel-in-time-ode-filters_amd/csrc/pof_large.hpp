@@ -1,10 +1,10 @@
 // Large-state IEKS engine: the same solve as the per-element kernels, for state
 // dimensions whose elements do not fit one worker's registers (Lorenz-96 with
 // d = 32, q = 3: D = 128).  Every scan level runs as batched primitives over all
-// its combines: a blocked Householder LQ (panel kernel plus a one-pass trailing
-// update on the FP64 matrix cores), a strided-batched MFMA GEMM for the plain
-// products, a triangular-solve kernel, and small element-wise kernels.  The host
-// drives JAX's odd/even recursion.
+// its combines: a blocked Householder LQ (one wave per matrix, strips of 16 rows
+// in registers, block reflectors on the FP64 matrix cores), a strided-batched MFMA
+// GEMM for the plain products, a triangular-solve kernel, and small element-wise
+// kernels.  The host drives JAX's odd/even recursion.
 #pragma once
 
 #include <hip/hip_runtime.h>

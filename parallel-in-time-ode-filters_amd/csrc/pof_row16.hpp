@@ -13,8 +13,10 @@
 // LDS and every lane repeating the pivot's scalar part: about 5,300 instructions per combine became
 // about 4,300 per four (5,100 with a wait in front of every group and groups of at most eight), and at
 // D = 12 a level of 32,768 combines went from 364 to 91 us (up) and from 205 to 61 us (down), the latency
-// of one combine from 19 to 13 us and from 13 to 9.5 us.  What bounds it is FP64 issue: two waves per SIMD
-// (221 registers), 2.5 ns per instruction.
+// of one combine from 19 to 13 us and from 13 to 9.5 us.  A narrow level is bound by the instructions of one combine
+// in order (a wave issues an FP64 operation every 8.5 to 9 cycles).  A wide one has two waves per SIMD (221 registers) and
+// takes 2.5 ns per instruction, against the 1.67 ns of the FP64 peak: the counters show the vector ALUs 46 to 50 % busy
+// and 12 of 16 lanes hold a row at D = 12; what holds the two waves back from there is not known.
 //
 // Lanes r >= D of a row repeat row 0; only lanes r < D are ever the source of a broadcast or store.
 // A whole row is active or not (a worker past the end returns as a whole), so a broadcast never
@@ -334,7 +336,9 @@ struct Pivot {
 };
 
 // norm and 1 / norm of x > 0: the hardware's estimate y (about 2^-24) and one third-order step,
-// e = 1 - x y^2, (1 - e)^(-1/2) = 1 + e / 2 + 3 e^2 / 8 + O(e^3): 2^-72 before rounding.
+// e = 1 - x y^2, (1 - e)^(-1/2) = 1 + e / 2 + 3 e^2 / 8 + O(e^3): 2^-72 before rounding.  Rounded, over 4 million x from
+// 1e-290 to 1e290: the norm within 0.75 ulp (mean 0.27), its reciprocal within 0.99 (0.28).  sqrt_rsqrt, which the D > 16
+// kernels use, has 0.50 (0.25) and 1.61 (0.31): one step more for the norm, one less for the reciprocal.
 __device__ __forceinline__ void norm_rnorm(double x, double& n, double& rn) {
   const double y = __builtin_amdgcn_rsq(x);
   const double g = x * y;
@@ -344,7 +348,7 @@ __device__ __forceinline__ void norm_rnorm(double x, double& n, double& rn) {
   rn = fma(y, q, y);
 }
 
-// 1 / x for normal x: the estimate and one third-order step (1 + e + e^2)
+// 1 / x for normal x: the estimate and one third-order step (1 + e + e^2); within 0.50 ulp over the same x
 __device__ __forceinline__ double rcp3(double x) {
   const double r = __builtin_amdgcn_rcp(x);
   const double e = fma(-x, r, 1.0);
@@ -696,7 +700,8 @@ struct ObsRow<D, d, true> {
   static constexpr int NR = 0;  // noise columns
   Obs<D, d, true> o;
   double c[d];
-  // (the parameters are read where they are: a local copy indexed by the field's cases would go through scratch)
+  // (the parameters are read where they are.  The dual numbers of the field are an array that its cases index at run time: with
+  // three equations it takes 152 B of scratch per lane, with four 232 B, in every kernel that linearises.)
   __device__ __forceinline__ void load(const GroupArgs& g, int j, long long base, int k, int) {
     const double* lin = (g.cur[j] ? g.means1 : g.means0) + (size_t)base * D;
     o.load_at(g.kind[j], g.params + (size_t)j * kMaxParams, g.Pd + (size_t)j * D, lin + (size_t)(k + 1) * D);

@@ -196,7 +196,7 @@ def context(device=None):
             raise PofError(f"pof_ctx_create(device={device}) failed with status {rc}")
         c = h
         _ctx[key] = c
-        # the autotuner's cached kernel-form widths (pof/tuning_gfx950.json), if any
+        # the autotuner's cached scan-level widths (pof/tuning_gfx950.json), if any
         from . import autotune
 
         autotune.apply_cache(c)

@@ -1,13 +1,13 @@
-"""The two forms of the scan kernels give bitwise the same results.
+"""Scan levels give bitwise the same results in launches of their own and sharing launches.
 
-Each scan kernel of state dimension D <= 16 has a latency form (a matrix row
-split over 2 or 4 lanes) and a throughput form (one lane per row that
-reproduces the split form's reduction order: the same partial sums, chains and
-combination order).  Which one a scan level runs is a performance choice
-(pof_tuning_set, the autotuner's cache); results must not depend on it.  Here
-every level runs in one form, then in the other, for each (D, d) of the
-batched mix, and the outputs must be identical (torch.equal), as must the
-batch results against solves alone whatever form each level took.
+A scan level of a state dimension D <= 16 has a launch of its own (here: the
+throughput form) or shares one with the levels above it, each block carrying
+its combines through up to five (the latency form).  Which of the two a level
+takes is a performance choice (pof_tuning_set, the autotuner's cache); results
+must not depend on it.  Here every level runs in one form, then in the other,
+for each (D, d) of the batched mix, and the outputs must be identical
+(torch.equal), as must the batch results against solves alone whatever form
+each level took.
 """
 import numpy as np
 import pytest
