@@ -612,12 +612,13 @@ struct Uploader {
   }
   void maps() { add(b->maps_map, b->maps_dev, b->hmaps.size() * sizeof(int)); }
   void flush() {
-    if (n == 0 || status != hipSuccess) return;
-    const unsigned blocks = (unsigned)std::min<size_t>((most + 255) / 256, 256);
-    hipLaunchKernelGGL(k_upload, dim3(blocks, n), dim3(256), 0, b->st, a);
-    status = hipGetLastError();
-    if (status == hipSuccess) status = hipEventRecord(b->up_ev, b->st);
-    n = 0;
+    if (n > 0 && status == hipSuccess) {
+      const unsigned blocks = (unsigned)std::min<size_t>((most + 255) / 256, 256);
+      hipLaunchKernelGGL(k_upload, dim3(blocks, n), dim3(256), 0, b->st, a);
+      status = hipGetLastError();
+      if (status == hipSuccess) status = hipEventRecord(b->up_ev, b->st);
+    }
+    n = 0;  // (what follows a failed launch goes nowhere, and must not run over the table)
     most = 0;
   }
 };

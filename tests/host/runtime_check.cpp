@@ -212,6 +212,32 @@ static void failed_launch() {
   CHECK(stand_in::live == 0);
 }
 
+// More parts than one upload launch takes, the first of whose launches fails: the others go nowhere, and the retry has all
+static void failed_upload_of_many() {
+  pof_ctx* ctx = nullptr;
+  CHECK(pof_ctx_create(0, &ctx) == POF_OK);
+  constexpr int kIvps = 60;
+  pof_batch* b = nullptr;
+  CHECK(pof_batch_create(ctx, 12, 3, 4096, kIvps, &b) == POF_OK);
+  stand_in::on_launch = count_words;
+  std::vector<double> ts = grid(5), y0(3, 1.0);
+  pof_problem p = problem(POF_RIGID_BODY, 3, 3, ts, y0);
+  p.init = POF_INIT_PRIOR;  // initial means from the host: a part each
+  pof_opts o{};
+  o.maxiters = o.fixed_iters = 2;
+  std::vector<pof_out> out(kIvps);
+  for (auto& x : out) CHECK(pof_batch_admit(b, &p, &o, &x, nullptr) == POF_OK);
+  stand_in::fail_launch = "k_upload";
+  CHECK(pof_batch_launch(b) == POF_E_HIP);
+  g_words = 0;
+  CHECK(pof_batch_launch(b) == POF_OK);
+  CHECK(g_words > (size_t)kIvps * 5 * 12 * 2);
+  stand_in::on_launch = nullptr;
+  pof_batch_destroy(b);
+  pof_ctx_destroy(ctx);
+  CHECK(stand_in::live == 0);
+}
+
 // A call on a stream that its caller is capturing is refused before anything is enqueued: what it enqueued would
 // stay in the caller's graph, over memory that the refused call gives back
 static void captured_stream() {
@@ -307,6 +333,7 @@ int main(int argc, char** argv) {
   else if (what == "captured_stream") captured_stream();
   else if (what == "large_shapes") large_shapes();
   else if (what == "failed_call") failed_call();
+  else if (what == "failed_upload_of_many") failed_upload_of_many();
   else CHECK(!"a known check");
   std::printf("%s: %d failures\n", what.c_str(), failures);
   return failures == 0 ? 0 : 1;

@@ -32,8 +32,8 @@ def driver(tmp_path_factory):
     return exe
 
 
-@pytest.mark.parametrize("check", ["kept_memory", "kept_bound", "failed_call", "failed_launch", "captured_stream",
-                                   "large_shapes"])
+@pytest.mark.parametrize("check", ["kept_memory", "kept_bound", "failed_call", "failed_launch", "failed_upload_of_many",
+                                   "captured_stream", "large_shapes"])
 def test_runtime_check(driver, check):
     r = subprocess.run([str(driver), check], capture_output=True, text=True, timeout=300)
     assert r.returncode == 0, (r.stdout[-2000:], r.stderr[-4000:])
